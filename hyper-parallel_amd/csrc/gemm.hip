@@ -30,12 +30,14 @@
 #include <atomic>
 #include <type_traits>
 
+#include "gemm_skinny.h"
+#include "gemm_tile.h"
 #include "hpfp8_device.h"
 #include "hpfp8_host.h"
 
 namespace hpfp8 {
 
-constexpr int BM = 256, BN = 256, BK = 128;
+constexpr int BM = 256, BN = 256;
 constexpr int kGemmThreads = 512;
 constexpr int kTileBytes = 256 * BK;          // one operand tile in LDS (32 KB)
 // LDS: two buffers for the a tile, then kBStages buffers for the b tile.  The b operand is the one
@@ -81,38 +83,6 @@ struct GemmParams {
   float* q_scale;
   float* q_scale_inv;
 };
-
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
-
-// XOR applied to the 16-byte chunk index of tile row r.  ds_read_b128 is served 16 lanes at a time
-// and the 16 are not consecutive: per half-wave the lane quads {0,3,5,6} go together and {1,2,4,7}
-// go together (measured with SQ_LDS_BANK_CONFLICT on pairs of active lanes).  With the fragment
-// mapping lane -> (row = lane%16, k-chunk pair = lane/16) each such group holds all 16 rows once,
-// rows 4..11 with one k-chunk and the other rows with the neighbouring one; shifting the usual
-// (r/2)%8 pattern by 6 sends those two row sets to disjoint chunk ranges, so the 16 lanes hit 16
-// different bank groups.
-__device__ __forceinline__ int row_swizzle(int r) { return (((r >> 1) & 7) + 6) & 7; }
-
-__device__ __forceinline__ v4i lds_read16(const uint8_t* p) {
-  return *reinterpret_cast<const v4i*>(p);
-}
-
-__device__ __forceinline__ v8i frag_read(const uint8_t* row_base, int pc0) {
-  v4i lo = lds_read16(row_base + pc0 * 16);
-  v4i hi = lds_read16(row_base + (pc0 ^ 1) * 16);
-  v8i r;
-  r[0] = lo[0]; r[1] = lo[1]; r[2] = lo[2]; r[3] = lo[3];
-  r[4] = hi[0]; r[5] = hi[1]; r[6] = hi[2]; r[7] = hi[3];
-  return r;
-}
-
-// two floats -> two bf16 in one word (a low, b high): one v_cvt_pk_bf16_f32 (converted one by one, each
-// value costs a conversion, a shift and an or)
-__device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
-  typedef float f32x2 __attribute__((ext_vector_type(2)));
-  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
-}
 
 // Tile number -> (m tile, n tile).  Consecutive numbers (one XCD's CUs at any moment) cover
 // gm x gn rectangles of tiles (gm * gn = 32), n fastest inside a rectangle, so the L2 of that XCD
@@ -1094,6 +1064,21 @@ static bool use_small_kernel(int64_t M, int64_t N) {
   return 2 * big < cus && small > big && small < (int64_t)0x7FFFFFFF;
 }
 
+// Few rows of a (decode): bound by reading b once, which the tile kernels do not reach (gemm_skinny.hip; 8 rows of
+// [7168, 16384]: 60 us with 64 x 128 tiles, 22 us; 64 rows: 64 and 36 us; 37 rows of [36864, 7168]: 81 us with 256 x 256
+// tiles, 63 us).  Hands the problem over if it is one; otherwise false.
+static bool try_skinny(const GemmParams& p, bool tensor, int out_type, hipStream_t stream, int& rc) {
+  if (p.M > kSkinnyMaxRows || p.K < kSkinnyMinK || p.accumulate || g_small_gemm_mode.load(std::memory_order_relaxed) != 0) return false;
+  const int cus = persistent_grid((int64_t)1 << 40);
+  if ((int64_t)p.N > (int64_t)cus * (kSkinnyMaxCols - 64)) return false;
+  SkinnyParams q{};
+  q.a = p.a; q.b = p.b; q.sa = p.sa; q.sb = p.sb; q.lda = p.lda; q.ldb = p.ldb;
+  q.sa_sm = p.sa_sm; q.sa_sk = p.sa_sk; q.sb_sn = p.sb_sn; q.sb_sk = p.sb_sk;
+  q.bias = p.bias; q.c = p.c; q.ldc = p.ldc; q.M = p.M; q.N = p.N; q.K = p.K;
+  rc = launch_skinny(q, tensor, out_type == HPFP8_OUT_F32, cus, stream);
+  return true;
+}
+
 template <int MODE>
 static int launch_small(const GemmParams& p, int out_type, hipStream_t stream) {
   const int64_t tiles = (((int64_t)p.M + kSmallTile - 1) / kSmallTile) * (p.N / kSmallTile);
@@ -1202,6 +1187,7 @@ static int gemm_blockwise_impl(const void* a, int64_t lda, const float* sa, int6
   const int64_t tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
   p.tiles = (int)tiles;
   if (sb_gran == 128) {
+    if (try_skinny(p, false, out_type, (hipStream_t)stream, rc)) return rc;
     if (pow2) return launch<kScalePow2, kDense>(p, out_type, tiles, (hipStream_t)stream);
     if (!accumulate && use_small_kernel(M, N)) return launch_small<kScaleBlock>(p, out_type, (hipStream_t)stream);
     return launch<kScaleBlock, kDense>(p, out_type, tiles, (hipStream_t)stream);
@@ -1295,6 +1281,7 @@ int hpfp8_gemm_per_tensor(const void* a, int64_t lda, const float* sa_inv, const
   p.M = (int)M; p.N = (int)N; p.K = (int)K;
   const int64_t tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
   p.tiles = (int)tiles;
+  if (try_skinny(p, true, out_type, (hipStream_t)stream, rc)) return rc;
   if (use_small_kernel(M, N)) return launch_small<kScaleTensor>(p, out_type, (hipStream_t)stream);
   return launch<kScaleTensor, kDense>(p, out_type, tiles, (hipStream_t)stream);
 }

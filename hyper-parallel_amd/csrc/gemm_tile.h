@@ -1,0 +1,42 @@
+// What the FP8 GEMM kernels share: the LDS image of an operand tile (128 bytes of one k-block per row, 16-byte chunks
+// XOR-swizzled by row), fragment reads from it, bf16 packing.
+#pragma once
+#include "hpfp8_device.h"
+
+namespace hpfp8 {
+
+constexpr int BK = 128;
+
+typedef __attribute__((address_space(3))) void* lds_ptr_t;
+
+// XOR applied to the 16-byte chunk index of tile row r.  ds_read_b128 is served 16 lanes at a time
+// and the 16 are not consecutive: per half-wave the lane quads {0,3,5,6} go together and {1,2,4,7}
+// go together (measured with SQ_LDS_BANK_CONFLICT on pairs of active lanes).  With the fragment
+// mapping lane -> (row = lane%16, k-chunk pair = lane/16) each such group holds all 16 rows once,
+// rows 4..11 with one k-chunk and the other rows with the neighbouring one; shifting the usual
+// (r/2)%8 pattern by 6 sends those two row sets to disjoint chunk ranges, so the 16 lanes hit 16
+// different bank groups.
+__device__ __forceinline__ int row_swizzle(int r) { return (((r >> 1) & 7) + 6) & 7; }
+
+__device__ __forceinline__ v4i lds_read16(const uint8_t* p) {
+  return *reinterpret_cast<const v4i*>(p);
+}
+
+__device__ __forceinline__ v8i frag_read(const uint8_t* row_base, int pc0) {
+  v4i lo = lds_read16(row_base + pc0 * 16);
+  v4i hi = lds_read16(row_base + (pc0 ^ 1) * 16);
+  v8i r;
+  r[0] = lo[0]; r[1] = lo[1]; r[2] = lo[2]; r[3] = lo[3];
+  r[4] = hi[0]; r[5] = hi[1]; r[6] = hi[2]; r[7] = hi[3];
+  return r;
+}
+
+// two floats -> two bf16 in one word (a low, b high): one v_cvt_pk_bf16_f32 (converted one by one, each
+// value costs a conversion, a shift and an or)
+__device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
+}
+
+}  // namespace hpfp8
