@@ -22,6 +22,9 @@ def _flags():
         "-fno-fast-math", "-ffp-contract=off", "-fno-gpu-flush-denormals-to-zero",
         "-fhip-fp32-correctly-rounded-divide-sqrt",
         "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+        # matrix instructions write their results to vector registers also where a kernel could have more of them
+        # (4-wave GEMM kernels): through accumulation registers every promotion FMA would need a move
+        "-mllvm", "-amdgpu-mfma-vgpr-form",
         "-Wno-unused-command-line-argument",
     ]
 

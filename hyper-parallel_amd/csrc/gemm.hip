@@ -14,6 +14,9 @@
 //     are DMA'd global -> LDS with 128-bit buffer loads (out-of-range rows read as zero), 16-byte
 //     chunks XOR-swizzled by row so that both the DMA writes and the ds_read_b128 fragment reads
 //     are bank-conflict free.
+//   * Where a launch would leave compute units idle the tile is smaller: 128 x 256 or 128 x 128 with four waves (wave
+//     tiles 64 x 128 and 64 x 64), the same template (WM, NS) and the same results bit for bit; pick_shape has the rule
+//     and the figures.
 //   * The grid is persistent: one workgroup per CU walks a list of tiles, and the rounds of
 //     consecutive tiles follow each other without a gap.  Each XCD (own L2) owns a contiguous run
 //     of tile numbers.
@@ -38,8 +41,6 @@
 namespace hpfp8 {
 
 constexpr int BM = 256, BN = 256;
-constexpr int kGemmThreads = 512;
-constexpr int kTileBytes = 256 * BK;          // one operand tile in LDS (32 KB)
 // LDS: two buffers for the a tile, then kBStages buffers for the b tile.  The b operand is the one
 // that streams from HBM (each weight panel is used by one XCD only), so where LDS allows it gets a
 // third buffer and its transfers run two k-blocks ahead; a's re-reads come from the Infinity Cache.
@@ -142,20 +143,27 @@ __device__ __forceinline__ int expert_end(int off, int prev, int total_rows) {
   return lo < total_rows ? lo : total_rows;
 }
 
+// WM, NS: the tile has 64 WM rows (WM pairs of waves) and 32 NS columns (a wave: NS subtiles of 16).
 // SA4: the activation scales have unit stride over rows (the k-block-major layout), so a lane's four
 // of them are one 16-byte load.
 // EPI: 0 = c is the GEMM's result; 1 / 2 = the gate/up projection of a SwiGLU MLP with the activation and its
 // 1x128 quantization as the epilogue (1: exactly specified silu, 2: hardware exponential and reciprocal).  A tile's
 // 256 columns are then the 128 gate columns and the 128 up columns of one scaling group of the activation: the b
 // tile's upper 128 rows come from `inter` rows further down, the two waves that share 64 rows hold gate and up.
-template <int MODE, int GROUPED, bool OUT_F32, bool ACC, bool SA4, int EPI = 0>
-__global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) {
+template <int MODE, int GROUPED, bool OUT_F32, bool ACC, bool SA4, int EPI = 0, int WM = 4, int NS = 8>
+__global__ __launch_bounds__(128 * WM) void gemm_kernel(const GemmParams p) {
+  constexpr int TM = 64 * WM, TN = 32 * NS;            // the tile
+  constexpr int kWaves = 2 * WM;
+  constexpr int kATile = TM * BK, kBTile = TN * BK;    // one operand tile in LDS
+  constexpr int NB = TN / 8 / kWaves;                  // b transfers per wave and k-block (a: always 4)
+  constexpr int kSlice = kBTile / kWaves;              // a wave's part of a b buffer
+  static_assert(EPI == 0 || NS == 8, "SwiGLU epilogue: 128 gate and 128 up columns per tile");
   static_assert(EPI == 0 || ((MODE == kScaleBlock || MODE == kScalePow2) && GROUPED == kDense && !OUT_F32 && !ACC),
                 "SwiGLU epilogue: dense block-scaled forward");
   static_assert(!ACC || (OUT_F32 && MODE != kScaleTensor), "accumulating onto c: fp32 output, sums that start from c's values");
   static_assert(GROUPED != kGroupedK || (!ACC && (MODE == kScaleRow || MODE == kScalePow2Row)),
                 "grouped along the contraction: the wgrad form");
-  constexpr int kBStages = b_stages(MODE);
+  constexpr int kBStages = WM == 4 ? b_stages(MODE) : 3;
   constexpr bool kRowScales = MODE == kScaleRow || MODE == kScalePow2Row;   // per-row b scales, staged in LDS
   constexpr bool kPromote = MODE == kScaleBlock || MODE == kScaleRow;       // partial sums scaled by FMAs
   constexpr bool kHwScale = MODE == kScalePow2 || MODE == kScalePow2Row;    // scales applied by the MFMA
@@ -163,16 +171,17 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) 
   // One LDS object for everything.  (With a second __shared__ array the compiler tells the two apart
   // with alias scopes, and from then on makes every LDS read wait for all transfers into the array it
   // reads, those to other buffers included: the transfers' latency would be paid in every round.)
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[(2 + kBStages) * kTileBytes + (kRowScales ? 3 * BN * 4 : 0)];
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * kATile + kBStages * kBTile + (kRowScales ? 3 * 256 * 4 : 0)];
   // per-row scales of the b operand for one k-block (wgrad form), three stages of 256 floats: the
   // stage of k-block kb+1 is filled while slower waves may still read that of kb-1
-  float* const sb_lds = reinterpret_cast<float*>(lds + (2 + kBStages) * kTileBytes);
+  float* const sb_lds = reinterpret_cast<float*>(lds + 2 * kATile + kBStages * kBTile);
+  uint8_t* const b_lds = lds + 2 * kATile;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int K = p.K, N = p.N;
   const int kblocks = K / BK;
-  const int tiles_n = (N + BN - 1) / BN;
+  const int tiles_n = (N + TN - 1) / TN;
 
   // ---- the tile list of this workgroup.  The grid is persistent (one workgroup per CU); tiles are
   // numbered so that consecutive numbers cover rectangles of 32 tiles (rect_map), each XCD (workgroup ids
@@ -185,7 +194,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) 
     int prev = 0, mt = 0;
     for (int e = 0; e < p.experts; ++e) {
       const int end = expert_end(p.offs[e], prev, p.M);
-      mt += (end - prev + BM - 1) / BM;
+      mt += (end - prev + TM - 1) / TM;
       prev = end;
     }
     total_tiles = mt * tiles_n;
@@ -211,7 +220,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) 
     }
   }
   if (my_tiles == 0) return;
-  const int n_pad = tiles_n * BN;
+  const int n_pad = tiles_n * TN;
   // grouped: forward-only search state (tile numbers are asked for in increasing order)
   int g_e = 0, g_prev = 0, g_first = 0;
   auto lookup = [&](int k, TileInfo& ti) {
@@ -224,15 +233,15 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) 
         expert = p.layout[4 * p.experts + i];
         kb0 = p.layout[4 * expert + 2];
         kbn = p.layout[4 * expert + 3];
-        rect_map(t - i * p.tiles, (p.M + BM - 1) / BM, tiles_n, tm, tn);
-        row0 = tm * BM;
-        row_end = row0 + BM < p.M ? row0 + BM : p.M;
-        n0 = tn * BN;
+        rect_map(t - i * p.tiles, (p.M + TM - 1) / TM, tiles_n, tm, tn);
+        row0 = tm * TM;
+        row_end = row0 + TM < p.M ? row0 + TM : p.M;
+        n0 = tn * TN;
       } else if (GROUPED == kGroupedRows) {
         int end = 0, cnt = 0;
         while (g_e < p.experts) {
           end = expert_end(p.offs[g_e], g_prev, p.M);
-          cnt = (end - g_prev + BM - 1) / BM;
+          cnt = (end - g_prev + TM - 1) / TM;
           if (t < g_first + cnt * tiles_n) break;
           g_first += cnt * tiles_n;
           g_prev = end;
@@ -241,16 +250,16 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) 
         if (g_e < p.experts) {
           rect_map(t - g_first, cnt, tiles_n, tm, tn);
           expert = g_e;
-          row0 = g_prev + tm * BM;
+          row0 = g_prev + tm * TM;
           row_end = end < p.M ? end : p.M;
-          if (row0 + BM < row_end) row_end = row0 + BM;
-          n0 = tn * BN;
+          if (row0 + TM < row_end) row_end = row0 + TM;
+          n0 = tn * TN;
         }
       } else {
-        rect_map(t, (p.M + BM - 1) / BM, tiles_n, tm, tn);
-        row0 = tm * BM;
-        row_end = row0 + BM < p.M ? row0 + BM : p.M;
-        n0 = tn * BN;
+        rect_map(t, (p.M + TM - 1) / TM, tiles_n, tm, tn);
+        row0 = tm * TM;
+        row_end = row0 + TM < p.M ? row0 + TM : p.M;
+        n0 = tn * TN;
       }
     }
     // (values found through the expert search sit in vector registers; as scalars they keep the
@@ -291,7 +300,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) 
     const uint8_t* base = p.b + (GROUPED == kGroupedRows ? (int64_t)ti.expert * p.b_se : 0) + (int64_t)(rows ? brow0 : 0) * p.ldb;
     return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, span_bytes(rows, p.ldb), 0x00020000);
   };
-  uint32_t a_off[4], b_off[4];
+  uint32_t a_off[4], b_off[NB];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int q = wave * 4 + i;                       // 8-row group inside the tile
@@ -303,6 +312,11 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) 
     // rows of c.  (The b tile keeps its order.)
     const int ra = (r & ~63) + (r & 15) * 4 + ((r >> 4) & 3);
     a_off[i] = (uint32_t)ra * (uint32_t)p.lda + chunk * 16;
+  }
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    const int r = (wave * NB + i) * 8 + (lane >> 3);
+    const int chunk = (lane & 7) ^ row_swizzle(r);
     b_off[i] = (uint32_t)(EPI && r >= 128 ? r - 128 + p.inter : r) * (uint32_t)p.ldb + chunk * 16;
   }
   // wgrad form: the 256 per-row scales of the b tile for one k-block are one more 1 KB transfer
@@ -311,23 +325,28 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) 
       (void*)p.sb, 0, kRowScales ? (int)((((int64_t)kblocks - 1) * p.sb_sk + N) * 4) : 0, 0x00020000);
   auto issue_sb_load = [&](const TileInfo& ti, int kb, int stage) {      // kb counted inside the tile's own contraction
     if (kRowScales && wave == 0)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_sb, (lds_ptr_t)(sb_lds + stage * BN), 16,
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_sb, (lds_ptr_t)(sb_lds + stage * 256), 16,
                                                (uint32_t)(ti.n0 + lane * 4) * 4u,
                                                (int)(((GROUPED == kGroupedK ? ti.kb0 : 0) + kb) * p.sb_sk * 4), 0, 0);
   };
-  // One transfer = 8 rows x 128 B per wave; `sub` (0..3) selects which of the wave's four 8-row groups
-  // of the 256-row tile.  The four transfers of one operand tile share one LDS base (M0) and differ
-  // in the instruction's immediate offset, which the hardware adds to both the LDS and the memory
-  // address; the memory side is compensated in the lane offset.
-  auto issue_tile = [&](const __amdgpu_buffer_rsrc_t& rs, const uint32_t (&off)[4], int buf, int kb, int sub) {
-    uint8_t* sbase = lds + wave * 4096 + buf * kTileBytes;
-    const uint32_t voff = off[sub] - sub * 1024;
-    switch (sub) {   // the immediate must be a literal; sub is a compile-time constant after unrolling
+  // One transfer = 8 rows x 128 B per wave; `sub` selects which of the wave's 8-row groups of the tile.
+  // Four transfers share one LDS base (M0) and differ in the instruction's immediate offset, which the
+  // hardware adds to both the LDS and the memory address; the memory side is compensated in the lane offset.
+  auto transfer = [&](const __amdgpu_buffer_rsrc_t& rs, uint32_t off, uint8_t* base, int kb, int sub) {
+    uint8_t* sbase = base + (sub >> 2) * 4096;
+    const uint32_t voff = off - (sub & 3) * 1024;
+    switch (sub & 3) {   // the immediate must be a literal; sub is a compile-time constant after unrolling
       case 0: __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)sbase, 16, voff, kb * BK, 0, 0); break;
       case 1: __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)sbase, 16, voff, kb * BK, 1024, 0); break;
       case 2: __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)sbase, 16, voff, kb * BK, 2048, 0); break;
       default: __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)sbase, 16, voff, kb * BK, 3072, 0); break;
     }
+  };
+  auto issue_a = [&](const __amdgpu_buffer_rsrc_t& rs, int buf, int kb, int sub) {
+    transfer(rs, a_off[sub], lds + buf * kATile + wave * 4096, kb, sub);
+  };
+  auto issue_b = [&](const __amdgpu_buffer_rsrc_t& rs, int buf, int kb, int sub) {
+    transfer(rs, b_off[sub], b_lds + buf * kBTile + wave * kSlice, kb, sub);
   };
 
   // ---- fragment addressing
@@ -335,7 +354,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) 
   const int l16 = lane & 15, g = lane >> 4;
   const int pc0 = (2 * g) ^ row_swizzle(l16);
   const int a_frag_off = (wm * 64 + l16) * BK;               // + j * 16 rows
-  const int b_frag_off = (wn * 128 + l16) * BK;               // + i * 16 rows, inside a b buffer
+  const int b_frag_off = (wn * (TN / 2) + l16) * BK;               // + i * 16 rows, inside a b buffer
 
   // ---- scales.  Raw values for one k-block are loaded at the top of the round before it and only
   // combined (sa * sb) at its end, so nothing waits on global memory in between.
@@ -356,7 +375,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) 
       // (SA4 does not clamp: words past the end of the array read as zero, and rows past M are never stored)
       sa_voff[j] = SA4 ? (uint32_t)r * 4u : (uint32_t)(r < p.M ? r : p.M - 1) * (uint32_t)((int)p.sa_sm * 4);
     }
-    int nblk_idx = EPI ? (ti.n0 >> 8) + wn * (p.inter >> 7) : (ti.n0 + wn * 128) >> 7;
+    int nblk_idx = EPI ? (ti.n0 >> 8) + wn * (p.inter >> 7) : (ti.n0 + wn * (TN / 2)) >> 7;
     if (nblk_idx > (N >> 7) - 1) nblk_idx = (N >> 7) - 1;
     sb_soff = ((GROUPED == kGroupedRows ? ti.expert * (int)p.sb_se : 0) + nblk_idx * (int)p.sb_sn) * 4;
   };
@@ -395,7 +414,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) 
   // load.  The resource ends with the tensor: rows past it (and the tiles past the end of the list)
   // read as zero.
   auto rsrc_c_of = [&](const TileInfo& ti) {
-    const int ncol = ti.n0 + wn * 128;
+    const int ncol = ti.n0 + wn * (TN / 2);
     const bool ok = ti.row_end > ti.row0 && ncol < N;
     int64_t bytes = ok ? (((int64_t)p.M - ti.row0 - 1) * p.ldc + N - ncol) * 4 : 0;
     if (bytes > (int64_t)0x7FFFF000) bytes = 0x7FFFF000;       // 256 rows always fit (host check)
@@ -407,19 +426,19 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) 
     return __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rs, lane_off + i * 64, j * c_jstep, 0));
   };
   const v4f zero = {0.f, 0.f, 0.f, 0.f};
-  v4f acc[8][4];
+  v4f acc[NS][4];
   auto load_old_values = [&](const TileInfo& ti) {
     int lane_c = lane;
     asm volatile("" : "+v"(lane_c));    // (keeps the lane offset out of the registers held through the rounds)
     const __amdgpu_buffer_rsrc_t rc = rsrc_c_of(ti);
     const uint32_t c_lane = ((uint32_t)(wm * 64 + (lane_c & 15) * 4) * (uint32_t)p.ldc + (lane_c >> 4) * 4) * 4u;
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < NS; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) acc[i][j] = old_values(rc, c_lane, i, j);
   };
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < NS; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = zero;
 
@@ -436,27 +455,27 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) 
   {
     const __amdgpu_buffer_rsrc_t ra = rsrc_a_of(T0), rb = rsrc_b_of(T0);
 #pragma unroll
-    for (int sub = 0; sub < 4; ++sub) issue_tile(ra, a_off, 0, kfirst(T0), sub);
+    for (int sub = 0; sub < 4; ++sub) issue_a(ra, 0, kfirst(T0), sub);
 #pragma unroll
-    for (int sub = 0; sub < 4; ++sub) issue_tile(rb, b_off, 2, kfirst(T0), sub);
+    for (int sub = 0; sub < NB; ++sub) issue_b(rb, 0, kfirst(T0), sub);
     int kb1;
     const TileInfo t1 = pick_tile(tiles_ahead(0, 1, kcount(T0), kcount(T1), kb1), T0, T1, T2);
     kb1 += kfirst(t1);
     if (kBAhead == 2) {
       const __amdgpu_buffer_rsrc_t rb1 = rsrc_b_of(t1);
 #pragma unroll
-      for (int sub = 0; sub < 4; ++sub) issue_tile(rb1, b_off, 3, kb1, sub);
+      for (int sub = 0; sub < NB; ++sub) issue_b(rb1, 1, kb1, sub);
     }
     issue_sb_load(T0, 0, 0);
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
     __syncthreads();
     const __amdgpu_buffer_rsrc_t ra1 = rsrc_a_of(t1);
-    issue_tile(ra1, a_off, 1, kb1, 0);
-    issue_tile(ra1, a_off, 1, kb1, 1);
+    issue_a(ra1, 1, kb1, 0);
+    issue_a(ra1, 1, kb1, 1);
     if (kBAhead == 1) {
       const __amdgpu_buffer_rsrc_t rb1 = rsrc_b_of(t1);
-      issue_tile(rb1, b_off, 3, kb1, 0);
-      issue_tile(rb1, b_off, 3, kb1, 1);
+      issue_b(rb1, 1, kb1, 0);
+      issue_b(rb1, 1, kb1, 1);
     }
   }
 
@@ -468,10 +487,10 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) 
   // Rounds follow each other without a gap across tiles: the last rounds of a tile already fetch
   // the first k-blocks of the next one, and its stores drain while the next tile computes.
   v8i xf[4], wf_n0, wf_n1;
-  wf_n0 = frag_read(lds + 2 * kTileBytes + b_frag_off, pc0);
+  wf_n0 = frag_read(b_lds + b_frag_off, pc0);
 #pragma unroll
   for (int j = 0; j < 4; ++j) xf[j] = frag_read(lds + a_frag_off + j * 16 * BK, pc0);
-  wf_n1 = frag_read(lds + 2 * kTileBytes + b_frag_off + 16 * BK, pc0);
+  wf_n1 = frag_read(b_lds + b_frag_off + 16 * BK, pc0);
 
   constexpr bool kCarry = MODE == kScaleBlock;   // promote subtile 7 inside the next round's first group
   v4f part_c[4] = {zero, zero, zero, zero};
@@ -522,44 +541,59 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) 
     kb1 += kfirst(tile_1);
     kb2 += kofs_2;
     load_scales(kb1, s_raw);
-    const uint8_t* bcur = lds + (2 + bbuf) * kTileBytes;
+    const uint8_t* bcur = b_lds + bbuf * kBTile;
     int bnext = bbuf + 1 == kBStages ? 0 : bbuf + 1;           // holds the next k-block
     int bbuf_issue = bbuf + kBAhead;                           // receives the k-block kBAhead ahead
     if (bbuf_issue >= kBStages) bbuf_issue -= kBStages;
-    const uint8_t* bnxt = lds + (2 + bnext) * kTileBytes;
-    const uint8_t* anxt = lds + (stage ^ 1) * kTileBytes;
+    const uint8_t* bnxt = b_lds + bnext * kBTile;
+    const uint8_t* anxt = lds + (stage ^ 1) * kATile;
     int snext = sbuf + 1 == 3 ? 0 : sbuf + 1;
     // Per round, with three b buffers: the rest of the next a tile at subtiles 0,1; the b tile two
-    // rounds ahead at 2..5; after the barrier the first half of the a tile after next, into the
+    // rounds ahead at 2..5 (with four subtiles in all: 0 and 1); after the barrier the first half of the a tile after next, into the
     // buffer whose fragments every wave has just left behind.  One transfer per subtile: a burst
     // would queue up in the texture path ahead of the LDS reads.
     // With two b buffers (wgrad form) the b tile has to land within one round like the a tile, so
     // both go out in the four subtiles that follow the barrier, one transfer of each per subtile.
     auto issue_slot = [&](int i) {
-      if (kBAhead == 2) {
-        if (i < 2) issue_tile(rs_a1, a_off, stage ^ 1, kb1, i + 2);
-        else if (i < 6) issue_tile(rs_b2, b_off, 2 + bbuf_issue, kb2, i - 2);
-        else issue_tile(rs_a2, a_off, stage, kb2, i - 6);
+      if (kBAhead == 2 && NS == 8) {
+        if (i < 2) {
+          issue_a(rs_a1, stage ^ 1, kb1, i + 2);
+        } else if (i < 6) {
+#pragma unroll
+          for (int t = 0; t < NB / 4; ++t) issue_b(rs_b2, bbuf_issue, kb2, (i - 2) * (NB / 4) + t);
+        } else {
+          issue_a(rs_a2, stage, kb2, i - 6);
+        }
+      } else if (kBAhead == 2) {               // (four n-subtiles)
+        if (i == 0) {
+          issue_a(rs_a1, stage ^ 1, kb1, 2);
+          issue_a(rs_a1, stage ^ 1, kb1, 3);
+        } else if (i == 1) {
+#pragma unroll
+          for (int t = 0; t < NB; ++t) issue_b(rs_b2, bbuf_issue, kb2, t);
+        } else {
+          issue_a(rs_a2, stage, kb2, i - 2);
+        }
       } else if (i < 2) {
-        issue_tile(rs_a1, a_off, stage ^ 1, kb1, i + 2);
-        issue_tile(rs_b1, b_off, 2 + bnext, kb1, i + 2);
+        issue_a(rs_a1, stage ^ 1, kb1, i + 2);
+        issue_b(rs_b1, bnext, kb1, i + 2);
       } else if (i >= 6) {
-        issue_tile(rs_a2, a_off, stage, kb2, i - 6);
-        issue_tile(rs_b2, b_off, 2 + bbuf, kb2, i - 6);
+        issue_a(rs_a2, stage, kb2, i - 6);
+        issue_b(rs_b2, bbuf, kb2, i - 6);
       }
     };
     auto round_sync = [&]() {
       // Own transfers for the next round have landed and own LDS reads of this round's buffers are
-      // done; then everyone's.  With three b buffers the four b transfers of this round (the
+      // done; then everyone's.  With three b buffers the NB b transfers of this round (the
       // youngest vector-memory operations) are for the round after next and may stay in flight.
-      if (kBAhead == 2) __builtin_amdgcn_s_waitcnt(0x0074);  // vmcnt(4) lgkmcnt(0)
+      if (kBAhead == 2) __builtin_amdgcn_s_waitcnt(0x0070 | NB);  // vmcnt(NB) lgkmcnt(0)
       else __builtin_amdgcn_s_waitcnt(0x0070);               // vmcnt(0) lgkmcnt(0)
       __builtin_amdgcn_s_barrier();
     };
     // weight fragment of subtile i + 2 (the first two of the next round once past the barrier)
     auto read_ahead = [&](int i) {
-      return i + 2 < 8 ? frag_read(bcur + b_frag_off + (i + 2) * 16 * BK, pc0)
-                       : frag_read(bnxt + b_frag_off + (i + 2 - 8) * 16 * BK, pc0);
+      return i + 2 < NS ? frag_read(bcur + b_frag_off + (i + 2) * 16 * BK, pc0)
+                       : frag_read(bnxt + b_frag_off + (i + 2 - NS) * 16 * BK, pc0);
     };
     if (kPromote) {
       // Software pipeline over the 8 n-subtiles: the matrix instructions of subtile i are issued
@@ -572,14 +606,14 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) 
 #pragma unroll
       for (int j = 0; j < 4; ++j) part[1][j] = part_c[j];
       // wgrad form: the four per-row b scales of subtile i for this lane's four n
-      const float* sb_row = sb_lds + sbuf * BN + wn * 128 + g * 4;
+      const float* sb_row = sb_lds + sbuf * 256 + wn * (TN / 2) + g * 4;
       v4f sbv[2];
       if (MODE == kScaleRow) sbv[0] = *reinterpret_cast<const v4f*>(sb_row);
       if (MODE == kScaleRow) issue_sb_load(tile_1, kb1_rel, snext);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        if (i == 6) round_sync();
+      for (int i = 0; i < NS; ++i) {
+        if (i == NS - 2) round_sync();
         wf[(i + 2) % 3] = read_ahead(i);
         if (MODE == kScaleRow && i > 0) sbv[i & 1] = *reinterpret_cast<const v4f*>(sb_row + i * 16);   // used by the FMAs of group i+1
         issue_slot(i);
@@ -588,7 +622,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) 
         for (int j = 0; j < 4; ++j) {
           part[i & 1][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[i % 3], xf[j], zero, 0, 0, 0, 0, 0, 0);
           if (i > 0 || kCarry) {
-            const int ip = (i + 7) & 7;     // subtile being promoted; for i = 0 the last one of the previous round
+            const int ip = (i + NS - 1) % NS;     // subtile being promoted; for i = 0 the last one of the previous round
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
               float pv = part[(i - 1) & 1][j][r];
@@ -596,7 +630,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) 
               acc[ip][j][r] = __builtin_fmaf(pv, i == 0 ? s_old[j] : s_cur[j], acc[ip][j][r]);
             }
           }
-          if (i == 7) xf[j] = frag_read(anxt + a_frag_off + j * 16 * BK, pc0);
+          if (i == NS - 1) xf[j] = frag_read(anxt + a_frag_off + j * 16 * BK, pc0);
           __builtin_amdgcn_sched_barrier(0);   // keep this (MFMA, FMAs) group together, in this order
         }
       }
@@ -610,25 +644,25 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) 
           for (int r = 0; r < 4; ++r) {
             float pv = part[1][j][r];
             if (MODE == kScaleRow) pv *= sbv[1][r];
-            acc[7][j][r] = __builtin_fmaf(pv, s_cur[j], acc[7][j][r]);
+            acc[NS - 1][j][r] = __builtin_fmaf(pv, s_cur[j], acc[NS - 1][j][r]);
           }
       }
-      wf_n0 = wf[8 % 3];
-      wf_n1 = wf[9 % 3];
+      wf_n0 = wf[NS % 3];
+      wf_n1 = wf[(NS + 1) % 3];
     } else {
       v8i wf[3];
       wf[0] = wf_n0;
       wf[1] = wf_n1;
       // per-row b scales: this lane's row of subtile i is row i * 16 + l16 of the wave's 128
-      const float* sb_lane = sb_lds + sbuf * BN + wn * 128 + l16;
+      const float* sb_lane = sb_lds + sbuf * 256 + wn * (TN / 2) + l16;
       int e_bi[2] = {127, 127};
       if (MODE == kScalePow2Row) e_bi[0] = (int)(__builtin_bit_cast(uint32_t, sb_lane[0]) >> 23);
       if (MODE == kScalePow2Row) issue_sb_load(tile_1, kb1_rel, snext);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        if (i == 6) round_sync();
+      for (int i = 0; i < NS; ++i) {
+        if (i == NS - 2) round_sync();
         wf[(i + 2) % 3] = read_ahead(i);
-        if (MODE == kScalePow2Row && i < 7) e_bi[(i + 1) & 1] = (int)(__builtin_bit_cast(uint32_t, sb_lane[(i + 1) * 16]) >> 23);
+        if (MODE == kScalePow2Row && i < NS - 1) e_bi[(i + 1) & 1] = (int)(__builtin_bit_cast(uint32_t, sb_lane[(i + 1) * 16]) >> 23);
         issue_slot(i);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -640,12 +674,12 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) 
                                                                         MODE == kScalePow2 ? e_b : e_bi[i & 1], 0, e_a[j]);
           else
             acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[i % 3], xf[j], acc[i][j], 0, 0, 0, 0, 0, 0);
-          if (i == 7) xf[j] = frag_read(anxt + a_frag_off + j * 16 * BK, pc0);
+          if (i == NS - 1) xf[j] = frag_read(anxt + a_frag_off + j * 16 * BK, pc0);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
-      wf_n0 = wf[8 % 3];
-      wf_n1 = wf[9 % 3];
+      wf_n0 = wf[NS % 3];
+      wf_n1 = wf[(NS + 1) % 3];
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -660,7 +694,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) 
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) acc[7][j][r] = __builtin_fmaf(part_c[j][r], s_old[j], acc[7][j][r]);
+      for (int r = 0; r < 4; ++r) acc[NS - 1][j][r] = __builtin_fmaf(part_c[j][r], s_old[j], acc[NS - 1][j][r]);
 #pragma unroll
     for (int j = 0; j < 4; ++j) part_c[j] = zero;
   }
@@ -676,27 +710,27 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) 
   int lane_e = lane;
   asm volatile("" : "+v"(lane_e));
   const int l16e = lane_e & 15, ge = lane_e >> 4;
-  uint8_t* stg = lds + (2 + (bbuf == 0 ? kBStages - 1 : bbuf - 1)) * kTileBytes + wave * 4096;
+  uint8_t* stg = b_lds + (bbuf == 0 ? kBStages - 1 : bbuf - 1) * kBTile + wave * kSlice;
   // With two b buffers the lower half of that slice already receives the next transfers: rows 0..7
   // then go to its upper half and rows 8..15 to the upper half of this wave's slice of the a buffer
   // that is being refilled (its upper half is filled after these stores).
-  uint8_t* stg_hi = kBAhead == 1 ? lds + (stage ^ 1) * kTileBytes + wave * 4096 + 2048 : stg + 2048;
+  uint8_t* stg_hi = kBAhead == 1 ? lds + (stage ^ 1) * kATile + wave * 4096 + 2048 : stg + 2048;
   if (kBAhead == 1) stg += 2048;
   auto stg_row = [&](int row) { return (row < 8 ? stg : stg_hi) + (row & 7) * 256; };   // (row = l16e: the write side)
-  const int ncol = n0 + wn * 128;                 // first column of the wave tile
+  const int ncol = n0 + wn * (TN / 2);                 // first column of the wave tile
   const bool cols_ok = ncol < N;
-  constexpr int kHalves = OUT_F32 ? 2 : 1;       // fp32 rows of 128 columns take two slices
-  constexpr int kPerHalf = 8 / kHalves;           // n-subtiles per slice
+  constexpr int kHalves = OUT_F32 && NS == 8 ? 2 : 1;       // fp32 rows of 128 columns take two slices
+  constexpr int kPerHalf = NS / kHalves;           // n-subtiles per slice
   const uint32_t stg_w = (uint32_t)(uintptr_t)(lds_ptr_t)stg_row(l16e);   // LDS byte address of this lane's row
   // Rows leave through a buffer resource that starts at the wave tile's first element and ends with the
   // tile's last valid row: the lane part of a store address is one offset computed once per tile, the
   // rest scalar, and rows past the end of a ragged tile (or of an expert) are dropped by the range check.
   constexpr int kEsize = OUT_F32 ? 4 : 2;
-  const int rows_valid = row_end - row0 < BM ? row_end - row0 : BM;
+  const int rows_valid = row_end - row0 < TM ? row_end - row0 : TM;
   const __amdgpu_buffer_rsrc_t rsrc_st = __builtin_amdgcn_make_buffer_rsrc(
       (void*)(reinterpret_cast<uint8_t*>(p.c) +
               ((int64_t)row0 * p.ldc + ncol + (GROUPED == kGroupedK ? (int64_t)T0.expert * p.c_se : 0)) * kEsize), 0,
-      cols_ok && rows_valid > 0 ? (int)((((int64_t)rows_valid - 1) * p.ldc + 128) * kEsize) : 0, 0x00020000);
+      cols_ok && rows_valid > 0 ? (int)((((int64_t)rows_valid - 1) * p.ldc + TN / 2) * kEsize) : 0, 0x00020000);
   const uint32_t st_lane = (uint32_t)(((wm * 64 + ge * 4) * (int)p.ldc) * kEsize + l16e * 16);
   const int st_row = (int)p.ldc * kEsize;        // bytes from one row of c to the next
   auto store_tile = [&](auto with_bias) {
@@ -746,7 +780,9 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) 
             // staging row s of pass j is tile row 4 s + j (s = 4 (k2 + k) + ge: the ge part is in st_lane).
             // Streaming stores: the output is not read again here, and as ordinary stores a tile's
             // 128-256 KB would push operand panels out of the L2.
-            __builtin_amdgcn_raw_buffer_store_b128(val[k], rsrc_st, st_lane, (16 * (k2 + k) + j) * st_row + h * 256, 2);
+            // (64 columns of bf16 are 128 bytes: half of the lanes hold a row)
+            if (OUT_F32 || NS == 8 || l16e < 8)
+              __builtin_amdgcn_raw_buffer_store_b128(val[k], rsrc_st, st_lane, (16 * (k2 + k) + j) * st_row + h * 256, 2);
           }
           // A 128-bit store reads its data registers over several cycles after it has issued, and a vector instruction
           // right behind it must not write them yet.  The compiler inserts the wait states for that only where the
@@ -766,8 +802,8 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) 
     // the activation exactly as the stand-alone kernel does on a bf16 gate/up tensor.  A second barrier keeps the
     // next pass's writes (and, after the last pass, the next tile's transfers) off slices still being read.
     static_assert(kBStages == 3, "staging rows 0..15 of a wave are contiguous");
-    const uint8_t* gate_s = stg - wave * 4096 + (wave & ~1) * 4096;
-    const uint8_t* up_s = gate_s + 4096;
+    const uint8_t* gate_s = stg - (wave & 1) * kSlice;
+    const uint8_t* up_s = gate_s + kSlice;
     const uint32_t stg_we = (uint32_t)(uintptr_t)(lds_ptr_t)(stg + l16e * 256);   // this lane's staging row
     const int gcol = n0 >> 1;                        // first activation column of the tile's scaling group
     const __amdgpu_buffer_rsrc_t rsrc_q = __builtin_amdgcn_make_buffer_rsrc(
@@ -782,7 +818,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) 
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
 #pragma unroll
-      for (int ii = 0; ii < 8; ++ii) {
+      for (int ii = 0; ii < NS; ++ii) {
         u32x2 o;
         o[0] = pack_bf16x2(acc[ii][j][0], acc[ii][j][1]);
         o[1] = pack_bf16x2(acc[ii][j][2], acc[ii][j][3]);
@@ -823,7 +859,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) 
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int i = 0; i < 8; ++i) acc[i][j] = zero;
+      for (int i = 0; i < NS; ++i) acc[i][j] = zero;
   }
   T0 = T1;
   T1 = T2;
@@ -836,24 +872,22 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmParams p) 
 }
 
 // ---------------------------------------------------------------------------------------------
-// small problems: fewer 256 x 256 tiles than compute units
+// small problems: at most one 64 x 128 tile per compute unit
 // ---------------------------------------------------------------------------------------------
-// One 128 x 128 output tile per workgroup of 4 waves (2 x 2, wave tile 64 x 64), no persistence: four times as
-// many workgroups as the kernel above has tiles, each with a quarter of the matrix work per k-block.  Same
-// operand layout in LDS (global -> LDS transfers, swizzle, fragment reads), five stages of one a tile and one b
-// tile (16 KB each), transfers four k-blocks ahead, one barrier per k-block.  Same arithmetic in the same order as
-// the kernel above (one matrix instruction per 16 x 16 subtile and k-block; block form: acc += partial * (sa * sb)),
-// so the two give identical results.  Per-tensor and 128x128-block scale forms, dense, bf16 or fp32 output, bias.
+// One 64 x 128 output tile per workgroup of 4 waves (2 x 2, wave tile 32 x 64), no persistence.  Same operand layout
+// in LDS as above (global -> LDS transfers, swizzle, fragment reads), five stages of one a tile and one b tile (24 KB),
+// transfers four k-blocks ahead, one barrier per k-block.  Same arithmetic in the same order as the kernel above (one
+// matrix instruction per 16 x 16 subtile and k-block; block form: acc += partial * (sa * sb)), so the two give identical
+// results.  Per-tensor and 128x128-block scale forms, dense, bf16 or fp32 output, bias.
 constexpr int kSmallThreads = 256;
-constexpr int kSmallTile = 128;
+constexpr int kSmallTile = 128;      // columns
+constexpr int kSmallRows = 64;
 constexpr int kSmallStages = 5;
 
-// TM: rows of the tile, 128 or 64.  With 64 (wave tile 32 x 64) a problem has twice as many workgroups: the form for
-// problems whose 128 x 128 tiles would leave compute units idle (cfg 1: 128 tiles on 256 compute units).
-template <int MODE, bool OUT_F32, int TM = 128>
+template <int MODE, bool OUT_F32>
 __global__ __launch_bounds__(kSmallThreads) void gemm_small_kernel(const GemmParams p) {
   static_assert(MODE == kScaleTensor || MODE == kScaleBlock, "per-tensor or block scales");
-  static_assert(TM == 128 || TM == 64, "tile rows");
+  constexpr int TM = kSmallRows;
   constexpr int kStageBytes = (TM + kSmallTile) * BK;     // a tile + b tile
   constexpr int NA = TM / 32;                             // a transfers per wave and k-block; also m-subtiles per wave
   __shared__ __attribute__((aligned(1024))) uint8_t lds[kSmallStages * kStageBytes];
@@ -879,15 +913,18 @@ __global__ __launch_bounds__(kSmallThreads) void gemm_small_kernel(const GemmPar
   const __amdgpu_buffer_rsrc_t rs_b = __builtin_amdgcn_make_buffer_rsrc((void*)(p.b + (int64_t)n0 * p.ldb), 0,
                                                                       span(p.N - n0, p.ldb), 0x00020000);
   const __amdgpu_buffer_rsrc_t rs_none = __builtin_amdgcn_make_buffer_rsrc((void*)p.a, 0, 0, 0x00020000);
-  uint32_t a_off[4], b_off[4];
+  uint32_t a_off[NA], b_off[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int r = (wave * 4 + i) * 8 + (lane >> 3);
     const int chunk = (lane & 7) ^ row_swizzle(r);
     b_off[i] = (uint32_t)r * (uint32_t)p.ldb + chunk * 16 - i * 1024;
-    const int ra = (wave * NA + (i < NA ? i : 0)) * 8 + (lane >> 3);
-    const int chunk_a = (lane & 7) ^ row_swizzle(ra);
-    a_off[i] = (uint32_t)ra * (uint32_t)p.lda + chunk_a * 16 - (i < NA ? i : 0) * 1024;
+  }
+#pragma unroll
+  for (int i = 0; i < NA; ++i) {
+    const int r = (wave * NA + i) * 8 + (lane >> 3);
+    const int chunk = (lane & 7) ^ row_swizzle(r);
+    a_off[i] = (uint32_t)r * (uint32_t)p.lda + chunk * 16 - i * 1024;
   }
   auto issue_stage = [&](int kb, int stage) {
     const bool ok = kb < kblocks;
@@ -896,10 +933,6 @@ __global__ __launch_bounds__(kSmallThreads) void gemm_small_kernel(const GemmPar
     uint8_t* sb_base = lds + stage * kStageBytes + TM * BK + wave * 4096;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)sa_base, 16, a_off[0], kb * BK, 0, 0);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)sa_base, 16, a_off[1], kb * BK, 1024, 0);
-    if (NA == 4) {
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)sa_base, 16, a_off[2], kb * BK, 2048, 0);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)sa_base, 16, a_off[3], kb * BK, 3072, 0);
-    }
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)sb_base, 16, b_off[0], kb * BK, 0, 0);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)sb_base, 16, b_off[1], kb * BK, 1024, 0);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)sb_base, 16, b_off[2], kb * BK, 2048, 0);
@@ -955,9 +988,7 @@ __global__ __launch_bounds__(kSmallThreads) void gemm_small_kernel(const GemmPar
     // stage that is refilled next
     // (in flight and allowed to stay so: the transfers of three k-blocks, NA + 4 each, and in the block form the scale
     // loads of two, NA + 1 each)
-    if (MODE == kScaleBlock && NA == 4) asm volatile("s_waitcnt vmcnt(34)\n\ts_barrier" ::: "memory");
-    else if (MODE == kScaleBlock) asm volatile("s_waitcnt vmcnt(24)\n\ts_barrier" ::: "memory");
-    else if (NA == 4) asm volatile("s_waitcnt vmcnt(24)\n\ts_barrier" ::: "memory");
+    if (MODE == kScaleBlock) asm volatile("s_waitcnt vmcnt(24)\n\ts_barrier" ::: "memory");
     else asm volatile("s_waitcnt vmcnt(18)\n\ts_barrier" ::: "memory");
     load_scales(kb + 3, s_ring[(Q + 3) & 3]);
     asm volatile("" ::: "memory");       // (keeps the scale loads ahead of the transfers, as the wait above counts them)
@@ -1035,8 +1066,8 @@ __global__ __launch_bounds__(kSmallThreads) void gemm_small_kernel(const GemmPar
   }
 }
 
-// 0: the small-tile kernel serves problems with fewer 256 x 256 tiles than half the compute units (and more
-// 128 x 128 tiles than that); 1: never; 2: whenever its forms allow (test hook)
+// Test hook.  0: pick_shape and use_small_kernel choose the tile; 1: always 256 x 256; 2: 64 x 128 where 128 x 128 tiles
+// would be fewer than the compute units and 128 x 128 otherwise, whenever the form allows it
 static std::atomic<int> g_small_gemm_mode{0};   // (atomic: the test hook may be called from any thread)
 
 // Workgroups to launch for `tiles` tiles: one per CU, a multiple of 8 (one share per XCD) unless
@@ -1054,14 +1085,61 @@ static int persistent_grid(int64_t tiles) {
   return (int)g;
 }
 
+// The tile of a GEMM: 256 x 256 (8 waves), 128 x 256 or 128 x 128 (4 waves); a wave's part has 64 rows in each.
+enum TileShape { k256x256, k128x256, k128x128 };
+
+static int64_t tile_count(int64_t M, int64_t N, TileShape shape) {
+  const int tm = shape == k256x256 ? 256 : 128, tn = shape == k128x128 ? 128 : 256;
+  return ((M + tm - 1) / tm) * ((N + tn - 1) / tn);
+}
+
+// The smallest tile with which the problem is still one round, one tile per compute unit; problems of several rounds
+// take 256 x 256, which moves the fewest bytes through L2 and LDS per product.  A workgroup's round trip per k-block
+// is bound by what its compute unit's vector-memory path and LDS move, so with idle units a smaller tile is less work
+// on the same critical path.  us with 256 x 256 / 128 x 256 / 128 x 128 tiles:
+//   block  1000 x 7168 x 7168 (112 / 224 / 448 tiles)    79 / 61 / 61-69   (128 x 128 without pipelining: 91)
+//   block  1531 x 2048 x 7168 ( 48 /  96 / 192)          70 / 50 / 43
+//   block   300 x 14336 x 7168 (112 / 168 / 336)         78 / 56 / 86
+//   pow2   2048 x 4096 x 7168 (128 / 256 / 512)          67 / 50 / 54
+//   rows   2048 x 1024 x 4096 ( 32 /  64 / 128)          54 / 38 / 30
+//   rows, onto c  1024 x 1024 x 8192 (16 / 32 / 64)     104 / 74 / 54
+//   more than one round: block 4096 x 4096 x 4096 58 / 68 / 69, 3000 x 3072 x 3072 39 / 48 / 44, 1531 x 7168 x 2048
+//   (168 / 336 / 672 tiles) 29 / 36 / 32, pow2 2048 x 7168 x 4096 48 / 56 / 61
+static TileShape pick_shape(int64_t M, int64_t N) {
+  const int mode = g_small_gemm_mode.load(std::memory_order_relaxed);
+  if (mode == 1) return k256x256;
+  if (mode == 2) return k128x128;
+  const int64_t cus = persistent_grid((int64_t)1 << 40);
+  if (tile_count(M, N, k128x128) <= cus) return k128x128;
+  if (tile_count(M, N, k128x256) <= cus) return k128x256;
+  return k256x256;
+}
+
+// SwiGLU epilogue: a tile's columns are the gate and the up half of one scaling group, 256 in all
+// (500 x 8192 x 4096: 52 us with 64 tiles of 256 rows, 37 with 128 of 128 rows; 1000 x 12288 x 4096, 192 and 384: 62, 81).
+static TileShape pick_shape_swiglu(int64_t M, int64_t N) {
+  if (g_small_gemm_mode.load(std::memory_order_relaxed) != 0) return k256x256;
+  return tile_count(M, N, k128x256) <= persistent_grid((int64_t)1 << 40) ? k128x256 : k256x256;
+}
+
+// Grouped by rows: every expert ends in a partial tile, so with few rows per expert most of a 256-row tile is padding,
+// which costs as much as real rows (32 experts [4096, 7168], 64 / 512 / 2048 / 8192 / 16384 rows in all: 186 / 225 / 287 /
+// 389 / 531 us with 256 x 256 tiles, 147 / 176 / 214 / 344 / 606 with 128 x 256).  The rows of an expert are known on the
+// device only: the rule goes by their average, and by whether even the largest number of tiles is one round.
+static TileShape pick_shape_grouped(int64_t M, int64_t N, int experts) {
+  if (g_small_gemm_mode.load(std::memory_order_relaxed) == 1) return k256x256;
+  const int64_t most = (M / 128 + experts) * ((N + 255) / 256);
+  return M <= (int64_t)256 * experts || most <= persistent_grid((int64_t)1 << 40) ? k128x256 : k256x256;
+}
+
+// 64 x 128 tiles, where that is still one round (dense, per tensor or by blocks; 256 x 7168 x 7168: 30 us against 41
+// with 128 x 128 tiles, 700 x 1024 x 8192: 32 against 46).
 static bool use_small_kernel(int64_t M, int64_t N) {
   const int mode = g_small_gemm_mode.load(std::memory_order_relaxed);
   if (mode == 1) return false;
-  if (mode == 2) return true;
-  const int64_t big = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-  const int64_t small = ((M + kSmallTile - 1) / kSmallTile) * (N / kSmallTile);
-  const int cus = persistent_grid((int64_t)1 << 40);
-  return 2 * big < cus && small > big && small < (int64_t)0x7FFFFFFF;
+  const int64_t cus = persistent_grid((int64_t)1 << 40);
+  if (mode == 2) return tile_count(M, N, k128x128) < cus;
+  return ((M + kSmallRows - 1) / kSmallRows) * (N / kSmallTile) <= cus;
 }
 
 // Few rows of a (decode): bound by reading b once, which the tile kernels do not reach (gemm_skinny.hip; 8 rows of
@@ -1081,44 +1159,51 @@ static bool try_skinny(const GemmParams& p, bool tensor, int out_type, hipStream
 
 template <int MODE>
 static int launch_small(const GemmParams& p, int out_type, hipStream_t stream) {
-  const int64_t tiles = (((int64_t)p.M + kSmallTile - 1) / kSmallTile) * (p.N / kSmallTile);
-  dim3 block(kSmallThreads);
-  // fewer 128 x 128 tiles than compute units: tiles of 64 rows, twice as many workgroups (the same results)
-  if (tiles < persistent_grid((int64_t)1 << 40)) {
-    dim3 grid((unsigned)((((int64_t)p.M + 63) / 64) * (p.N / kSmallTile)));
-    if (out_type == HPFP8_OUT_F32) gemm_small_kernel<MODE, true, 64><<<grid, block, 0, stream>>>(p);
-    else gemm_small_kernel<MODE, false, 64><<<grid, block, 0, stream>>>(p);
-    return check_launch("gemm (small tiles)");
-  }
-  dim3 grid((unsigned)tiles);
+  dim3 grid((unsigned)((((int64_t)p.M + kSmallRows - 1) / kSmallRows) * (p.N / kSmallTile))), block(kSmallThreads);
   if (out_type == HPFP8_OUT_F32) gemm_small_kernel<MODE, true><<<grid, block, 0, stream>>>(p);
   else gemm_small_kernel<MODE, false><<<grid, block, 0, stream>>>(p);
   return check_launch("gemm (small tiles)");
 }
 
-template <int MODE, int GROUPED, bool SA4>
+template <int MODE, int GROUPED, bool SA4, int WM, int NS>
 static int launch_sa(const GemmParams& p, int out_type, int64_t tiles, hipStream_t stream) {
-  dim3 grid((unsigned)persistent_grid(tiles)), block(kGemmThreads);
+  dim3 grid((unsigned)persistent_grid(tiles)), block(128 * WM);
   if (out_type == HPFP8_OUT_F32) {
     if constexpr (MODE != kScaleTensor && GROUPED == kDense) {   // (the per-tensor and grouped entry points have no accumulate)
       if (p.accumulate) {
-        gemm_kernel<MODE, GROUPED, true, true, SA4><<<grid, block, 0, stream>>>(p);
+        gemm_kernel<MODE, GROUPED, true, true, SA4, 0, WM, NS><<<grid, block, 0, stream>>>(p);
         return check_launch("gemm");
       }
     }
-    gemm_kernel<MODE, GROUPED, true, false, SA4><<<grid, block, 0, stream>>>(p);
+    gemm_kernel<MODE, GROUPED, true, false, SA4, 0, WM, NS><<<grid, block, 0, stream>>>(p);
   } else {
-    gemm_kernel<MODE, GROUPED, false, false, SA4><<<grid, block, 0, stream>>>(p);
+    gemm_kernel<MODE, GROUPED, false, false, SA4, 0, WM, NS><<<grid, block, 0, stream>>>(p);
   }
   return check_launch("gemm");
 }
 
-template <int MODE, int GROUPED>
-static int launch(const GemmParams& p, int out_type, int64_t tiles, hipStream_t stream) {
+template <int MODE, int GROUPED, int WM, int NS>
+static int launch_shape(const GemmParams& p, int out_type, int64_t tiles, hipStream_t stream) {
   if constexpr (MODE != kScaleTensor) {
-    if (p.sa_sm == 1) return launch_sa<MODE, GROUPED, true>(p, out_type, tiles, stream);
+    if (p.sa_sm == 1) return launch_sa<MODE, GROUPED, true, WM, NS>(p, out_type, tiles, stream);
   }
-  return launch_sa<MODE, GROUPED, false>(p, out_type, tiles, stream);
+  return launch_sa<MODE, GROUPED, false, WM, NS>(p, out_type, tiles, stream);
+}
+
+template <int MODE, int GROUPED>
+static int launch(GemmParams p, int out_type, TileShape shape, hipStream_t stream) {
+  int64_t tiles = tile_count(p.M, p.N, shape);
+  p.tiles = (int)tiles;                        // (grouped by rows: the kernel counts the experts' own tiles)
+  if (GROUPED == kGroupedK) tiles *= p.experts;
+  // upper bound on row tiles: every expert may add one partial tile
+  if (GROUPED == kGroupedRows) tiles = (p.M / (shape == k256x256 ? 256 : 128) + p.experts) * ((p.N + 255) / 256);
+  if constexpr (GROUPED != kGroupedK) {
+    if (shape == k128x256) return launch_shape<MODE, GROUPED, 2, 8>(p, out_type, tiles, stream);
+  }
+  if constexpr (GROUPED == kDense) {
+    if (shape == k128x128) return launch_shape<MODE, GROUPED, 2, 4>(p, out_type, tiles, stream);
+  }
+  return launch_shape<MODE, GROUPED, 4, 8>(p, out_type, tiles, stream);
 }
 
 static int check_common(const char* what, const void* a, int64_t lda, const void* b, int64_t ldb, const float* sa,
@@ -1184,13 +1269,11 @@ static int gemm_blockwise_impl(const void* a, int64_t lda, const float* sa, int6
   p.sb_bytes = (int)(((N / kBlock - 1) * sb_stride_n + (K / BK - 1) * sb_stride_k + 1) * 4);
   p.c = c; p.ldc = ldc; p.bias = (const uint16_t*)bias;
   p.M = (int)M; p.N = (int)N; p.K = (int)K; p.accumulate = accumulate;
-  const int64_t tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-  p.tiles = (int)tiles;
   if (sb_gran == 128) {
     if (try_skinny(p, false, out_type, (hipStream_t)stream, rc)) return rc;
-    if (pow2) return launch<kScalePow2, kDense>(p, out_type, tiles, (hipStream_t)stream);
+    if (pow2) return launch<kScalePow2, kDense>(p, out_type, pick_shape(M, N), (hipStream_t)stream);
     if (!accumulate && use_small_kernel(M, N)) return launch_small<kScaleBlock>(p, out_type, (hipStream_t)stream);
-    return launch<kScaleBlock, kDense>(p, out_type, tiles, (hipStream_t)stream);
+    return launch<kScaleBlock, kDense>(p, out_type, pick_shape(M, N), (hipStream_t)stream);
   }
   // per-row b scales travel to LDS as one contiguous 1 KB piece per k-block
   if (K == BK) sb_stride_k = N;     // a single k-block: the stride between k-blocks is never used
@@ -1200,8 +1283,8 @@ static int gemm_blockwise_impl(const void* a, int64_t lda, const float* sa, int6
                 "16-byte aligned rows)");
   HPFP8_REQUIRE(((K / BK - 1) * sb_stride_k + N) * 4 < (int64_t)0x7FFFFFFF, HPFP8_ERR_SHAPE,
                 "gemm_blockwise: b scale array too large");
-  if (pow2) return launch<kScalePow2Row, kDense>(p, out_type, tiles, (hipStream_t)stream);
-  return launch<kScaleRow, kDense>(p, out_type, tiles, (hipStream_t)stream);
+  if (pow2) return launch<kScalePow2Row, kDense>(p, out_type, pick_shape(M, N), (hipStream_t)stream);
+  return launch<kScaleRow, kDense>(p, out_type, pick_shape(M, N), (hipStream_t)stream);
 }
 
 int hpfp8_gemm_blockwise(const void* a, int64_t lda, const float* sa, int64_t sa_stride_m, int64_t sa_stride_k,
@@ -1251,12 +1334,17 @@ int hpfp8_gemm_blockwise_swiglu_quantize(const void* a, int64_t lda, const float
   p.c = q; p.ldc = ldq;
   p.M = (int)M; p.N = (int)(2 * inter); p.K = (int)K;
   p.inter = (int)inter; p.pow2_out = pow2_out; p.q_scale = scale; p.q_scale_inv = scale_inv;
-  const int64_t tiles = ((M + BM - 1) / BM) * (inter / kBlock);
+  const TileShape shape = pick_shape_swiglu(M, 2 * inter);
+  const int64_t tiles = tile_count(M, 2 * inter, shape);
   p.tiles = (int)tiles;
-  dim3 grid((unsigned)persistent_grid(tiles)), block(kGemmThreads);
+  dim3 grid((unsigned)persistent_grid(tiles)), block(shape == k256x256 ? 512 : 256);
   hipStream_t st = (hipStream_t)stream;
   const bool sa4 = sa_stride_m == 1;
-#define HPFP8_LAUNCH_EPI(MODE, SA4, EPI) gemm_kernel<MODE, kDense, false, false, SA4, EPI><<<grid, block, 0, st>>>(p)
+#define HPFP8_LAUNCH_EPI(MODE, SA4, EPI) \
+  do { \
+    if (shape == k256x256) gemm_kernel<MODE, kDense, false, false, SA4, EPI, 4><<<grid, block, 0, st>>>(p); \
+    else gemm_kernel<MODE, kDense, false, false, SA4, EPI, 2><<<grid, block, 0, st>>>(p); \
+  } while (0)
   if (pow2) {
     if (sa4) { if (fast) HPFP8_LAUNCH_EPI(kScalePow2, true, 2); else HPFP8_LAUNCH_EPI(kScalePow2, true, 1); }
     else { if (fast) HPFP8_LAUNCH_EPI(kScalePow2, false, 2); else HPFP8_LAUNCH_EPI(kScalePow2, false, 1); }
@@ -1279,11 +1367,9 @@ int hpfp8_gemm_per_tensor(const void* a, int64_t lda, const float* sa_inv, const
   p.a = (const uint8_t*)a; p.b = (const uint8_t*)b; p.sa = sa_inv; p.sb = sb_inv; p.lda = lda; p.ldb = ldb;
   p.c = c; p.ldc = ldc; p.bias = (const uint16_t*)bias;
   p.M = (int)M; p.N = (int)N; p.K = (int)K;
-  const int64_t tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-  p.tiles = (int)tiles;
   if (try_skinny(p, true, out_type, (hipStream_t)stream, rc)) return rc;
   if (use_small_kernel(M, N)) return launch_small<kScaleTensor>(p, out_type, (hipStream_t)stream);
-  return launch<kScaleTensor, kDense>(p, out_type, tiles, (hipStream_t)stream);
+  return launch<kScaleTensor, kDense>(p, out_type, pick_shape(M, N), (hipStream_t)stream);
 }
 
 static int gemm_grouped_impl(const void* a, int64_t lda, const float* sa, int64_t sa_stride_m, int64_t sa_stride_k,
@@ -1310,10 +1396,8 @@ static int gemm_grouped_impl(const void* a, int64_t lda, const float* sa, int64_
   p.sb_bytes = (int)sb_span;
   p.c = c; p.ldc = ldc; p.offs = offs; p.experts = experts;
   p.M = (int)total_m; p.N = (int)N; p.K = (int)K;
-  // upper bound on row tiles: every expert may add one partial tile
-  const int64_t tiles = (total_m / BM + experts) * ((N + BN - 1) / BN);
-  if (pow2) return launch<kScalePow2, kGroupedRows>(p, out_type, tiles, (hipStream_t)stream);
-  return launch<kScaleBlock, kGroupedRows>(p, out_type, tiles, (hipStream_t)stream);
+  if (pow2) return launch<kScalePow2, kGroupedRows>(p, out_type, pick_shape_grouped(total_m, N, experts), (hipStream_t)stream);
+  return launch<kScaleBlock, kGroupedRows>(p, out_type, pick_shape_grouped(total_m, N, experts), (hipStream_t)stream);
 }
 
 int hpfp8_gemm_grouped_blockwise(const void* a, int64_t lda, const float* sa, int64_t sa_stride_m, int64_t sa_stride_k,
@@ -1365,9 +1449,7 @@ int hpfp8_gemm_grouped_wgrad(const void* a, int64_t lda, const float* sa, const 
   p.sb_sn = 1; p.sb_sk = K;          // [padded / 128, K]
   p.c = c; p.ldc = K; p.c_se = N * K; p.layout = layout; p.experts = experts;
   p.M = (int)N; p.N = (int)K; p.K = (int)padded;
-  const int64_t per_expert = ((N + BM - 1) / BM) * ((K + BN - 1) / BN);
-  p.tiles = (int)per_expert;
-  return launch<kScaleRow, kGroupedK>(p, out_type, per_expert * experts, (hipStream_t)stream);
+  return launch<kScaleRow, kGroupedK>(p, out_type, k256x256, (hipStream_t)stream);
 }
 
 }  // extern "C"

@@ -354,11 +354,11 @@ int hpfp8_gemm_per_tensor(const void* a, int64_t lda, const float* sa_inv, const
                           const float* sb_inv, int64_t M, int64_t N, int64_t K, const void* bias, void* c,
                           int64_t ldc, int out_type, hpfp8_stream_t stream);
 
-/* Small problems.  When a problem has fewer 256 x 256 output tiles than half the GPU's compute units (cfg-1-sized
- * layers, decode-sized M), hpfp8_gemm_per_tensor and hpfp8_gemm_blockwise (sb_gran = 128, no accumulate) run a
- * kernel with 128 x 128 tiles instead, four times as many workgroups; same arithmetic in the same order, identical
- * results.  Test hook, not part of the path: mode 0 = that rule (default), 1 = never, 2 = whenever the form allows
- * (process-wide, stored atomically, takes effect with the next launch). */
+/* Tiles.  The GEMMs take the smallest output tile with which a problem is still one tile per compute unit (64 x 128 for
+ * hpfp8_gemm_per_tensor and hpfp8_gemm_blockwise with sb_gran = 128 and plain scales; 128 x 128; 128 x 256) and 256 x 256
+ * otherwise; the grouped forms take 128 x 256 for few rows per expert.  Same arithmetic in the same order, identical
+ * results.  Test hook, not part of the path: mode 0 = that rule (default), 1 = always 256 x 256, 2 = always a small tile
+ * where the form has one (process-wide, stored atomically, takes effect with the next launch). */
 void hpfp8_debug_set_small_gemm(int mode);
 
 /* MoE grouped form (one rank's local experts; no counterpart in the reference, whose expert

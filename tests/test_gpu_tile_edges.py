@@ -92,3 +92,66 @@ def test_grouped_gemm_with_few_rows_is_exact_on_integer_inputs(gpu, counts, n, k
     assert bool((out[r:] == 7.0).all())
     y = ops.gemm_grouped_blockwise(a, sa, b.view(e, n, k), sb.view(e, n // 128, kb), offs)
     assert torch.equal(y[:r], out[:r].to(torch.bfloat16))
+
+
+def _strided_rows(t, pad, gpu):
+    """The same rows with a row stride of pad elements more."""
+    wide = torch.zeros((t.shape[0], t.shape[1] + pad), dtype=t.dtype, device=gpu)
+    wide[:, :t.shape[1]] = t
+    return wide[:, :t.shape[1]]
+
+
+@pytest.mark.parametrize("m,n", [(300, 6784), (385, 5504), (256, 16384), (300, 14208), (129, 32512), (257, 10880)])
+@pytest.mark.parametrize("k", [128, 256, 640])
+def test_gemm_tiles_are_exact_on_integer_inputs(gpu, m, n, k):
+    """Problems that take 128 x 128 tiles (the first three) and 128 x 256 tiles (the last three) under the default rule,
+    with ragged rows, an odd number of 128-column blocks, contractions of one, two and five k-blocks; every scale form,
+    output type, bias and accumulation.  Exact for the reason above (with scales on both operands' rows sums are multiples
+    of 2^-4 too)."""
+    from hpfp8 import ops
+    a, b = _ints((m, k), 1, gpu), _ints((n, k), 2, gpu)
+    kb = k // 128
+    sa, sb = _pow2((kb, m), 3, gpu).t(), _pow2((n // 128, kb), 4, gpu)
+    sr = _pow2((kb, n), 6, gpu).t()
+    bias = _pow2((n,), 5, gpu).to(torch.bfloat16)
+    av = _dequantized(a, sa.contiguous(), 1)
+    want = av @ _dequantized(b, sb, 128).t()
+    rows = av @ _dequantized(b, sr.contiguous(), 1).t()
+    for pow2 in (False, True):
+        assert torch.equal(ops.gemm_blockwise(a, sa, b, sb, pow2_scales=pow2, out_dtype=torch.float32).double(), want)
+        assert torch.equal(ops.gemm_blockwise(_strided_rows(a, 16, gpu), sa.contiguous(), b, sb, bias=bias, pow2_scales=pow2),
+                           (want + bias.double()).to(torch.bfloat16))
+        assert torch.equal(ops.gemm_blockwise(a, sa, b, sr, sb_gran=1, pow2_scales=pow2), rows.to(torch.bfloat16))
+        c = torch.full((m, n), 3.0, dtype=torch.float32, device=gpu)
+        ops.gemm_blockwise(a, sa, b, sr, sb_gran=1, out=c, accumulate=True, pow2_scales=pow2)
+        assert torch.equal(c.double(), rows + 3.0)
+        ops.gemm_blockwise(a, sa, b, sb, out=c, accumulate=True, pow2_scales=pow2)
+        assert torch.equal(c.double(), rows + 3.0 + want)
+    one = a.double() @ b.double().t() * 0.125
+    ta, tb = torch.tensor(0.5, device=gpu), torch.tensor(0.25, device=gpu)
+    assert torch.equal(ops.gemm_per_tensor(a, ta, b, tb, out_dtype=torch.float32).double(), one)
+    assert torch.equal(ops.gemm_per_tensor(a, ta, b, tb, bias=bias), (one + bias.double()).to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("m,inter,k", [(65, 128, 128), (127, 384, 384), (129, 1280, 256), (300, 10752, 128)])
+@pytest.mark.parametrize("fast,pow2", [(True, False), (False, True)])
+def test_swiglu_epilogue_is_the_same_with_both_tile_heights(gpu, m, inter, k, fast, pow2):
+    from hpfp8 import _lib, ops
+    x, w = randn_bf16((m, k), 1).to(gpu), randn_bf16((2 * inter, k), 2, 0.05).to(gpu)
+    xq, sx = ops.quantize_1x128(x, kmajor=True, pow2=pow2)
+    wq, sw = ops.quantize_128x128(w, pow2=pow2)
+    got = ops.gemm_blockwise_swiglu_quantize(xq, sx, wq, sw, fast=fast, pow2_scales=pow2, want_scale=True)
+    _lib.load().hpfp8_debug_set_small_gemm(1)
+    try:
+        want = ops.gemm_blockwise_swiglu_quantize(xq, sx, wq, sw, fast=fast, pow2_scales=pow2, want_scale=True)
+    finally:
+        _lib.load().hpfp8_debug_set_small_gemm(0)
+    assert torch.equal(got[0].view(torch.uint8), want[0].view(torch.uint8))
+    assert torch.equal(got[1], want[1]) and torch.equal(got[2], want[2])
+
+
+@pytest.mark.parametrize("counts", [[127, 128, 129, 0, 1, 255, 257], [0, 0, 1000, 3], [2048, 0, 1, 700]])
+@pytest.mark.parametrize("n,k", [(128, 128), (640, 384)])
+def test_grouped_tiles_are_exact_on_integer_inputs(gpu, counts, n, k):
+    """Row counts around the 128-row tile of the grouped form, the tile it takes for few rows per expert."""
+    test_grouped_gemm_with_few_rows_is_exact_on_integer_inputs(gpu, counts, n, k)
