@@ -728,7 +728,13 @@ __device__ __forceinline__ float column_sum_of_tile(const float (*s_cs)[128], in
 
 // With COLSUM the kernel also writes colsum_part[tr * k + column] = the fp32 sum of the tile's 128 rows per column
 // (tile_column_sums): the per-block partial sums of a bias gradient, from the same read of grad_out.
-template <bool KMAJOR, bool DUAL, int SW = 0, bool GROUPED = false, bool COLSUM = false>
+// ROWS: which rows of a tile exist.  Whole: all.  By expert: the layout table says.  Ragged: m need not be a multiple of
+// 128; rows past m count as zeros, as if x had been filled up with zero rows, and are written in the transposed form
+// only.  (A variant of its own, so that the whole form's loads stay unconditional.)  A ragged training step used to copy
+// x and grad_out into zero-padded buffers (fill + copy, 25 us for [1531, 7168] and [1531, 2048]) and to read each once
+// more for its 1x128 form and for the bias gradient.
+enum TileRows { kWholeRows = 0, kRowsByExpert = 1, kRaggedRows = 2 };
+template <bool KMAJOR, bool DUAL, int SW = 0, int ROWS = kWholeRows, bool COLSUM = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void quant_128x1_t_kernel(const uint16_t* __restrict__ x, int64_t ld_src, int m, int k,
                                                             uint8_t* __restrict__ qt, int64_t ld_t,
                                                             float* __restrict__ scale_t,
@@ -738,8 +744,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void q
                                                             const int32_t* __restrict__ layout = nullptr, int experts = 0,
                                                             int padded_blocks = 0, const uint16_t* __restrict__ dact = nullptr,
                                                             float* __restrict__ colsum_part = nullptr) {
+  constexpr bool GROUPED = ROWS == kRowsByExpert;
+  constexpr bool PARTIAL = ROWS != kWholeRows;
   static_assert(!COLSUM || (SW == 0 && !GROUPED), "column sums: plain dense source only");
-  const int kb = k >> 7, mb = GROUPED ? padded_blocks : m >> 7;
+  const int kb = k >> 7, mb = GROUPED ? padded_blocks : (m + 127) >> 7;
   const int cg = threadIdx.x & 15, rq = threadIdx.x >> 4;
   const int wave = threadIdx.x >> 6;
   __shared__ uint32_t part[4][64];  // [wave][cg*4 + word]
@@ -758,6 +766,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void q
     g_valid = layout[4 * e + 1] - j * 128;
     g_valid = g_valid < 0 ? 0 : (g_valid > 128 ? 128 : g_valid);
   }
+  if (ROWS == kRaggedRows) g_valid = m - g_row0 < 128 ? m - g_row0 : 128;
   // byte offset of this thread's first element inside the source tile, and the row stride in bytes
   const uint32_t ld_b = (uint32_t)ld_src * 2u;
   const uint32_t t_off = (uint32_t)(4 * rq) * ld_b + (uint32_t)cg * 16u;
@@ -774,6 +783,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void q
     const uint32_t d_off = (uint32_t)(4 * rq) * ldd_b + (uint32_t)cg * 16u;
 #pragma unroll
     for (int p = 0; p < 8; ++p) {
+      v[p] = make_uint4(0, 0, 0, 0);
+      if (PARTIAL && tile_row(rq, p) >= g_valid) continue;
       const uint4 gv = nt_load16(gbase + row_off(p));
       const uint4 dv = nt_load16(dbase + d_off + (uint32_t)((p >> 2) * 64 + (p & 3)) * ldd_b);
       uint32_t unused;
@@ -794,10 +805,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void q
     const char* sbase = reinterpret_cast<const char*>(x + (int64_t)g_row0 * ld_src + tc * 128);
 #pragma unroll
     for (int p = 0; p < 8; ++p)
-      v[p] = (!GROUPED || tile_row(rq, p) < g_valid) ? nt_load16(sbase + row_off(p)) : make_uint4(0, 0, 0, 0);
+      v[p] = (!PARTIAL || tile_row(rq, p) < g_valid) ? nt_load16(sbase + row_off(p)) : make_uint4(0, 0, 0, 0);
     if (SW) {
 #pragma unroll
       for (int p = 0; p < 8; ++p) {
+        if (PARTIAL && tile_row(rq, p) >= g_valid) continue;      // (stays zero)
         const uint4 u = nt_load16(sbase + (uint32_t)k * 2u + row_off(p));
         v[p].x = swiglu2<SW == 2>(v[p].x, u.x);
         v[p].y = swiglu2<SW == 2>(v[p].y, u.y);
@@ -837,7 +849,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void q
 #pragma unroll
       for (int p = 0; p < 4; ++p) {
         const int row = tile_row(rq, 4 * half + p);
-        if (!GROUPED || row < g_valid)
+        if (!PARTIAL || row < g_valid)
           nt_store8(qbase + q_off + (uint32_t)(half * 64 + p) * (uint32_t)k, cvt8<false>(v[4 * half + p], s[p]));
       }
       if (cg < 4) {
@@ -852,7 +864,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void q
     const int row = threadIdx.x - 128;
     const int64_t r_abs = (int64_t)g_row0 + row;
     const int64_t o = KMAJOR ? (int64_t)tc * m + r_abs : r_abs * kb + tc;
-    if (!GROUPED || row < g_valid) {
+    if (!PARTIAL || row < g_valid) {
       if (scale_r) scale_r[o] = s_row[row];
       scale_inv_r[o] = s_row[128 + row];
     }
@@ -1370,10 +1382,10 @@ static int quantize_128x1_t_impl(const char* what, bool kmajor, const void* x, i
   if (colsum_part) {
     HPFP8_REQUIRE(kmajor, HPFP8_ERR_ARG, "%s: the column sums come with the k-block-major scale layout only", what);
     if (q)
-      quant_128x1_t_kernel<true, true, 0, false, true><<<grid, 256, 0, s>>>(xs, k, (int)m, (int)k, qt8, ld_t, scale_t, scale_inv_t, q8,
+      quant_128x1_t_kernel<true, true, 0, kWholeRows, true><<<grid, 256, 0, s>>>(xs, k, (int)m, (int)k, qt8, ld_t, scale_t, scale_inv_t, q8,
                                                                             scale, scale_inv, pow2, ak, nullptr, 0, 0, nullptr, colsum_part);
     else
-      quant_128x1_t_kernel<true, false, 0, false, true><<<grid, 256, 0, s>>>(xs, k, (int)m, (int)k, qt8, ld_t, scale_t, scale_inv_t, nullptr,
+      quant_128x1_t_kernel<true, false, 0, kWholeRows, true><<<grid, 256, 0, s>>>(xs, k, (int)m, (int)k, qt8, ld_t, scale_t, scale_inv_t, nullptr,
                                                                              nullptr, nullptr, pow2, ak, nullptr, 0, 0, nullptr, colsum_part);
   } else if (q) {
     if (kmajor)
@@ -1470,13 +1482,97 @@ int hpfp8_quantize_128x1_t_grouped_bf16(const void* x, int64_t total_m, int64_t 
   int ak = 0;
   const dim3 grid = transpose_grid(padded_blocks, k / kBlock, k * 2, q ? 2 : 1, ak);
   if (q)
-    quant_128x1_t_kernel<true, true, 0, true><<<grid, 256, 0, s>>>(
+    quant_128x1_t_kernel<true, true, 0, kRowsByExpert><<<grid, 256, 0, s>>>(
         (const uint16_t*)x, k, (int)total_m, (int)k, (uint8_t*)q_t, ld_t, nullptr, scale_inv_t, (uint8_t*)q, nullptr, scale_inv, 0,
         ak, layout, experts, (int)padded_blocks);
   else
-    quant_128x1_t_kernel<true, false, 0, true><<<grid, 256, 0, s>>>(
+    quant_128x1_t_kernel<true, false, 0, kRowsByExpert><<<grid, 256, 0, s>>>(
         (const uint16_t*)x, k, (int)total_m, (int)k, (uint8_t*)q_t, ld_t, nullptr, scale_inv_t, nullptr, nullptr, nullptr, 0,
         ak, layout, experts, (int)padded_blocks);
+  return check_launch(what);
+}
+
+// What the three entry points for any number of rows check: the dense forms' rules but for the row count.
+static int check_rows(const char* what, int64_t m, int64_t k, const void* x, int64_t ld, const void* q, const float* scale_inv,
+                      const void* q_t, int64_t ld_t, const float* scale_inv_t) {
+  HPFP8_REQUIRE(m >= 0 && k >= 0, HPFP8_ERR_SHAPE, "%s: negative shape", what);
+  HPFP8_REQUIRE(k % kBlock == 0, HPFP8_ERR_SHAPE, "%s: width %lld is not a multiple of 128", what, (long long)k);
+  HPFP8_REQUIRE(m < (1 << 30) && k < (1 << 24) && ld < (1 << 24) && ld_t < (1 << 24), HPFP8_ERR_SHAPE,
+                "%s: dimension too large (at most 2^30 rows; width and row strides below 2^24)", what);
+  const int64_t mb = (m + kBlock - 1) / kBlock, blocks = mb * (k / kBlock);
+  if (blocks == 0) return HPFP8_OK;
+  HPFP8_REQUIRE(blocks <= 0x7FFFFFFF, HPFP8_ERR_SHAPE, "%s: tensor too large", what);
+  HPFP8_REQUIRE(x && q_t && scale_inv_t, HPFP8_ERR_ARG, "%s: null buffer", what);
+  HPFP8_REQUIRE(aligned16(x) && aligned16(q_t), HPFP8_ERR_ALIGN, "%s: buffers must be 16-byte aligned", what);
+  HPFP8_REQUIRE(ld % 8 == 0, HPFP8_ERR_SHAPE, "%s: the row stride must be a multiple of 8", what);
+  HPFP8_REQUIRE(ld_t >= mb * kBlock && ld_t % 16 == 0, HPFP8_ERR_SHAPE,
+                "%s: ld_t=%lld must be a multiple of 16 and at least the rows rounded up to 128", what, (long long)ld_t);
+  HPFP8_REQUIRE(!q || (scale_inv && aligned16(q)), HPFP8_ERR_ARG, "%s: q needs scale_inv and 16-byte alignment", what);
+  return 1;
+}
+
+int hpfp8_quantize_rows_128x1_t_bf16(const void* x, int64_t m, int64_t k, void* q, float* scale_inv, void* q_t, int64_t ld_t,
+                                     float* scale_inv_t, int pow2, float* colsum_partial, hpfp8_stream_t stream) {
+  const char* what = "quantize_rows_128x1_t";
+  int rc = check_rows(what, m, k, x, k, q, scale_inv, q_t, ld_t, scale_inv_t);
+  if (rc <= 0) return rc;
+  if (m % kBlock == 0)
+    return quantize_128x1_t_impl(what, true, x, m, k, q_t, ld_t, nullptr, scale_inv_t, stream, q, nullptr, scale_inv, pow2 ? 1 : 0,
+                                 colsum_partial);
+  int ak = 0;
+  const dim3 grid = transpose_grid((m + kBlock - 1) / kBlock, k / kBlock, k * 2, q ? 2 : 1, ak);
+#define HPFP8_RAGGED(DUAL, COLSUM) \
+  quant_128x1_t_kernel<true, DUAL, 0, kRaggedRows, COLSUM><<<grid, 256, 0, (hipStream_t)stream>>>( \
+      (const uint16_t*)x, k, (int)m, (int)k, (uint8_t*)q_t, ld_t, nullptr, scale_inv_t, (uint8_t*)q, nullptr, scale_inv, pow2 ? 1 : 0, \
+      ak, nullptr, 0, 0, nullptr, colsum_partial)
+  if (q && colsum_partial) HPFP8_RAGGED(true, true);
+  else if (q) HPFP8_RAGGED(true, false);
+  else if (colsum_partial) HPFP8_RAGGED(false, true);
+  else HPFP8_RAGGED(false, false);
+#undef HPFP8_RAGGED
+  return check_launch(what);
+}
+
+int hpfp8_swiglu_quantize_rows_128x1_t_bf16(const void* h, int64_t rows, int64_t inter, int64_t ld_h, int fast, void* q,
+                                            float* scale_inv, void* q_t, int64_t ld_t, float* scale_inv_t, hpfp8_stream_t stream) {
+  const char* what = "swiglu_quantize_rows_128x1_t";
+  int rc = check_rows(what, rows, inter, h, ld_h, q, scale_inv, q_t, ld_t, scale_inv_t);
+  if (rc <= 0) return rc;
+  HPFP8_REQUIRE(q, HPFP8_ERR_ARG, "%s: null buffer", what);
+  HPFP8_REQUIRE(ld_h >= 2 * inter, HPFP8_ERR_SHAPE, "%s: ld_h=%lld must be at least twice the width", what, (long long)ld_h);
+  if (rows % kBlock == 0)
+    return hpfp8_swiglu_quantize_1x128_and_128x1_t_bf16(h, rows, inter, ld_h, fast, q, nullptr, scale_inv, q_t, ld_t, nullptr,
+                                                        scale_inv_t, stream);
+  int ak = 0;
+  const dim3 grid = transpose_grid((rows + kBlock - 1) / kBlock, inter / kBlock, ld_h * 2, 2, ak);
+  if (fast)
+    quant_128x1_t_kernel<true, true, 2, kRaggedRows><<<grid, 256, 0, (hipStream_t)stream>>>(
+        (const uint16_t*)h, ld_h, (int)rows, (int)inter, (uint8_t*)q_t, ld_t, nullptr, scale_inv_t, (uint8_t*)q, nullptr, scale_inv, 0, ak);
+  else
+    quant_128x1_t_kernel<true, true, 1, kRaggedRows><<<grid, 256, 0, (hipStream_t)stream>>>(
+        (const uint16_t*)h, ld_h, (int)rows, (int)inter, (uint8_t*)q_t, ld_t, nullptr, scale_inv_t, (uint8_t*)q, nullptr, scale_inv, 0, ak);
+  return check_launch(what);
+}
+
+int hpfp8_swiglu_backward_quantize_rows_128x1_t_bf16(const void* h, int64_t rows, int64_t inter, int64_t ld_h, const void* dact,
+                                                     void* q, float* scale_inv, void* q_t, int64_t ld_t, float* scale_inv_t,
+                                                     hpfp8_stream_t stream) {
+  const char* what = "swiglu_backward_quantize_rows_128x1_t";
+  HPFP8_REQUIRE(inter < (1 << 23) && inter % kBlock == 0, HPFP8_ERR_SHAPE, "%s: width %lld is not a multiple of 128 below 2^23", what,
+                (long long)inter);
+  int rc = check_rows(what, rows, 2 * inter, h, ld_h, q, scale_inv, q_t, ld_t, scale_inv_t);
+  if (rc <= 0) return rc;
+  HPFP8_REQUIRE(q && dact, HPFP8_ERR_ARG, "%s: null buffer", what);
+  HPFP8_REQUIRE(aligned16(dact), HPFP8_ERR_ALIGN, "%s: buffers must be 16-byte aligned", what);
+  HPFP8_REQUIRE(ld_h >= 2 * inter, HPFP8_ERR_SHAPE, "%s: ld_h=%lld must be at least twice the width", what, (long long)ld_h);
+  if (rows % kBlock == 0)
+    return hpfp8_swiglu_backward_quantize_1x128_and_128x1_t_bf16(h, rows, inter, ld_h, dact, q, nullptr, scale_inv, q_t, ld_t, nullptr,
+                                                                 scale_inv_t, stream);
+  int ak = 0;
+  const dim3 grid = transpose_grid((rows + kBlock - 1) / kBlock, 2 * inter / kBlock, ld_h * 2, 2, ak);
+  quant_128x1_t_kernel<true, true, 3, kRaggedRows><<<grid, 256, 0, (hipStream_t)stream>>>(
+      (const uint16_t*)h, ld_h, (int)rows, (int)(2 * inter), (uint8_t*)q_t, ld_t, nullptr, scale_inv_t, (uint8_t*)q, nullptr,
+      scale_inv, 0, ak, nullptr, 0, 0, (const uint16_t*)dact);
   return check_launch(what);
 }
 

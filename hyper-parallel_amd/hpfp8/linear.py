@@ -82,9 +82,15 @@ def _flatten(x: torch.Tensor):
 
 def _pad_rows(t: torch.Tensor) -> torch.Tensor:
     """t[M, C] with zero rows appended up to the next multiple of 128: tokens that contribute nothing to a
-    weight gradient, so that the 128x1 groups along the tokens are whole (the last one holds fewer real values)."""
+    weight gradient, so that the contraction over them is whole k-blocks."""
     pad = -t.shape[0] % ops.BLOCK
     return torch.nn.functional.pad(t, (0, 0, 0, pad)) if pad else t
+
+
+def _both_forms(t: torch.Tensor, pow2: bool = False, column_sum: bool = False):
+    """The 1x128 and the transposed 128x1 form of t[M, C] from one read of it, for any M > 0 (k-block-major scales)."""
+    form = ops.quantize_1x128_and_128x1_t_rows if t.shape[0] % ops.BLOCK else ops.quantize_1x128_and_128x1_t
+    return form(t, pow2=pow2, column_sum=column_sum)
 
 
 def _empty_batch_grads(ctx, go):
@@ -114,12 +120,11 @@ class _Fp8LinearBlockwise(torch.autograd.Function):
         # Parameter has requires_grad set under torch.no_grad() too; without a backward to come nothing is
         # prepared or kept for it.
         need_dx, need_dw = grad_mode and x.requires_grad, grad_mode and weight.requires_grad
-        # With a weight gradient to come and a token count that allows it, x is read once: its 1x128
-        # codes for this GEMM and its transposed 128x1 codes for wgrad, which are what is kept for
-        # backward (1 byte per element instead of the bf16 source).
-        fused = need_dw and m % ops.BLOCK == 0 and m > 0
-        if fused:
-            xq, sx, xt, sxt = ops.quantize_1x128_and_128x1_t(x2.contiguous(), kmajor=True, pow2=pow2)
+        # With a weight gradient to come x is read once: its 1x128 codes for this GEMM and its transposed 128x1
+        # codes for wgrad, which are what is kept for backward (1 byte per element instead of the bf16 source).
+        # The 128x1 groups run along the tokens; a ragged token count is filled up with zero rows by the kernel.
+        if need_dw and m > 0:
+            xq, sx, xt, sxt = _both_forms(x2, pow2=pow2)
         else:
             xq, sx = ops.quantize_1x128(x2, kmajor=True, pow2=pow2)
             xt = sxt = None
@@ -131,7 +136,7 @@ class _Fp8LinearBlockwise(torch.autograd.Function):
         elif need_dx and wqt is None:
             wqt = ops.transpose_codes(wq)
         y = ops.gemm_blockwise(xq, sx, wq, sw, bias=bias, pow2_scales=pow2)
-        ctx.save_for_backward(x2 if (need_dw and not fused) else None, xt, sxt, wqt if need_dx else None, sw)
+        ctx.save_for_backward(xt, sxt, wqt if need_dx else None, sw)
         ctx.x_shape = x.shape
         ctx.w_shape = weight.shape
         ctx.has_bias = bias is not None
@@ -140,7 +145,7 @@ class _Fp8LinearBlockwise(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_out):
-        x2, xt, sxt, wqt, sw = ctx.saved_tensors
+        xt, sxt, wqt, sw = ctx.saved_tensors
         need_dx, need_dw = ctx.need
         pow2 = ctx.pow2
         go = _flatten(grad_out)
@@ -150,19 +155,18 @@ class _Fp8LinearBlockwise(torch.autograd.Function):
         m = go.shape[0]
         if m == 0:
             return _empty_batch_grads(ctx, go) + (None, None, None, None, None, None)
-        ragged = m % ops.BLOCK != 0            # wgrad then runs on zero-padded token rows
         dx = dw = db = None
         goq = sgo = got = sgot = None
-        if need_dx and need_dw and not ragged:
+        if need_dx and need_dw:
             if ctx.has_bias:                   # one read of grad_out: both operand forms and the bias gradient
-                goq, sgo, got, sgot, db = ops.quantize_1x128_and_128x1_t(go, kmajor=True, pow2=pow2, column_sum=True)
+                goq, sgo, got, sgot, db = _both_forms(go, pow2=pow2, column_sum=True)
             else:
-                goq, sgo, got, sgot = ops.quantize_1x128_and_128x1_t(go, kmajor=True, pow2=pow2)
+                goq, sgo, got, sgot = _both_forms(go, pow2=pow2)
         else:
             if need_dx:
                 goq, sgo = ops.quantize_1x128(go, kmajor=True, pow2=pow2)
             if need_dw:
-                got, sgot = ops.quantize_128x1_t(_pad_rows(go), kmajor=True, pow2=pow2)
+                got, sgot = ops.quantize_128x1_t_rows(go, pow2=pow2)
             if ctx.has_bias:
                 db = ops.column_sum(go)
         if need_dx:
@@ -171,8 +175,6 @@ class _Fp8LinearBlockwise(torch.autograd.Function):
             dx = ops.gemm_blockwise(goq, sgo, wqt, sw.t(), pow2_scales=pow2).reshape(ctx.x_shape)
         if need_dw:
             # dW[N,K] = go^T[N,M] . x[M,K]: contraction over tokens, both operands 1x128 along M
-            if xt is None:
-                xt, sxt = ops.quantize_128x1_t(_pad_rows(x2), kmajor=True, pow2=pow2)
             param = ctx.main_grad_of
             if param is None:
                 dw = ops.gemm_blockwise(got, sgot, xt, sxt, sb_gran=1, pow2_scales=pow2)
@@ -521,11 +523,10 @@ class _Fp8SwiGLUDown(torch.autograd.Function):
     def forward(ctx, h, weight, fast=True, wq=None, sw=None, wqt=None):
         h2 = _flatten(h)
         m = h2.shape[0]
-        # With a weight gradient to come and a token count that allows it, the gate/up output is read once for
-        # both forms of the activation: its 1x128 codes for this GEMM and its transposed 128x1 codes, kept for wgrad.
-        fused = weight.requires_grad and m % ops.BLOCK == 0 and m > 0
-        if fused:
-            aq, sa, at, sat = ops.swiglu_quantize_1x128_and_128x1_t(h2, fast=fast)
+        # With a weight gradient to come the gate/up output is read once for both forms of the activation: its
+        # 1x128 codes for this GEMM and its transposed 128x1 codes, kept for wgrad.
+        if weight.requires_grad and m > 0:
+            aq, sa, at, sat = ops.swiglu_quantize_1x128_and_128x1_t_rows(h2, fast=fast)
         else:
             aq, sa = ops.swiglu_quantize_1x128(h2, kmajor=True, fast=fast)
             at = sat = None
@@ -537,8 +538,7 @@ class _Fp8SwiGLUDown(torch.autograd.Function):
         elif h.requires_grad and wqt is None:
             wqt = ops.transpose_codes(wq)
         y = ops.gemm_blockwise(aq, sa, wq, sw)
-        ctx.save_for_backward(h2 if h.requires_grad or (weight.requires_grad and not fused) else None, wqt, sw, at, sat)
-        ctx.fast = fast
+        ctx.save_for_backward(h2 if h.requires_grad else None, wqt, sw, at, sat)
         ctx.h_shape = h.shape
         ctx.x_shape, ctx.w_shape, ctx.has_bias = h.shape, weight.shape, False
         ctx.need = (h.requires_grad, weight.requires_grad)
@@ -555,22 +555,16 @@ class _Fp8SwiGLUDown(torch.autograd.Function):
         m = go.shape[0]
         if m == 0:
             return _empty_batch_grads(ctx, go)[:2] + (None, None, None, None)
-        ragged = m % ops.BLOCK != 0            # wgrad then runs on zero-padded token rows
         dh = dw = None
         goq = sgo = got = sgot = None
-        if need_dh and need_dw and not ragged:
-            goq, sgo, got, sgot = ops.quantize_1x128_and_128x1_t(go, kmajor=True)
+        if need_dh and need_dw:
+            goq, sgo, got, sgot = _both_forms(go)
         else:
             if need_dh:
                 goq, sgo = ops.quantize_1x128(go, kmajor=True)
             if need_dw:
-                got, sgot = ops.quantize_128x1_t(_pad_rows(go), kmajor=True)
+                got, sgot = ops.quantize_128x1_t_rows(go)
         if need_dw:
-            if at is None:
-                # the activation again (bf16 this time), for its 128x1 codes along the tokens
-                _, _, act = ops.swiglu_quantize_1x128(h2, kmajor=True, want_act=True, fast=ctx.fast)
-                at, sat = ops.quantize_128x1_t(_pad_rows(act), kmajor=True)
-                del act
             dw = ops.gemm_blockwise(got, sgot, at, sat, sb_gran=1)
         if need_dh:
             dact = ops.gemm_blockwise(goq, sgo, wqt, sw.t())
@@ -580,16 +574,16 @@ class _Fp8SwiGLUDown(torch.autograd.Function):
 
 class _Fp8SwiGLUMLPBlock(torch.autograd.Function):
     """The whole block y = F.linear(silu(gate) * up, w_down), gate | up = F.linear(x, w_gate_up), as one autograd node
-    (blockwise recipe, both weights trained, token count a multiple of 128).  Every bf16 tensor between the GEMMs is
+    (blockwise recipe, both weights trained).  Every bf16 tensor between the GEMMs is
     read once: x, the gate/up output and grad_out each give both of their operand forms in one pass, and in backward
     the gradient of SwiGLU is quantized for the gate/up projection's two GEMMs as it is computed, so d gate | d up is
     never written in bf16."""
 
     @staticmethod
     def forward(ctx, x, w_gate_up, w_down, fast, gu8, dn8):
-        x2 = _flatten(x).contiguous()
+        x2 = _flatten(x)
         need_dx = x.requires_grad
-        xq, sx, xt, sxt = ops.quantize_1x128_and_128x1_t(x2, kmajor=True)
+        xq, sx, xt, sxt = _both_forms(x2)
 
         def forms(w, f8):
             if f8 is None:
@@ -598,7 +592,7 @@ class _Fp8SwiGLUMLPBlock(torch.autograd.Function):
         gq, gs, gqt = forms(w_gate_up, gu8)
         dq, ds, dqt = forms(w_down, dn8)
         h = ops.gemm_blockwise(xq, sx, gq, gs)
-        aq, sa, at, sat = ops.swiglu_quantize_1x128_and_128x1_t(h, fast=fast)
+        aq, sa, at, sat = ops.swiglu_quantize_1x128_and_128x1_t_rows(h, fast=fast)
         y = ops.gemm_blockwise(aq, sa, dq, ds)
         ctx.save_for_backward(h, xt, sxt, gqt if need_dx else None, gs, dqt, ds, at, sat)
         ctx.x_shape, ctx.need_dx = x.shape, need_dx
@@ -610,10 +604,10 @@ class _Fp8SwiGLUMLPBlock(torch.autograd.Function):
         go = _flatten(grad_out)
         if go.dtype != torch.bfloat16:
             go = go.to(torch.bfloat16)
-        goq, sgo, got, sgot = ops.quantize_1x128_and_128x1_t(go.contiguous(), kmajor=True)
+        goq, sgo, got, sgot = _both_forms(go)
         dw_down = ops.gemm_blockwise(got, sgot, at, sat, sb_gran=1)
         dact = ops.gemm_blockwise(goq, sgo, dqt, ds.t())
-        dhq, sdh, dht, sdht = ops.swiglu_backward_quantize_1x128_and_128x1_t(h, dact)
+        dhq, sdh, dht, sdht = ops.swiglu_backward_quantize_1x128_and_128x1_t_rows(h, dact)
         dx = ops.gemm_blockwise(dhq, sdh, gqt, gs.t()).reshape(ctx.x_shape) if ctx.need_dx else None
         dw_gate_up = ops.gemm_blockwise(dht, sdht, xt, sxt, sb_gran=1)
         return dx, dw_gate_up, dw_down, None, None, None
@@ -653,7 +647,7 @@ def fp8_swiglu_mlp(input: torch.Tensor, w_gate_up, w_down, *, fast: bool = True,
         if input.shape[-1] != w_gate_up.shape[1]:
             raise ValueError(f"input last dim {input.shape[-1]} != w_gate_up in_features {w_gate_up.shape[1]}")
         rows = input.numel() // max(input.shape[-1], 1)
-        if (w_gate_up.requires_grad and w_down.requires_grad and rows > 0 and rows % ops.BLOCK == 0
+        if (w_gate_up.requires_grad and w_down.requires_grad and rows > 0
                 and input.dtype == torch.bfloat16 and w_gate_up.dtype == torch.bfloat16 and w_down.dtype == torch.bfloat16):
             return _Fp8SwiGLUMLPBlock.apply(input, w_gate_up, w_down, fast, gate_up_fp8, d8)
         h = fp8_linear(input, w_gate_up, weight_fp8=gate_up_fp8)

@@ -253,18 +253,27 @@ def swiglu_quantize_1x128_and_128x1_t(h: torch.Tensor, fast: bool = False):
     """Both quantized forms of act = silu(gate) * up from one read of h[M, 2I] = gate | up:
     (codes[M, I], scale_inv[M, I/128], codes_t[I, M], scale_inv_t[I, M/128]), k-block-major scales, bit-identical to
     ``swiglu_quantize_1x128(h, fast=fast)`` and to ``quantize_128x1_t`` of its activation.  M and I multiples of 128."""
-    h = _check_bf16(h, "h", contiguous=False)
-    if h.dim() != 2 or h.shape[1] % (2 * BLOCK) or h.shape[0] % BLOCK:
+    if isinstance(h, torch.Tensor) and h.dim() == 2 and h.shape[0] % BLOCK:
         raise ValueError("h must be [M, 2I] with M and I multiples of 128")
+    return swiglu_quantize_1x128_and_128x1_t_rows(h, fast)
+
+
+def swiglu_quantize_1x128_and_128x1_t_rows(h: torch.Tensor, fast: bool = False):
+    """`swiglu_quantize_1x128_and_128x1_t` for any M: the transposed form is that of the activation filled up with zero rows
+    to the next multiple of 128 (codes_t[I, Mp], scale_inv_t[I, Mp/128])."""
+    h = _check_bf16(h, "h", contiguous=False)
+    if h.dim() != 2 or h.shape[1] % (2 * BLOCK):
+        raise ValueError("h must be [M, 2I] with I a multiple of 128")
     if h.stride(1) != 1 or h.stride(0) % 8 or h.data_ptr() % 16:
         h = h.contiguous()
     m, inter = h.shape[0], h.shape[1] // 2
     q = torch.empty((m, inter), dtype=FP8, device=h.device)
-    qt = _empty_codes_t(inter, m, h.device)
+    mp = _rows_up(m)
+    qt = _empty_codes_t(inter, mp, h.device)
     s_inv = torch.empty((inter // BLOCK, m), dtype=torch.float32, device=h.device)
-    st_inv = torch.empty((m // BLOCK, inter), dtype=torch.float32, device=h.device)
-    _lib.call("hpfp8_swiglu_quantize_1x128_and_128x1_t_bf16", _ptr(h), m, inter, h.stride(0) if m > 1 else 2 * inter,
-              int(fast), _ptr(q), None, _ptr(s_inv), _ptr(qt), _ld(qt), None, _ptr(st_inv), _stream())
+    st_inv = torch.empty((mp // BLOCK, inter), dtype=torch.float32, device=h.device)
+    _lib.call("hpfp8_swiglu_quantize_rows_128x1_t_bf16", _ptr(h), m, inter, h.stride(0) if m > 1 else 2 * inter,
+              int(fast), _ptr(q), _ptr(s_inv), _ptr(qt), _ld(qt), _ptr(st_inv), _stream())
     return q, s_inv.t(), qt, st_inv.t()
 
 
@@ -287,19 +296,28 @@ def swiglu_backward_quantize_1x128_and_128x1_t(h: torch.Tensor, dact: torch.Tens
     """`swiglu_backward` fused with both quantized forms of its result dh = [d gate | d up] ([M, 2I]; never written in
     bf16): (codes[M, 2I], scale_inv[M, 2I/128], codes_t[2I, M], scale_inv_t[2I, M/128]), k-block-major scales,
     bit-identical to ``quantize_1x128_and_128x1_t(swiglu_backward(h, dact))``.  M and I multiples of 128."""
+    if isinstance(h, torch.Tensor) and h.dim() == 2 and h.shape[0] % BLOCK:
+        raise ValueError("h must be [M, 2I] with M and I multiples of 128 and dact [M, I]")
+    return swiglu_backward_quantize_1x128_and_128x1_t_rows(h, dact)
+
+
+def swiglu_backward_quantize_1x128_and_128x1_t_rows(h: torch.Tensor, dact: torch.Tensor):
+    """`swiglu_backward_quantize_1x128_and_128x1_t` for any M: the transposed form is that of dh filled up with zero rows to
+    the next multiple of 128 (codes_t[2I, Mp], scale_inv_t[2I, Mp/128])."""
     h = _check_bf16(h, "h", contiguous=False)
     dact = _check_bf16(dact, "dact")
-    if h.dim() != 2 or h.shape[1] % (2 * BLOCK) or h.shape[0] % BLOCK or dact.shape != (h.shape[0], h.shape[1] // 2):
-        raise ValueError("h must be [M, 2I] with M and I multiples of 128 and dact [M, I]")
+    if h.dim() != 2 or h.shape[1] % (2 * BLOCK) or dact.shape != (h.shape[0], h.shape[1] // 2):
+        raise ValueError("h must be [M, 2I] with I a multiple of 128 and dact [M, I]")
     if h.stride(1) != 1 or h.stride(0) % 8 or h.data_ptr() % 16:
         h = h.contiguous()
     m, inter = dact.shape
     q = torch.empty((m, 2 * inter), dtype=FP8, device=h.device)
-    qt = _empty_codes_t(2 * inter, m, h.device)
+    mp = _rows_up(m)
+    qt = _empty_codes_t(2 * inter, mp, h.device)
     s_inv = torch.empty((2 * inter // BLOCK, m), dtype=torch.float32, device=h.device)
-    st_inv = torch.empty((m // BLOCK, 2 * inter), dtype=torch.float32, device=h.device)
-    _lib.call("hpfp8_swiglu_backward_quantize_1x128_and_128x1_t_bf16", _ptr(h), m, inter, h.stride(0) if m > 1 else 2 * inter,
-              _ptr(dact), _ptr(q), None, _ptr(s_inv), _ptr(qt), _ld(qt), None, _ptr(st_inv), _stream())
+    st_inv = torch.empty((mp // BLOCK, 2 * inter), dtype=torch.float32, device=h.device)
+    _lib.call("hpfp8_swiglu_backward_quantize_rows_128x1_t_bf16", _ptr(h), m, inter, h.stride(0) if m > 1 else 2 * inter,
+              _ptr(dact), _ptr(q), _ptr(s_inv), _ptr(qt), _ld(qt), _ptr(st_inv), _stream())
     return q, s_inv.t(), qt, st_inv.t()
 
 
@@ -343,27 +361,51 @@ def quantize_128x1_t(x: torch.Tensor, want_scale: bool = False, kmajor: bool = F
     return (qt, scale, scale_inv) if want_scale else (qt, scale_inv)
 
 
-def quantize_128x1_t_rows(x: torch.Tensor):
+def _rows_up(m: int) -> int:
+    return (m + BLOCK - 1) // BLOCK * BLOCK
+
+
+def quantize_128x1_t_rows(x: torch.Tensor, pow2: bool = False):
     """`quantize_128x1_t(..., kmajor=True)` of x[M, K] for any M > 0: the last group of a ragged M is filled up with
-    zero rows.  Only those last rows are copied for the padding; the whole groups are quantized where they lie.
+    zero rows (by the kernel, nothing is copied).
     Returns (codes_t[K, Mp], scale_inv_t[K, Mp/128]) with Mp = M rounded up to a multiple of 128."""
     x = _check_bf16(x, "x")
     if x.dim() != 2 or x.shape[1] % BLOCK or x.shape[0] == 0:
         raise ValueError("x must be [M, K] with M > 0 and K a multiple of 128")
+    if x.data_ptr() % 16:                  # (a view that starts between two vectors)
+        x = x.clone()
     m, k = x.shape
-    main = m // BLOCK * BLOCK
-    mp = main + (BLOCK if m > main else 0)
+    mp = _rows_up(m)
     qt = _empty_codes_t(k, mp, x.device)
     scale_inv = torch.empty((mp // BLOCK, k), dtype=torch.float32, device=x.device)
-    if main:
-        _lib.call("hpfp8_quantize_128x1_t_kmajor_bf16", _ptr(x), main, k, _ptr(qt), qt.stride(0), None, _ptr(scale_inv),
-                  _stream())
-    if m > main:
-        tail = torch.zeros((BLOCK, k), dtype=torch.bfloat16, device=x.device)
-        tail[:m - main] = x[main:]
-        _lib.call("hpfp8_quantize_128x1_t_kmajor_bf16", _ptr(tail), BLOCK, k, qt.data_ptr() + main, qt.stride(0), None,
-                  scale_inv.data_ptr() + main // BLOCK * k * 4, _stream())
+    _lib.call("hpfp8_quantize_rows_128x1_t_bf16", _ptr(x), m, k, None, None, _ptr(qt), _ld(qt), _ptr(scale_inv), int(pow2), None,
+              _stream())
     return qt, scale_inv.t()
+
+
+def quantize_1x128_and_128x1_t_rows(x: torch.Tensor, pow2: bool = False, column_sum: bool = False):
+    """`quantize_1x128_and_128x1_t` (k-block-major scales) of x[M, K] for any M > 0, from one read of x: the transposed form
+    is that of `quantize_128x1_t_rows`, codes_t[K, Mp] and scale_inv_t[K, Mp/128] with Mp = M rounded up to a multiple of
+    128; the other results have M rows."""
+    x = _check_bf16(x, "x")
+    if x.dim() != 2 or x.shape[1] % BLOCK or x.shape[0] == 0:
+        raise ValueError("x must be [M, K] with M > 0 and K a multiple of 128")
+    if x.data_ptr() % 16:                  # (a view that starts between two vectors)
+        x = x.clone()
+    m, k = x.shape
+    mp = _rows_up(m)
+    q = torch.empty((m, k), dtype=FP8, device=x.device)
+    qt = _empty_codes_t(k, mp, x.device)
+    s_inv = torch.empty((k // BLOCK, m), dtype=torch.float32, device=x.device)
+    st_inv = torch.empty((mp // BLOCK, k), dtype=torch.float32, device=x.device)
+    part = torch.empty((mp // BLOCK, k), dtype=torch.float32, device=x.device) if column_sum else None
+    _lib.call("hpfp8_quantize_rows_128x1_t_bf16", _ptr(x), m, k, _ptr(q), _ptr(s_inv), _ptr(qt), _ld(qt), _ptr(st_inv), int(pow2),
+              _ptr(part), _stream())
+    if not column_sum:
+        return q, s_inv.t(), qt, st_inv.t()
+    total = torch.empty((k,), dtype=torch.bfloat16, device=x.device)
+    _lib.call("hpfp8_column_sum_finish", _ptr(part), mp // BLOCK, k, _ptr(total), None, _stream())
+    return q, s_inv.t(), qt, st_inv.t(), total
 
 
 def quantize_1x128_and_128x1_t(x: torch.Tensor, kmajor: bool = True, pow2: bool = False, column_sum: bool = False):

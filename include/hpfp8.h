@@ -240,6 +240,20 @@ int hpfp8_swiglu_backward_quantize_1x128_and_128x1_t_bf16(const void* h, int64_t
                                                           void* q_t, int64_t ld_t, float* scale_t, float* scale_inv_t,
                                                           hpfp8_stream_t stream);
 
+/* The three dual quantizers above (k-block-major scales, scale_inv only) for any number of rows m.  The 128x1 groups run
+ * down the rows; the last one of a ragged m is filled up with zero rows: q_t [k, mb * 128] (row stride ld_t >= mb * 128)
+ * and scale_inv_t [mb, k] with mb = ceil(m / 128) are those of the source with zero rows appended, q [m, k] and scale_inv
+ * [k / 128, m] those of the source.  hpfp8_quantize_rows_128x1_t_bf16 without q (and scale_inv) makes the transposed form
+ * alone; colsum_partial (may be NULL) receives the column sums per 128-row block, [mb, k], for hpfp8_column_sum_finish. */
+int hpfp8_quantize_rows_128x1_t_bf16(const void* x, int64_t m, int64_t k, void* q, float* scale_inv, void* q_t, int64_t ld_t,
+                                     float* scale_inv_t, int pow2, float* colsum_partial, hpfp8_stream_t stream);
+int hpfp8_swiglu_quantize_rows_128x1_t_bf16(const void* h, int64_t rows, int64_t inter, int64_t ld_h, int fast, void* q,
+                                            float* scale_inv, void* q_t, int64_t ld_t, float* scale_inv_t, hpfp8_stream_t stream);
+int hpfp8_swiglu_backward_quantize_rows_128x1_t_bf16(const void* h, int64_t rows, int64_t inter, int64_t ld_h, const void* dact,
+                                                     void* q, float* scale_inv, void* q_t, int64_t ld_t, float* scale_inv_t,
+                                                     hpfp8_stream_t stream);
+
+
 /* Byte transpose of a code matrix: q[rows, cols] (row stride ld) -> q_t[cols, rows] (row stride ld_t);
  * rows, cols multiples of 128.  128x128 scaling blocks are symmetric, so this turns the codes of a
  * weight into its dgrad operand without requantizing, e.g. after FP8 shards were all-gathered: the

@@ -155,3 +155,59 @@ def test_swiglu_epilogue_is_the_same_with_both_tile_heights(gpu, m, inter, k, fa
 def test_grouped_tiles_are_exact_on_integer_inputs(gpu, counts, n, k):
     """Row counts around the 128-row tile of the grouped form, the tile it takes for few rows per expert."""
     test_grouped_gemm_with_few_rows_is_exact_on_integer_inputs(gpu, counts, n, k)
+
+
+@pytest.mark.parametrize("m", [1, 63, 64, 65, 127, 128, 129, 383])
+@pytest.mark.parametrize("k", [128, 640, 2048])
+@pytest.mark.parametrize("pow2", [False, True])
+def test_dual_quantizers_of_ragged_rows_equal_those_of_zero_padded_rows(gpu, m, k, pow2):
+    """Both row quads of a tile partly or wholly missing, one tile and several, both walking orders (row stride a multiple
+    of 4 KB or not): every result bit for bit that of the source with zero rows appended, whose own rows are unchanged."""
+    from hpfp8 import ops
+    u8 = torch.uint8
+    mp = (m + 127) // 128 * 128
+    x = torch.full((mp + 8, k), 77.0, dtype=torch.bfloat16, device=gpu)      # what lies behind the rows must not be read
+    x[:m] = randn_bf16((m, k), m, 1.0, 0.01, 50.0).to(gpu)
+    pad = torch.zeros((mp, k), dtype=torch.bfloat16, device=gpu)
+    pad[:m] = x[:m]
+    q, s, qt, st, cs = ops.quantize_1x128_and_128x1_t_rows(x[:m], pow2=pow2, column_sum=True)
+    w = ops.quantize_1x128_and_128x1_t(pad, pow2=pow2, column_sum=True)
+    assert torch.equal(q.view(u8), w[0][:m].view(u8)) and torch.equal(s, w[1][:m])
+    assert torch.equal(qt.view(u8), w[2].view(u8)) and torch.equal(st, w[3]) and torch.equal(cs, ops.column_sum(x[:m]))
+    for a, b in zip(ops.quantize_1x128_and_128x1_t_rows(x[:m], pow2=pow2), (q, s, qt, st)):
+        assert torch.equal(a.float(), b.float())
+    qt2, st2 = ops.quantize_128x1_t_rows(x[:m], pow2=pow2)
+    assert torch.equal(qt2.view(u8), qt.view(u8)) and torch.equal(st2, st)
+    if pow2:
+        return
+    inter = k
+    h = torch.full((mp + 8, 2 * inter), 77.0, dtype=torch.bfloat16, device=gpu)
+    h[:m] = randn_bf16((m, 2 * inter), m + 1).to(gpu)
+    dact = randn_bf16((m, inter), m + 2).to(gpu)
+    hp, dp = torch.zeros((mp, 2 * inter), dtype=torch.bfloat16, device=gpu), torch.zeros((mp, inter), dtype=torch.bfloat16, device=gpu)
+    hp[:m], dp[:m] = h[:m], dact
+    for got, want in [(ops.swiglu_quantize_1x128_and_128x1_t_rows(h[:m], fast=f), ops.swiglu_quantize_1x128_and_128x1_t(hp, fast=f))
+                      for f in (False, True)] + [(ops.swiglu_backward_quantize_1x128_and_128x1_t_rows(h[:m], dact),
+                                                  ops.swiglu_backward_quantize_1x128_and_128x1_t(hp, dp))]:
+        assert torch.equal(got[0].view(u8), want[0][:m].view(u8)) and torch.equal(got[1], want[1][:m])
+        assert torch.equal(got[2].view(u8), want[2].view(u8)) and torch.equal(got[3], want[3])
+
+
+@pytest.mark.parametrize("rows", [1, 100, 129])
+def test_mlp_block_of_ragged_tokens_is_that_of_its_two_linears(gpu, rows):
+    """The one-node training path of the MLP block at a ragged token count gives the bits of the linear and SwiGLU nodes
+    it replaces (which a frozen weight still selects)."""
+    import hpfp8
+    x0, gu0, dn0, go = (randn_bf16(s, i, sd).to(gpu) for i, (s, sd) in enumerate((((rows, 256), 1.0), ((512, 256), 0.05),
+                                                                               ((384, 256), 0.05), ((rows, 384), 0.1))))
+    x, gu, dn = (t.clone().requires_grad_(True) for t in (x0, gu0, dn0))
+    y = hpfp8.fp8_swiglu_mlp(x, gu, dn)
+    dx, dgu, ddn = torch.autograd.grad(y, (x, gu, dn), go)
+    x2, gu2 = (t.clone().requires_grad_(True) for t in (x0, gu0))
+    y2 = hpfp8.fp8_swiglu_mlp(x2, gu2, dn0)                      # frozen down projection
+    dx2, dgu2 = torch.autograd.grad(y2, (x2, gu2), go)
+    x3, dn3 = (t.clone().requires_grad_(True) for t in (x0, dn0))
+    y3 = hpfp8.fp8_swiglu_mlp(x3, gu0, dn3)                      # frozen gate/up projection
+    dx3, ddn3 = torch.autograd.grad(y3, (x3, dn3), go)
+    for a, b in ((y, y2), (y, y3), (dx, dx2), (dx, dx3), (dgu, dgu2), (ddn, ddn3)):
+        assert torch.equal(a, b)
