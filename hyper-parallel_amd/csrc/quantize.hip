@@ -155,14 +155,15 @@ constexpr int kFusedThreads = 1024;
 constexpr int kFusedMaxVec = 8;
 constexpr int64_t kFusedMaxElems = (int64_t)kFusedMaxBlocks * kFusedThreads * kFusedMaxVec * 8;   // 4 Mi elements
 
-// maximum over a workgroup of 1024 threads; part: 16 words of LDS
+// maximum over a workgroup of WAVES waves (a power of two, at most 16); part: 16 words of LDS
+template <int WAVES = 16>
 __device__ __forceinline__ uint32_t block_max_u32(uint32_t m, uint32_t* part) {
   m = row16_max_u32(m);
   m = umax(m, (uint32_t)__shfl_xor((int)m, 16));
   m = umax(m, (uint32_t)__shfl_xor((int)m, 32));
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
   __syncthreads();
-  m = row16_max_u32(part[threadIdx.x & 15]);
+  m = row16_max_u32(part[threadIdx.x & (WAVES - 1)]);
   __syncthreads();
   return m;                       // the same in every thread
 }
@@ -176,6 +177,44 @@ __device__ __forceinline__ uint32_t block_max_u32(uint32_t m, uint32_t* part) {
 // one to leave clears slots and count.  No word needs clearing before the launch, and the results go to their own
 // outputs (amax_out, scale_out, scale_inv_out).  (A workgroup whose wait ran out computes the maximum alone.)
 constexpr uint32_t kSlotValid = 0x80000000u;
+// The first wave of every workgroup: publish this workgroup's maximum m, wait for the grid's; s_amax is the maximum of
+// the slots seen, s_alone whether the wait ran out.  A barrier follows.
+__device__ __forceinline__ void slots_agree(uint32_t m, uint32_t* slots, uint32_t spin_limit, uint32_t* s_amax, uint32_t* s_alone) {
+  const uint32_t lane = threadIdx.x, grid = gridDim.x;            // lane l watches slot l
+  // (Relaxed accesses: a slot's value is all that is communicated -- nothing else is published with it, nothing
+  // else of another workgroup's is read after it -- so no cache needs writing back or invalidating; a release or
+  // an acquire at device scope does that to the XCD's whole L2.)
+  if (lane == 0) __hip_atomic_store(slots + blockIdx.x, kSlotValid | m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  uint32_t spins = 0, slot = 0;
+  bool all = false;
+  while (true) {
+    slot = lane < grid ? __hip_atomic_load(slots + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : kSlotValid;
+    all = __ballot((slot & kSlotValid) != 0) == ~0ull;
+    if (all || spins++ >= spin_limit) break;
+    __builtin_amdgcn_s_sleep(1);
+  }
+  uint32_t mx = (slot & kSlotValid) ? (slot & 0xFFFFu) : 0u;
+  mx = row16_max_u32(mx);
+  mx = umax(mx, (uint32_t)__shfl_xor((int)mx, 16));
+  mx = umax(mx, (uint32_t)__shfl_xor((int)mx, 32));
+  if (lane == 0) {
+    *s_amax = mx;
+    *s_alone = all ? 0u : 1u;
+  }
+}
+// The first wave, at a workgroup's end: it has read the slots for the last time (before a barrier: the values had
+// arrived, they were used); the last one to say so clears them for the next launch.
+__device__ __forceinline__ void slots_leave(uint32_t* slots, uint32_t* count) {
+  uint32_t last = 0;
+  if (threadIdx.x == 0)
+    last = __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u == gridDim.x ? 1u : 0u;
+  last = (uint32_t)__shfl((int)last, 0);
+  if (last) {
+    __hip_atomic_store(slots + threadIdx.x, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x == 0) __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
 template <int VEC, bool SYNC3 = false>
 __global__ __launch_bounds__(kFusedThreads) void quant_per_tensor_fused_kernel(const uint16_t* __restrict__ x, int64_t n,
                                                                      uint32_t* __restrict__ amax_word,
@@ -208,30 +247,7 @@ __global__ __launch_bounds__(kFusedThreads) void quant_per_tensor_fused_kernel(c
   m = block_max_u32(m, part);
   const uint32_t grid = gridDim.x;
   if (SYNC3) {
-    if (threadIdx.x < 64) {              // the first wave: lane l watches slot l
-      const uint32_t lane = threadIdx.x;
-      // (Relaxed accesses: a slot's value is all that is communicated -- nothing else is published with it, nothing
-      // else of another workgroup's is read after it -- so no cache needs writing back or invalidating; a release or
-      // an acquire at device scope does that to the XCD's whole L2.)
-      if (lane == 0) __hip_atomic_store(amax_word + blockIdx.x, kSlotValid | m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      uint32_t spins = 0, slot = 0;
-      bool all = false;
-      while (true) {
-        slot = lane < grid ? __hip_atomic_load(amax_word + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : kSlotValid;
-        all = __ballot((slot & kSlotValid) != 0) == ~0ull;
-        if (all || spins++ >= spin_limit) break;
-        __builtin_amdgcn_s_sleep(1);
-      }
-      uint32_t mx = (slot & kSlotValid) ? (slot & 0xFFFFu) : 0u;
-      mx = row16_max_u32(mx);
-      mx = umax(mx, (uint32_t)__shfl_xor((int)mx, 16));
-      mx = umax(mx, (uint32_t)__shfl_xor((int)mx, 32));
-      if (lane == 0) {
-        s_amax = mx;
-        s_alone = all ? 0u : 1u;
-        s_repair = 0u;
-      }
-    }
+    if (threadIdx.x < 64) slots_agree(m, amax_word, spin_limit, &s_amax, &s_alone);
   } else if (threadIdx.x == 0) {
     if ((m << 16) > __hip_atomic_load(amax_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
       __hip_atomic_fetch_max(amax_word, m << 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -270,18 +286,7 @@ __global__ __launch_bounds__(kFusedThreads) void quant_per_tensor_fused_kernel(c
       if (scale_out) *scale_out = scale;
       if (scale_inv_out) *scale_inv_out = scale_inv;
     }
-    // this workgroup has read the slots for the last time (before the barrier above: the values had arrived, they
-    // were used); the last one to say so clears them for the next launch
-    if (threadIdx.x < 64) {
-      uint32_t last = 0;
-      if (threadIdx.x == 0)
-        last = __hip_atomic_fetch_add(count_word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u == grid ? 1u : 0u;
-      last = (uint32_t)__shfl((int)last, 0);
-      if (last) {
-        __hip_atomic_store(amax_word + threadIdx.x, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (threadIdx.x == 0) __hip_atomic_store(count_word, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-    }
+    if (threadIdx.x < 64) slots_leave(amax_word, count_word);
     return;
   }
   if (threadIdx.x == 0 && (blockIdx.x == 0 || s_repair)) {
@@ -542,8 +547,9 @@ __device__ __forceinline__ void byte_transpose4(const uint32_t in[4], uint32_t o
 // Writes the thread's codes c[p] (8 codes of tile row tile_row(rq,p)) into the transposed LDS
 // tile (row = tile column, 128 B; 16-byte chunks XOR-swizzled by the column group), then the
 // workgroup streams the tile out as 128 rows of dst (row stride ld bytes) with 128-bit stores.
+// tid: the thread's number among the tile's 256.  Every thread of the workgroup comes here (a barrier); ok: there is a tile.
 __device__ __forceinline__ void store_tile_transposed(uint8_t* tile, const uint2 c[8], int cg, int rq,
-                                                      uint8_t* __restrict__ dst, int64_t ld) {
+                                                      uint8_t* __restrict__ dst, int64_t ld, int tid, bool ok) {
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const uint32_t lo[4] = {c[4 * h].x, c[4 * h + 1].x, c[4 * h + 2].x, c[4 * h + 3].x};
@@ -558,10 +564,11 @@ __device__ __forceinline__ void store_tile_transposed(uint8_t* tile, const uint2
       *reinterpret_cast<uint32_t*>(&tile[(cg * 8 + j) * 128 + pc * 16 + (rword & 3) * 4]) = wcol[j];
   }
   __syncthreads();
+  if (!ok) return;
 #pragma unroll
   for (int pass = 0; pass < 4; ++pass) {
-    const int col = pass * 32 + (threadIdx.x >> 3);
-    const int pc = threadIdx.x & 7;
+    const int col = pass * 32 + (tid >> 3);
+    const int pc = tid & 7;
     const int chunk = pc ^ ((col >> 3) & 7);
     uint4 o = *reinterpret_cast<const uint4*>(&tile[col * 128 + pc * 16]);
     nt_store16(reinterpret_cast<char*>(dst) + ((uint32_t)col * (uint32_t)ld + (uint32_t)chunk * 16u), o);
@@ -618,7 +625,7 @@ __global__ __launch_bounds__(256) void quant_128x128_kernel(const uint16_t* __re
     c[p] = cvt8<false>(v[p], s);
     nt_store8(qbase + ((uint32_t)tile_row(rq, p) * ucols + (uint32_t)cg * 8u), c[p]);
   }
-  if (WITH_T) store_tile_transposed(tile, c, cg, rq, qt + (int64_t)bc * 128 * ld_t + br * 128, ld_t);
+  if (WITH_T) store_tile_transposed(tile, c, cg, rq, qt + (int64_t)bc * 128 * ld_t + br * 128, ld_t, threadIdx.x, true);
 }
 
 // Without the transposed copy and for a large matrix with an even number of tile columns: two neighbouring 128x128
@@ -704,7 +711,7 @@ __device__ __forceinline__ void wave_column_sums(float cs[8], int cg, int wave, 
     cs[i] += __shfl_xor(cs[i], 16);
     cs[i] += __shfl_xor(cs[i], 32);
   }
-  if ((threadIdx.x & 63) < 16) {
+  if ((threadIdx.x & 63) < 16) {      // (wave: 0..3 among the tile's four)
     *reinterpret_cast<float4*>(&s_cs[wave][cg * 8]) = make_float4(cs[0], cs[1], cs[2], cs[3]);
     *reinterpret_cast<float4*>(&s_cs[wave][cg * 8 + 4]) = make_float4(cs[4], cs[5], cs[6], cs[7]);
   }
@@ -908,10 +915,92 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void q
     c[p].y = hi;
   }
   if (COLSUM) wave_column_sums(cs, cg, wave, s_cs);
-  store_tile_transposed(tile, c, cg, rq, qt + (int64_t)tc * 128 * ld_t + tr * 128, ld_t);
+  store_tile_transposed(tile, c, cg, rq, qt + (int64_t)tc * 128 * ld_t + tr * 128, ld_t, threadIdx.x, true);
   // (the barrier inside store_tile_transposed has also made every wave's column sums visible)
   if (COLSUM && threadIdx.x < 128)
     colsum_part[(int64_t)tr * k + tc * 128 + threadIdx.x] = column_sum_of_tile(s_cs, threadIdx.x);
+}
+
+// ---------------------------------------------------------------------------------------------
+// per tensor, both operand forms: codes [m, k] and transposed codes [k, m rounded up to 128] from one read of x
+// ---------------------------------------------------------------------------------------------
+// With one scale per tensor the transposed codes are the codes transposed; made in the cast they cost no second pass
+// over the codes and no launch.  256 threads hold one 128 x 128 tile of x in registers, as in quant_128x1_t_kernel (a
+// ragged m: rows past it count as zeros, in the transposed form only).  COLSUM: the tile's column sums as there.
+//   TILES > 0 : a workgroup has TILES tiles and the grid, at most 64 workgroups, agrees on the maximum through `sync`
+//               (slots_agree) before it casts what it still holds: one launch, for tensors of up to 256 tiles.
+//   TILES == 0: one tile per workgroup, the maximum is at `amax`.
+// Measured: x[2048, 1024] 11.1 us where quantizer and byte transpose took 8.1 + 3.1 and two launches (bound by latency: load,
+// agree, store); with the launches, x[4096, 7168] 57 us where amax, cast and transpose took 62, x[4096, 16384] 88 and 98.
+template <int TILES, bool COLSUM>
+__global__ __launch_bounds__(TILES ? 256 * TILES : 256) void quant_per_tensor_tiles_kernel(
+    const uint16_t* __restrict__ x, int m, int k, const float* __restrict__ amax, uint32_t* __restrict__ sync, uint32_t spin_limit,
+    uint8_t* __restrict__ q, uint8_t* __restrict__ qt, int64_t ld_t, float* __restrict__ scale_out, float* __restrict__ scale_inv_out,
+    float* __restrict__ colsum_part, int along_k) {
+  constexpr int T = TILES ? TILES : 1;
+  const int tid = threadIdx.x & 255, group = threadIdx.x >> 8;
+  const int cg = tid & 15, rq = tid >> 4, wave = tid >> 6;
+  const int mb = (m + 127) >> 7, kb = k >> 7;
+  __shared__ uint32_t part[16];
+  __shared__ uint32_t s_amax, s_alone;
+  __shared__ __attribute__((aligned(16))) float s_cs[COLSUM ? T : 1][COLSUM ? 4 : 1][128];
+  __shared__ __attribute__((aligned(16))) uint8_t tile[T][128 * 128];
+  int tr, tc;
+  bool ok = true;
+  if (TILES) {                                           // tiles along a row of x follow each other
+    const int t = blockIdx.x * T + group;
+    ok = t < mb * kb;
+    tr = ok ? t / kb : 0;
+    tc = ok ? t % kb : 0;
+  } else {
+    tr = along_k ? blockIdx.y : blockIdx.x;
+    tc = along_k ? blockIdx.x : blockIdx.y;
+  }
+  const int valid = !ok ? 0 : (m - tr * 128 < 128 ? m - tr * 128 : 128);
+  const char* sbase = reinterpret_cast<const char*>(x + (int64_t)tr * 128 * k + tc * 128);
+  uint4 v[8];
+#pragma unroll
+  for (int p = 0; p < 8; ++p) {
+    const int row = tile_row(rq, p);
+    v[p] = row < valid ? nt_load16(sbase + ((uint32_t)row * (uint32_t)k + (uint32_t)cg * 8u) * 2u) : make_uint4(0, 0, 0, 0);
+  }
+  float scale, scale_inv;
+  if (TILES) {
+    uint32_t mx = 0;
+#pragma unroll
+    for (int p = 0; p < 8; ++p) mx = umax(mx, mag8(v[p]));
+    mx = block_max_u32<4 * T>(mx, part);
+    if (threadIdx.x < 64) slots_agree(mx, sync, spin_limit, &s_amax, &s_alone);
+    __syncthreads();
+    uint32_t amax16 = s_amax;
+    if (s_alone) {                // (uniform over the workgroup) the wait ran out: the whole tensor's maximum, alone
+      const uint4* xv = reinterpret_cast<const uint4*>(x);
+      const int64_t nvec = (int64_t)m * k >> 3;
+      for (int64_t i = threadIdx.x; i < nvec; i += 256 * T) mx = umax(mx, mag8(xv[i]));
+      amax16 = block_max_u32<4 * T>(mx, part);
+    }
+    scales_from_amax(__uint_as_float(amax16 << 16), scale, scale_inv);
+  } else {
+    scales_from_amax(*amax, scale, scale_inv);
+  }
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
+    if (scale_out) *scale_out = scale;
+    *scale_inv_out = scale_inv;
+  }
+  char* qbase = reinterpret_cast<char*>(q + (int64_t)tr * 128 * k + tc * 128);
+  uint2 c[8];
+#pragma unroll
+  for (int p = 0; p < 8; ++p) {
+    const int row = tile_row(rq, p);
+    c[p] = cvt8<true>(v[p], scale);
+    if (row < valid) nt_store8(qbase + ((uint32_t)row * (uint32_t)k + (uint32_t)cg * 8u), c[p]);
+    else c[p] = make_uint2(0, 0);                        // (zeros, whatever the scale is)
+  }
+  if (COLSUM) tile_column_sums(v, cg, wave, s_cs[COLSUM ? group : 0]);
+  store_tile_transposed(tile[group], c, cg, rq, qt + (int64_t)tc * 128 * ld_t + (int64_t)tr * 128, ld_t, tid, ok);
+  // (the barrier inside store_tile_transposed has also made every wave's column sums visible)
+  if (COLSUM && ok && tid < 128) colsum_part[(int64_t)tr * k + tc * 128 + tid] = column_sum_of_tile(s_cs[COLSUM ? group : 0], tid);
+  if (TILES && threadIdx.x < 64) slots_leave(sync, sync + 64);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1008,7 +1097,7 @@ __global__ __launch_bounds__(256) void transpose_codes_kernel(const uint8_t* __r
         reinterpret_cast<const u32x2*>(src + ((uint32_t)tile_row(rq, p) * (uint32_t)ld + (uint32_t)cg * 8u)));
     c[p] = make_uint2(t.x, t.y);
   }
-  store_tile_transposed(tile, c, cg, rq, qt + (int64_t)bc * 128 * ld_t + br * 128, ld_t);
+  store_tile_transposed(tile, c, cg, rq, qt + (int64_t)bc * 128 * ld_t + br * 128, ld_t, threadIdx.x, true);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1573,6 +1662,52 @@ int hpfp8_swiglu_backward_quantize_rows_128x1_t_bf16(const void* h, int64_t rows
   quant_128x1_t_kernel<true, true, 3, kRaggedRows><<<grid, 256, 0, (hipStream_t)stream>>>(
       (const uint16_t*)h, ld_h, (int)rows, (int)(2 * inter), (uint8_t*)q_t, ld_t, nullptr, scale_inv_t, (uint8_t*)q, nullptr,
       scale_inv, 0, ak, nullptr, 0, 0, (const uint16_t*)dact);
+  return check_launch(what);
+}
+
+int hpfp8_quantize_per_tensor_t_bf16(const void* x, int64_t m, int64_t k, void* q, void* q_t, int64_t ld_t, float* amax,
+                                     float* scale, float* scale_inv, uint32_t* sync, float* colsum_partial, hpfp8_stream_t stream) {
+  const char* what = "quantize_per_tensor_t";
+  HPFP8_REQUIRE(m > 0 && k > 0, HPFP8_ERR_SHAPE, "%s: empty or negative shape", what);
+  int rc = check_rows(what, m, k, x, k, q, scale_inv, q_t, ld_t, scale_inv);
+  if (rc <= 0) return rc;
+  HPFP8_REQUIRE(q, HPFP8_ERR_ARG, "%s: null buffer", what);
+  const int64_t mb = (m + kBlock - 1) / kBlock, tiles = mb * (k / kBlock);
+  hipStream_t s = (hipStream_t)stream;
+  const uint16_t* xs = (const uint16_t*)x;
+  uint8_t *q8 = (uint8_t*)q, *qt8 = (uint8_t*)q_t;
+  // (a launch of 64 workgroups at most, one per slot; four tiles of 16 KB of LDS each are what 1024 threads hold)
+  if (sync && tiles <= 4 * kFusedMaxBlocks) {
+    HPFP8_REQUIRE((reinterpret_cast<uintptr_t>(sync) & 255u) == 0, HPFP8_ERR_ALIGN, "%s: sync must be 256-byte aligned", what);
+    const uint32_t spin = g_spin_limit.load(std::memory_order_relaxed);
+    const int per = tiles <= kFusedMaxBlocks ? 1 : (tiles <= 2 * kFusedMaxBlocks ? 2 : 4);
+    const unsigned grid = (unsigned)((tiles + per - 1) / per);
+#define HPFP8_PT(TILES, COLSUM) \
+  quant_per_tensor_tiles_kernel<TILES, COLSUM><<<grid, 256 * TILES, 0, s>>>(xs, (int)m, (int)k, nullptr, sync, spin, q8, qt8, ld_t, scale, \
+                                                                           scale_inv, colsum_partial, 0)
+    if (colsum_partial) {
+      if (per == 1) HPFP8_PT(1, true);
+      else if (per == 2) HPFP8_PT(2, true);
+      else HPFP8_PT(4, true);
+    } else {
+      if (per == 1) HPFP8_PT(1, false);
+      else if (per == 2) HPFP8_PT(2, false);
+      else HPFP8_PT(4, false);
+    }
+#undef HPFP8_PT
+    return check_launch(what);
+  }
+  HPFP8_REQUIRE(amax, HPFP8_ERR_ARG, "%s: null amax word", what);
+  rc = hpfp8_amax_bf16(x, m * k, amax, stream);
+  if (rc != HPFP8_OK) return rc;
+  int ak = 0;
+  const dim3 grid = transpose_grid(mb, k / kBlock, k * 2, 2, ak);
+  if (colsum_partial)
+    quant_per_tensor_tiles_kernel<0, true><<<grid, 256, 0, s>>>(xs, (int)m, (int)k, amax, nullptr, 0, q8, qt8, ld_t, scale, scale_inv,
+                                                                colsum_partial, ak);
+  else
+    quant_per_tensor_tiles_kernel<0, false><<<grid, 256, 0, s>>>(xs, (int)m, (int)k, amax, nullptr, 0, q8, qt8, ld_t, scale, scale_inv,
+                                                                 nullptr, ak);
   return check_launch(what);
 }
 

@@ -39,6 +39,7 @@ SIGNATURES = {
     "hpfp8_bucket_pack_quantize_bf16": [_vp, _vp, _vp, ctypes.c_int, ctypes.c_int, _i64, _vp, _vp, _vp, _vp],
     "hpfp8_bucket_unpack_dequantize_bf16": [_vp, _vp, _vp, ctypes.c_int, _i64, _vp, _vp, ctypes.c_float, _vp],
     "hpfp8_quantize_1x128_and_128x1_t_bf16": [_vp, _i64, _i64, ctypes.c_int, _vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp],
+    "hpfp8_quantize_per_tensor_t_bf16": [_vp, _i64, _i64, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp],
     "hpfp8_quantize_rows_128x1_t_bf16": [_vp, _i64, _i64, _vp, _vp, _vp, _i64, _vp, _int, _vp, _vp],
     "hpfp8_swiglu_quantize_rows_128x1_t_bf16": [_vp, _i64, _i64, _i64, _int, _vp, _vp, _vp, _i64, _vp, _vp],
     "hpfp8_swiglu_backward_quantize_rows_128x1_t_bf16": [_vp, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _i64, _vp, _vp],

@@ -80,13 +80,6 @@ def _flatten(x: torch.Tensor):
     return x.reshape(-1, x.shape[-1])
 
 
-def _pad_rows(t: torch.Tensor) -> torch.Tensor:
-    """t[M, C] with zero rows appended up to the next multiple of 128: tokens that contribute nothing to a
-    weight gradient, so that the contraction over them is whole k-blocks."""
-    pad = -t.shape[0] % ops.BLOCK
-    return torch.nn.functional.pad(t, (0, 0, 0, pad)) if pad else t
-
-
 def _both_forms(t: torch.Tensor, pow2: bool = False, column_sum: bool = False):
     """The 1x128 and the transposed 128x1 form of t[M, C] from one read of it, for any M > 0 (k-block-major scales)."""
     form = ops.quantize_1x128_and_128x1_t_rows if t.shape[0] % ops.BLOCK else ops.quantize_1x128_and_128x1_t
@@ -191,26 +184,30 @@ class _Fp8LinearBlockwise(torch.autograd.Function):
 
 class _Fp8LinearPerTensor(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, x, weight, bias, wq=None, sw=None):
+    def forward(ctx, x, weight, bias, wq=None, sw=None, grad_mode=True):
         x2 = _flatten(x)
-        xq, _, sx = ops.quantize_per_tensor(x2)
-        if wq is None:                          # no prequantized form of the weight was passed in
-            wq, _, sw = ops.quantize_per_tensor(weight)
-        y = ops.gemm_per_tensor(xq, sx, wq, sw, bias=bias)
-        # With one scale per tensor the codes of a transposed tensor are the transposed codes, so backward
-        # needs no second quantization of x and W: it keeps the codes (1 byte per element) where their
-        # shapes allow the byte transpose, and the bf16 tensors otherwise.
         m = x2.shape[0]
-        can_t = m % ops.BLOCK == 0 and m > 0
-        ctx.codes_saved = can_t
-        if can_t:
-            ctx.save_for_backward(xq if weight.requires_grad else None, sx, wq if x.requires_grad else None, sw)
+        # (grad_mode: as in the blockwise form)
+        need_dx, need_dw = grad_mode and x.requires_grad, grad_mode and weight.requires_grad
+        # With one scale per tensor the codes of a transposed tensor are the transposed codes: what a gradient will
+        # need transposed is written beside the codes in the same pass, and kept (1 byte per element).
+        xt = wqt = None
+        if need_dw and m > 0:
+            xq, sx, xt = ops.quantize_per_tensor_t(x2)
         else:
-            ctx.save_for_backward(x2, weight)
+            xq, _, sx = ops.quantize_per_tensor(x2)
+        if wq is None:                          # no prequantized form of the weight was passed in
+            if need_dx and m > 0:
+                wq, sw, wqt = ops.quantize_per_tensor_t(weight)
+            else:
+                wq, _, sw = ops.quantize_per_tensor(weight)
+        y = ops.gemm_per_tensor(xq, sx, wq, sw, bias=bias)
+        ctx.w_transposed = wqt is not None
+        ctx.save_for_backward(xt, sx, (wqt if wqt is not None else wq) if need_dx else None, sw)
         ctx.x_shape = x.shape
         ctx.w_shape = weight.shape
         ctx.has_bias = bias is not None
-        ctx.need = (x.requires_grad, weight.requires_grad)
+        ctx.need = (need_dx, need_dw)
         return y.reshape(x.shape[:-1] + (weight.shape[0],))
 
     @staticmethod
@@ -221,28 +218,23 @@ class _Fp8LinearPerTensor(torch.autograd.Function):
             go = go.to(torch.bfloat16)
         go = go.contiguous()
         if go.shape[0] == 0:
-            return _empty_batch_grads(ctx, go) + (None, None)
-        dx = dw = db = None
-        if ctx.codes_saved:
-            xq, sx, wq, sw = ctx.saved_tensors
-            goq, _, sgo = ops.quantize_per_tensor(go)
-            if need_dx:
-                dx = ops.gemm_per_tensor(goq, sgo, ops.transpose_codes(wq), sw).reshape(ctx.x_shape)
-            if need_dw:
-                dw = ops.gemm_per_tensor(ops.transpose_codes(goq), sgo, ops.transpose_codes(xq), sx)
+            return _empty_batch_grads(ctx, go) + (None, None, None)
+        xt, sx, w, sw = ctx.saved_tensors
+        dx = dw = db = goq = sgo = got = None
+        if need_dw and ctx.has_bias:
+            goq, sgo, got, db = ops.quantize_per_tensor_t(go, column_sum=True)
+        elif need_dw:
+            goq, sgo, got = ops.quantize_per_tensor_t(go)
         else:
-            x2, weight = ctx.saved_tensors
             if need_dx:
                 goq, _, sgo = ops.quantize_per_tensor(go)
-                wtq, _, swt = ops.quantize_per_tensor(weight.t().contiguous())
-                dx = ops.gemm_per_tensor(goq, sgo, wtq, swt).reshape(ctx.x_shape)
-            if need_dw:
-                gotq, _, sgot = ops.quantize_per_tensor(_pad_rows(go).t().contiguous())
-                xtq, _, sxt = ops.quantize_per_tensor(_pad_rows(x2).t().contiguous())
-                dw = ops.gemm_per_tensor(gotq, sgot, xtq, sxt)
-        if ctx.has_bias:
-            db = ops.column_sum(go)
-        return dx, dw, db, None, None
+            if ctx.has_bias:
+                db = ops.column_sum(go)
+        if need_dx:
+            dx = ops.gemm_per_tensor(goq, sgo, w if ctx.w_transposed else ops.transpose_codes(w), sw).reshape(ctx.x_shape)
+        if need_dw:
+            dw = ops.gemm_per_tensor(got, sgo, xt, sx)     # (contraction over the tokens, filled up with zero codes)
+        return dx, dw, db, None, None, None
 
 
 def fp8_linear(input: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, *,
@@ -292,7 +284,7 @@ def fp8_linear(input: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.T
         if recipe == "per_tensor":
             if weight_fp8.scale_inv.numel() != 1:
                 raise ValueError("weight_fp8 was not quantized with one scale per tensor")
-            return _Fp8LinearPerTensor.apply(input, weight, bias, weight_fp8.codes, weight_fp8.scale_inv)
+            return _Fp8LinearPerTensor.apply(input, weight, bias, weight_fp8.codes, weight_fp8.scale_inv, torch.is_grad_enabled())
         if weight_fp8.scale_inv.dim() != 2:
             raise ValueError("weight_fp8 was quantized with one scale per tensor")
         if bool(weight_fp8.pow2) != pow2:
@@ -302,7 +294,7 @@ def fp8_linear(input: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.T
     if recipe != "per_tensor":
         return _Fp8LinearBlockwise.apply(input, weight, bias, None, None, None, apply_grad_on_fp32_main_grad, pow2,
                                          torch.is_grad_enabled())
-    return _Fp8LinearPerTensor.apply(input, weight, bias)
+    return _Fp8LinearPerTensor.apply(input, weight, bias, None, None, torch.is_grad_enabled())
 
 
 _FP8_LINEAR_DEFAULTS = dict(recipe="blockwise", weight_fp8=None, apply_grad_on_fp32_main_grad=False)

@@ -159,6 +159,35 @@ def quantize_per_tensor(x: torch.Tensor, amax_in: Optional[torch.Tensor] = None
     return q, scale, scale_inv
 
 
+_ONE_PASS_TILES = 256         # 128 x 128 tiles the one-launch form of quantize_per_tensor_t holds
+
+
+def quantize_per_tensor_t(x: torch.Tensor, column_sum: bool = False):
+    """`quantize_per_tensor` of x[M, K] (K a multiple of 128, any M > 0) with the transposed codes from the same read:
+    (codes[M, K], scale_inv, codes_t[K, Mp]), Mp = M rounded up to a multiple of 128, the codes of the rows past M zero.
+    With ``column_sum`` a fourth result, the bits of `column_sum(x)`."""
+    x = _check_bf16(x, "x")
+    if x.dim() != 2 or x.shape[1] % BLOCK or x.numel() == 0:
+        raise ValueError("x must be [M, K] with M > 0 and K a positive multiple of 128")
+    if x.data_ptr() % 16:                  # (a view that starts between two vectors)
+        x = x.clone()
+    m, k = x.shape
+    mp = _rows_up(m)
+    q = torch.empty((m, k), dtype=FP8, device=x.device)
+    qt = _empty_codes_t(k, mp, x.device)
+    scale_inv = torch.empty((), dtype=torch.float32, device=x.device)
+    part = torch.empty((mp // BLOCK, k), dtype=torch.float32, device=x.device) if column_sum else None
+    sync = _sync_words(x.device) if (mp // BLOCK) * (k // BLOCK) <= _ONE_PASS_TILES else None
+    am = torch.empty((), dtype=torch.float32, device=x.device) if sync is None else None
+    _lib.call("hpfp8_quantize_per_tensor_t_bf16", _ptr(x), m, k, _ptr(q), _ptr(qt), _ld(qt), _ptr(am), None, _ptr(scale_inv),
+              _ptr(sync), _ptr(part), _stream())
+    if not column_sum:
+        return q, scale_inv, qt
+    total = torch.empty((k,), dtype=torch.bfloat16, device=x.device)
+    _lib.call("hpfp8_column_sum_finish", _ptr(part), mp // BLOCK, k, _ptr(total), None, _stream())
+    return q, scale_inv, qt, total
+
+
 def quantize_1x128(x: torch.Tensor, want_scale: bool = False, kmajor: bool = False, pow2: bool = False):
     """x[..., C] -> (codes, scale_inv[..., C/128]) (plus scale when ``want_scale``).
 

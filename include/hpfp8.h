@@ -240,6 +240,14 @@ int hpfp8_swiglu_backward_quantize_1x128_and_128x1_t_bf16(const void* h, int64_t
                                                           void* q_t, int64_t ld_t, float* scale_t, float* scale_inv_t,
                                                           hpfp8_stream_t stream);
 
+/* Per tensor, both operand forms of x[m, k] (k a multiple of 128, any m > 0) from one read of it: q [m, k] and q_t
+ * [k, ceil(m / 128) * 128] (row stride ld_t), the codes of hpfp8_quantize_per_tensor_bf16 and their transpose with zero
+ * codes for the rows past m; scale may be NULL.  One launch when the matrix has at most 256 tiles of 128 x 128 and `sync`
+ * is given (512 bytes, 256-byte aligned, the rules of hpfp8_quantize_per_tensor_sync_bf16); otherwise through the word at
+ * `amax`.  colsum_partial (may be NULL): the column sums per 128-row block for hpfp8_column_sum_finish. */
+int hpfp8_quantize_per_tensor_t_bf16(const void* x, int64_t m, int64_t k, void* q, void* q_t, int64_t ld_t, float* amax,
+                                     float* scale, float* scale_inv, uint32_t* sync, float* colsum_partial, hpfp8_stream_t stream);
+
 /* The three dual quantizers above (k-block-major scales, scale_inv only) for any number of rows m.  The 128x1 groups run
  * down the rows; the last one of a ragged m is filled up with zero rows: q_t [k, mb * 128] (row stride ld_t >= mb * 128)
  * and scale_inv_t [mb, k] with mb = ceil(m / 128) are those of the source with zero rows appended, q [m, k] and scale_inv

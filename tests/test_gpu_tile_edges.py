@@ -211,3 +211,33 @@ def test_mlp_block_of_ragged_tokens_is_that_of_its_two_linears(gpu, rows):
     dx3, ddn3 = torch.autograd.grad(y3, (x3, dn3), go)
     for a, b in ((y, y2), (y, y3), (dx, dx2), (dx, dx3), (dgu, dgu2), (ddn, ddn3)):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("m,k", [(1, 128), (127, 128), (129, 384), (1024, 1024), (1000, 2048), (2048, 1024), (2049, 2048), (4096, 1024),
+                                 (4097, 1024), (300, 16384)])
+@pytest.mark.parametrize("one_launch,polls", [(True, None), (True, 0), (False, None)])
+def test_per_tensor_codes_with_their_transpose(gpu, m, k, one_launch, polls, monkeypatch):
+    """One, two and four tiles per workgroup with whole and partly empty last workgroups, the first sizes past 256 tiles,
+    ragged rows, workgroups that stop waiting for the others and find the maximum alone (no polls), and the form without a
+    block to agree through: the codes and scale of the plain quantizer, their transpose, the column sums; twice in a row,
+    since the block must have been left as it was found."""
+    from hpfp8 import _lib, ops
+    x = torch.full((m + 8, k), 1e30, dtype=torch.bfloat16, device=gpu)       # what lies behind the rows must not be read
+    x[:m] = randn_bf16((m, k), m, 1.0, 0.001, 50.0).to(gpu)
+    x = x[:m]
+    want, _, si = ops.quantize_per_tensor(x)
+    mp = (m + 127) // 128 * 128
+    if not one_launch:
+        monkeypatch.setattr(ops, "_sync_words", lambda device: None)
+    if polls is not None:
+        _lib.load().hpfp8_debug_set_spin_limit(polls)
+    try:
+        for column_sum in (False, True):
+            out = ops.quantize_per_tensor_t(x, column_sum=column_sum)
+            assert torch.equal(out[0].view(torch.uint8), want.view(torch.uint8)) and torch.equal(out[1], si)
+            t = out[2].view(torch.uint8)
+            assert tuple(t.shape) == (k, mp) and torch.equal(t[:, :m].t(), want.view(torch.uint8)) and not t[:, m:].any()
+            if column_sum:
+                assert torch.equal(out[3], ops.column_sum(x))
+    finally:
+        _lib.load().hpfp8_debug_set_spin_limit(256)
