@@ -119,7 +119,7 @@ def load():
 
 
 def call(name: str, *args) -> None:
-    lib = load()
+    lib = _lib if _lib is not None else load()
     rc = getattr(lib, name)(*args)
     if rc != 0:
         msg = lib.hpfp8_last_error().decode("utf-8", "replace")

@@ -67,8 +67,9 @@ class Fp8GradBucket:
         if len(tensors) != len(self.numels):
             raise ValueError(f"expected {len(self.numels)} tensors, got {len(tensors)}")
         ptrs = (ctypes.c_void_p * max(len(tensors), 1))()
+        current = torch.cuda.current_device()
         for e, (t, n) in enumerate(zip(tensors, per_tensor_elems)):
-            if not t.is_cuda or t.device.index != torch.cuda.current_device() or t.dtype != torch.bfloat16 or not t.is_contiguous():
+            if not t.is_cuda or t.get_device() != current or t.dtype != torch.bfloat16 or not t.is_contiguous():
                 raise TypeError(f"gradient {e} must be a contiguous bfloat16 tensor on the current GPU")
             if t.numel() != n:
                 raise ValueError(f"gradient {e} has {t.numel()} elements, expected {n}")
@@ -84,7 +85,7 @@ class Fp8GradBucket:
         scale_inv = torch.empty((self.shard_size, self.row_elems // ops.BLOCK), dtype=torch.float32, device=dev)
         _lib.call("hpfp8_bucket_pack_quantize_bf16", ptrs, self._numels_c, self._offsets_c, len(self.numels),
                   self.shard_size, self.row_elems, q.data_ptr(), None, scale_inv.data_ptr(),
-                  torch.cuda.current_stream().cuda_stream)
+                  ops._stream())
         return q, scale_inv
 
     def unpack(self, codes_row: torch.Tensor, scale_inv_row: torch.Tensor, outs: Sequence[torch.Tensor]):
@@ -100,5 +101,5 @@ class Fp8GradBucket:
         ptrs = self._ptr_table(outs, self.numels)
         _lib.call("hpfp8_bucket_unpack_dequantize_bf16", ptrs, self._numels_c, self._offsets_c, len(self.numels),
                   self.row_elems, codes_row.data_ptr(), scale_inv_row.data_ptr(), ctypes.c_float(self.grad_scale),
-                  torch.cuda.current_stream().cuda_stream)
+                  ops._stream())
         return list(outs)
