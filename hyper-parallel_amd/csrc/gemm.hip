@@ -1143,8 +1143,8 @@ static bool use_small_kernel(int64_t M, int64_t N) {
 }
 
 // Few rows of a (decode): bound by reading b once, which the tile kernels do not reach (gemm_skinny.hip; 8 rows of
-// [7168, 16384]: 60 us with 64 x 128 tiles, 22 us; 64 rows: 64 and 36 us; 37 rows of [36864, 7168]: 81 us with 256 x 256
-// tiles, 63 us).  Hands the problem over if it is one; otherwise false.
+// [7168, 16384]: 60 us with 64 x 128 tiles, 20 us; 64 rows: 64 and 31 us; 37 rows of [36864, 7168]: 81 us with 256 x 256
+// tiles, 57 us).  Hands the problem over if it is one; otherwise false.
 static bool try_skinny(const GemmParams& p, bool tensor, int out_type, hipStream_t stream, int& rc) {
   if (p.M > kSkinnyMaxRows || p.K < kSkinnyMinK || p.accumulate || g_small_gemm_mode.load(std::memory_order_relaxed) != 0) return false;
   const int cus = persistent_grid((int64_t)1 << 40);

@@ -23,8 +23,8 @@ struct SkinnyParams {
 constexpr int kSkinnyMaxRows = 64;
 constexpr int kSkinnyMaxCols = 1024;      // columns per compute unit (the bias of a workgroup's columns is kept in LDS)
 constexpr int kSkinnyMinK = 2048;         // shorter contractions leave too few k-blocks per wave: the tile kernels
-constexpr int kSkinnyWide = 128;          // from this many columns per compute unit on, units are 64 columns wide (up to 32 rows;
-                                          // 32 rows of [36864, 7168]: 57 us with 32 columns, 54.5 with 64)
+constexpr int kSkinnyWide = 128;          // from this many columns per compute unit on, units are 64 columns wide, which reads a half as often
+                                          // (32 / 37 / 64 rows of [36864, 7168]: 55.1 / 59.1 / 74.4 us with 32 columns, 52.9 / 56.5 / 65.4)
 
 int launch_skinny(const SkinnyParams& p, bool tensor, bool out_f32, int cus, hipStream_t stream);
 

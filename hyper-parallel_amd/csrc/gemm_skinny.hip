@@ -15,9 +15,10 @@
 //   * a wave begins its quarter at a k-block that depends on the workgroup: begun at the same one, 256 workgroups whose
 //     units start a multiple of 16 KB apart ask the same memory channels at the same time (8 rows of [7168, 16384]: 28
 //     us, 22 us with it).
-// Measured (weights rotating beyond the Infinity Cache): 8 rows of [7168, 16384] 60 -> 22 us (5.3 TB/s), of [36864, 7168]
-// 80 -> 47 us (5.6 TB/s); from about 40 rows on the vector-memory path of a compute unit, which carries a's rows once per
-// 32 columns, is the bound (64 rows of [7168, 16384]: 64 -> 36 us).
+//   * a is moved in pieces of 8 rows, so that 37 rows cost 40 and not 48 (27.3 -> 26.4 us on [7168, 16384]).
+// Measured (weights rotating beyond the Infinity Cache): 8 rows of [7168, 16384] 60 -> 20 us (5.8 TB/s), of [36864, 7168]
+// 80 -> 47 us (5.6 TB/s); from about 24 rows on the vector-memory path of a compute unit, which carries a's rows once per
+// unit, is the bound (64 rows of [7168, 16384]: 64 -> 31 us, of [36864, 7168] 65 us).
 // Transfers past the end go through an empty resource: they fetch nothing, write zeros and keep the number of
 // operations in flight constant, which is what the waits count.  (A result store in between adds to the count, which
 // makes a wait stricter, never looser.)
@@ -30,17 +31,23 @@ namespace hpfp8 {
 
 constexpr int kSkinnyWaves = 4;
 constexpr int kSkinnyThreads = kSkinnyWaves * 64;
-// LDS of one workgroup: the four rings, the partial sums of one unit, the bias of the workgroup's columns.
-// U k-blocks per ring: what 160 KB have room for, and at most 6 (more in flight gains nothing).
+// ME: 8-row pieces of a, one transfer each (M <= 8 ME); NF: 16-column fragments of a unit.
+// LDS of one workgroup: the four rings, the partial sums of the fragments added up at a time, the bias of the workgroup's
+// columns.  U k-blocks per ring: what 160 KB have room for, and at most 6 (more in flight gains nothing).
 constexpr int kSkinnyBiasBytes = kSkinnyMaxCols * 2;
-constexpr int skinny_stage_bytes(int mf, int nf) { return (nf + mf) * 2048 + 256; }
-constexpr int skinny_sum_bytes(int mf, int nf) { return kSkinnyWaves * nf * mf * 1024; }
-constexpr int skinny_stages(int mf, int nf) {
-  const int fit = (160 * 1024 - skinny_sum_bytes(mf, nf) - kSkinnyBiasBytes) / (kSkinnyWaves * skinny_stage_bytes(mf, nf));
+constexpr int skinny_frags(int me, int nf) { return nf * ((me + 1) / 2); }
+constexpr int skinny_sum_frags(int me, int nf) {      // fragments summed between two barriers
+  const int f = skinny_frags(me, nf);
+  return f <= 8 ? f : (f == 12 ? 6 : 4);
+}
+constexpr int skinny_stage_bytes(int me, int nf) { return (2 * nf + me + me % 2) * 1024 + 256; }
+constexpr int skinny_sum_bytes(int me, int nf) { return kSkinnyWaves * skinny_sum_frags(me, nf) * 1024; }
+constexpr int skinny_stages(int me, int nf) {
+  const int fit = (160 * 1024 - skinny_sum_bytes(me, nf) - kSkinnyBiasBytes) / (kSkinnyWaves * skinny_stage_bytes(me, nf));
   return fit > 6 ? 6 : fit;
 }
-constexpr int skinny_lds_bytes(int mf, int nf) {
-  return kSkinnyWaves * skinny_stages(mf, nf) * skinny_stage_bytes(mf, nf) + skinny_sum_bytes(mf, nf) + kSkinnyBiasBytes;
+constexpr int skinny_lds_bytes(int me, int nf) {
+  return kSkinnyWaves * skinny_stages(me, nf) * skinny_stage_bytes(me, nf) + skinny_sum_bytes(me, nf) + kSkinnyBiasBytes;
 }
 
 // one wave's transfer global -> LDS: lane i's 16 bytes (at its own offset) go to dst + 16 i; NT: streamed, read once
@@ -59,16 +66,17 @@ __device__ __forceinline__ void transfer_256(__amdgpu_buffer_rsrc_t rs, uint8_t*
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)dst, 4, lane_off, off, 0, 0);
 }
 
-// MF: 16-row fragments of a (M <= 16 MF); NF: 16-column fragments of a unit
-template <bool TENSOR, bool OUT_F32, int MF, int NF>
+// (Rows of a fragment past the last piece hold what the LDS held: a row of the product depends on its own row of a alone.)
+template <bool TENSOR, bool OUT_F32, int ME, int NF>
 __global__ __launch_bounds__(kSkinnyThreads) void gemm_skinny_kernel(const SkinnyParams p) {
-  constexpr int U = skinny_stages(MF, NF);
+  constexpr int MF = (ME + 1) / 2;                              // 16-row fragments of a
+  constexpr int U = skinny_stages(ME, NF);
   constexpr int kCols = 16 * NF;
-  constexpr int kStage = skinny_stage_bytes(MF, NF);            // one k-block: b's rows, a's rows, a's scales
-  constexpr int kOps = 2 * (NF + MF) + (TENSOR ? 0 : 1);        // transfers of one k-block
+  constexpr int kStage = skinny_stage_bytes(ME, NF);            // one k-block: b's rows, a's rows, a's scales
+  constexpr int kOps = 2 * NF + ME + (TENSOR ? 0 : 1);          // transfers of one k-block
   constexpr int kLeft = (U - 1) * kOps;                         // in flight behind the oldest k-block
   static_assert(U >= 2 && kLeft <= 63, "the wait counter holds 63");
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[skinny_lds_bytes(MF, NF)];
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[skinny_lds_bytes(ME, NF)];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, g = lane >> 4;
@@ -76,7 +84,7 @@ __global__ __launch_bounds__(kSkinnyThreads) void gemm_skinny_kernel(const Skinn
   const int steps = (kblocks + kSkinnyWaves - 1) / kSkinnyWaves;
   uint8_t* const ring = lds + wave * (U * kStage);
   v4f* const red = reinterpret_cast<v4f*>(lds + kSkinnyWaves * U * kStage);      // [wave][fragment][lane]
-  uint16_t* const bias_lds = reinterpret_cast<uint16_t*>(lds + kSkinnyWaves * U * kStage + skinny_sum_bytes(MF, NF));
+  uint16_t* const bias_lds = reinterpret_cast<uint16_t*>(lds + kSkinnyWaves * U * kStage + skinny_sum_bytes(ME, NF));
 
   // this workgroup's units: a contiguous run
   const int units = p.N / kCols, base = units / (int)gridDim.x, more = units % (int)gridDim.x;
@@ -86,14 +94,14 @@ __global__ __launch_bounds__(kSkinnyThreads) void gemm_skinny_kernel(const Skinn
     for (int i = tid; i < count * kCols; i += kSkinnyThreads) bias_lds[i] = p.bias[unit0 * kCols + i];
 
   // a transfer moves 8 rows; lane i delivers to the i-th 16 bytes and fetches the chunk whose swizzled home that is
-  uint32_t b_off[2 * NF], a_off[2 * MF];
+  uint32_t b_off[2 * NF], a_off[ME];
 #pragma unroll
   for (int i = 0; i < 2 * NF; ++i) {
     const int r = i * 8 + (lane >> 3);
     b_off[i] = (uint32_t)r * (uint32_t)p.ldb + ((lane & 7) ^ row_swizzle(r)) * 16;
   }
 #pragma unroll
-  for (int i = 0; i < 2 * MF; ++i) {
+  for (int i = 0; i < ME; ++i) {
     const int r = i * 8 + (lane >> 3);
     a_off[i] = (uint32_t)(r < p.M ? r : p.M - 1) * (uint32_t)p.lda + ((lane & 7) ^ row_swizzle(r)) * 16;
   }
@@ -120,7 +128,7 @@ __global__ __launch_bounds__(kSkinnyThreads) void gemm_skinny_kernel(const Skinn
 #pragma unroll
     for (int i = 0; i < 2 * NF; ++i) transfer_1k<true>(rb, dst + i * 1024, b_off[i], kb * BK);
 #pragma unroll
-    for (int i = 0; i < 2 * MF; ++i) transfer_1k<false>(ra, dst + NF * 2048 + i * 1024, a_off[i], kb * BK);
+    for (int i = 0; i < ME; ++i) transfer_1k<false>(ra, dst + NF * 2048 + i * 1024, a_off[i], kb * BK);
     if (!TENSOR) {
       const __amdgpu_buffer_rsrc_t rsa = __builtin_amdgcn_make_buffer_rsrc((void*)p.sa, 0, ok ? sa_bytes : 0, 0x00020000);
       transfer_256(rsa, dst + (NF + MF) * 2048, sa_off, (int)(kb * p.sa_sk * 4));
@@ -185,53 +193,61 @@ __global__ __launch_bounds__(kSkinnyThreads) void gemm_skinny_kernel(const Skinn
       slot = slot + 1 == U ? 0 : slot + 1;
     }
     // the unit's sums: every wave puts down its own, then each fragment is added up by one wave
+    constexpr int G = skinny_sum_frags(ME, NF);
+    static_assert(F % G == 0, "whole groups of fragments");
 #pragma unroll
-    for (int i = 0; i < F; ++i) {
-      red[(wave * F + i) * 64 + lane] = acc[i];
-      acc[i] = zero;
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");     // (not __syncthreads, which waits for the transfers)
-    for (int i = wave; i < F; i += kSkinnyWaves) {
-      v4f s = red[i * 64 + lane];
+    for (int i0 = 0; i0 < F; i0 += G) {
 #pragma unroll
-      for (int v = 1; v < kSkinnyWaves; ++v) s += red[(v * F + i) * 64 + lane];
-      if (TENSOR) s *= tensor_scale;
-      const int f = i / MF, j = i % MF, row = j * 16 + l16, col = f * 16 + g * 4;
-      if (p.bias) {
-        const uint2 braw = *reinterpret_cast<const uint2*>(bias_lds + unit * kCols + col);
-        s[0] += bf16lo(braw.x); s[1] += bf16hi(braw.x); s[2] += bf16lo(braw.y); s[3] += bf16hi(braw.y);
+      for (int i = 0; i < G; ++i) {
+        red[(wave * G + i) * 64 + lane] = acc[i0 + i];
+        acc[i0 + i] = zero;
       }
-      if (row < p.M) {
-        const int64_t o = (int64_t)row * p.ldc + n0 + col;
-        if (OUT_F32) *reinterpret_cast<v4f*>(reinterpret_cast<float*>(p.c) + o) = s;
-        else *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(p.c) + o) = u32x2{pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3])};
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");     // (not __syncthreads, which waits for the transfers)
+      for (int i = wave; i < G; i += kSkinnyWaves) {
+        v4f s = red[i * 64 + lane];
+#pragma unroll
+        for (int v = 1; v < kSkinnyWaves; ++v) s += red[(v * G + i) * 64 + lane];
+        if (TENSOR) s *= tensor_scale;
+        const int f = (i0 + i) / MF, j = (i0 + i) % MF, row = j * 16 + l16, col = f * 16 + g * 4;
+        if (p.bias) {
+          const uint2 braw = *reinterpret_cast<const uint2*>(bias_lds + unit * kCols + col);
+          s[0] += bf16lo(braw.x); s[1] += bf16hi(braw.x); s[2] += bf16lo(braw.y); s[3] += bf16hi(braw.y);
+        }
+        if (row < p.M) {
+          const int64_t o = (int64_t)row * p.ldc + n0 + col;
+          if (OUT_F32) *reinterpret_cast<v4f*>(reinterpret_cast<float*>(p.c) + o) = s;
+          else *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(p.c) + o) = u32x2{pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3])};
+        }
       }
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");     // the sums have been read
     }
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");     // the sums have been read
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);   // the empty transfers still write to this workgroup's LDS
 }
 
-template <bool TENSOR, bool OUT_F32, int MF, int NF>
+template <bool TENSOR, bool OUT_F32, int ME>
 static void launch_skinny_form(const SkinnyParams& p, int cus, hipStream_t stream) {
-  const int units = p.N / (16 * NF);
-  gemm_skinny_kernel<TENSOR, OUT_F32, MF, NF>
-      <<<dim3((unsigned)(units < cus ? units : cus)), dim3(kSkinnyThreads), 0, stream>>>(p);
+  if (p.N >= kSkinnyWide * cus) {
+    const int units = p.N / 64;
+    gemm_skinny_kernel<TENSOR, OUT_F32, ME, 4><<<dim3((unsigned)(units < cus ? units : cus)), dim3(kSkinnyThreads), 0, stream>>>(p);
+  } else {
+    const int units = p.N / 32;
+    gemm_skinny_kernel<TENSOR, OUT_F32, ME, 2><<<dim3((unsigned)(units < cus ? units : cus)), dim3(kSkinnyThreads), 0, stream>>>(p);
+  }
 }
 
 template <bool TENSOR, bool OUT_F32>
 static void launch_skinny_rows(const SkinnyParams& p, int cus, hipStream_t stream) {
-  const bool wide = p.N >= kSkinnyWide * cus;
-  if (p.M <= 16) {
-    if (wide) launch_skinny_form<TENSOR, OUT_F32, 1, 4>(p, cus, stream);
-    else launch_skinny_form<TENSOR, OUT_F32, 1, 2>(p, cus, stream);
-  } else if (p.M <= 32) {
-    if (wide) launch_skinny_form<TENSOR, OUT_F32, 2, 4>(p, cus, stream);
-    else launch_skinny_form<TENSOR, OUT_F32, 2, 2>(p, cus, stream);
-  } else if (p.M <= 48) {
-    launch_skinny_form<TENSOR, OUT_F32, 3, 2>(p, cus, stream);
-  } else {
-    launch_skinny_form<TENSOR, OUT_F32, 4, 2>(p, cus, stream);
+  static_assert(kSkinnyMaxRows == 64, "one form per eight rows");
+  switch ((p.M + 7) / 8) {
+    case 1: launch_skinny_form<TENSOR, OUT_F32, 1>(p, cus, stream); break;
+    case 2: launch_skinny_form<TENSOR, OUT_F32, 2>(p, cus, stream); break;
+    case 3: launch_skinny_form<TENSOR, OUT_F32, 3>(p, cus, stream); break;
+    case 4: launch_skinny_form<TENSOR, OUT_F32, 4>(p, cus, stream); break;
+    case 5: launch_skinny_form<TENSOR, OUT_F32, 5>(p, cus, stream); break;
+    case 6: launch_skinny_form<TENSOR, OUT_F32, 6>(p, cus, stream); break;
+    case 7: launch_skinny_form<TENSOR, OUT_F32, 7>(p, cus, stream); break;
+    default: launch_skinny_form<TENSOR, OUT_F32, 8>(p, cus, stream); break;
   }
 }
 
