@@ -124,14 +124,15 @@ __global__ __launch_bounds__(kSkinnyThreads) void gemm_skinny_kernel(const Skinn
     const uint8_t* const b0 = p.b + (int64_t)((unit0 + (ok ? l_unit : 0)) * kCols) * p.ldb;
     const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)b0, 0, ok ? b_bytes : 0, 0x00020000);
     const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)p.a, 0, ok ? a_bytes : 0, 0x00020000);
+    const int off = ok ? kb * BK : 0;           // (an empty resource with no offset: out of range in any lane)
     uint8_t* const dst = ring + l_slot * kStage;
 #pragma unroll
-    for (int i = 0; i < 2 * NF; ++i) transfer_1k<true>(rb, dst + i * 1024, b_off[i], kb * BK);
+    for (int i = 0; i < 2 * NF; ++i) transfer_1k<true>(rb, dst + i * 1024, b_off[i], off);
 #pragma unroll
-    for (int i = 0; i < ME; ++i) transfer_1k<false>(ra, dst + NF * 2048 + i * 1024, a_off[i], kb * BK);
+    for (int i = 0; i < ME; ++i) transfer_1k<false>(ra, dst + NF * 2048 + i * 1024, a_off[i], off);
     if (!TENSOR) {
       const __amdgpu_buffer_rsrc_t rsa = __builtin_amdgcn_make_buffer_rsrc((void*)p.sa, 0, ok ? sa_bytes : 0, 0x00020000);
-      transfer_256(rsa, dst + (NF + MF) * 2048, sa_off, (int)(kb * p.sa_sk * 4));
+      transfer_256(rsa, dst + (NF + MF) * 2048, sa_off, ok ? (int)(kb * p.sa_sk * 4) : 0);
     }
     l_slot = l_slot + 1 == U ? 0 : l_slot + 1;
     if (++l_t == steps) {
