@@ -45,7 +45,6 @@ constexpr int BM = 256, BN = 256;
 // that streams from HBM (each weight panel is used by one XCD only), so where LDS allows it gets a
 // third buffer and its transfers run two k-blocks ahead; a's re-reads come from the Infinity Cache.
 __host__ __device__ constexpr int b_stages(int mode) { return (mode == 2 || mode == 4) /* per-row b scales: LDS also holds them */ ? 2 : 3; }
-constexpr int kXcds = 8;
 constexpr int kRectTiles = 32;              // tiles of the rectangle one XCD (32 CUs) works on at a time
 
 // kScalePow2: scales laid out as for kScaleBlock but every one a power of two; the matrix instruction
@@ -1144,17 +1143,15 @@ static bool use_small_kernel(int64_t M, int64_t N) {
 }
 
 // Few rows of a (decode): bound by reading b once, which the tile kernels do not reach (gemm_skinny.hip; 8 rows of
-// [7168, 16384]: 60 us with 64 x 128 tiles, 20 us; 64 rows: 64 and 31 us; 37 rows of [36864, 7168]: 81 us with 256 x 256
-// tiles, 57 us).  Hands the problem over if it is one; otherwise false.
-static bool try_skinny(const GemmParams& p, bool tensor, int out_type, hipStream_t stream, int& rc) {
+// [7168, 16384]: 60 us with 64 x 128 tiles, 20.6 us; 64 rows: 64 and 26.8 us; 37 rows of [36864, 7168]: 81 us with 256 x 256
+// tiles, 41.6 us), with the same bits.  Hands the problem over if it is one; otherwise false.
+static bool try_skinny(const GemmParams& p, SkinnyMode mode, int out_type, hipStream_t stream, int& rc) {
   if (p.M > kSkinnyMaxRows || p.K < kSkinnyMinK || p.accumulate || g_small_gemm_mode.load(std::memory_order_relaxed) != 0) return false;
-  const int cus = persistent_grid((int64_t)1 << 40);
-  if ((int64_t)p.N > (int64_t)cus * (kSkinnyMaxCols - 64)) return false;
   SkinnyParams q{};
   q.a = p.a; q.b = p.b; q.sa = p.sa; q.sb = p.sb; q.lda = p.lda; q.ldb = p.ldb;
-  q.sa_sm = p.sa_sm; q.sa_sk = p.sa_sk; q.sb_sn = p.sb_sn; q.sb_sk = p.sb_sk;
-  q.bias = p.bias; q.c = p.c; q.ldc = p.ldc; q.M = p.M; q.N = p.N; q.K = p.K;
-  rc = launch_skinny(q, tensor, out_type == HPFP8_OUT_F32, cus, stream);
+  q.sa_sm = p.sa_sm; q.sa_sk = p.sa_sk; q.sb_sn = p.sb_sn; q.sb_sk = p.sb_sk; q.sb_bytes = p.sb_bytes;
+  q.bias = p.bias; q.c = p.c; q.ldc = p.ldc; q.M = p.M; q.N = p.N; q.K = p.K; q.out_f32 = out_type == HPFP8_OUT_F32;
+  rc = launch_skinny(q, mode, persistent_grid((int64_t)1 << 40), stream);
   return true;
 }
 
@@ -1271,7 +1268,7 @@ static int gemm_blockwise_impl(const void* a, int64_t lda, const float* sa, int6
   p.c = c; p.ldc = ldc; p.bias = (const uint16_t*)bias;
   p.M = (int)M; p.N = (int)N; p.K = (int)K; p.accumulate = accumulate;
   if (sb_gran == 128) {
-    if (try_skinny(p, false, out_type, (hipStream_t)stream, rc)) return rc;
+    if (try_skinny(p, pow2 ? kSkinnyPow2 : kSkinnyBlock, out_type, (hipStream_t)stream, rc)) return rc;
     if (pow2) return launch<kScalePow2, kDense>(p, out_type, pick_shape(M, N), (hipStream_t)stream);
     if (!accumulate && use_small_kernel(M, N)) return launch_small<kScaleBlock>(p, out_type, (hipStream_t)stream);
     return launch<kScaleBlock, kDense>(p, out_type, pick_shape(M, N), (hipStream_t)stream);
@@ -1368,7 +1365,7 @@ int hpfp8_gemm_per_tensor(const void* a, int64_t lda, const float* sa_inv, const
   p.a = (const uint8_t*)a; p.b = (const uint8_t*)b; p.sa = sa_inv; p.sb = sb_inv; p.lda = lda; p.ldb = ldb;
   p.c = c; p.ldc = ldc; p.bias = (const uint16_t*)bias;
   p.M = (int)M; p.N = (int)N; p.K = (int)K;
-  if (try_skinny(p, true, out_type, (hipStream_t)stream, rc)) return rc;
+  if (try_skinny(p, kSkinnyTensor, out_type, (hipStream_t)stream, rc)) return rc;
   if (use_small_kernel(M, N)) return launch_small<kScaleTensor>(p, out_type, (hipStream_t)stream);
   return launch<kScaleTensor, kDense>(p, out_type, pick_shape(M, N), (hipStream_t)stream);
 }

@@ -5,7 +5,10 @@
 
 namespace hpfp8 {
 
-// c[m, n] = sum_kb sa(m, kb) * sb(n / 128, kb) * (A_kb . B_kb^T) (+ bias), or with `tensor` one scale each (sa[0], sb[0]).
+// c[m, n] = sum_kb sa(m, kb) * sb(n / 128, kb) * (A_kb . B_kb^T) (+ bias); kSkinnyPow2: power-of-two scales, applied by the
+// matrix instruction; kSkinnyTensor: one scale each (sa[0], sb[0]).
+enum SkinnyMode { kSkinnyBlock, kSkinnyPow2, kSkinnyTensor };
+
 struct SkinnyParams {
   const uint8_t* a;
   const uint8_t* b;
@@ -14,18 +17,20 @@ struct SkinnyParams {
   int64_t lda, ldb;       // row strides of a and b in bytes
   int64_t sa_sm, sa_sk;   // element strides of sa over (row, k-block)
   int64_t sb_sn, sb_sk;   // element strides of sb over (128-row block, k-block)
+  int sb_bytes;           // span of sb
   const uint16_t* bias;
   void* c;
   int64_t ldc;
   int M, N, K;
+  int out_f32;
 };
 
-constexpr int kSkinnyMaxRows = 64;
-constexpr int kSkinnyMaxCols = 1024;      // columns per compute unit (the bias of a workgroup's columns is kept in LDS)
-constexpr int kSkinnyMinK = 2048;         // shorter contractions leave too few k-blocks per wave: the tile kernels
-constexpr int kSkinnyWide = 128;          // from this many columns per compute unit on, units are 64 columns wide, which reads a half as often
-                                          // (32 / 37 / 64 rows of [36864, 7168]: 55.1 / 59.1 / 74.4 us with 32 columns, 52.9 / 56.5 / 65.4)
+constexpr int kSkinnyMaxRows = 64;        // four fragments of 16 rows; one row more takes tiles (64 rows of [7168, 16384]: 27 us here,
+                                          // 64 us with the 64 x 128 tiles that 65 rows take)
+// Contractions from here on.  Measured, 16 rows of [4096, K] with tiles / here: K = 256 4.9 / 4.9 us, 512 5.6 / 5.3, 1024 7.2 /
+// 5.1, 1920 10.1 / 5.1; of [36864, 512] 10.3 / 6.4: below 512 there is nothing to gain, from 512 to here there would be.
+constexpr int kSkinnyMinK = 2048;
 
-int launch_skinny(const SkinnyParams& p, bool tensor, bool out_f32, int cus, hipStream_t stream);
+int launch_skinny(const SkinnyParams& p, SkinnyMode mode, int cus, hipStream_t stream);
 
 }  // namespace hpfp8

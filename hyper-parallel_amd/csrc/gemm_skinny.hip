@@ -2,26 +2,28 @@
 //
 // Bound by reading b once.  A tile kernel has one workgroup per 128 columns here: 56 of 256 compute units on
 // N = 7168, each limited by what its vector-memory path delivers (about 25 bytes per clock).  Here
-//   * a unit of work is 32 columns (64 of a wide matrix); one workgroup per compute unit walks a contiguous run of units.
-//   * operands go global -> LDS -> registers, each wave through a ring of its own of U k-blocks (no barriers: a wave
-//     waits for its own transfers), and the ring runs on across units: while the sums of one are added up, the first
-//     k-blocks of the next are under way.  The transfers are there for their shape: one moves 8 rows x 128 bytes, whole
-//     cache lines, where loads straight into the matrix instruction's register layout (16 rows x 64 bytes) reach half
-//     the rate per compute unit.
-//   * each of a workgroup's four waves takes a contiguous quarter of the k-blocks (no wave waits for another before the
-//     end) and the four sums meet in LDS, added in wave order: the result differs from a tile kernel's, which adds all
-//     k-blocks in one chain, in the last bits of fp32.  (Kept in one chain -- the waves hand their partial products to
-//     one another round by round -- 37 rows of [36864, 7168] take 85 us instead of 63.)
-//   * a wave begins its quarter at a k-block that depends on the workgroup: begun at the same one, 256 workgroups whose
-//     units start a multiple of 16 KB apart ask the same memory channels at the same time (8 rows of [7168, 16384]: 28
-//     us, 22 us with it).
-//   * a is moved in pieces of 8 rows, so that 37 rows cost 40 and not 48 (27.3 -> 26.4 us on [7168, 16384]).
-// Measured (weights rotating beyond the Infinity Cache): 8 rows of [7168, 16384] 60 -> 20 us (5.8 TB/s), of [36864, 7168]
-// 80 -> 47 us (5.6 TB/s); from about 24 rows on the vector-memory path of a compute unit, which carries a's rows once per
-// unit, is the bound (64 rows of [7168, 16384]: 64 -> 31 us, of [36864, 7168] 65 us).
-// Transfers past the end go through an empty resource: they fetch nothing, write zeros and keep the number of
-// operations in flight constant, which is what the waits count.  (A result store in between adds to the count, which
-// makes a wait stricter, never looser.)
+//   * a workgroup has F 16-column fragments at a time, as many as give every compute unit its columns in few runs
+//     (skinny_fragments has the rule), and a's rows travel once per run.
+//   * four waves fetch, four multiply.  Operands go global -> LDS -> registers through a ring of stages of KS k-blocks
+//     that runs on across the runs of columns; one barrier per stage says that the stage has arrived and that the one
+//     before has been read, whose slot is refilled.  (With four waves doing both in turn the issue of the transfers and
+//     the multiplication add up: 8 rows of [36864, 7168] 59 us, 41 with them apart.)  The transfers are there for their
+//     shape: one moves 8 rows x 128 bytes, whole cache lines, where loads straight into the matrix instruction's
+//     register layout (16 rows x 64 bytes) reach half the rate per compute unit.
+//   * the waves share the matrix work by fragments of the result, never by k-blocks: a sum runs over the k-blocks in
+//     their order in one chain with the matrix instruction, scales and roundings of the tile kernels, so an element of c
+//     has the same bits here and there -- whatever the number of rows, the column it stands in, the width of b (a column
+//     shard) and the number of compute units.
+//   * all workgroups walk through k in step, so with rows a power of two apart they ask few memory channels at a time.
+//     Two things spread that: an XCD's workgroups have neighbouring columns (8 rows of [7168, 16384] 26.4 -> 21.7 us, of
+//     [8192, 8192] 19.8 -> 13.6), and a stage is as many k-blocks as LDS has three of (8 rather than 4 k-blocks on
+//     [7168, 16384]: 21.4 -> 20.4 us; 4 rather than 2 for 64 rows of it: 31.7 -> 26.8).
+//   * a is moved in pieces of 8 rows, so that 37 rows cost 40 and not 48.
+// Measured (weights rotating beyond the Infinity Cache): 8 rows of [7168, 16384] 20.6 us (5.7 TB/s), of [36864, 7168] 39.5
+// us (6.7 TB/s); 37 rows of the latter 41.6, 64 rows 44.0.  64 rows of [7168, 16384] 26.8 us: a's rows are then two
+// thirds of what passes a compute unit's vector-memory path.
+// Transfers past the end go through an empty resource (with no scalar offset: out of range in any lane): they fetch
+// nothing, write zeros and keep the number of operations in flight constant, which is what the waits count.
 #include "gemm_skinny.h"
 #include "gemm_tile.h"
 #include "hpfp8_device.h"
@@ -29,25 +31,17 @@
 
 namespace hpfp8 {
 
-constexpr int kSkinnyWaves = 4;
-constexpr int kSkinnyThreads = kSkinnyWaves * 64;
-// ME: 8-row pieces of a, one transfer each (M <= 8 ME); NF: 16-column fragments of a unit.
-// LDS of one workgroup: the four rings, the partial sums of the fragments added up at a time, the bias of the workgroup's
-// columns.  U k-blocks per ring: what 160 KB have room for, and at most 6 (more in flight gains nothing).
-constexpr int kSkinnyBiasBytes = kSkinnyMaxCols * 2;
-constexpr int skinny_frags(int me, int nf) { return nf * ((me + 1) / 2); }
-constexpr int skinny_sum_frags(int me, int nf) {      // fragments summed between two barriers
-  const int f = skinny_frags(me, nf);
-  return f <= 8 ? f : (f == 12 ? 6 : 4);
-}
-constexpr int skinny_stage_bytes(int me, int nf) { return (2 * nf + me + me % 2) * 1024 + 256; }
-constexpr int skinny_sum_bytes(int me, int nf) { return kSkinnyWaves * skinny_sum_frags(me, nf) * 1024; }
-constexpr int skinny_stages(int me, int nf) {
-  const int fit = (160 * 1024 - skinny_sum_bytes(me, nf) - kSkinnyBiasBytes) / (kSkinnyWaves * skinny_stage_bytes(me, nf));
-  return fit > 6 ? 6 : fit;
-}
-constexpr int skinny_lds_bytes(int me, int nf) {
-  return kSkinnyWaves * skinny_stages(me, nf) * skinny_stage_bytes(me, nf) + skinny_sum_bytes(me, nf) + kSkinnyBiasBytes;
+constexpr int kSkinnyWaves = 4;                         // so many fetch, so many multiply
+constexpr int kSkinnyThreads = 2 * kSkinnyWaves * 64;
+// ME: 8-row pieces of a, one transfer each (M <= 8 ME); F: 16-column fragments of a workgroup.
+// A stage: KS k-blocks, each b's rows, a's rows, the scales of a's rows (64) and of the fragments.
+constexpr int skinny_kstep(int me, int f) { return 2 * f + me <= 6 ? 8 : (2 * f + me <= 12 ? 4 : 2); }
+constexpr int skinny_block_bytes(int me, int f) { return (2 * f + me) * 1024 + 512; }
+constexpr int skinny_stage_bytes(int me, int f) { return skinny_kstep(me, f) * skinny_block_bytes(me, f); }
+constexpr int kSkinnySpare = 1024;       // behind the ring: where a transfer without a piece of its own goes
+constexpr int skinny_stages(int me, int f) {
+  const int fit = (160 * 1024 - kSkinnySpare) / skinny_stage_bytes(me, f);
+  return fit > 8 ? 8 : fit;
 }
 
 // one wave's transfer global -> LDS: lane i's 16 bytes (at its own offset) go to dst + 16 i; NT: streamed, read once
@@ -66,200 +60,262 @@ __device__ __forceinline__ void transfer_256(__amdgpu_buffer_rsrc_t rs, uint8_t*
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)dst, 4, lane_off, off, 0, 0);
 }
 
-// (Rows of a fragment past the last piece hold what the LDS held: a row of the product depends on its own row of a alone.)
-template <bool TENSOR, bool OUT_F32, int ME, int NF>
-__global__ __launch_bounds__(kSkinnyThreads) void gemm_skinny_kernel(const SkinnyParams p) {
+// (Rows of a fragment past the last piece hold what lies behind it in the LDS: a row of the product depends on its own
+// row of a alone, and rows past M are not stored.)
+template <int MODE, int ME, int F>
+__global__ __launch_bounds__(kSkinnyThreads) void gemm_skinny_kernel(const SkinnyParams p, int units) {
   constexpr int MF = (ME + 1) / 2;                              // 16-row fragments of a
-  constexpr int U = skinny_stages(ME, NF);
-  constexpr int kCols = 16 * NF;
-  constexpr int kStage = skinny_stage_bytes(ME, NF);            // one k-block: b's rows, a's rows, a's scales
-  constexpr int kOps = 2 * NF + ME + (TENSOR ? 0 : 1);          // transfers of one k-block
-  constexpr int kLeft = (U - 1) * kOps;                         // in flight behind the oldest k-block
-  static_assert(U >= 2 && kLeft <= 63, "the wait counter holds 63");
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[skinny_lds_bytes(ME, NF)];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  constexpr int KS = skinny_kstep(ME, F), U = skinny_stages(ME, F);
+  constexpr int kBlockBytes = skinny_block_bytes(ME, F), kStage = skinny_stage_bytes(ME, F);
+  constexpr int kA = 2 * F * 1024, kScales = (2 * F + ME) * 1024;     // a's rows and the scales inside a k-block's bytes
+  constexpr int kCols = 16 * F;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[U * kStage + kSkinnySpare];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, g = lane >> 4;
   const int kblocks = p.K >> 7;
-  const int steps = (kblocks + kSkinnyWaves - 1) / kSkinnyWaves;
-  uint8_t* const ring = lds + wave * (U * kStage);
-  v4f* const red = reinterpret_cast<v4f*>(lds + kSkinnyWaves * U * kStage);      // [wave][fragment][lane]
-  uint16_t* const bias_lds = reinterpret_cast<uint16_t*>(lds + kSkinnyWaves * U * kStage + skinny_sum_bytes(ME, NF));
+  const int stages = (kblocks + KS - 1) / KS;                   // of one unit (a run of kCols columns)
+  // this workgroup's units: first, first + step, ..; the workgroups of an XCD (ids congruent mod 8) have neighbouring ones
+  const int step = gridDim.x, xcd = blockIdx.x % kXcds;
+  const int first = xcd * (step / kXcds) + (xcd < step % kXcds ? xcd : step % kXcds) + blockIdx.x / kXcds;
 
-  // this workgroup's units: a contiguous run
-  const int units = p.N / kCols, base = units / (int)gridDim.x, more = units % (int)gridDim.x;
-  const int wg = blockIdx.x;
-  const int unit0 = wg * base + (wg < more ? wg : more), count = base + (wg < more ? 1 : 0);
-  if (p.bias)
-    for (int i = tid; i < count * kCols; i += kSkinnyThreads) bias_lds[i] = p.bias[unit0 * kCols + i];
-
-  // a transfer moves 8 rows; lane i delivers to the i-th 16 bytes and fetches the chunk whose swizzled home that is
-  uint32_t b_off[2 * NF], a_off[ME];
+  if (wave < kSkinnyWaves) {
+    // ---- fetching.  A transfer moves 8 rows; lane i delivers to the i-th 16 bytes and fetches the chunk whose swizzled
+    // home that is.  Offsets inside a resource: rows per lane, the k-block (less than a row) scalar.
+    constexpr int KW = KS > kSkinnyWaves ? KS / kSkinnyWaves : 1;       // k-blocks a wave fetches per stage
+    constexpr int W = KS < kSkinnyWaves ? kSkinnyWaves / KS : 1;        // waves that fetch one k-block together
+    constexpr int NBP = (2 * F + W - 1) / W, NAP = (ME + W - 1) / W;    // a wave's transfers of b and of a per k-block
+    constexpr int kScaleOps = MODE == kSkinnyTensor ? 0 : (W == 1 ? 2 : 1);
+    constexpr int kLeft = (U - 2) * KW * (NBP + NAP + kScaleOps);       // in flight behind the oldest stage
+    static_assert(U >= 3 && kLeft <= 63, "the wait counter holds 63");
+    static_assert(W <= 2, "every wave of a k-block has scales to fetch");
+    const int h = wave % W, kb0 = wave / W * KW;
+    uint32_t b_off[NBP], a_off[NAP];
 #pragma unroll
-  for (int i = 0; i < 2 * NF; ++i) {
-    const int r = i * 8 + (lane >> 3);
-    b_off[i] = (uint32_t)r * (uint32_t)p.ldb + ((lane & 7) ^ row_swizzle(r)) * 16;
-  }
-#pragma unroll
-  for (int i = 0; i < ME; ++i) {
-    const int r = i * 8 + (lane >> 3);
-    a_off[i] = (uint32_t)(r < p.M ? r : p.M - 1) * (uint32_t)p.lda + ((lane & 7) ^ row_swizzle(r)) * 16;
-  }
-  const uint32_t sa_off = (uint32_t)(lane < p.M ? lane : p.M - 1) * (uint32_t)p.sa_sm * 4u;
-  const int a_bytes = (int)((p.M - 1) * p.lda + p.K), b_bytes = (int)((kCols - 1) * p.ldb + p.K);
-  const int sa_bytes = TENSOR ? 0 : (int)(((p.M - 1) * p.sa_sm + (kblocks - 1) * p.sa_sk + 1) * 4);
-  const int rot = (int)((blockIdx.x >> 3) * 5u % (unsigned)steps);
-
-  // the k-block a wave touches in its t-th step on a unit (past the end of the contraction: kblocks)
-  auto kb_of = [&](int t) {
-    int r = t + rot;
-    if (r >= steps) r -= steps;
-    const int kb = wave * steps + r;
-    return kb < kblocks ? kb : kblocks;
-  };
-  int l_t = 0, l_unit = 0, l_slot = 0;          // the next step to fetch: step of the unit, unit of the run, ring slot
-  auto fetch = [&]() {
-    const int kb = kb_of(l_t);
-    const bool ok = l_unit < count && kb < kblocks;
-    const uint8_t* const b0 = p.b + (int64_t)((unit0 + (ok ? l_unit : 0)) * kCols) * p.ldb;
-    const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)b0, 0, ok ? b_bytes : 0, 0x00020000);
-    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)p.a, 0, ok ? a_bytes : 0, 0x00020000);
-    const int off = ok ? kb * BK : 0;           // (an empty resource with no offset: out of range in any lane)
-    uint8_t* const dst = ring + l_slot * kStage;
-#pragma unroll
-    for (int i = 0; i < 2 * NF; ++i) transfer_1k<true>(rb, dst + i * 1024, b_off[i], off);
-#pragma unroll
-    for (int i = 0; i < ME; ++i) transfer_1k<false>(ra, dst + NF * 2048 + i * 1024, a_off[i], off);
-    if (!TENSOR) {
-      const __amdgpu_buffer_rsrc_t rsa = __builtin_amdgcn_make_buffer_rsrc((void*)p.sa, 0, ok ? sa_bytes : 0, 0x00020000);
-      transfer_256(rsa, dst + (NF + MF) * 2048, sa_off, ok ? (int)(kb * p.sa_sk * 4) : 0);
+    for (int i = 0; i < NBP; ++i) {
+      const int r = (i * W + h) * 8 + (lane >> 3);
+      b_off[i] = (uint32_t)r * (uint32_t)p.ldb + ((lane & 7) ^ row_swizzle(r)) * 16;
     }
-    l_slot = l_slot + 1 == U ? 0 : l_slot + 1;
-    if (++l_t == steps) {
-      l_t = 0;
-      ++l_unit;
+#pragma unroll
+    for (int i = 0; i < NAP; ++i) {                             // (rows past M lie past the end of the resource)
+      const int r = (i * W + h) * 8 + (lane >> 3);
+      a_off[i] = (uint32_t)r * (uint32_t)p.lda + ((lane & 7) ^ row_swizzle(r)) * 16;
     }
-  };
+    const uint32_t sa_off = (uint32_t)(lane < p.M ? lane : p.M - 1) * (uint32_t)p.sa_sm * 4u;
+    const int a_bytes = (int)((p.M - 1) * p.lda + p.K);
+    const int sa_bytes = MODE == kSkinnyTensor ? 0 : (int)(((p.M - 1) * p.sa_sm + (kblocks - 1) * p.sa_sk + 1) * 4);
+    const int sa_step = (int)p.sa_sk * 4, sb_step = (int)p.sb_sk * 4;
+    int unit = first, kb = kb0, slot = 0;                       // the next stage to fetch
+    const uint8_t* b0;
+    int b_bytes;
+    uint32_t sb_off;
+    auto enter = [&]() {                                        // the unit's part of b (past the last unit: nothing)
+      const int n0 = unit < units ? unit * kCols : 0;
+      const int rows = p.N - n0 < kCols ? p.N - n0 : kCols;
+      b0 = p.b + (int64_t)n0 * p.ldb;
+      b_bytes = unit < units ? (int)((rows - 1) * p.ldb + p.K) : 0;
+      const int n = n0 + (lane < F ? lane : F - 1) * 16;        // lane i: the scale of fragment i (past the last: of the last)
+      sb_off = (uint32_t)((n < p.N ? n : p.N - 1) >> 7) * (uint32_t)p.sb_sn * 4u;
+    };
+    enter();
+    auto fetch = [&]() {
+#pragma unroll
+      for (int j = 0; j < KW; ++j) {
+        const bool ok = kb + j < kblocks && b_bytes != 0;
+        const int off = ok ? (kb + j) * BK : 0;
+        uint8_t* const dst = lds + slot * kStage + (kb0 + j) * kBlockBytes;
+#pragma unroll
+        for (int i = 0; i < NBP; ++i) {                         // (2 F is a multiple of W: every wave has as many)
+          const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)b0, 0, ok ? b_bytes : 0, 0x00020000);
+          transfer_1k<true>(rb, dst + (i * W + h) * 1024, b_off[i], off);
+        }
+#pragma unroll
+        for (int i = 0; i < NAP; ++i) {
+          const bool in = ME % W == 0 || i * W + h < ME;
+          const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)p.a, 0, ok && in ? a_bytes : 0, 0x00020000);
+          transfer_1k<false>(ra, in ? dst + kA + (i * W + h) * 1024 : lds + U * kStage, a_off[i], in ? off : 0);
+        }
+        if (MODE != kSkinnyTensor) {
+          const __amdgpu_buffer_rsrc_t rsa = __builtin_amdgcn_make_buffer_rsrc((void*)p.sa, 0, ok ? sa_bytes : 0, 0x00020000);
+          const __amdgpu_buffer_rsrc_t rsb = __builtin_amdgcn_make_buffer_rsrc((void*)p.sb, 0, ok ? p.sb_bytes : 0, 0x00020000);
+          if (h == 0) transfer_256(rsa, dst + kScales, sa_off, ok ? (kb + j) * sa_step : 0);
+          if (h == W - 1) transfer_256(rsb, dst + kScales + 256, sb_off, ok ? (kb + j) * sb_step : 0);
+        }
+      }
+      slot = slot + 1 == U ? 0 : slot + 1;
+      kb += KS;
+      if (kb - kb0 >= kblocks) {
+        kb = kb0;
+        unit += step;
+        enter();
+      }
+    };
+    for (int u = 0; u < U - 1; ++u) fetch();
+    for (int u = first; u < units; u += step)
+      for (int t = 0; t < stages; ++t) {
+        // own transfers of this stage have landed; then everyone's, and the stage before has been read
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kLeft) : "memory");
+        fetch();
+      }
+    __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the empty transfers still write to this workgroup's LDS
+    return;
+  }
+
+  // ---- multiplying.  WF waves along the fragments of b, WJ along those of a; FW x JW results per wave (the last ones of
+  // an uneven split are computed twice and stored once)
+  constexpr int WF = F >= 3 ? 4 : F, WJ = kSkinnyWaves / WF;
+  constexpr int FW = (F + WF - 1) / WF, JW = (MF + WJ - 1) / WJ;
+  const int wf = (wave - kSkinnyWaves) % WF, wj = (wave - kSkinnyWaves) / WF;
+  const bool active = wf < F && wj < MF;
+  int frag[FW], rows16[JW];                                     // this wave's fragments of b and of a
+#pragma unroll
+  for (int q = 0; q < FW; ++q) frag[q] = wf + WF * q < F ? wf + WF * q : F - 1;
+#pragma unroll
+  for (int r = 0; r < JW; ++r) rows16[r] = wj + WJ * r < MF ? wj + WJ * r : MF - 1;
   const v4f zero = {0.f, 0.f, 0.f, 0.f};
-  constexpr int F = NF * MF;
-  v4f acc[F];
+  v4f acc[FW][JW];
 #pragma unroll
-  for (int i = 0; i < F; ++i) acc[i] = zero;
+  for (int q = 0; q < FW; ++q)
+#pragma unroll
+    for (int r = 0; r < JW; ++r) acc[q][r] = zero;
   const int pc0 = (2 * g) ^ row_swizzle(l16);
   float tensor_scale = 1.f;
-  if (TENSOR) tensor_scale = p.sa[0] * p.sb[0];
-  __syncthreads();                              // the bias is there (and no load but the transfers is in flight)
-  for (int u = 0; u < U; ++u) fetch();
+  if (MODE == kSkinnyTensor) tensor_scale = p.sa[0] * p.sb[0];
+
+  // one k-block of a stage: the arithmetic of gemm_kernel, operation for operation
+  auto k_block = [&](const uint8_t* src) {
+    v8i w[FW], x[JW];
+    float sa[JW], sb[FW];
+#pragma unroll
+    for (int q = 0; q < FW; ++q) {
+      w[q] = frag_read(src + frag[q] * 2048 + l16 * BK, pc0);
+      if (MODE != kSkinnyTensor) sb[q] = *reinterpret_cast<const float*>(src + kScales + 256 + frag[q] * 4);
+    }
+#pragma unroll
+    for (int r = 0; r < JW; ++r) {
+      x[r] = frag_read(src + kA + rows16[r] * 2048 + l16 * BK, pc0);
+      if (MODE != kSkinnyTensor) sa[r] = *reinterpret_cast<const float*>(src + kScales + (rows16[r] * 16 + l16) * 4);
+    }
+#pragma unroll
+    for (int q = 0; q < FW; ++q)
+#pragma unroll
+      for (int r = 0; r < JW; ++r) {
+        if (MODE == kSkinnyTensor) {
+          acc[q][r] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w[q], x[r], acc[q][r], 0, 0, 0, 0, 0, 0);
+        } else if (MODE == kSkinnyPow2) {
+          acc[q][r] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w[q], x[r], acc[q][r], 0, 0, 0,
+                                                                      (int)(__builtin_bit_cast(uint32_t, sb[q]) >> 23), 0,
+                                                                      (int)(__builtin_bit_cast(uint32_t, sa[r]) >> 23));
+        } else {
+          const v4f part = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w[q], x[r], zero, 0, 0, 0, 0, 0, 0);
+          const float s = sa[r] * sb[q];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[q][r][e] = __builtin_fmaf(part[e], s, acc[q][r][e]);
+        }
+      }
+  };
 
   int slot = 0;
-  for (int unit = 0; unit < count; ++unit) {
-    const int n0 = (unit0 + unit) * kCols;
-    // (a scalar load: the scale of the unit's 128-row block of b)
-    typedef const __attribute__((address_space(4))) float* const_f32_t;
-    const const_f32_t sb_row = (const_f32_t)(uintptr_t)(p.sb + (TENSOR ? 0 : (int64_t)(n0 >> 7) * p.sb_sn));
-    for (int t = 0; t < steps; ++t) {
-      const int kb = kb_of(t);
-      const float sb = TENSOR ? 1.f : sb_row[(int64_t)(kb < kblocks ? kb : 0) * p.sb_sk];
-      __builtin_amdgcn_s_waitcnt((kLeft & 15) | ((kLeft >> 4) << 14) | 0x0F70);     // vmcnt(kLeft): this slot has arrived
-      asm volatile("" ::: "memory");
+  for (int unit = first; unit < units; unit += step) {
+    for (int t = 0; t < stages; ++t) {
       __builtin_amdgcn_sched_barrier(0);
-      const uint8_t* const src = ring + slot * kStage;
-      v8i w[NF], x[MF];
-      float sa[MF];
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // the stage is there; the one before has been read
+      __builtin_amdgcn_sched_barrier(0);
+      if (active) {
+        const uint8_t* const src = lds + slot * kStage;
+        if ((t + 1) * KS <= kblocks) {
 #pragma unroll
-      for (int f = 0; f < NF; ++f) w[f] = frag_read(src + l16 * BK + f * 2048, pc0);
-#pragma unroll
-      for (int j = 0; j < MF; ++j) {
-        x[j] = frag_read(src + l16 * BK + (NF + j) * 2048, pc0);
-        if (!TENSOR) sa[j] = *reinterpret_cast<const float*>(src + (NF + MF) * 2048 + (j * 16 + l16) * 4);
-      }
-#pragma unroll
-      for (int j = 0; j < MF; ++j) {
-        const float s = TENSOR ? 1.f : sa[j] * sb;
-#pragma unroll
-        for (int f = 0; f < NF; ++f) {
-          const int i = f * MF + j;
-          if (TENSOR) {
-            acc[i] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w[f], x[j], acc[i], 0, 0, 0, 0, 0, 0);
-          } else {
-            const v4f part = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w[f], x[j], zero, 0, 0, 0, 0, 0, 0);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[i][r] = __builtin_fmaf(part[r], s, acc[i][r]);
-          }
+          for (int i = 0; i < KS; ++i) k_block(src + i * kBlockBytes);
+        } else {
+          for (int i = 0; t * KS + i < kblocks; ++i) k_block(src + i * kBlockBytes);
         }
       }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");        // the slot has been read: it may be refilled
-      __builtin_amdgcn_sched_barrier(0);
-      fetch();
       slot = slot + 1 == U ? 0 : slot + 1;
     }
-    // the unit's sums: every wave puts down its own, then each fragment is added up by one wave
-    constexpr int G = skinny_sum_frags(ME, NF);
-    static_assert(F % G == 0, "whole groups of fragments");
+    // the unit's results: a lane holds four consecutive columns of one row
+    if (!active) continue;
 #pragma unroll
-    for (int i0 = 0; i0 < F; i0 += G) {
+    for (int q = 0; q < FW; ++q) {
+      const int col = unit * kCols + (wf + WF * q) * 16 + g * 4;
+      const bool col_ok = wf + WF * q < F && col < p.N;
+      uint2 braw = make_uint2(0, 0);
+      if (p.bias && col_ok) braw = *reinterpret_cast<const uint2*>(p.bias + col);
 #pragma unroll
-      for (int i = 0; i < G; ++i) {
-        red[(wave * G + i) * 64 + lane] = acc[i0 + i];
-        acc[i0 + i] = zero;
-      }
-      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");     // (not __syncthreads, which waits for the transfers)
-      for (int i = wave; i < G; i += kSkinnyWaves) {
-        v4f s = red[i * 64 + lane];
-#pragma unroll
-        for (int v = 1; v < kSkinnyWaves; ++v) s += red[(v * G + i) * 64 + lane];
-        if (TENSOR) s *= tensor_scale;
-        const int f = (i0 + i) / MF, j = (i0 + i) % MF, row = j * 16 + l16, col = f * 16 + g * 4;
+      for (int r = 0; r < JW; ++r) {
+        v4f s = acc[q][r];
+        acc[q][r] = zero;
+        const int row = (wj + WJ * r) * 16 + l16;
+        if (MODE == kSkinnyTensor) s *= tensor_scale;
         if (p.bias) {
-          const uint2 braw = *reinterpret_cast<const uint2*>(bias_lds + unit * kCols + col);
           s[0] += bf16lo(braw.x); s[1] += bf16hi(braw.x); s[2] += bf16lo(braw.y); s[3] += bf16hi(braw.y);
         }
-        if (row < p.M) {
-          const int64_t o = (int64_t)row * p.ldc + n0 + col;
-          if (OUT_F32) *reinterpret_cast<v4f*>(reinterpret_cast<float*>(p.c) + o) = s;
+        if (col_ok && row < p.M) {
+          const int64_t o = (int64_t)row * p.ldc + col;
+          if (p.out_f32) *reinterpret_cast<v4f*>(reinterpret_cast<float*>(p.c) + o) = s;
           else *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(p.c) + o) = u32x2{pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3])};
         }
       }
-      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");     // the sums have been read
     }
   }
-  __builtin_amdgcn_s_waitcnt(0x0F70);   // the empty transfers still write to this workgroup's LDS
 }
 
-template <bool TENSOR, bool OUT_F32, int ME>
+// Fragments per workgroup.  A run costs what is larger, b's part of the memory bandwidth or what passes the compute unit's
+// vector-memory path (1.4 : 1 per KB), and 1.4 times that where a stage is fewer than four k-blocks; taken is the form whose
+// runs cost least, the narrowest of equals.  Over 10 widths from 4096 to 36864, 4 contractions from 4096 to 16384 and 5 row
+// counts this is 0.7 % slower on average than the best of the six forms of each, 14 % at most (24 rows of [18432, 7168]).
+static int skinny_fragments(int64_t N, int me, int cus) {
+  const int forms[] = {1, 2, 3, 4, 6, 9};
+  int best = 0;
+  int64_t best_cost = 0;
+  for (int f : forms) {
+    const int64_t units = (N / 16 + f - 1) / f, runs = (units + cus - 1) / cus;
+    const int64_t run = 14 * 2 * f > 10 * (2 * f + me) ? 14 * 2 * f : 10 * (2 * f + me);
+    const int64_t cost = runs * run * (skinny_kstep(me, f) >= 4 ? 10 : 14);
+    if (!best || cost < best_cost) {
+      best = f;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
+template <int MODE, int ME, int F>
 static void launch_skinny_form(const SkinnyParams& p, int cus, hipStream_t stream) {
-  if (p.N >= kSkinnyWide * cus) {
-    const int units = p.N / 64;
-    gemm_skinny_kernel<TENSOR, OUT_F32, ME, 4><<<dim3((unsigned)(units < cus ? units : cus)), dim3(kSkinnyThreads), 0, stream>>>(p);
-  } else {
-    const int units = p.N / 32;
-    gemm_skinny_kernel<TENSOR, OUT_F32, ME, 2><<<dim3((unsigned)(units < cus ? units : cus)), dim3(kSkinnyThreads), 0, stream>>>(p);
+  const int units = (p.N / 16 + F - 1) / F;
+  gemm_skinny_kernel<MODE, ME, F><<<dim3((unsigned)(units < cus ? units : cus)), dim3(kSkinnyThreads), 0, stream>>>(p, units);
+}
+
+template <int MODE, int ME>
+static void launch_skinny_cols(const SkinnyParams& p, int cus, hipStream_t stream) {
+  switch (skinny_fragments(p.N, ME, cus)) {
+    case 1: launch_skinny_form<MODE, ME, 1>(p, cus, stream); break;
+    case 2: launch_skinny_form<MODE, ME, 2>(p, cus, stream); break;
+    case 3: launch_skinny_form<MODE, ME, 3>(p, cus, stream); break;
+    case 4: launch_skinny_form<MODE, ME, 4>(p, cus, stream); break;
+    case 6: launch_skinny_form<MODE, ME, 6>(p, cus, stream); break;
+    default: launch_skinny_form<MODE, ME, 9>(p, cus, stream); break;
   }
 }
 
-template <bool TENSOR, bool OUT_F32>
+template <int MODE>
 static void launch_skinny_rows(const SkinnyParams& p, int cus, hipStream_t stream) {
   static_assert(kSkinnyMaxRows == 64, "one form per eight rows");
   switch ((p.M + 7) / 8) {
-    case 1: launch_skinny_form<TENSOR, OUT_F32, 1>(p, cus, stream); break;
-    case 2: launch_skinny_form<TENSOR, OUT_F32, 2>(p, cus, stream); break;
-    case 3: launch_skinny_form<TENSOR, OUT_F32, 3>(p, cus, stream); break;
-    case 4: launch_skinny_form<TENSOR, OUT_F32, 4>(p, cus, stream); break;
-    case 5: launch_skinny_form<TENSOR, OUT_F32, 5>(p, cus, stream); break;
-    case 6: launch_skinny_form<TENSOR, OUT_F32, 6>(p, cus, stream); break;
-    case 7: launch_skinny_form<TENSOR, OUT_F32, 7>(p, cus, stream); break;
-    default: launch_skinny_form<TENSOR, OUT_F32, 8>(p, cus, stream); break;
+    case 1: launch_skinny_cols<MODE, 1>(p, cus, stream); break;
+    case 2: launch_skinny_cols<MODE, 2>(p, cus, stream); break;
+    case 3: launch_skinny_cols<MODE, 3>(p, cus, stream); break;
+    case 4: launch_skinny_cols<MODE, 4>(p, cus, stream); break;
+    case 5: launch_skinny_cols<MODE, 5>(p, cus, stream); break;
+    case 6: launch_skinny_cols<MODE, 6>(p, cus, stream); break;
+    case 7: launch_skinny_cols<MODE, 7>(p, cus, stream); break;
+    default: launch_skinny_cols<MODE, 8>(p, cus, stream); break;
   }
 }
 
-int launch_skinny(const SkinnyParams& p, bool tensor, bool out_f32, int cus, hipStream_t stream) {
-  if (tensor) {
-    if (out_f32) launch_skinny_rows<true, true>(p, cus, stream);
-    else launch_skinny_rows<true, false>(p, cus, stream);
-  } else {
-    if (out_f32) launch_skinny_rows<false, true>(p, cus, stream);
-    else launch_skinny_rows<false, false>(p, cus, stream);
-  }
+int launch_skinny(const SkinnyParams& p, SkinnyMode mode, int cus, hipStream_t stream) {
+  if (mode == kSkinnyTensor) launch_skinny_rows<kSkinnyTensor>(p, cus, stream);
+  else if (mode == kSkinnyPow2) launch_skinny_rows<kSkinnyPow2>(p, cus, stream);
+  else launch_skinny_rows<kSkinnyBlock>(p, cus, stream);
   return check_launch("gemm (few rows)");
 }
 

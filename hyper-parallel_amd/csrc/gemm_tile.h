@@ -6,6 +6,7 @@
 namespace hpfp8 {
 
 constexpr int BK = 128;
+constexpr int kXcds = 8;             // workgroup ids congruent mod 8 share an XCD and its L2
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 

@@ -50,9 +50,8 @@ def _dequantized(q, s, rows, cols=128):
 @pytest.mark.parametrize("n,k", [(128, 128), (256, 640), (1152, 1152), (33024, 384), (384, 2048), (256, 2432), (33024, 2048)])
 def test_gemm_with_few_rows_is_exact_on_integer_inputs(gpu, m, n, k):
     """Every row-fragment count of the few-rows GEMM and the first row count beyond it; contractions on both sides of the
-    shortest it takes, k-blocks that divide among its waves and that do not; fewer units of columns than compute units,
-    uneven runs of them, and wide ones.  All
-    partial sums are integers below 2^24 (k / 128 blocks of 128 products of at most 16, times scales of at most 16 in
+    shortest it takes, k-blocks that divide into its stages and that do not; fewer runs of columns than compute units and
+    more.  All partial sums are integers below 2^24 (k / 128 blocks of 128 products of at most 16, times scales of at most 16 in
     steps of 2^-4), so every order of summation gives the exact result."""
     from hpfp8 import ops
     a, b = _ints((m, k), 1, gpu), _ints((n, k), 2, gpu)
@@ -67,6 +66,161 @@ def test_gemm_with_few_rows_is_exact_on_integer_inputs(gpu, m, n, k):
     ta, tb = torch.tensor(0.5, device=gpu), torch.tensor(0.25, device=gpu)
     assert torch.equal(ops.gemm_per_tensor(a, ta, b, tb, out_dtype=torch.float32).double(), one)
     assert torch.equal(ops.gemm_per_tensor(a, ta, b, tb, bias=bias), (one + bias.double()).to(torch.bfloat16))
+
+
+# (n, k) of the few-rows form: with the row counts below every number of fragments per workgroup (1, 2, 3, 4, 6 and 9 on 256
+# compute units) in one run and in several, last runs that are partly missing, stages of two, four and eight k-blocks that
+# divide the contraction and that do not
+FEW_ROWS_SHAPES = [(128, 2048), (1152, 2432), (8320, 2176), (12160, 2304), (16384, 2432), (24704, 2176), (36736, 2432), (38400, 2176)]
+
+
+def _normal(shape, seed, gpu, std=1.0, outliers=False):
+    """Normal values drawn on the GPU (the wide weights here would take seconds on the CPU)."""
+    g = torch.Generator(device=gpu).manual_seed(seed)
+    x = torch.empty(shape, dtype=torch.bfloat16, device=gpu).normal_(0.0, std, generator=g)
+    if outliers:
+        x.view(-1)[torch.randint(0, x.numel(), (1 + x.numel() // 1000,), device=gpu, generator=g)] *= 50.0
+    return x
+
+
+def _both_tiles(run):
+    """What `run` gives under the default rule and with the 256 x 256 tiles of the general form."""
+    from hpfp8 import _lib
+    got = run()
+    _lib.load().hpfp8_debug_set_small_gemm(1)
+    try:
+        return got, run()
+    finally:
+        _lib.load().hpfp8_debug_set_small_gemm(0)
+
+
+@pytest.mark.parametrize("m", [1, 8, 9, 23, 37, 48, 57, 64])
+@pytest.mark.parametrize("n,k", FEW_ROWS_SHAPES)
+def test_gemm_with_few_rows_has_the_bits_of_the_general_form(gpu, m, n, k):
+    """Random values, so that the order and the rounding of the sums show: an element of c does not depend on how many
+    rows there are or which kernel computes it.  Against 64 bits: what the matrix instruction leaves of products some 2^12
+    times smaller than the largest of its 128 (test_gpu_gemm.py measures that and derives the 1e-4 used here)."""
+    from hpfp8 import ops
+    x, w = _normal((m, k), 1, gpu, outliers=True), _normal((n, k), 2, gpu, 0.02)
+    bias = _normal((n,), 3, gpu)
+    for pow2 in (False, True):
+        a, sa = ops.quantize_1x128(x, kmajor=True, pow2=pow2)
+        b, sb = ops.quantize_128x128(w, pow2=pow2)
+        got, want = _both_tiles(lambda: ops.gemm_blockwise(a, sa, b, sb, pow2_scales=pow2, out_dtype=torch.float32))
+        assert torch.equal(got, want)
+        exact = _dequantized(a, sa.contiguous(), 1) @ _dequantized(b, sb, 128).t()
+        assert float((got.double() - exact).norm() / exact.norm()) < 1e-4
+        got, want = _both_tiles(lambda: ops.gemm_blockwise(a, sa.contiguous(), b, sb, bias=bias, pow2_scales=pow2))
+        assert torch.equal(got, want)
+    a, _, sa = ops.quantize_per_tensor(x)
+    b, _, sb = ops.quantize_per_tensor(w)
+    got, want = _both_tiles(lambda: ops.gemm_per_tensor(a, sa, b, sb, out_dtype=torch.float32))
+    assert torch.equal(got, want)
+    got, want = _both_tiles(lambda: ops.gemm_per_tensor(a, sa, b, sb, bias=bias))
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("m", [1, 17, 40, 64])
+@pytest.mark.parametrize("n,k", [(1152, 2432), (8320, 2176), (16384, 2432)])
+def test_gemm_with_few_rows_on_rows_with_strides(gpu, m, n, k):
+    """Row strides of a, b and c beyond the width: the same bits, and c untouched outside its columns and rows."""
+    from hpfp8 import _lib, ops
+    x, w = _normal((m, k), 1, gpu), _normal((n, k), 2, gpu, 0.02)
+    a, sa = ops.quantize_1x128(x, kmajor=True)
+    b, sb = ops.quantize_128x128(w)
+    want = ops.gemm_blockwise(a, sa, b, sb)
+    a8, b8 = _strided_rows(a.view(torch.uint8), 48, gpu), _strided_rows(b.view(torch.uint8), 16, gpu)
+    c = torch.full((m + 3, n + 24), 7.0, dtype=torch.bfloat16, device=gpu)
+    _lib.call("hpfp8_gemm_blockwise", a8.data_ptr(), a8.stride(0), sa.data_ptr(), sa.stride(0), sa.stride(1), b8.data_ptr(),
+              b8.stride(0), sb.data_ptr(), sb.stride(0), sb.stride(1), 128, m, n, k, None, c.data_ptr(), c.stride(0), _lib.OUT_BF16, 0,
+              ops._stream())
+    assert torch.equal(c[:m, :n], want)
+    assert bool((c[:m, n:] == 7.0).all()) and bool((c[m:] == 7.0).all())
+
+
+@pytest.mark.parametrize("m", [2, 9, 33, 64])
+@pytest.mark.parametrize("pow2", [False, True])
+def test_gemm_with_few_rows_keeps_nan_and_infinity_to_their_rows(gpu, m, pow2):
+    """A NaN code, a NaN scale and an infinite scale in a row of a, a NaN code in a row of b: that row or column of c as the
+    general form has it, every other element unchanged."""
+    from hpfp8 import ops
+    n, k = 8320, 2432
+    x, w = _normal((m, k), 1, gpu), _normal((n, k), 2, gpu, 0.02)
+    a, sa = ops.quantize_1x128(x, kmajor=True, pow2=pow2)
+    b, sb = ops.quantize_128x128(w, pow2=pow2)
+    clean = ops.gemm_blockwise(a, sa, b, sb, pow2_scales=pow2)
+    bad = m // 2
+    for what in ("code", "nan", "inf", "weight"):
+        a2, s2, b2 = a.clone(), sa.t().clone().t(), b.clone()
+        if what == "code":
+            a2.view(torch.uint8)[bad, 200] = 0x7F
+        elif what == "weight":
+            b2.view(torch.uint8)[4000, k - 1] = 0xFF
+        else:
+            s2[bad, 3] = float(what)
+        got, want = _both_tiles(lambda: ops.gemm_blockwise(a2, s2, b2, sb, pow2_scales=pow2))
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16)) or torch.equal(got.nan_to_num(7.0), want.nan_to_num(7.0))
+        keep = torch.ones((m, n), dtype=torch.bool, device=gpu)
+        if what == "weight":
+            assert bool(got[:, 4000].isnan().all())
+            keep[:, 4000] = False
+        else:
+            assert not bool(got[bad].isfinite().all())
+            keep[bad] = False
+        assert torch.equal(got[keep], clean[keep])
+
+
+def test_gemm_with_few_rows_and_power_of_two_scales_whose_product_is_out_of_range(gpu):
+    """Two scales of 2^80: their product is no fp32 number, but a product of codes that is zero stays zero."""
+    from hpfp8 import ops
+    m, n, k = 5, 256, 2048
+    a, b = _ints((m, k), 1, gpu), _ints((n, k), 2, gpu)
+    a.view(torch.uint8)[:, 128:256] = 0
+    sa = torch.ones((m, k // 128), dtype=torch.float32, device=gpu)
+    sb = torch.ones((n // 128, k // 128), dtype=torch.float32, device=gpu)
+    want = ops.gemm_blockwise(a, sa, b, sb, pow2_scales=True, out_dtype=torch.float32)
+    sa[:, 1], sb[:, 1] = 2.0 ** 80, 2.0 ** 80
+    assert torch.equal(ops.gemm_blockwise(a, sa, b, sb, pow2_scales=True, out_dtype=torch.float32), want)
+
+
+def test_gemm_with_few_rows_does_not_depend_on_the_column_or_the_batch(gpu):
+    """The same rows of b in other places (a column shard, a rolled weight) and more rows of a: the same bits."""
+    from hpfp8 import ops
+    n, k = 7168, 16384
+    x, w = _normal((65, k), 1, gpu), _normal((n, k), 2, gpu, 0.02)
+    a, sa = ops.quantize_1x128(x, kmajor=True)
+    b, sb = ops.quantize_128x128(w)
+    c = ops.gemm_blockwise(a, sa, b, sb)
+    for m in (1, 8, 37, 64):
+        am, sm = ops.quantize_1x128(x[:m], kmajor=True)
+        assert torch.equal(ops.gemm_blockwise(am, sm, b, sb), c[:m])
+        half = ops.gemm_blockwise(am, sm, b[n // 2:], sb[n // 256:])
+        assert torch.equal(half, c[:m, n // 2:])
+        rolled = ops.gemm_blockwise(am, sm, b.view(torch.uint8).roll(1280, 0).view(b.dtype), sb.roll(10, 0))
+        assert torch.equal(rolled, c[:m].roll(1280, 1))
+
+
+@pytest.mark.parametrize("m", [1, 37, 64, 65])
+@pytest.mark.parametrize("fast", [False, True])
+@pytest.mark.parametrize("pow2_in,pow2_out", [(False, False), (True, False), (False, True), (True, True)])
+def test_swiglu_epilogue_is_its_two_calls_at_decode_row_counts(gpu, m, fast, pow2_in, pow2_out):
+    """What `hpfp8_gemm_blockwise_swiglu_quantize` promises, on both sides of the few-rows GEMM's last row count: bit for bit
+    the GEMM followed by the SwiGLU quantizer, by the C entry point and by the operator, which takes two launches there."""
+    from hpfp8 import _lib, ops
+    k, inter = 7168, 4608
+    x, w = _normal((m, k), 1, gpu), _normal((2 * inter, k), 2, gpu, 0.05)
+    a, sa = ops.quantize_1x128(x, kmajor=True, pow2=pow2_in)
+    b, sb = ops.quantize_128x128(w, pow2=pow2_in)
+    h = ops.gemm_blockwise(a, sa, b, sb, pow2_scales=pow2_in)
+    q, si = ops.swiglu_quantize_1x128(h, fast=fast, pow2=pow2_out)
+    cq = torch.zeros((m, inter), dtype=torch.uint8, device=gpu)
+    cs, csi = (torch.zeros((inter // 128, m), dtype=torch.float32, device=gpu) for _ in range(2))
+    _lib.call("hpfp8_gemm_blockwise_swiglu_quantize", a.data_ptr(), k, sa.data_ptr(), sa.stride(0), sa.stride(1), b.data_ptr(), k,
+              sb.data_ptr(), sb.stride(0), sb.stride(1), m, inter, k, int(fast), int(pow2_in), int(pow2_out), cq.data_ptr(), inter,
+              cs.data_ptr(), csi.data_ptr(), ops._stream())
+    assert torch.equal(cq, q.view(torch.uint8)) and torch.equal(csi.t(), si)
+    got = ops.gemm_blockwise_swiglu_quantize(a, sa, b, sb, fast=fast, pow2_scales=pow2_in, pow2_out=pow2_out, want_scale=True)
+    assert torch.equal(got[0].view(torch.uint8), cq) and torch.equal(got[1], si) and torch.equal(got[2], cs.t())
 
 
 @pytest.mark.parametrize("counts", [[1], [0, 1, 0], [16, 17, 32, 0, 33], [48, 49, 0, 64, 65, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0],
