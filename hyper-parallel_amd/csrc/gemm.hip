@@ -1144,9 +1144,13 @@ static bool use_small_kernel(int64_t M, int64_t N) {
 
 // Few rows of a (decode): bound by reading b once, which the tile kernels do not reach (gemm_skinny.hip; 8 rows of
 // [7168, 16384]: 60 us with 64 x 128 tiles, 20.6 us; 64 rows: 64 and 26.8 us; 37 rows of [36864, 7168]: 81 us with 256 x 256
-// tiles, 41.6 us), with the same bits.  Hands the problem over if it is one; otherwise false.
+// tiles, 41.6 us), with the same bits.  try_skinny hands the problem over if it is one; otherwise false.
+static int64_t few_rows(int64_t K) {        // the most rows that count as few
+  return K >= kSkinnyMinK && g_small_gemm_mode.load(std::memory_order_relaxed) == 0 ? kSkinnyMaxRows : 0;
+}
+
 static bool try_skinny(const GemmParams& p, SkinnyMode mode, int out_type, hipStream_t stream, int& rc) {
-  if (p.M > kSkinnyMaxRows || p.K < kSkinnyMinK || p.accumulate || g_small_gemm_mode.load(std::memory_order_relaxed) != 0) return false;
+  if (p.accumulate || p.M > few_rows(p.K)) return false;
   SkinnyParams q{};
   q.a = p.a; q.b = p.b; q.sa = p.sa; q.sb = p.sb; q.lda = p.lda; q.ldb = p.ldb;
   q.sa_sm = p.sa_sm; q.sa_sk = p.sa_sk; q.sb_sn = p.sb_sn; q.sb_sk = p.sb_sk; q.sb_bytes = p.sb_bytes;
@@ -1355,6 +1359,8 @@ int hpfp8_gemm_blockwise_swiglu_quantize(const void* a, int64_t lda, const float
 }
 
 void hpfp8_debug_set_small_gemm(int mode) { g_small_gemm_mode.store(mode == 1 || mode == 2 ? mode : 0, std::memory_order_relaxed); }
+
+int64_t hpfp8_gemm_few_rows(int64_t K) { return few_rows(K); }
 
 int hpfp8_gemm_per_tensor(const void* a, int64_t lda, const float* sa_inv, const void* b, int64_t ldb,
                           const float* sb_inv, int64_t M, int64_t N, int64_t K, const void* bias, void* c,

@@ -78,6 +78,7 @@ SIGNATURES = {
 SIZE_FUNCTIONS = {
     "hpfp8_grouped_padded_rows": [_int, _i64],
     "hpfp8_grouped_layout_words": [_int, _i64],
+    "hpfp8_gemm_few_rows": [_i64],
 }
 
 OUT_BF16, OUT_F32 = 0, 1

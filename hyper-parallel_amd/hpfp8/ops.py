@@ -17,7 +17,6 @@ import torch
 from . import _lib
 
 BLOCK = 128
-_FEW_ROWS, _FEW_ROWS_K = 64, 2048      # up to so many rows of a, from this contraction on, a GEMM takes its few-rows form
 FP8 = torch.float8_e4m3fn
 
 
@@ -637,10 +636,10 @@ def gemm_blockwise_swiglu_quantize(a: torch.Tensor, sa: torch.Tensor, b: torch.T
     q = torch.empty((m, inter), dtype=FP8, device=a.device)
     s_inv = torch.empty((inter // BLOCK, m), dtype=torch.float32, device=a.device)
     s = torch.empty_like(s_inv) if want_scale else None
-    if 0 < m <= _FEW_ROWS and k >= _FEW_ROWS_K:
+    if 0 < m <= _lib.load().hpfp8_gemm_few_rows(k):
         # A decode step: the GEMM is bound by reading the weight, which its few-rows form does at twice the rate of the
         # 256 x 256 tiles the epilogue belongs to; gate | up is a few megabytes (37 rows of a [36864, 7168] weight: 86 us
-        # for the epilogue form, 57 + 4 us for the two launches).
+        # for the epilogue form, 42 + 5 us for the two launches, the same bits).
         h = gemm_blockwise(a, sa, b, sb, pow2_scales=pow2_scales)
         if fast:
             _lib.call("hpfp8_swiglu_quantize_1x128_fast_bf16", _ptr(h), m, inter, n, 1, int(pow2_out), _ptr(q), _ptr(s), _ptr(s_inv),

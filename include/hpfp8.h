@@ -385,6 +385,11 @@ int hpfp8_gemm_per_tensor(const void* a, int64_t lda, const float* sa_inv, const
  * where the form has one (process-wide, stored atomically, takes effect with the next launch). */
 void hpfp8_debug_set_small_gemm(int mode);
 
+/* The largest number of rows of a with which hpfp8_gemm_blockwise[_pow2] (sb_gran = 128, no accumulate) and
+ * hpfp8_gemm_per_tensor take their few-rows form at contraction K (0: none): a caller that can choose between a fused call
+ * and one of these followed by another launch asks here. */
+int64_t hpfp8_gemm_few_rows(int64_t K);
+
 /* MoE grouped form (one rank's local experts; no counterpart in the reference, whose expert
  * parallelism is unimplemented): rows of a[total_m, K] (row stride lda) are sorted by expert; offs[e] (int32,
  * device) is the inclusive prefix sum of per-expert row counts, a count may be 0, rows past

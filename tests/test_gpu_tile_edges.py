@@ -223,6 +223,27 @@ def test_swiglu_epilogue_is_its_two_calls_at_decode_row_counts(gpu, m, fast, pow
     assert torch.equal(got[0].view(torch.uint8), cq) and torch.equal(got[1], si) and torch.equal(got[2], cs.t())
 
 
+@pytest.mark.parametrize("m", [64, 65])
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_swiglu_operator_takes_two_launches_where_the_gemm_takes_few_rows(gpu, m, mode, monkeypatch):
+    """One rule for both, the library's: the operator splits exactly where the GEMM would take its few-rows form, so a tile
+    that the test hook asks for reaches the epilogue it belongs to."""
+    from hpfp8 import _lib, ops
+    k, inter = 2048, 128
+    a, sa = ops.quantize_1x128(_normal((m, k), 1, gpu), kmajor=True)
+    b, sb = ops.quantize_128x128(_normal((2 * inter, k), 2, gpu, 0.05))
+    names, call = [], _lib.call
+    monkeypatch.setattr(_lib, "call", lambda name, *args: (names.append(name), call(name, *args))[1])
+    _lib.load().hpfp8_debug_set_small_gemm(mode)
+    try:
+        few = m <= _lib.load().hpfp8_gemm_few_rows(k)
+        ops.gemm_blockwise_swiglu_quantize(a, sa, b, sb)
+    finally:
+        _lib.load().hpfp8_debug_set_small_gemm(0)
+    assert few == (m == 64 and mode == 0)
+    assert names == (["hpfp8_gemm_blockwise", "hpfp8_swiglu_quantize_1x128_bf16"] if few else ["hpfp8_gemm_blockwise_swiglu_quantize"])
+
+
 @pytest.mark.parametrize("counts", [[1], [0, 1, 0], [16, 17, 32, 0, 33], [48, 49, 0, 64, 65, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0],
                                     [200] + [0] * 69 + [3, 0, 7], [5] * 130])
 @pytest.mark.parametrize("n,k", [(128, 128), (384, 640), (256, 2176)])
