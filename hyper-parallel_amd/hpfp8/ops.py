@@ -636,7 +636,8 @@ def gemm_blockwise_swiglu_quantize(a: torch.Tensor, sa: torch.Tensor, b: torch.T
     q = torch.empty((m, inter), dtype=FP8, device=a.device)
     s_inv = torch.empty((inter // BLOCK, m), dtype=torch.float32, device=a.device)
     s = torch.empty_like(s_inv) if want_scale else None
-    if 0 < m <= _lib.load().hpfp8_gemm_few_rows(k):
+    # (a weight that spans 2 GiB or more is left to the fused call, which refuses it at every row count)
+    if 0 < m <= _lib.load().hpfp8_gemm_few_rows(k) and n * _ld(b) < 0x7FFFF000:
         # A decode step: the GEMM is bound by reading the weight, which its few-rows form does at twice the rate of the
         # 256 x 256 tiles the epilogue belongs to; gate | up is a few megabytes (37 rows of a [36864, 7168] weight: 86 us
         # for the epilogue form, 42 + 5 us for the two launches, the same bits).

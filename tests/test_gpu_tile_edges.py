@@ -244,6 +244,18 @@ def test_swiglu_operator_takes_two_launches_where_the_gemm_takes_few_rows(gpu, m
     assert names == (["hpfp8_gemm_blockwise", "hpfp8_swiglu_quantize_1x128_bf16"] if few else ["hpfp8_gemm_blockwise_swiglu_quantize"])
 
 
+@pytest.mark.parametrize("m", [1, 64, 65])
+def test_swiglu_operator_refuses_a_weight_of_two_gib_at_every_row_count(gpu, m):
+    """512 rows of codes 4 MiB apart: what the fused call refuses is not taken on where the operator would split it."""
+    from hpfp8 import _lib, ops
+    k = 2048
+    b = torch.empty(512 << 22, dtype=torch.uint8, device=gpu).view(512, 1 << 22)[:, :k]
+    a = torch.zeros((m, k), dtype=torch.uint8, device=gpu)
+    sa, sb = torch.ones((m, k // 128), device=gpu), torch.ones((4, k // 128), device=gpu)
+    with pytest.raises(_lib.Hpfp8Error, match="2 GiB"):
+        ops.gemm_blockwise_swiglu_quantize(a, sa, b, sb)
+
+
 @pytest.mark.parametrize("counts", [[1], [0, 1, 0], [16, 17, 32, 0, 33], [48, 49, 0, 64, 65, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0],
                                     [200] + [0] * 69 + [3, 0, 7], [5] * 130])
 @pytest.mark.parametrize("n,k", [(128, 128), (384, 640), (256, 2176)])
