@@ -1065,8 +1065,8 @@ __global__ __launch_bounds__(kSmallThreads) void gemm_small_kernel(const GemmPar
   }
 }
 
-// Test hook.  0: pick_shape and use_small_kernel choose the tile; 1: always 256 x 256; 2: 64 x 128 where 128 x 128 tiles
-// would be fewer than the compute units and 128 x 128 otherwise, whenever the form allows it
+// Test hook.  0: pick_shape and the rules below choose the form; 1: always 256 x 256 tiles; 2: the smallest tile a form has
+// (64 x 128 where 128 x 128 tiles would be fewer than the compute units); 3: 128 x 256 tiles where a form has them
 static std::atomic<int> g_small_gemm_mode{0};   // (atomic: the test hook may be called from any thread)
 
 // Workgroups to launch for `tiles` tiles: at most one per CU, a multiple of 8 (one share per XCD) unless there are fewer
@@ -1107,8 +1107,7 @@ static int64_t tile_count(int64_t M, int64_t N, TileShape shape) {
 //   (168 / 336 / 672 tiles) 29 / 36 / 32, pow2 2048 x 7168 x 4096 48 / 56 / 61
 static TileShape pick_shape(int64_t M, int64_t N) {
   const int mode = g_small_gemm_mode.load(std::memory_order_relaxed);
-  if (mode == 1) return k256x256;
-  if (mode == 2) return k128x128;
+  if (mode != 0) return mode == 1 ? k256x256 : (mode == 2 ? k128x128 : k128x256);
   const int64_t cus = persistent_grid((int64_t)1 << 40);
   if (tile_count(M, N, k128x128) <= cus) return k128x128;
   if (tile_count(M, N, k128x256) <= cus) return k128x256;
@@ -1118,7 +1117,8 @@ static TileShape pick_shape(int64_t M, int64_t N) {
 // SwiGLU epilogue: a tile's columns are the gate and the up half of one scaling group, 256 in all
 // (500 x 8192 x 4096: 52 us with 64 tiles of 256 rows, 37 with 128 of 128 rows; 1000 x 12288 x 4096, 192 and 384: 62, 81).
 static TileShape pick_shape_swiglu(int64_t M, int64_t N) {
-  if (g_small_gemm_mode.load(std::memory_order_relaxed) != 0) return k256x256;
+  const int mode = g_small_gemm_mode.load(std::memory_order_relaxed);
+  if (mode != 0) return mode == 1 ? k256x256 : k128x256;
   return tile_count(M, N, k128x256) <= persistent_grid((int64_t)1 << 40) ? k128x256 : k256x256;
 }
 
@@ -1127,7 +1127,8 @@ static TileShape pick_shape_swiglu(int64_t M, int64_t N) {
 // 389 / 531 us with 256 x 256 tiles, 147 / 176 / 214 / 344 / 606 with 128 x 256).  The rows of an expert are known on the
 // device only: the rule goes by their average, and by whether even the largest number of tiles is one round.
 static TileShape pick_shape_grouped(int64_t M, int64_t N, int experts) {
-  if (g_small_gemm_mode.load(std::memory_order_relaxed) == 1) return k256x256;
+  const int mode = g_small_gemm_mode.load(std::memory_order_relaxed);
+  if (mode != 0) return mode == 1 ? k256x256 : k128x256;
   const int64_t most = (M / 128 + experts) * ((N + 255) / 256);
   return M <= (int64_t)256 * experts || most <= persistent_grid((int64_t)1 << 40) ? k128x256 : k256x256;
 }
@@ -1136,7 +1137,7 @@ static TileShape pick_shape_grouped(int64_t M, int64_t N, int experts) {
 // with 128 x 128 tiles, 700 x 1024 x 8192: 32 against 46).
 static bool use_small_kernel(int64_t M, int64_t N) {
   const int mode = g_small_gemm_mode.load(std::memory_order_relaxed);
-  if (mode == 1) return false;
+  if (mode == 1 || mode == 3) return false;
   const int64_t cus = persistent_grid((int64_t)1 << 40);
   if (mode == 2) return tile_count(M, N, k128x128) < cus;
   return ((M + kSmallRows - 1) / kSmallRows) * (N / kSmallTile) <= cus;
@@ -1358,7 +1359,7 @@ int hpfp8_gemm_blockwise_swiglu_quantize(const void* a, int64_t lda, const float
   return check_launch(what);
 }
 
-void hpfp8_debug_set_small_gemm(int mode) { g_small_gemm_mode.store(mode == 1 || mode == 2 ? mode : 0, std::memory_order_relaxed); }
+void hpfp8_debug_set_small_gemm(int mode) { g_small_gemm_mode.store(mode >= 1 && mode <= 3 ? mode : 0, std::memory_order_relaxed); }
 
 int64_t hpfp8_gemm_few_rows(int64_t K) { return few_rows(K); }
 

@@ -381,8 +381,9 @@ int hpfp8_gemm_per_tensor(const void* a, int64_t lda, const float* sa_inv, const
  * 256 otherwise; the grouped forms take 128 x 256 for few rows per expert.  With at most 64 rows and K >= 2048
  * hpfp8_gemm_per_tensor and hpfp8_gemm_blockwise[_pow2] with sb_gran = 128 (no accumulate) take a form that reads b once at
  * the memory's rate.  Same arithmetic in the same order in all of them: an element of c has the same bits in each, so it
- * depends neither on the number of rows nor on where b's rows stand (a column shard).  Test hook, not part of the path: mode 0 = that rule (default), 1 = always 256 x 256, 2 = always a small tile
- * where the form has one (process-wide, stored atomically, takes effect with the next launch). */
+ * depends neither on the number of rows nor on where b's rows stand (a column shard).  Test hook, not part of the path: mode
+ * 0 = that rule (default), 1 = always 256 x 256 tiles, 2 = the smallest tile a form has, 3 = 128 x 256 tiles where a form has
+ * them; 1 to 3 without the few-rows form (process-wide, stored atomically, takes effect with the next launch). */
 void hpfp8_debug_set_small_gemm(int mode);
 
 /* The largest number of rows of a with which hpfp8_gemm_blockwise[_pow2] (sb_gran = 128, no accumulate) and

@@ -723,8 +723,8 @@ def test_small_tile_kernel_equals_the_large_tile_kernel_and_the_oracle(gpu, shap
     """The small-tile kernel (problems with few tiles: BASELINE configuration 1, decode-sized M) does the same
     arithmetic in the same order as the 256 x 256-tile kernel: identical bits for the block and the per-tensor
     form, fp32 and bf16 output, with and without bias, ragged M; and the fp32 output agrees with the oracle as the
-    large kernel's does.  Both of its tile heights are covered: 64 rows where 128 x 128 tiles would be fewer than the
-    256 compute units (the first six shapes), 128 rows otherwise (288 and 264 such tiles in the last two)."""
+    large kernel's does.  Mode 2 is that kernel (64 x 128 tiles) where 128 x 128 tiles would be fewer than the 256
+    compute units (the first six shapes) and 128 x 128 tiles of the large kernel otherwise (288 and 264 of them)."""
     import hpfp8
     m, n, k = shape
     x = U.randn_bf16((m, k), 40 + m, 1.0, 0.001, 30.0).to(gpu)

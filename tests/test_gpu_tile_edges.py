@@ -260,8 +260,9 @@ def test_swiglu_operator_refuses_a_weight_of_two_gib_at_every_row_count(gpu, m):
                                     [200] + [0] * 69 + [3, 0, 7], [5] * 130])
 @pytest.mark.parametrize("n,k", [(128, 128), (384, 640), (256, 2176)])
 def test_grouped_gemm_with_few_rows_is_exact_on_integer_inputs(gpu, counts, n, k):
-    """Row counts around every fragment count and around the 64-row chunks, empty experts, more experts than a wave has
-    lanes, fewer units than workgroups; rows past the last offset stay as they are.  Exact for the reason above."""
+    """Experts of a few rows each, so that every tile is a partial one; empty experts, many of them in a row, more experts
+    than a wave has lanes, fewer tiles than workgroups; rows past the last offset stay as they are.  Exact for the reason
+    above."""
     from hpfp8 import _lib, ops
     e, rows = len(counts), sum(counts) + 2
     a, b = _ints((rows, k), 1, gpu), _ints((e * n, k), 2, gpu)
@@ -318,6 +319,46 @@ def test_gemm_tiles_are_exact_on_integer_inputs(gpu, m, n, k):
     ta, tb = torch.tensor(0.5, device=gpu), torch.tensor(0.25, device=gpu)
     assert torch.equal(ops.gemm_per_tensor(a, ta, b, tb, out_dtype=torch.float32).double(), one)
     assert torch.equal(ops.gemm_per_tensor(a, ta, b, tb, bias=bias), (one + bias.double()).to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 128, 128), (127, 384, 256), (129, 640, 640), (300, 2432, 384), (1000, 1152, 1152)])
+def test_every_tile_shape_gives_the_same_bits(gpu, m, n, k):
+    """256 x 256, 128 x 256, 128 x 128 and 64 x 128 tiles, asked for one after the other (so whatever the number of compute
+    units) on random values: all scale forms, output types, bias, accumulation, the SwiGLU epilogue and experts."""
+    from hpfp8 import _lib, ops
+    x, w = _normal((m, k), 1, gpu, outliers=True), _normal((2 * n, k), 2, gpu, 0.05)
+    bias, c0 = _normal((n,), 3, gpu), _normal((m, n), 4, gpu).float()
+    rows = torch.tensor([m // 3, 0, m - m // 3]).cumsum(0).to(torch.int32).to(gpu)
+    out = {}
+    for mode in (1, 2, 3):
+        _lib.load().hpfp8_debug_set_small_gemm(mode)
+        try:
+            r = out[mode] = []
+            for pow2 in (False, True):
+                a, sa = ops.quantize_1x128(x, kmajor=True, pow2=pow2)
+                b, sb = ops.quantize_128x128(w, pow2=pow2)
+                br, sr = ops.quantize_1x128(w[:n], kmajor=True, pow2=pow2)
+                b1, sb1 = b[:n], sb[:n // 128]
+                r.append(ops.gemm_blockwise(a, sa, b1, sb1, pow2_scales=pow2, out_dtype=torch.float32))
+                r.append(ops.gemm_blockwise(a, sa.contiguous(), b1, sb1, bias=bias, pow2_scales=pow2))
+                r.append(ops.gemm_blockwise(a, sa, br, sr, sb_gran=1, pow2_scales=pow2))
+                for gran, bb, ss in ((128, b1, sb1), (1, br, sr)):
+                    r.append(ops.gemm_blockwise(a, sa, bb, ss, sb_gran=gran, out=c0.clone(), accumulate=True, pow2_scales=pow2))
+                r += ops.gemm_blockwise_swiglu_quantize(a, sa, b, sb, fast=pow2, pow2_scales=pow2, pow2_out=pow2, want_scale=True)
+                stack = b.view(2, n, k), sb.view(2, n // 128, k // 128)
+                experts = [torch.cat((t, t[:1])) if t.dtype == torch.float32 else torch.cat((t.view(torch.uint8), t[:1].view(torch.uint8)))
+                           for t in stack]
+                r.append(ops.gemm_grouped_blockwise(a, sa, *experts, rows, pow2_scales=pow2))
+            a, _, sa = ops.quantize_per_tensor(x)
+            b, _, sb = ops.quantize_per_tensor(w[:n])
+            r.append(ops.gemm_per_tensor(a, sa, b, sb, out_dtype=torch.float32))
+            r.append(ops.gemm_per_tensor(a, sa, b, sb, bias=bias))
+        finally:
+            _lib.load().hpfp8_debug_set_small_gemm(0)
+    for mode in (2, 3):
+        for got, want in zip(out[mode], out[1]):
+            assert torch.equal(got.view(torch.uint8) if got.dtype == torch.float8_e4m3fn else got,
+                               want.view(torch.uint8) if want.dtype == torch.float8_e4m3fn else want)
 
 
 @pytest.mark.parametrize("m,inter,k", [(65, 128, 128), (127, 384, 384), (129, 1280, 256), (300, 10752, 128)])
