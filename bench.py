@@ -31,18 +31,29 @@ PEAK_FP8_TFLOPS = 5000.0     # MI355X dense FP8 MFMA
 PEAK_HBM_GBS = 8000.0        # MI355X HBM3E
 # Bytes per GEMM launch that crossed the L2 <-> memory-fabric boundary come from rocprofv3 --pmc runs (FETCH_SIZE,
 # calibrated on a copy of known size, + WRITE_SIZE; and the requests among them destined for the memory controller)
-# whose summary is kept in PROFILE together with the sha256 of the kernel source it was measured on; the figure is
-# only reported while csrc/gemm.hip is still that source (otherwise `traffic` is null, with a line on stderr, until
-# the counters are collected again).
+# whose summary is kept in PROFILE together with the sha256 of the kernel it was measured on (its source, the headers that
+# it is made of, the compiler's options); the figure is only reported while that is still so (otherwise `traffic` is null,
+# with a line on stderr, until the counters are collected again).
 PROFILE = os.path.join(ROOT, "profiles", "bench_cfg2_gemm_blockwise_and_quantizers.md")
-GEMM_SOURCE = os.path.join(ROOT, "hyper-parallel_amd", "csrc", "gemm.hip")
+GEMM_SOURCES = [os.path.join(ROOT, "hyper-parallel_amd", "csrc", name) for name in ("gemm.hip", "gemm_tile.h", "hpfp8_device.h")]
 
 
-def gemm_source_digest(path=GEMM_SOURCE):
-    """sha256 of csrc/gemm.hip: the profile summary records the digest of the source its counters were collected on."""
+def gemm_source_digest(paths=None, flags=None):
+    """sha256 of csrc/gemm.hip, the headers it is made of and the compiler's options: the profile summary records the digest
+    of what its counters were collected on."""
     import hashlib
-    with open(path, "rb") as f:
-        return hashlib.sha256(f.read()).hexdigest()
+    import importlib.util
+    if flags is None:
+        spec = importlib.util.spec_from_file_location("hpfp8_build", os.path.join(ROOT, "hyper-parallel_amd", "build.py"))
+        build = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(build)
+        flags = build._flags()
+    h = hashlib.sha256()
+    for path in GEMM_SOURCES if paths is None else paths:
+        with open(path, "rb") as f:
+            h.update(f.read() + b"\0")
+    h.update("\0".join(flags).encode())
+    return h.hexdigest()
 
 
 def gemm_traffic_bytes():
@@ -58,7 +69,7 @@ def gemm_traffic_bytes():
     if not m:
         return None, "profile summary has no traffic line"
     if m.group(3) != gemm_source_digest():
-        why = ("profiles/%s was collected on another version of csrc/gemm.hip (its digest %s..., the source's %s...): "
+        why = ("profiles/%s was collected on another version of the GEMM (its digest %s..., the tree's %s...): "
                "collect FETCH_SIZE / WRITE_SIZE again" % (os.path.basename(PROFILE), m.group(3)[:12], gemm_source_digest()[:12]))
         print("bench.py: STALE TRAFFIC FIGURE NOT REPORTED: " + why, file=sys.stderr, flush=True)
         return None, why

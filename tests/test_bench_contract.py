@@ -56,3 +56,23 @@ def test_reported_gemm_traffic_belongs_to_the_kernel_as_it_is_now(tmp_path, monk
     if traffic is not None:
         assert traffic["tcc_ea"] > 2 * (4096 * 7168 + 36864 * 7168) and source.startswith("profiles/")      # at least the operands once
         assert 0 < traffic["dram_path"] <= traffic["tcc_ea"] * 1.05
+
+
+def test_gemm_digest_covers_the_headers_and_the_options(tmp_path):
+    """A counter figure belongs to the kernel that was measured: a change of the operand layout or the fragment reads, which
+    live in headers, or of an option of the compiler makes it another one."""
+    sys.path.insert(0, ROOT)
+    import bench
+    copies = []
+    for path in bench.GEMM_SOURCES:
+        copies.append(tmp_path / os.path.basename(path))
+        copies[-1].write_bytes(open(path, "rb").read())
+    digest = bench.gemm_source_digest([str(c) for c in copies])
+    assert digest == bench.gemm_source_digest()
+    assert {c.name for c in copies} >= {"gemm.hip", "gemm_tile.h", "hpfp8_device.h"}
+    for c in copies:
+        text = c.read_bytes()
+        c.write_bytes(text + b"// changed\n")
+        assert bench.gemm_source_digest([str(c) for c in copies]) != digest
+        c.write_bytes(text)
+    assert bench.gemm_source_digest(flags=["-O3"]) != digest
