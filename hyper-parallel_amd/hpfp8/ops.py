@@ -20,10 +20,16 @@ BLOCK = 128
 FP8 = torch.float8_e4m3fn
 
 
+# The current device and the handle of its current stream, asked for directly: the Stream object that
+# torch.cuda.current_stream() builds around the handle costs 3 us, more than a launch.  Both are private names of torch; one
+# that has them no longer is asked through the public ones.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda device: torch.cuda.current_stream(device).cuda_stream)
+_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
+
+
 def _stream() -> int:
-    """The handle of the current device's current stream (asked for directly: the Stream object that
-    torch.cuda.current_stream() builds around it costs 3 us, more than a launch)."""
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    """The handle of the current device's current stream."""
+    return _raw_stream(torch.cuda.current_device())
 
 
 def _ptr(t: Optional[torch.Tensor]):
@@ -35,7 +41,7 @@ def _check_device(x: torch.Tensor, name: str) -> None:
     GPU must be used under ``torch.cuda.device(x.device)``."""
     if not x.is_cuda:
         raise ValueError(f"{name} must live on the GPU (got device {x.device}); this path has no CPU fallback")
-    if x.get_device() != torch._C._cuda_getDevice():
+    if x.get_device() != _device():
         raise ValueError(f"{name} lives on {x.device} but the current device is cuda:{torch.cuda.current_device()}; "
                          f"call under torch.cuda.device({name}.device)")
 

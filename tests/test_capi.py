@@ -118,3 +118,20 @@ def test_python_wrappers_reject_cpu_tensors_and_bad_shapes():
         hpfp8.Fp8Linear(100, 128)
     with pytest.raises(ValueError):
         hpfp8.quantize_bucket(torch.zeros(100, dtype=torch.bfloat16))
+
+
+def test_operators_load_on_a_torch_without_the_private_stream_names(monkeypatch):
+    """The current stream and device are asked of torch by private names where it has them; without them the public ones
+    serve."""
+    import importlib.util
+    import torch
+    import hpfp8
+    from hpfp8 import ops
+    for name in ("_cuda_getCurrentRawStream", "_cuda_getDevice"):
+        monkeypatch.delattr(torch._C, name, raising=False)
+    spec = importlib.util.spec_from_file_location("hpfp8._ops_again", ops.__file__)
+    again = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(again)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 3)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: type("S", (), {"cuda_stream": 70 + device})())
+    assert again._stream() == 73
