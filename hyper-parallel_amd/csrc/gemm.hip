@@ -82,6 +82,7 @@ struct GemmParams {
   int pow2_out;
   float* q_scale;
   float* q_scale_inv;
+  int choose_cus;         // grouped by rows: launched with both tile heights, the kernel of the better one runs (0: the only one)
 };
 
 // Tile number -> (m tile, n tile).  Consecutive numbers (one XCD's CUs at any moment) cover
@@ -142,6 +143,35 @@ __device__ __forceinline__ int expert_end(int off, int prev, int total_rows) {
   return lo < total_rows ? lo : total_rows;
 }
 
+// Grouped by rows, launched with both tile heights: whether 128-row tiles are the better ones for the rows that the experts
+// have.  A round of them takes three fifths of one of 256-row tiles.  (64 experts at a time, one per lane: an expert's end is
+// the largest offset up to its own, as expert_end gives it one after the other.)
+__device__ __forceinline__ bool better_is_low(const GemmParams& p, int tiles_n, int lane) {
+  int carry = 0, low = 0, high = 0;
+  for (int e0 = 0; e0 < p.experts; e0 += 64) {
+    int end = e0 + lane < p.experts ? p.offs[e0 + lane] : 0;
+#pragma unroll
+    for (int d = 1; d < 64; d *= 2) {
+      const int before = __shfl_up(end, d);
+      if (lane >= d && before > end) end = before;
+    }
+    end = expert_end(end, carry, p.M);
+    int prev = __shfl_up(end, 1);
+    if (lane == 0) prev = carry;
+    low += (end - prev + 127) / 128;
+    high += (end - prev + 255) / 256;
+    carry = __shfl(end, 63);
+  }
+#pragma unroll
+  for (int d = 1; d < 64; d *= 2) {
+    low += __shfl_xor(low, d);
+    high += __shfl_xor(high, d);
+  }
+  const int low_rounds = (low * tiles_n + p.choose_cus - 1) / p.choose_cus;
+  const int high_rounds = (high * tiles_n + p.choose_cus - 1) / p.choose_cus;
+  return __builtin_amdgcn_readfirstlane(3 * low_rounds <= 5 * high_rounds ? 1 : 0) != 0;
+}
+
 // WM, NS: the tile has 64 WM rows (WM pairs of waves) and 32 NS columns (a wave: NS subtiles of 16).
 // SA4: the activation scales have unit stride over rows (the k-block-major layout), so a lane's four
 // of them are one 16-byte load.
@@ -189,6 +219,7 @@ __global__ __launch_bounds__(128 * WM) void gemm_kernel(const GemmParams p) {
   int total_tiles = p.tiles;
   if (GROUPED == kGroupedK) total_tiles = p.experts * p.tiles;
   if (GROUPED == kGroupedRows) {
+    if (p.choose_cus && better_is_low(p, tiles_n, lane) != (TM == 128)) return;
     // tiles are numbered expert by expert; an expert with no rows has none
     int prev = 0, mt = 0;
     for (int e = 0; e < p.experts; ++e) {
@@ -1122,15 +1153,27 @@ static TileShape pick_shape_swiglu(int64_t M, int64_t N) {
   return tile_count(M, N, k128x256) <= persistent_grid((int64_t)1 << 40) ? k128x256 : k256x256;
 }
 
-// Grouped by rows: every expert ends in a partial tile, so with few rows per expert most of a 256-row tile is padding,
-// which costs as much as real rows (32 experts [4096, 7168], 64 / 512 / 2048 / 8192 / 16384 rows in all: 186 / 225 / 287 /
-// 389 / 531 us with 256 x 256 tiles, 147 / 176 / 214 / 344 / 606 with 128 x 256).  The rows of an expert are known on the
-// device only: the rule goes by their average, and by whether even the largest number of tiles is one round.
-static TileShape pick_shape_grouped(int64_t M, int64_t N, int experts) {
+// Grouped by rows: every expert ends in a partial tile, which costs as much as a whole one, so with few rows per expert low
+// tiles are better, with many (or the rows of many with one expert) high ones.  The rows of an expert are known on the device
+// only.  Even the largest number of low tiles is one round: low.  Of more than 256 rows per expert on average: high.  Low
+// tiles are at most M / 129 row tiles more than high ones: where that is a quarter of a round, low.  In between both kernels
+// are launched, count both kinds of tiles and one of them returns at once (3 to 5 us).  us with 128 / 256 rows per tile, for rows
+// spread evenly / by Zipf's law / half with one expert / all with one:
+//   32 experts [4096, 7168],   512 rows   187 / 257   167 / 207   209 / 267    49 / 69
+//                             4096 rows   175 / 235   267 / 278   226 / 295   112 / 99
+//                             8192 rows   281 / 234   338 / 366   392 / 320   224 / 187
+//                            16384 rows               606 / 531
+//   8 experts  [4096, 7168],  2048 rows    58 / 81     98 / 78    102 / 79     57 / 76
+//   64 experts [2048, 2048], 16384 rows    95 / 83    111 / 125   132 / 102    76 / 70
+enum GroupedTiles { kLowTiles, kHighTiles, kEitherTiles };
+
+static GroupedTiles pick_grouped(int64_t M, int64_t N, int experts) {
   const int mode = g_small_gemm_mode.load(std::memory_order_relaxed);
-  if (mode != 0) return mode == 1 ? k256x256 : k128x256;
-  const int64_t most = (M / 128 + experts) * ((N + 255) / 256);
-  return M <= (int64_t)256 * experts || most <= persistent_grid((int64_t)1 << 40) ? k128x256 : k256x256;
+  if (mode != 0) return mode == 1 ? kHighTiles : kLowTiles;
+  const int64_t cus = persistent_grid((int64_t)1 << 40), tiles_n = (N + 255) / 256;
+  if ((M / 128 + experts) * tiles_n <= cus) return kLowTiles;
+  if (M > (int64_t)256 * experts) return kHighTiles;
+  return M / 129 * tiles_n <= cus / 4 ? kLowTiles : kEitherTiles;
 }
 
 // 64 x 128 tiles, where that is still one round (dense, per tensor or by blocks; 256 x 7168 x 7168: 30 us against 41
@@ -1207,6 +1250,17 @@ static int launch(GemmParams p, int out_type, TileShape shape, hipStream_t strea
     if (shape == k128x128) return launch_shape<MODE, GROUPED, 2, 4>(p, out_type, tiles, stream);
   }
   return launch_shape<MODE, GROUPED, 4, 8>(p, out_type, tiles, stream);
+}
+
+template <int MODE>
+static int launch_grouped(GemmParams p, int out_type, hipStream_t stream) {
+  const GroupedTiles tiles = pick_grouped(p.M, p.N, p.experts);
+  p.choose_cus = tiles == kEitherTiles ? persistent_grid((int64_t)1 << 40) : 0;
+  if (tiles != kHighTiles) {
+    const int rc = launch<MODE, kGroupedRows>(p, out_type, k128x256, stream);
+    if (rc != HPFP8_OK || tiles == kLowTiles) return rc;
+  }
+  return launch<MODE, kGroupedRows>(p, out_type, k256x256, stream);
 }
 
 static int check_common(const char* what, const void* a, int64_t lda, const void* b, int64_t ldb, const float* sa,
@@ -1401,8 +1455,8 @@ static int gemm_grouped_impl(const void* a, int64_t lda, const float* sa, int64_
   p.sb_bytes = (int)sb_span;
   p.c = c; p.ldc = ldc; p.offs = offs; p.experts = experts;
   p.M = (int)total_m; p.N = (int)N; p.K = (int)K;
-  if (pow2) return launch<kScalePow2, kGroupedRows>(p, out_type, pick_shape_grouped(total_m, N, experts), (hipStream_t)stream);
-  return launch<kScaleBlock, kGroupedRows>(p, out_type, pick_shape_grouped(total_m, N, experts), (hipStream_t)stream);
+  if (pow2) return launch_grouped<kScalePow2>(p, out_type, (hipStream_t)stream);
+  return launch_grouped<kScaleBlock>(p, out_type, (hipStream_t)stream);
 }
 
 int hpfp8_gemm_grouped_blockwise(const void* a, int64_t lda, const float* sa, int64_t sa_stride_m, int64_t sa_stride_k,

@@ -385,6 +385,31 @@ def test_grouped_tiles_are_exact_on_integer_inputs(gpu, counts, n, k):
     test_grouped_gemm_with_few_rows_is_exact_on_integer_inputs(gpu, counts, n, k)
 
 
+@pytest.mark.parametrize("rows,experts,n", [(513, 8, 4096), (2048, 8, 4096), (2049, 8, 4096), (4096, 32, 2048), (8192, 32, 4096),
+                                            (1024, 4, 16384)])
+@pytest.mark.parametrize("spread", ["even", "zipf", "half", "two", "one", "none"])
+def test_grouped_gemm_leaves_the_tile_height_to_the_device(gpu, rows, experts, n, spread):
+    """Row counts at which the host cannot know which tile height is better and both kernels are launched (and the first
+    beyond them, and some at which it knows): every row is computed, by one of them, with the bits of either."""
+    from hpfp8 import _lib, ops
+    k = 256
+    counts = {"even": [rows // experts] * experts, "zipf": [int(rows / 4 / (i + 1)) for i in range(experts)],
+              "half": [rows // 2] + [rows // 2 // experts] * (experts - 1), "two": [0, rows // 2] + [0] * (experts - 3) + [rows // 2],
+              "one": [0] * (experts - 1) + [rows], "none": [0] * experts}[spread]
+    a, sa = ops.quantize_1x128(_normal((rows, k), 1, gpu), kmajor=True)
+    b, sb = ops.quantize_128x128(_normal((experts * n, k), 2, gpu, 0.05))
+    offs = torch.tensor(counts).cumsum(0).clamp(max=rows).to(torch.int32).to(gpu)
+
+    def run():
+        out = torch.full((rows, n), 7.0, dtype=torch.bfloat16, device=gpu)
+        _lib.call("hpfp8_gemm_grouped_blockwise", a.data_ptr(), k, sa.data_ptr(), sa.stride(0), sa.stride(1), b.data_ptr(), sb.data_ptr(),
+                  offs.data_ptr(), experts, rows, n, k, out.data_ptr(), n, _lib.OUT_BF16, ops._stream())
+        return out
+    got, want = _both_tiles(run)
+    assert torch.equal(got, want)
+    assert bool((got[int(offs[-1]):] == 7.0).all())
+
+
 @pytest.mark.parametrize("m", [1, 63, 64, 65, 127, 128, 129, 383])
 @pytest.mark.parametrize("k", [128, 640, 2048])
 @pytest.mark.parametrize("pow2", [False, True])
