@@ -197,7 +197,7 @@ class _Fp8LinearPerTensor(torch.autograd.Function):
         else:
             xq, _, sx = ops.quantize_per_tensor(x2)
         if wq is None:                          # no prequantized form of the weight was passed in
-            if need_dx and m > 0:
+            if need_dx and m > 0 and weight.shape[0] > 0:
                 wq, sw, wqt = ops.quantize_per_tensor_t(weight)
             else:
                 wq, _, sw = ops.quantize_per_tensor(weight)

@@ -466,6 +466,16 @@ def test_mlp_block_of_ragged_tokens_is_that_of_its_two_linears(gpu, rows):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("m", [0, 1, 5, 128, 200])
+@pytest.mark.parametrize("x_grad,w_grad", [(True, True), (True, False), (False, True), (False, False)])
+def test_per_tensor_linear_without_output_features_has_an_empty_result(gpu, m, x_grad, w_grad):
+    """A weight of no rows: nothing to quantize in any form, whatever gradients are to come."""
+    import hpfp8
+    x, w = randn_bf16((m, 256), 1).to(gpu).requires_grad_(x_grad), torch.empty((0, 256), dtype=torch.bfloat16, device=gpu, requires_grad=w_grad)
+    for bias in (None, torch.empty((0,), dtype=torch.bfloat16, device=gpu)):
+        assert tuple(hpfp8.fp8_linear(x, w, bias, recipe="per_tensor").shape) == (m, 0)
+
+
 @pytest.mark.parametrize("m,k", [(1, 128), (127, 128), (129, 384), (1024, 1024), (1000, 2048), (2048, 1024), (2049, 2048), (4096, 1024),
                                  (4097, 1024), (300, 16384)])
 @pytest.mark.parametrize("one_launch,polls", [(True, None), (True, 0), (False, None)])
