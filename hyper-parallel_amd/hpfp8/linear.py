@@ -86,6 +86,12 @@ def _both_forms(t: torch.Tensor, pow2: bool = False, column_sum: bool = False):
     return form(t, pow2=pow2, column_sum=column_sum)
 
 
+def _for_weight_gradient_alone(go: torch.Tensor) -> torch.Tensor:
+    """A ragged grad_out from which only a weight gradient is made may start between two 16-byte vectors (a view): it is
+    copied then.  Everything else that starts there is refused by the quantizers, whatever its number of rows."""
+    return go.clone() if go.shape[0] % ops.BLOCK and go.data_ptr() % 16 else go
+
+
 def _empty_batch_grads(ctx, go):
     """(dx, dw, db) of a linear whose batch is empty: no token contributes, so the weight and bias gradients are
     zero (an fp32 main gradient is left as it is, or created as zeros)."""
@@ -159,7 +165,7 @@ class _Fp8LinearBlockwise(torch.autograd.Function):
             if need_dx:
                 goq, sgo = ops.quantize_1x128(go, kmajor=True, pow2=pow2)
             if need_dw:
-                got, sgot = ops.quantize_128x1_t_rows(go, pow2=pow2)
+                got, sgot = ops.quantize_128x1_t_rows(_for_weight_gradient_alone(go), pow2=pow2)
             if ctx.has_bias:
                 db = ops.column_sum(go)
         if need_dx:
@@ -224,7 +230,7 @@ class _Fp8LinearPerTensor(torch.autograd.Function):
         if need_dw and ctx.has_bias:
             goq, sgo, got, db = ops.quantize_per_tensor_t(go, column_sum=True)
         elif need_dw:
-            goq, sgo, got = ops.quantize_per_tensor_t(go)
+            goq, sgo, got = ops.quantize_per_tensor_t(go if need_dx else _for_weight_gradient_alone(go))
         else:
             if need_dx:
                 goq, _, sgo = ops.quantize_per_tensor(go)
@@ -555,7 +561,7 @@ class _Fp8SwiGLUDown(torch.autograd.Function):
             if need_dh:
                 goq, sgo = ops.quantize_1x128(go, kmajor=True)
             if need_dw:
-                got, sgot = ops.quantize_128x1_t_rows(go)
+                got, sgot = ops.quantize_128x1_t_rows(_for_weight_gradient_alone(go))
         if need_dw:
             dw = ops.gemm_blockwise(got, sgot, at, sat, sb_gran=1)
         if need_dh:

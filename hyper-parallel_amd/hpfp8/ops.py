@@ -176,8 +176,6 @@ def quantize_per_tensor_t(x: torch.Tensor, column_sum: bool = False):
     x = _check_bf16(x, "x")
     if x.dim() != 2 or x.shape[1] % BLOCK or x.numel() == 0:
         raise ValueError("x must be [M, K] with M > 0 and K a positive multiple of 128")
-    if x.data_ptr() % 16:                  # (a view that starts between two vectors)
-        x = x.clone()
     m, k = x.shape
     mp = _rows_up(m)
     q = torch.empty((m, k), dtype=FP8, device=x.device)
@@ -408,7 +406,7 @@ def quantize_128x1_t_rows(x: torch.Tensor, pow2: bool = False):
     x = _check_bf16(x, "x")
     if x.dim() != 2 or x.shape[1] % BLOCK or x.shape[0] == 0:
         raise ValueError("x must be [M, K] with M > 0 and K a multiple of 128")
-    if x.data_ptr() % 16:                  # (a view that starts between two vectors)
+    if x.shape[0] < BLOCK and x.data_ptr() % 16:      # (a view that starts between two vectors; a larger one is refused)
         x = x.clone()
     m, k = x.shape
     mp = _rows_up(m)
@@ -426,8 +424,6 @@ def quantize_1x128_and_128x1_t_rows(x: torch.Tensor, pow2: bool = False, column_
     x = _check_bf16(x, "x")
     if x.dim() != 2 or x.shape[1] % BLOCK or x.shape[0] == 0:
         raise ValueError("x must be [M, K] with M > 0 and K a multiple of 128")
-    if x.data_ptr() % 16:                  # (a view that starts between two vectors)
-        x = x.clone()
     m, k = x.shape
     mp = _rows_up(m)
     q = torch.empty((m, k), dtype=FP8, device=x.device)

@@ -476,6 +476,41 @@ def test_per_tensor_linear_without_output_features_has_an_empty_result(gpu, m, x
         assert tuple(hpfp8.fp8_linear(x, w, bias, recipe="per_tensor").shape) == (m, 0)
 
 
+def _between_vectors(t):
+    """The same values in memory that starts two bytes past a 16-byte boundary."""
+    buf = torch.empty(t.numel() + 8, dtype=t.dtype, device=t.device)
+    v = buf[1:1 + t.numel()].view(t.shape)
+    return v.copy_(t)
+
+
+@pytest.mark.parametrize("recipe", ["blockwise", "blockwise_pow2", "per_tensor"])
+@pytest.mark.parametrize("m", [5, 128, 200])
+def test_what_starts_between_two_vectors_is_refused_at_every_number_of_rows(gpu, recipe, m):
+    """Input, weight and grad_out of a training step: refused or taken alike for whole and for ragged token counts, but for a
+    ragged grad_out of which only the weight gradient is made."""
+    import hpfp8
+    from hpfp8 import _lib
+    x, w, go = (randn_bf16(s, i, sd).to(gpu) for i, (s, sd) in enumerate((((m, 256), 1.0), ((384, 256), 0.05), ((m, 384), 0.1))))
+    for x_grad, w_grad in ((True, True), (False, True)):
+        with pytest.raises(_lib.Hpfp8Error, match="16-byte aligned"):
+            hpfp8.fp8_linear(_between_vectors(x).requires_grad_(x_grad), w.clone().requires_grad_(w_grad), recipe=recipe)
+        with pytest.raises(_lib.Hpfp8Error, match="16-byte aligned"):
+            hpfp8.fp8_linear(x.clone().requires_grad_(x_grad), _between_vectors(w).requires_grad_(w_grad), recipe=recipe)
+        ins = [t for t, g in ((x.clone(), x_grad), (w.clone(), w_grad)) if t.requires_grad_(g).requires_grad]
+        y = hpfp8.fp8_linear(ins[0] if x_grad else x, ins[-1], recipe=recipe)
+        if x_grad or m == 128:
+            with pytest.raises(_lib.Hpfp8Error, match="16-byte aligned"):
+                torch.autograd.grad(y, ins, _between_vectors(go))
+        else:
+            want = torch.autograd.grad(y, ins, go, retain_graph=True)
+            assert torch.equal(torch.autograd.grad(y, ins, _between_vectors(go))[0], want[0])
+    if recipe == "blockwise":
+        dn = randn_bf16((256, 128), 4, 0.05).to(gpu)
+        w2, d2 = w[:256].clone().requires_grad_(True), dn.clone().requires_grad_(True)
+        with pytest.raises(_lib.Hpfp8Error, match="16-byte aligned"):
+            hpfp8.fp8_swiglu_mlp(_between_vectors(x), w2, d2)
+
+
 @pytest.mark.parametrize("m,k", [(1, 128), (127, 128), (129, 384), (1024, 1024), (1000, 2048), (2048, 1024), (2049, 2048), (4096, 1024),
                                  (4097, 1024), (300, 16384)])
 @pytest.mark.parametrize("one_launch,polls", [(True, None), (True, 0), (False, None)])
