@@ -1156,8 +1156,10 @@ static TileShape pick_shape_swiglu(int64_t M, int64_t N) {
 // Grouped by rows: every expert ends in a partial tile, which costs as much as a whole one, so with few rows per expert low
 // tiles are better, with many (or the rows of many with one expert) high ones.  The rows of an expert are known on the device
 // only.  Even the largest number of low tiles is one round: low.  Of more than 256 rows per expert on average: high.  Low
-// tiles are at most M / 129 row tiles more than high ones: where that is a quarter of a round, low.  In between both kernels
-// are launched, count both kinds of tiles and one of them returns at once (3 to 5 us).  us with 128 / 256 rows per tile, for rows
+// tiles are at most M / 129 row tiles more than high ones: where that is at most a quarter of a round, low; at that quarter what
+// is lost where they are just one round more (32 experts [2048, 7168], 1024 rows by Zipf's law: 264 / 256 tiles, 137 / 120
+// us) is about what a second launch would cost on every call.  In between both kernels are launched, count both kinds of tiles
+// and one of them returns at once (3 to 5 us).  us with 128 / 256 rows per tile, for rows
 // spread evenly / by Zipf's law / half with one expert / all with one:
 //   32 experts [4096, 7168],   512 rows   187 / 257   167 / 207   209 / 267    49 / 69
 //                             4096 rows   175 / 235   267 / 278   226 / 295   112 / 99

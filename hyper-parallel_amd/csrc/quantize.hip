@@ -737,9 +737,8 @@ __device__ __forceinline__ float column_sum_of_tile(const float (*s_cs)[128], in
 // (tile_column_sums): the per-block partial sums of a bias gradient, from the same read of grad_out.
 // ROWS: which rows of a tile exist.  Whole: all.  By expert: the layout table says.  Ragged: m need not be a multiple of
 // 128; rows past m count as zeros, as if x had been filled up with zero rows, and are written in the transposed form
-// only.  (A variant of its own, so that the whole form's loads stay unconditional.)  A ragged training step used to copy
-// x and grad_out into zero-padded buffers (fill + copy, 25 us for [1531, 7168] and [1531, 2048]) and to read each once
-// more for its 1x128 form and for the bias gradient.
+// only.  (A variant of its own, so that the whole form's loads stay unconditional.)  Copying a ragged source into a
+// zero-padded buffer first costs 25 us for [1531, 7168] and [1531, 2048], and one more read for the 1x128 form.
 enum TileRows { kWholeRows = 0, kRowsByExpert = 1, kRaggedRows = 2 };
 template <bool KMAJOR, bool DUAL, int SW = 0, int ROWS = kWholeRows, bool COLSUM = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void quant_128x1_t_kernel(const uint16_t* __restrict__ x, int64_t ld_src, int m, int k,
