@@ -14,9 +14,15 @@
 //     are DMA'd global -> LDS with 128-bit buffer loads (out-of-range rows read as zero), 16-byte
 //     chunks XOR-swizzled by row so that both the DMA writes and the ds_read_b128 fragment reads
 //     are bank-conflict free.
-//   * Where a launch would leave compute units idle the tile is smaller: 128 x 256 or 128 x 128 with four waves (wave
-//     tiles 64 x 128 and 64 x 64), the same template (WM, NS) and the same results bit for bit; pick_shape has the rule
-//     and the figures.
+//   * Where a launch would leave compute units idle the tile is smaller: 128 x 256, 128 x 128 or 64 x 128 with four
+//     multiplying waves (wave tiles 64 x 128, 64 x 64 and 64 x 32), the same template (WM, NS, WN) and the same results bit
+//     for bit; pick_shape has the rule and the figures.  There a SIMD has one wave that multiplies, which waits whenever a
+//     transfer it issues finds the memory path occupied (78 clocks per transfer while the first k-blocks arrive, 21 later), so
+//     four more waves do the transfers, 3, 4 and 6 k-blocks at a time in LDS, the scales with them.  us, transfers by the
+//     multiplying waves with two buffers of a / by waves of their own: 1000 x 7168 x 7168 62 / 54, 1531 x 2048 x 7168 41 / 33,
+//     500 x 7168 x 16384 106 / 75, by rows 1024 x 1024 x 2048 16.7 / 11.0.  What is left there is what a k-block's transfers
+//     take by themselves (0.54 us for 48 KB, 0.39 for 32 KB, with every compute unit at it) and a first microsecond or three in
+//     which code and the first tiles arrive through cold caches.
 //   * The grid is persistent: one workgroup per CU walks a list of tiles, and the rounds of
 //     consecutive tiles follow each other without a gap.  Each XCD (own L2) owns a contiguous run
 //     of tile numbers.
@@ -85,6 +91,17 @@ struct GemmParams {
   int choose_cus;         // grouped by rows: launched with both tile heights, the kernel of the better one runs (0: the only one)
 };
 
+// n / d for uniform values, without the compiler's division (some 30 dependent instructions; a tile lookup has four, and a
+// workgroup does nothing else before its first transfers)
+__device__ __forceinline__ int quotient(int n, int d) {
+  if (n >= (1 << 22)) return n / d;
+  int q = (int)((float)n * __builtin_amdgcn_rcpf((float)d));      // n and d exact in fp32, rcp within one ulp: off by one at most
+  const int rest = n - q * d;
+  q += rest >= d ? 1 : 0;
+  q -= rest < 0 ? 1 : 0;
+  return __builtin_amdgcn_readfirstlane(q);
+}
+
 // Tile number -> (m tile, n tile).  Consecutive numbers (one XCD's CUs at any moment) cover
 // gm x gn rectangles of tiles (gm * gn = 32), n fastest inside a rectangle, so the L2 of that XCD
 // serves each activation / weight panel to several CUs.  A panel of a is fetched once per column
@@ -95,12 +112,13 @@ struct GemmParams {
 __device__ __forceinline__ void rect_map(int t, int tiles_m, int tiles_n, int& tm, int& tn) {
   const int gm = tiles_m > tiles_n ? 4 : 8, gn_full = kRectTiles / gm;
   const int per_ngroup = gn_full * tiles_m;
-  const int ng = t / per_ngroup, rest = t % per_ngroup;
+  const int ng = quotient(t, per_ngroup), rest = t - ng * per_ngroup;
   const int gn = (tiles_n - ng * gn_full) < gn_full ? (tiles_n - ng * gn_full) : gn_full;
-  const int mg = rest / (gm * gn);
+  const int mg = quotient(rest, gm * gn);
   const int r3 = rest - mg * gm * gn;
-  tm = mg * gm + r3 / gn;
-  tn = ng * gn_full + r3 % gn;
+  const int row = quotient(r3, gn);
+  tm = mg * gm + row;
+  tn = ng * gn_full + r3 - row * gn;
 }
 
 // One output tile of a workgroup's list.  A tile with no rows (row0 == row_end, n0 >= N) stands for
@@ -136,55 +154,83 @@ __device__ __forceinline__ TileInfo pick_tile(int q, TileInfo t0, TileInfo t1, T
   return r;
 }
 
-// End row of an expert as the kernel uses it: offsets that decrease or run past the row count (a
-// malformed table) are clamped, so that every address derived from them stays inside a.
-__device__ __forceinline__ int expert_end(int off, int prev, int total_rows) {
-  const int lo = off > prev ? off : prev;
-  return lo < total_rows ? lo : total_rows;
+// Inclusive sum / maximum over the lanes of a wave, of values that are not negative (steps inside rows of 16 lanes, then
+// across the rows).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_or_zero(int x) { return __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xf, false); }
+template <class Op>
+__device__ __forceinline__ int wave_scan(int x, Op op) {
+  x = op(x, dpp_or_zero<0x111, 0xf>(x));   // row_shr:1
+  x = op(x, dpp_or_zero<0x112, 0xf>(x));
+  x = op(x, dpp_or_zero<0x114, 0xf>(x));
+  x = op(x, dpp_or_zero<0x118, 0xf>(x));
+  x = op(x, dpp_or_zero<0x142, 0xa>(x));   // row_bcast:15
+  x = op(x, dpp_or_zero<0x143, 0xc>(x));   // row_bcast:31
+  return x;
+}
+
+// Grouped by rows: 64 experts at a time, one per lane.  (One after the other, each behind the load of its offset, the experts
+// took longer than a small problem's products: 64 experts [2048, 2048], 64 rows, all with one of them 24.6 us, 13.1 so.)
+struct ExpertChunk {
+  int first, row, tile;   // the chunk's first expert, the rows and the tiles before it
+  int end, tile_end;      // this lane's expert: the row it ends with, the tiles up to its last one
+};
+
+// Offsets that decrease or run past the row count (a malformed table) are clamped, so that every address derived from them
+// stays inside a.
+__device__ __forceinline__ void load_experts(ExpertChunk& c, const GemmParams& p, int tile_rows, int tiles_n, int lane) {
+  int end = c.first + lane < p.experts ? p.offs[c.first + lane] : 0;
+  end = wave_scan(end > c.row ? end : c.row, [](int a, int b) { return a > b ? a : b; });
+  c.end = end < p.M ? end : p.M;
+  int prev = __shfl_up(c.end, 1);
+  if (lane == 0) prev = c.row;
+  c.tile_end = c.tile + wave_scan((c.end - prev + tile_rows - 1) / tile_rows, [](int a, int b) { return a + b; }) * tiles_n;
+}
+__device__ __forceinline__ bool next_experts(ExpertChunk& c, const GemmParams& p, int tile_rows, int tiles_n, int lane) {
+  if (c.first + 64 >= p.experts) return false;
+  c.first += 64;
+  c.row = __builtin_amdgcn_readlane(c.end, 63);
+  c.tile = __builtin_amdgcn_readlane(c.tile_end, 63);
+  load_experts(c, p, tile_rows, tiles_n, lane);
+  return true;
+}
+__device__ __forceinline__ int grouped_tiles(ExpertChunk& c, const GemmParams& p, int tile_rows, int tiles_n, int lane) {
+  c = ExpertChunk{0, 0, 0, 0, 0};
+  load_experts(c, p, tile_rows, tiles_n, lane);
+  while (next_experts(c, p, tile_rows, tiles_n, lane)) {}
+  return __builtin_amdgcn_readlane(c.tile_end, 63);
 }
 
 // Grouped by rows, launched with both tile heights: whether 128-row tiles are the better ones for the rows that the experts
-// have.  A round of them takes three fifths of one of 256-row tiles.  (64 experts at a time, one per lane: an expert's end is
-// the largest offset up to its own, as expert_end gives it one after the other.)
+// have.  A round of them takes three fifths of one of 256-row tiles.
 __device__ __forceinline__ bool better_is_low(const GemmParams& p, int tiles_n, int lane) {
-  int carry = 0, low = 0, high = 0;
-  for (int e0 = 0; e0 < p.experts; e0 += 64) {
-    int end = e0 + lane < p.experts ? p.offs[e0 + lane] : 0;
-#pragma unroll
-    for (int d = 1; d < 64; d *= 2) {
-      const int before = __shfl_up(end, d);
-      if (lane >= d && before > end) end = before;
-    }
-    end = expert_end(end, carry, p.M);
-    int prev = __shfl_up(end, 1);
-    if (lane == 0) prev = carry;
-    low += (end - prev + 127) / 128;
-    high += (end - prev + 255) / 256;
-    carry = __shfl(end, 63);
-  }
-#pragma unroll
-  for (int d = 1; d < 64; d *= 2) {
-    low += __shfl_xor(low, d);
-    high += __shfl_xor(high, d);
-  }
-  const int low_rounds = (low * tiles_n + p.choose_cus - 1) / p.choose_cus;
-  const int high_rounds = (high * tiles_n + p.choose_cus - 1) / p.choose_cus;
+  ExpertChunk c;
+  const int low = grouped_tiles(c, p, 128, tiles_n, lane), high = grouped_tiles(c, p, 256, tiles_n, lane);
+  const int low_rounds = (low + p.choose_cus - 1) / p.choose_cus;
+  const int high_rounds = (high + p.choose_cus - 1) / p.choose_cus;
   return __builtin_amdgcn_readfirstlane(3 * low_rounds <= 5 * high_rounds ? 1 : 0) != 0;
 }
 
-// WM, NS: the tile has 64 WM rows (WM pairs of waves) and 32 NS columns (a wave: NS subtiles of 16).
+// WM, NS, WN: WM x WN waves multiply, each 64 rows x NS subtiles of 16 columns.  Tiles of 64 and of 128 rows have four more
+// waves, which do the transfers.
+__host__ __device__ constexpr bool fetchers(int wm) { return wm <= 2; }
+__host__ __device__ constexpr int tile_threads(int wm, int wn) { return 64 * (wm * wn + (fetchers(wm) ? 4 : 0)); }
+
 // SA4: the activation scales have unit stride over rows (the k-block-major layout), so a lane's four
 // of them are one 16-byte load.
 // EPI: 0 = c is the GEMM's result; 1 / 2 = the gate/up projection of a SwiGLU MLP with the activation and its
 // 1x128 quantization as the epilogue (1: exactly specified silu, 2: hardware exponential and reciprocal).  A tile's
 // 256 columns are then the 128 gate columns and the 128 up columns of one scaling group of the activation: the b
 // tile's upper 128 rows come from `inter` rows further down, the two waves that share 64 rows hold gate and up.
-template <int MODE, int GROUPED, bool OUT_F32, bool ACC, bool SA4, int EPI = 0, int WM = 4, int NS = 8>
-__global__ __launch_bounds__(128 * WM) void gemm_kernel(const GemmParams p) {
-  constexpr int TM = 64 * WM, TN = 32 * NS;            // the tile
-  constexpr int kWaves = 2 * WM;
+template <int MODE, int GROUPED, bool OUT_F32, bool ACC, bool SA4, int EPI = 0, int WM = 4, int NS = 8, int WN = 2>
+__global__ __launch_bounds__(tile_threads(WM, WN)) void gemm_kernel(const GemmParams p) {
+  constexpr int TM = 64 * WM, TN = 16 * NS * WN;       // the tile
+  constexpr int WC = 16 * NS;                          // a wave's columns
+  constexpr int kWaves = WM * WN;                      // that multiply
+  constexpr bool kFetchers = fetchers(WM);             // four more do the transfers
+  constexpr int kFetchWaves = kFetchers ? 4 : kWaves;
   constexpr int kATile = TM * BK, kBTile = TN * BK;    // one operand tile in LDS
-  constexpr int NB = TN / 8 / kWaves;                  // b transfers per wave and k-block (a: always 4)
+  constexpr int NA = TM / 8 / kFetchWaves, NB = TN / 8 / kFetchWaves;     // transfers per wave and k-block
   constexpr int kSlice = kBTile / kWaves;              // a wave's part of a b buffer
   static_assert(EPI == 0 || NS == 8, "SwiGLU epilogue: 128 gate and 128 up columns per tile");
   static_assert(EPI == 0 || ((MODE == kScaleBlock || MODE == kScalePow2) && GROUPED == kDense && !OUT_F32 && !ACC),
@@ -192,7 +238,9 @@ __global__ __launch_bounds__(128 * WM) void gemm_kernel(const GemmParams p) {
   static_assert(!ACC || (OUT_F32 && MODE != kScaleTensor), "accumulating onto c: fp32 output, sums that start from c's values");
   static_assert(GROUPED != kGroupedK || (!ACC && (MODE == kScaleRow || MODE == kScalePow2Row)),
                 "grouped along the contraction: the wgrad form");
-  constexpr int kBStages = WM == 4 ? b_stages(MODE) : 3;
+  static_assert(!kFetchers || GROUPED != kGroupedK, "the fetching waves count k-blocks from 0");
+  constexpr int kBStages = !kFetchers ? b_stages(MODE) : (WM == 1 ? 6 : (TN == 256 ? 3 : 4));
+  constexpr int kAStages = kFetchers ? kBStages : 2;
   constexpr bool kRowScales = MODE == kScaleRow || MODE == kScalePow2Row;   // per-row b scales, staged in LDS
   constexpr bool kPromote = MODE == kScaleBlock || MODE == kScaleRow;       // partial sums scaled by FMAs
   constexpr bool kHwScale = MODE == kScalePow2 || MODE == kScalePow2Row;    // scales applied by the MFMA
@@ -200,14 +248,23 @@ __global__ __launch_bounds__(128 * WM) void gemm_kernel(const GemmParams p) {
   // One LDS object for everything.  (With a second __shared__ array the compiler tells the two apart
   // with alias scopes, and from then on makes every LDS read wait for all transfers into the array it
   // reads, those to other buffers included: the transfers' latency would be paid in every round.)
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * kATile + kBStages * kBTile + (kRowScales ? 3 * 256 * 4 : 0)];
+  // kFetchers: the scales of a k-block travel with its tiles, into a slot of one part per fetching wave: 256 bytes of sb (the
+  // scale of the left or of the right half's block; with per-row scales 64 of the tile's rows) and the upper or the lower 64
+  // rows of sa.
+  constexpr int kScaleOps = MODE == kScaleTensor ? 0 : 2, kScaleSlot = 2048, kScaleSlots = kBStages + 1;
+  constexpr int kScaleBytes = kFetchers ? (kScaleOps ? kScaleSlots * kScaleSlot : 0) : (kRowScales ? 3 * 256 * 4 : 0);
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[kAStages * kATile + kBStages * kBTile + kScaleBytes];
   // per-row scales of the b operand for one k-block (wgrad form), three stages of 256 floats: the
   // stage of k-block kb+1 is filled while slower waves may still read that of kb-1
-  float* const sb_lds = reinterpret_cast<float*>(lds + 2 * kATile + kBStages * kBTile);
-  uint8_t* const b_lds = lds + 2 * kATile;
+  uint8_t* const scale_lds = lds + kAStages * kATile + kBStages * kBTile;
+  float* const sb_lds = reinterpret_cast<float*>(scale_lds);
+  constexpr int kSbSlot = kFetchers ? kScaleSlot / 4 : 256;
+  uint8_t* const b_lds = lds + kAStages * kATile;
 
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave_id = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const bool fetching = kFetchers && wave_id >= kWaves;
+  const int wave = fetching ? wave_id - kWaves : wave_id;         // its part of a tile: of the transfers or of the products
   const int K = p.K, N = p.N;
   const int kblocks = K / BK;
   const int tiles_n = (N + TN - 1) / TN;
@@ -218,27 +275,28 @@ __global__ __launch_bounds__(128 * WM) void gemm_kernel(const GemmParams p) {
   // through that run side by side, so at any moment they work on one rectangle.
   int total_tiles = p.tiles;
   if (GROUPED == kGroupedK) total_tiles = p.experts * p.tiles;
+  ExpertChunk group;       // grouped by rows: the experts among which tiles are looked up (tile numbers are asked for in increasing order)
   if (GROUPED == kGroupedRows) {
     if (p.choose_cus && better_is_low(p, tiles_n, lane) != (TM == 128)) return;
     // tiles are numbered expert by expert; an expert with no rows has none
-    int prev = 0, mt = 0;
-    for (int e = 0; e < p.experts; ++e) {
-      const int end = expert_end(p.offs[e], prev, p.M);
-      mt += (end - prev + TM - 1) / TM;
-      prev = end;
+    total_tiles = grouped_tiles(group, p, TM, tiles_n, lane);
+    if (p.experts > 64) {
+      group = ExpertChunk{0, 0, 0, 0, 0};
+      load_experts(group, p, TM, tiles_n, lane);
     }
-    total_tiles = mt * tiles_n;
   }
   int my_tiles, t_first, t_step;
   {
     const int nwg = gridDim.x, pid = blockIdx.x;
-    const int xu = nwg < kXcds ? nwg : kXcds;        // the host launches a multiple of 8 workgroups, or fewer than 8
-    const int xcd = pid % xu, slot = pid / xu;
-    t_step = nwg / xu;
-    const int base = total_tiles / xu, big = total_tiles % xu;
+    // (the host launches a multiple of 8 workgroups, or fewer than 8)
+    const bool few = nwg < kXcds;
+    const int xcd = few ? pid : pid % kXcds, slot = few ? 0 : pid / kXcds;
+    t_step = few ? 1 : nwg / kXcds;
+    const int base = few ? quotient(total_tiles, nwg) : total_tiles / kXcds;
+    const int big = total_tiles - base * (few ? nwg : kXcds);
     const int cnt = base + (xcd < big ? 1 : 0);
     t_first = xcd * base + (xcd < big ? xcd : big) + slot;
-    my_tiles = slot < cnt ? (cnt - slot + t_step - 1) / t_step : 0;
+    my_tiles = slot < cnt ? quotient(cnt - slot + t_step - 1, t_step) : 0;
     if (GROUPED == kGroupedK) {
       // Tiles differ in length (an expert's contraction is its own token count) and are numbered longest expert
       // first.  They are dealt out in rounds of one tile per workgroup -- the XCD with index x takes positions
@@ -251,8 +309,6 @@ __global__ __launch_bounds__(128 * WM) void gemm_kernel(const GemmParams p) {
   }
   if (my_tiles == 0) return;
   const int n_pad = tiles_n * TN;
-  // grouped: forward-only search state (tile numbers are asked for in increasing order)
-  int g_e = 0, g_prev = 0, g_first = 0;
   auto lookup = [&](int k, TileInfo& ti) {
     int row0 = p.M, row_end = p.M, n0 = n_pad, expert = 0, kb0 = 0, kbn = GROUPED == kGroupedK ? 1 : kblocks;
     if (k < my_tiles) {
@@ -268,20 +324,15 @@ __global__ __launch_bounds__(128 * WM) void gemm_kernel(const GemmParams p) {
         row_end = row0 + TM < p.M ? row0 + TM : p.M;
         n0 = tn * TN;
       } else if (GROUPED == kGroupedRows) {
-        int end = 0, cnt = 0;
-        while (g_e < p.experts) {
-          end = expert_end(p.offs[g_e], g_prev, p.M);
-          cnt = (end - g_prev + TM - 1) / TM;
-          if (t < g_first + cnt * tiles_n) break;
-          g_first += cnt * tiles_n;
-          g_prev = end;
-          ++g_e;
-        }
-        if (g_e < p.experts) {
-          rect_map(t - g_first, cnt, tiles_n, tm, tn);
-          expert = g_e;
-          row0 = g_prev + tm * TM;
-          row_end = end < p.M ? end : p.M;
+        while (t >= __builtin_amdgcn_readlane(group.tile_end, 63) && next_experts(group, p, TM, tiles_n, lane)) {}
+        const int l = __builtin_popcountll(__ballot(group.tile_end <= t));    // (experts without rows end where the one before ends)
+        if (l < 64) {
+          const int end = __builtin_amdgcn_readlane(group.end, l), prev = l ? __builtin_amdgcn_readlane(group.end, l - 1) : group.row;
+          const int cnt = (end - prev + TM - 1) / TM;
+          rect_map(t - (__builtin_amdgcn_readlane(group.tile_end, l) - cnt * tiles_n), cnt, tiles_n, tm, tn);
+          expert = group.first + l;
+          row0 = prev + tm * TM;
+          row_end = end;
           if (row0 + TM < row_end) row_end = row0 + TM;
           n0 = tn * TN;
         }
@@ -301,12 +352,6 @@ __global__ __launch_bounds__(128 * WM) void gemm_kernel(const GemmParams p) {
     ti.kb0 = __builtin_amdgcn_readfirstlane(kb0);
     ti.kbn = __builtin_amdgcn_readfirstlane(kbn);
   };
-  // T0 is the tile being accumulated; transfers and scale loads run up to two k-blocks ahead and
-  // so reach into T1 (and into T2 when K is a single k-block).
-  TileInfo T0, T1, T2;
-  lookup(0, T0);
-  lookup(1, T1);
-  lookup(2, T2);
   // ---- global -> LDS tile DMA.  One wave instruction moves 8 rows x 128 B (lane i -> LDS slot
   // i); the lane picks the 16-byte global chunk whose swizzled home is its slot.  The buffer
   // resource of a transfer starts at the tile's first row and ends with the tensor, so lane
@@ -330,10 +375,10 @@ __global__ __launch_bounds__(128 * WM) void gemm_kernel(const GemmParams p) {
     const uint8_t* base = p.b + (GROUPED == kGroupedRows ? (int64_t)ti.expert * p.b_se : 0) + (int64_t)(rows ? brow0 : 0) * p.ldb;
     return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, span_bytes(rows, p.ldb), 0x00020000);
   };
-  uint32_t a_off[4], b_off[NB];
+  uint32_t a_off[NA], b_off[NB];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int q = wave * 4 + i;                       // 8-row group inside the tile
+  for (int i = 0; i < NA; ++i) {
+    const int q = wave * NA + i;                      // 8-row group inside the tile
     const int r = q * 8 + (lane >> 3);                // row inside the tile
     const int chunk = (lane & 7) ^ row_swizzle(r);    // logical 16-byte chunk of that row
     // The rows of the a tile are permuted on their way into LDS: LDS row 64 w + 16 j + l holds tile row
@@ -373,18 +418,18 @@ __global__ __launch_bounds__(128 * WM) void gemm_kernel(const GemmParams p) {
     }
   };
   auto issue_a = [&](const __amdgpu_buffer_rsrc_t& rs, int buf, int kb, int sub) {
-    transfer(rs, a_off[sub], lds + buf * kATile + wave * 4096, kb, sub);
+    transfer(rs, a_off[sub], lds + buf * kATile + wave * (NA * 1024), kb, sub);
   };
   auto issue_b = [&](const __amdgpu_buffer_rsrc_t& rs, int buf, int kb, int sub) {
-    transfer(rs, b_off[sub], b_lds + buf * kBTile + wave * kSlice, kb, sub);
+    transfer(rs, b_off[sub], b_lds + buf * kBTile + wave * (NB * 1024), kb, sub);
   };
 
   // ---- fragment addressing
-  const int wn = wave & 1, wm = wave >> 1;
+  const int wn = wave % WN, wm = wave / WN;
   const int l16 = lane & 15, g = lane >> 4;
   const int pc0 = (2 * g) ^ row_swizzle(l16);
   const int a_frag_off = (wm * 64 + l16) * BK;               // + j * 16 rows
-  const int b_frag_off = (wn * (TN / 2) + l16) * BK;               // + i * 16 rows, inside a b buffer
+  const int b_frag_off = (wn * WC + l16) * BK;               // + i * 16 rows, inside a b buffer
 
   // ---- scales.  Raw values for one k-block are loaded at the top of the round before it and only
   // combined (sa * sb) at its end, so nothing waits on global memory in between.
@@ -405,7 +450,7 @@ __global__ __launch_bounds__(128 * WM) void gemm_kernel(const GemmParams p) {
       // (SA4 does not clamp: words past the end of the array read as zero, and rows past M are never stored)
       sa_voff[j] = SA4 ? (uint32_t)r * 4u : (uint32_t)(r < p.M ? r : p.M - 1) * (uint32_t)((int)p.sa_sm * 4);
     }
-    int nblk_idx = EPI ? (ti.n0 >> 8) + wn * (p.inter >> 7) : (ti.n0 + wn * (TN / 2)) >> 7;
+    int nblk_idx = EPI ? (ti.n0 >> 8) + wn * (p.inter >> 7) : (ti.n0 + wn * WC) >> 7;
     if (nblk_idx > (N >> 7) - 1) nblk_idx = (N >> 7) - 1;
     sb_soff = ((GROUPED == kGroupedRows ? ti.expert * (int)p.sb_se : 0) + nblk_idx * (int)p.sb_sn) * 4;
   };
@@ -423,6 +468,91 @@ __global__ __launch_bounds__(128 * WM) void gemm_kernel(const GemmParams p) {
           raw[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc_sa, sa_voff[j], kb * sa_kstep, 0));
       }
     }
+  };
+  if constexpr (kFetchers) {
+    if (fetching) {
+      // ---- the fetching waves: the k-blocks of the tile list one after the other, kBStages of them at a time in LDS.  After a
+      // round's barrier the multiplying waves have left the buffers of its k-block, which are filled again at once; past
+      // the end of the list nothing is fetched.
+      constexpr int kOps = NA + NB + kScaleOps;          // a wave's transfers per k-block
+      int f_tile = 0, f_kb = 0, buf = 0, slot = 0;
+      __amdgpu_buffer_rsrc_t ra, rb;
+      uint32_t sa_off, sb_off = 0;
+      int sb_first = 0;
+      auto enter = [&](const TileInfo& ti) {
+        ra = rsrc_a_of(ti);
+        rb = rsrc_b_of(ti);
+        const int row = ti.row0 + (wave >> 1) * 64 + lane;       // (rows past M repeat the last one's scale: they are not stored)
+        sa_off = (uint32_t)(row < p.M ? row : p.M - 1) * (uint32_t)((int)p.sa_sm * 4);
+        if (kRowScales) {
+          sb_off = (uint32_t)(ti.n0 + wave * 64 + lane) * 4u;        // (past N: columns that are not stored)
+        } else {
+          int blk = EPI ? (ti.n0 >> 8) + (wave & 1) * (p.inter >> 7) : (ti.n0 + (wave & 1) * (TN / 2)) >> 7;
+          if (blk > (N >> 7) - 1) blk = (N >> 7) - 1;
+          sb_first = ((GROUPED == kGroupedRows ? ti.expert * (int)p.sb_se : 0) + blk * (int)p.sb_sn) * 4;
+        }
+      };
+      auto fetch_a = [&]() {
+#pragma unroll
+        for (int sub = 0; sub < NA; ++sub) issue_a(ra, buf, f_kb, sub);
+      };
+      auto fetch_rest = [&]() {
+#pragma unroll
+        for (int sub = 0; sub < NB; ++sub) issue_b(rb, buf, f_kb, sub);
+        if (kScaleOps) {
+          uint8_t* const dst = scale_lds + slot * kScaleSlot + wave * 256;
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(kRowScales ? rsrc_sb : rsrc_sbb, (lds_ptr_t)dst, 4, sb_off,
+                                                   sb_first + f_kb * sb_kstep, 0, 0);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_sa, (lds_ptr_t)(dst + 1024), 4, sa_off, f_kb * sa_kstep, 0, 0);
+        }
+        buf = buf + 1 == kBStages ? 0 : buf + 1;
+        slot = slot + 1 == kScaleSlots ? 0 : slot + 1;
+        if (++f_kb == kblocks) {
+          f_kb = 0;
+          TileInfo next;
+          lookup(++f_tile, next);
+          enter(next);
+        }
+      };
+      {
+        TileInfo first;
+        lookup(0, first);
+        enter(first);
+      }
+      // (two k-blocks ahead of the first wait and not all: the first has to land through cold caches and what is queued up
+      // behind it keeps these waves from the barrier)
+      for (int k = 0; k < kBStages; ++k) {
+        fetch_a();
+        fetch_rest();
+        if (k == 1) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kOps) : "memory");
+      }
+      for (int tile = 0; tile < my_tiles; ++tile) {
+        for (int kb = 0; kb < kblocks; ++kb) {
+          // the next k-block has landed; everyone has left this one
+          asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((kBStages - 2) * kOps) : "memory");
+          fetch_a();
+          // the last b buffer of a tile is what its results are staged in: it is filled again when they have been read
+          if (kb == kblocks - 1) {
+            if (EPI) {
+              for (int i = 0; i < 8; ++i) asm volatile("s_barrier" ::: "memory");
+            } else {
+              asm volatile("s_barrier" ::: "memory");
+            }
+          }
+          fetch_rest();
+        }
+      }
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the last transfers fetch nothing but write to this workgroup's LDS
+      return;
+    }
+  }
+  auto read_scales = [&](int slot, float raw[5]) {      // (kFetchers)
+    if (MODE == kScaleTensor) return;
+    const uint8_t* const src = scale_lds + slot * kScaleSlot + (wm * 2 + wn * 2 / WN) * 256;
+    const v4f four = *reinterpret_cast<const v4f*>(src + 1024 + l16 * 16);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) raw[j] = four[j];
+    if (!kRowScales) raw[4] = *reinterpret_cast<const float*>(src);
   };
   // kScalePow2: the exponent fields of the scales of the current k-block, which are their E8M0 codes:
   // e_a[j] for the activation rows j * 16 + l16 of this lane, e_b for the weight block
@@ -444,7 +574,7 @@ __global__ __launch_bounds__(128 * WM) void gemm_kernel(const GemmParams p) {
   // load.  The resource ends with the tensor: rows past it (and the tiles past the end of the list)
   // read as zero.
   auto rsrc_c_of = [&](const TileInfo& ti) {
-    const int ncol = ti.n0 + wn * (TN / 2);
+    const int ncol = ti.n0 + wn * WC;
     const bool ok = ti.row_end > ti.row0 && ncol < N;
     int64_t bytes = ok ? (((int64_t)p.M - ti.row0 - 1) * p.ldc + N - ncol) * 4 : 0;
     if (bytes > (int64_t)0x7FFFF000) bytes = 0x7FFFF000;       // 256 rows always fit (host check)
@@ -479,15 +609,24 @@ __global__ __launch_bounds__(128 * WM) void gemm_kernel(const GemmParams p) {
   // own k-blocks start at its expert's first block kb0; otherwise kb0 is 0)
   auto kfirst = [](const TileInfo& ti) { return GROUPED == kGroupedK ? ti.kb0 : 0; };
   auto kcount = [&](const TileInfo& ti) { return GROUPED == kGroupedK ? ti.kbn : kblocks; };
-  scale_target(T0);
-  load_scales(kfirst(T0), s_raw);
-  combine_scales(s_raw, s_cur);
-  {
+  // T0 is the tile being accumulated; transfers and scale loads run up to two k-blocks ahead and
+  // so reach into T1 (and into T2 when K is a single k-block).
+  TileInfo T0, T1, T2;
+  lookup(0, T0);
+  if constexpr (kFetchers) {
+    asm volatile("s_barrier" ::: "memory");        // the first k-block is there
+    read_scales(0, s_raw);
+    combine_scales(s_raw, s_cur);
+  } else {
     const __amdgpu_buffer_rsrc_t ra = rsrc_a_of(T0), rb = rsrc_b_of(T0);
 #pragma unroll
     for (int sub = 0; sub < 4; ++sub) issue_a(ra, 0, kfirst(T0), sub);
 #pragma unroll
     for (int sub = 0; sub < NB; ++sub) issue_b(rb, 0, kfirst(T0), sub);
+    scale_target(T0);
+    load_scales(kfirst(T0), s_raw);
+    lookup(1, T1);
+    lookup(2, T2);
     int kb1;
     const TileInfo t1 = pick_tile(tiles_ahead(0, 1, kcount(T0), kcount(T1), kb1), T0, T1, T2);
     kb1 += kfirst(t1);
@@ -497,8 +636,11 @@ __global__ __launch_bounds__(128 * WM) void gemm_kernel(const GemmParams p) {
       for (int sub = 0; sub < NB; ++sub) issue_b(rb1, 1, kb1, sub);
     }
     issue_sb_load(T0, 0, 0);
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    __builtin_amdgcn_sched_barrier(0);
+    // k-block 0 has landed (with three b buffers the next one of b may be under way)
+    __builtin_amdgcn_s_waitcnt(kBAhead == 2 ? 0x0F70 | NB : 0x0F70);
     __syncthreads();
+    combine_scales(s_raw, s_cur);
     const __amdgpu_buffer_rsrc_t ra1 = rsrc_a_of(t1);
     issue_a(ra1, 1, kb1, 0);
     issue_a(ra1, 1, kb1, 1);
@@ -549,7 +691,7 @@ __global__ __launch_bounds__(128 * WM) void gemm_kernel(const GemmParams p) {
     // two rounds of a tile does a target move on to the next tile of the list; its resource is
     // rebuilt then and stays valid when that tile becomes the current one.
     int kb1 = kb + 1, kb2 = kb + 2;
-    if (kb2 >= kbn0) {
+    if (!kFetchers && kb2 >= kbn0) {
       const int o1 = tile + tiles_ahead(kb, 1, kbn0, kcount(T1), kb1);
       const int o2 = tile + tiles_ahead(kb, 2, kbn0, kcount(T1), kb2);
       if (o1 != ord_1) {
@@ -570,39 +712,29 @@ __global__ __launch_bounds__(128 * WM) void gemm_kernel(const GemmParams p) {
     const int kb1_rel = kb1;             // inside tile_1's own contraction (what issue_sb_load counts in)
     kb1 += kfirst(tile_1);
     kb2 += kofs_2;
-    load_scales(kb1, s_raw);
+    if (!kFetchers) load_scales(kb1, s_raw);
     const uint8_t* bcur = b_lds + bbuf * kBTile;
     int bnext = bbuf + 1 == kBStages ? 0 : bbuf + 1;           // holds the next k-block
     int bbuf_issue = bbuf + kBAhead;                           // receives the k-block kBAhead ahead
     if (bbuf_issue >= kBStages) bbuf_issue -= kBStages;
     const uint8_t* bnxt = b_lds + bnext * kBTile;
-    const uint8_t* anxt = lds + (stage ^ 1) * kATile;
-    int snext = sbuf + 1 == 3 ? 0 : sbuf + 1;
+    const uint8_t* anxt = lds + (kFetchers ? bnext : stage ^ 1) * kATile;
+    int snext = sbuf + 1 == (kFetchers ? kScaleSlots : 3) ? 0 : sbuf + 1;
     // Per round, with three b buffers: the rest of the next a tile at subtiles 0,1; the b tile two
-    // rounds ahead at 2..5 (with four subtiles in all: 0 and 1); after the barrier the first half of the a tile after next, into the
+    // rounds ahead at 2..5; after the barrier the first half of the a tile after next, into the
     // buffer whose fragments every wave has just left behind.  One transfer per subtile: a burst
     // would queue up in the texture path ahead of the LDS reads.
     // With two b buffers (wgrad form) the b tile has to land within one round like the a tile, so
     // both go out in the four subtiles that follow the barrier, one transfer of each per subtile.
     auto issue_slot = [&](int i) {
-      if (kBAhead == 2 && NS == 8) {
+      if (kFetchers) return;
+      if (kBAhead == 2) {
         if (i < 2) {
           issue_a(rs_a1, stage ^ 1, kb1, i + 2);
         } else if (i < 6) {
-#pragma unroll
-          for (int t = 0; t < NB / 4; ++t) issue_b(rs_b2, bbuf_issue, kb2, (i - 2) * (NB / 4) + t);
+          issue_b(rs_b2, bbuf_issue, kb2, i - 2);
         } else {
           issue_a(rs_a2, stage, kb2, i - 6);
-        }
-      } else if (kBAhead == 2) {               // (four n-subtiles)
-        if (i == 0) {
-          issue_a(rs_a1, stage ^ 1, kb1, 2);
-          issue_a(rs_a1, stage ^ 1, kb1, 3);
-        } else if (i == 1) {
-#pragma unroll
-          for (int t = 0; t < NB; ++t) issue_b(rs_b2, bbuf_issue, kb2, t);
-        } else {
-          issue_a(rs_a2, stage, kb2, i - 2);
         }
       } else if (i < 2) {
         issue_a(rs_a1, stage ^ 1, kb1, i + 2);
@@ -616,6 +748,11 @@ __global__ __launch_bounds__(128 * WM) void gemm_kernel(const GemmParams p) {
       // Own transfers for the next round have landed and own LDS reads of this round's buffers are
       // done; then everyone's.  With three b buffers the NB b transfers of this round (the
       // youngest vector-memory operations) are for the round after next and may stay in flight.
+      // (kFetchers: the fetching waves wait for them)
+      if (kFetchers) {
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        return;
+      }
       if (kBAhead == 2) __builtin_amdgcn_s_waitcnt(0x0070 | NB);  // vmcnt(NB) lgkmcnt(0)
       else __builtin_amdgcn_s_waitcnt(0x0070);               // vmcnt(0) lgkmcnt(0)
       __builtin_amdgcn_s_barrier();
@@ -636,15 +773,16 @@ __global__ __launch_bounds__(128 * WM) void gemm_kernel(const GemmParams p) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) part[1][j] = part_c[j];
       // wgrad form: the four per-row b scales of subtile i for this lane's four n
-      const float* sb_row = sb_lds + sbuf * 256 + wn * (TN / 2) + g * 4;
+      const float* sb_row = sb_lds + sbuf * kSbSlot + wn * WC + g * 4;
       v4f sbv[2];
       if (MODE == kScaleRow) sbv[0] = *reinterpret_cast<const v4f*>(sb_row);
-      if (MODE == kScaleRow) issue_sb_load(tile_1, kb1_rel, snext);
+      if (MODE == kScaleRow && !kFetchers) issue_sb_load(tile_1, kb1_rel, snext);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int i = 0; i < NS; ++i) {
         if (i == NS - 2) round_sync();
         wf[(i + 2) % 3] = read_ahead(i);
+        if (kFetchers && i == NS - 2) read_scales(snext, s_raw);
         if (MODE == kScaleRow && i > 0) sbv[i & 1] = *reinterpret_cast<const v4f*>(sb_row + i * 16);   // used by the FMAs of group i+1
         issue_slot(i);
         __builtin_amdgcn_sched_barrier(0);
@@ -684,14 +822,15 @@ __global__ __launch_bounds__(128 * WM) void gemm_kernel(const GemmParams p) {
       wf[0] = wf_n0;
       wf[1] = wf_n1;
       // per-row b scales: this lane's row of subtile i is row i * 16 + l16 of the wave's 128
-      const float* sb_lane = sb_lds + sbuf * 256 + wn * (TN / 2) + l16;
+      const float* sb_lane = sb_lds + sbuf * kSbSlot + wn * WC + l16;
       int e_bi[2] = {127, 127};
       if (MODE == kScalePow2Row) e_bi[0] = (int)(__builtin_bit_cast(uint32_t, sb_lane[0]) >> 23);
-      if (MODE == kScalePow2Row) issue_sb_load(tile_1, kb1_rel, snext);
+      if (MODE == kScalePow2Row && !kFetchers) issue_sb_load(tile_1, kb1_rel, snext);
 #pragma unroll
       for (int i = 0; i < NS; ++i) {
         if (i == NS - 2) round_sync();
         wf[(i + 2) % 3] = read_ahead(i);
+        if (kFetchers && i == NS - 2) read_scales(snext, s_raw);
         if (MODE == kScalePow2Row && i < NS - 1) e_bi[(i + 1) & 1] = (int)(__builtin_bit_cast(uint32_t, sb_lane[(i + 1) * 16]) >> 23);
         issue_slot(i);
         __builtin_amdgcn_sched_barrier(0);
@@ -747,7 +886,7 @@ __global__ __launch_bounds__(128 * WM) void gemm_kernel(const GemmParams p) {
   uint8_t* stg_hi = kBAhead == 1 ? lds + (stage ^ 1) * kATile + wave * 4096 + 2048 : stg + 2048;
   if (kBAhead == 1) stg += 2048;
   auto stg_row = [&](int row) { return (row < 8 ? stg : stg_hi) + (row & 7) * 256; };   // (row = l16e: the write side)
-  const int ncol = n0 + wn * (TN / 2);                 // first column of the wave tile
+  const int ncol = n0 + wn * WC;                 // first column of the wave tile
   const bool cols_ok = ncol < N;
   constexpr int kHalves = OUT_F32 && NS == 8 ? 2 : 1;       // fp32 rows of 128 columns take two slices
   constexpr int kPerHalf = NS / kHalves;           // n-subtiles per slice
@@ -760,7 +899,7 @@ __global__ __launch_bounds__(128 * WM) void gemm_kernel(const GemmParams p) {
   const __amdgpu_buffer_rsrc_t rsrc_st = __builtin_amdgcn_make_buffer_rsrc(
       (void*)(reinterpret_cast<uint8_t*>(p.c) +
               ((int64_t)row0 * p.ldc + ncol + (GROUPED == kGroupedK ? (int64_t)T0.expert * p.c_se : 0)) * kEsize), 0,
-      cols_ok && rows_valid > 0 ? (int)((((int64_t)rows_valid - 1) * p.ldc + TN / 2) * kEsize) : 0, 0x00020000);
+      cols_ok && rows_valid > 0 ? (int)((((int64_t)rows_valid - 1) * p.ldc + WC) * kEsize) : 0, 0x00020000);
   const uint32_t st_lane = (uint32_t)(((wm * 64 + ge * 4) * (int)p.ldc) * kEsize + l16e * 16);
   const int st_row = (int)p.ldc * kEsize;        // bytes from one row of c to the next
   auto store_tile = [&](auto with_bias) {
@@ -810,8 +949,8 @@ __global__ __launch_bounds__(128 * WM) void gemm_kernel(const GemmParams p) {
             // staging row s of pass j is tile row 4 s + j (s = 4 (k2 + k) + ge: the ge part is in st_lane).
             // Streaming stores: the output is not read again here, and as ordinary stores a tile's
             // 128-256 KB would push operand panels out of the L2.
-            // (64 columns of bf16 are 128 bytes: half of the lanes hold a row)
-            if (OUT_F32 || NS == 8 || l16e < 8)
+            // (rows of fewer than 256 bytes: the first lanes hold them)
+            if (WC * kEsize >= 256 || l16e < WC * kEsize / 16)
               __builtin_amdgcn_raw_buffer_store_b128(val[k], rsrc_st, st_lane, (16 * (k2 + k) + j) * st_row + h * 256, 2);
           }
           // A 128-bit store reads its data registers over several cycles after it has issued, and a vector instruction
@@ -891,9 +1030,15 @@ __global__ __launch_bounds__(128 * WM) void gemm_kernel(const GemmParams p) {
 #pragma unroll
       for (int i = 0; i < NS; ++i) acc[i][j] = zero;
   }
+  if constexpr (kFetchers) {
+    // this tile's results have been read from the b buffer that the fetching waves fill next
+    if (!EPI) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    lookup(tile + 1, T0);
+  } else {
   T0 = T1;
   T1 = T2;
   lookup(tile + 3, T2);
+  }
   }
 
   // Transfers issued past the end of the list (they fetch nothing) still target this workgroup's
@@ -901,203 +1046,8 @@ __global__ __launch_bounds__(128 * WM) void gemm_kernel(const GemmParams p) {
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
 }
 
-// ---------------------------------------------------------------------------------------------
-// small problems: at most one 64 x 128 tile per compute unit
-// ---------------------------------------------------------------------------------------------
-// One 64 x 128 output tile per workgroup of 4 waves (2 x 2, wave tile 32 x 64), no persistence.  Same operand layout
-// in LDS as above (global -> LDS transfers, swizzle, fragment reads), five stages of one a tile and one b tile (24 KB),
-// transfers four k-blocks ahead, one barrier per k-block.  Same arithmetic in the same order as the kernel above (one
-// matrix instruction per 16 x 16 subtile and k-block; block form: acc += partial * (sa * sb)), so the two give identical
-// results.  Per-tensor and 128x128-block scale forms, dense, bf16 or fp32 output, bias.
-constexpr int kSmallThreads = 256;
-constexpr int kSmallTile = 128;      // columns
-constexpr int kSmallRows = 64;
-constexpr int kSmallStages = 5;
-
-template <int MODE, bool OUT_F32>
-__global__ __launch_bounds__(kSmallThreads) void gemm_small_kernel(const GemmParams p) {
-  static_assert(MODE == kScaleTensor || MODE == kScaleBlock, "per-tensor or block scales");
-  constexpr int TM = kSmallRows;
-  constexpr int kStageBytes = (TM + kSmallTile) * BK;     // a tile + b tile
-  constexpr int NA = TM / 32;                             // a transfers per wave and k-block; also m-subtiles per wave
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[kSmallStages * kStageBytes];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wn = wave & 1, wm = wave >> 1;
-  const int l16 = lane & 15, g = lane >> 4;
-  const int kblocks = p.K / BK;
-  const int tiles_n = p.N / kSmallTile;
-  const int tm = blockIdx.x / tiles_n, tn = blockIdx.x % tiles_n;
-  const int row0 = tm * TM, n0 = tn * kSmallTile;
-  const int rows_valid = p.M - row0 < TM ? p.M - row0 : TM;
-
-  // transfers: as in gemm_kernel, a wave moves 8 rows x 128 B per instruction, four per operand tile and k-block;
-  // the resources start at the tile's first row and end with the tensor (rows past it read as zero); k-blocks
-  // past the end go through an empty resource and fetch nothing
-  auto span = [&](int64_t rows, int64_t ld) {
-    const int64_t bytes = rows > 0 ? (rows - 1) * ld + p.K : 0;
-    return (int)(bytes < (int64_t)0x7FFFF000 ? bytes : (int64_t)0x7FFFF000);
-  };
-  const __amdgpu_buffer_rsrc_t rs_a = __builtin_amdgcn_make_buffer_rsrc((void*)(p.a + (int64_t)row0 * p.lda), 0,
-                                                                      span(p.M - row0, p.lda), 0x00020000);
-  const __amdgpu_buffer_rsrc_t rs_b = __builtin_amdgcn_make_buffer_rsrc((void*)(p.b + (int64_t)n0 * p.ldb), 0,
-                                                                      span(p.N - n0, p.ldb), 0x00020000);
-  const __amdgpu_buffer_rsrc_t rs_none = __builtin_amdgcn_make_buffer_rsrc((void*)p.a, 0, 0, 0x00020000);
-  uint32_t a_off[NA], b_off[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = (wave * 4 + i) * 8 + (lane >> 3);
-    const int chunk = (lane & 7) ^ row_swizzle(r);
-    b_off[i] = (uint32_t)r * (uint32_t)p.ldb + chunk * 16 - i * 1024;
-  }
-#pragma unroll
-  for (int i = 0; i < NA; ++i) {
-    const int r = (wave * NA + i) * 8 + (lane >> 3);
-    const int chunk = (lane & 7) ^ row_swizzle(r);
-    a_off[i] = (uint32_t)r * (uint32_t)p.lda + chunk * 16 - i * 1024;
-  }
-  auto issue_stage = [&](int kb, int stage) {
-    const bool ok = kb < kblocks;
-    const __amdgpu_buffer_rsrc_t ra = ok ? rs_a : rs_none, rb = ok ? rs_b : rs_none;
-    uint8_t* sa_base = lds + stage * kStageBytes + wave * (NA * 1024);
-    uint8_t* sb_base = lds + stage * kStageBytes + TM * BK + wave * 4096;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)sa_base, 16, a_off[0], kb * BK, 0, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)sa_base, 16, a_off[1], kb * BK, 1024, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)sb_base, 16, b_off[0], kb * BK, 0, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)sb_base, 16, b_off[1], kb * BK, 1024, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)sb_base, 16, b_off[2], kb * BK, 2048, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)sb_base, 16, b_off[3], kb * BK, 3072, 0);
-  };
-  const int pc0 = (2 * g) ^ row_swizzle(l16);
-  const int a_frag = (wm * (TM / 2) + l16) * BK, b_frag = TM * BK + (wn * 64 + l16) * BK;
-
-  // scales of the block form: this lane's four rows of a (clamped: rows past M are never stored), the tile's
-  // one 128-row block of b
-  const float* sa_row[NA];
-#pragma unroll
-  for (int j = 0; j < NA; ++j) {
-    const int r = row0 + wm * (TM / 2) + j * 16 + l16;
-    sa_row[j] = p.sa + (int64_t)(r < p.M ? r : p.M - 1) * p.sa_sm;
-  }
-  const float* sb_blk = p.sb + (int64_t)(n0 >> 7) * p.sb_sn;
-
-  const v4f zero = {0.f, 0.f, 0.f, 0.f};
-  v4f acc[4][NA];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < NA; ++j) acc[i][j] = zero;
-
-  // Transfers run four k-blocks ahead (five stages); the block form's scales are fetched three k-blocks ahead
-  // into a ring of registers, so that waiting for them never waits for a transfer that is not needed yet
-  // (vector-memory operations complete in order).  Issue order per iteration i: wait + barrier, scale loads of
-  // k-block i + 3, transfers of k-block i + 4.
-  float s_ring[4][5];
-  auto load_scales = [&](int kb, float raw[5]) {
-    if (MODE == kScaleBlock) {
-      const int kk = kb < kblocks ? kb : kblocks - 1;
-      raw[4] = sb_blk[(int64_t)kk * p.sb_sk];
-#pragma unroll
-      for (int j = 0; j < NA; ++j) raw[j] = sa_row[j][(int64_t)kk * p.sa_sk];
-    }
-  };
-  issue_stage(0, 0);
-  load_scales(0, s_ring[0]);
-  issue_stage(1, 1);
-  load_scales(1, s_ring[1]);
-  issue_stage(2, 2);
-  load_scales(2, s_ring[2]);
-  issue_stage(3, 3);
-  int st = 0, st_issue = 4;
-  // one k-block; Q = kb % 4 is the ring slot that holds its scales (static, so the ring needs no register moves:
-  // a move would have to wait for the load it moves)
-  auto k_block = [&](int kb, auto q_tag) {
-    constexpr int Q = decltype(q_tag)::value;
-    // all but the youngest transfers of three k-blocks (and, block form, the scale loads issued between them)
-    // have landed: this k-block's tiles of this wave; after the barrier everyone's, and everyone has left the
-    // stage that is refilled next
-    // (in flight and allowed to stay so: the transfers of three k-blocks, NA + 4 each, and in the block form the scale
-    // loads of two, NA + 1 each)
-    if (MODE == kScaleBlock) asm volatile("s_waitcnt vmcnt(24)\n\ts_barrier" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(18)\n\ts_barrier" ::: "memory");
-    load_scales(kb + 3, s_ring[(Q + 3) & 3]);
-    asm volatile("" ::: "memory");       // (keeps the scale loads ahead of the transfers, as the wait above counts them)
-    issue_stage(kb + 4, st_issue);
-    const uint8_t* base = lds + st * kStageBytes;
-    st = st == kSmallStages - 1 ? 0 : st + 1;
-    st_issue = st_issue == kSmallStages - 1 ? 0 : st_issue + 1;
-    v8i xf[NA], wf[4];
-#pragma unroll
-    for (int j = 0; j < NA; ++j) xf[j] = frag_read(base + a_frag + j * 16 * BK, pc0);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) wf[i] = frag_read(base + b_frag + i * 16 * BK, pc0);
-    if (MODE == kScaleTensor) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < NA; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[i], xf[j], acc[i][j], 0, 0, 0, 0, 0, 0);
-    } else {
-      v4f part[4][NA];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < NA; ++j)
-          part[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[i], xf[j], zero, 0, 0, 0, 0, 0, 0);
-      float s[NA];
-#pragma unroll
-      for (int j = 0; j < NA; ++j) s[j] = s_ring[Q][j] * s_ring[Q][4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < NA; ++j)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) acc[i][j][r] = __builtin_fmaf(part[i][j][r], s[j], acc[i][j][r]);
-    }
-  };
-  for (int kb = 0; kb < kblocks; kb += 4) {
-    k_block(kb, std::integral_constant<int, 0>{});
-    if (kb + 1 < kblocks) k_block(kb + 1, std::integral_constant<int, 1>{});
-    if (kb + 2 < kblocks) k_block(kb + 2, std::integral_constant<int, 2>{});
-    if (kb + 3 < kblocks) k_block(kb + 3, std::integral_constant<int, 3>{});
-  }
-  __builtin_amdgcn_s_waitcnt(0x0F70);   // the transfers past the last k-block (they fetch nothing) still target this LDS
-
-  // store: a lane holds, per subtile, four consecutive columns of one row
-  float tensor_scale = 1.f;
-  if (MODE == kScaleTensor) tensor_scale = p.sa[0] * p.sb[0];
-#pragma unroll
-  for (int j = 0; j < NA; ++j) {
-    const int r = wm * (TM / 2) + j * 16 + l16;
-    if (r >= rows_valid) continue;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int col = n0 + wn * 64 + i * 16 + g * 4;
-      float v[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        v[q] = acc[i][j][q];
-        if (MODE == kScaleTensor) v[q] *= tensor_scale;
-      }
-      if (p.bias) {
-        const uint2 braw = *reinterpret_cast<const uint2*>(p.bias + col);
-        v[0] += bf16lo(braw.x); v[1] += bf16hi(braw.x); v[2] += bf16lo(braw.y); v[3] += bf16hi(braw.y);
-      }
-      const int64_t o = (int64_t)(row0 + r) * p.ldc + col;
-      if (OUT_F32) {
-        *reinterpret_cast<v4f*>(reinterpret_cast<float*>(p.c) + o) = v4f{v[0], v[1], v[2], v[3]};
-      } else {
-        u32x2 w2;
-        w2[0] = pack_bf16x2(v[0], v[1]);
-        w2[1] = pack_bf16x2(v[2], v[3]);
-        *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(p.c) + o) = w2;
-      }
-    }
-  }
-}
-
-// Test hook.  0: pick_shape and the rules below choose the form; 1: always 256 x 256 tiles; 2: the smallest tile a form has
-// (64 x 128 where 128 x 128 tiles would be fewer than the compute units); 3: 128 x 256 tiles where a form has them
+// Test hook.  0: pick_shape and the rules below choose the form; 1: always 256 x 256 tiles; 2: the smallest tile a form has;
+// 3: 128 x 256 and 4: 128 x 128 tiles where a form has them
 static std::atomic<int> g_small_gemm_mode{0};   // (atomic: the test hook may be called from any thread)
 
 // Workgroups to launch for `tiles` tiles: at most one per CU, a multiple of 8 (one share per XCD) unless there are fewer
@@ -1116,30 +1066,30 @@ static int persistent_grid(int64_t tiles) {
   return (int)(up < most ? up : most);
 }
 
-// The tile of a GEMM: 256 x 256 (8 waves), 128 x 256 or 128 x 128 (4 waves); a wave's part has 64 rows in each.
-enum TileShape { k256x256, k128x256, k128x128 };
+// The tile of a GEMM: 256 x 256 (8 waves), or 128 x 256, 128 x 128 or 64 x 128 (4 waves that multiply, 4 that fetch).
+enum TileShape { k256x256, k128x256, k128x128, k64x128 };
 
 static int64_t tile_count(int64_t M, int64_t N, TileShape shape) {
-  const int tm = shape == k256x256 ? 256 : 128, tn = shape == k128x128 ? 128 : 256;
+  const int tm = shape == k256x256 ? 256 : (shape == k64x128 ? 64 : 128), tn = shape == k128x128 || shape == k64x128 ? 128 : 256;
   return ((M + tm - 1) / tm) * ((N + tn - 1) / tn);
 }
 
 // The smallest tile with which the problem is still one round, one tile per compute unit; problems of several rounds
 // take 256 x 256, which moves the fewest bytes through L2 and LDS per product.  A workgroup's round trip per k-block
 // is bound by what its compute unit's vector-memory path and LDS move, so with idle units a smaller tile is less work
-// on the same critical path.  us with 256 x 256 / 128 x 256 / 128 x 128 tiles:
-//   block  1000 x 7168 x 7168 (112 / 224 / 448 tiles)    79 / 61 / 61-69   (128 x 128 without pipelining: 91)
-//   block  1531 x 2048 x 7168 ( 48 /  96 / 192)          70 / 50 / 43
-//   block   300 x 14336 x 7168 (112 / 168 / 336)         78 / 56 / 86
-//   pow2   2048 x 4096 x 7168 (128 / 256 / 512)          67 / 50 / 54
-//   rows   2048 x 1024 x 4096 ( 32 /  64 / 128)          54 / 38 / 30
-//   rows, onto c  1024 x 1024 x 8192 (16 / 32 / 64)     104 / 74 / 54
-//   more than one round: block 4096 x 4096 x 4096 58 / 68 / 69, 3000 x 3072 x 3072 39 / 48 / 44, 1531 x 7168 x 2048
-//   (168 / 336 / 672 tiles) 29 / 36 / 32, pow2 2048 x 7168 x 4096 48 / 56 / 61
+// on the same critical path.  us with 256 x 256 / 128 x 256 / 128 x 128 / 64 x 128 tiles (tiles of the one taken):
+//   block   256 x 7168 x 7168    80 / 53 / 39 / 30 (224)         512 x 7168 x 7168    79 / 52 / 39 / 51 (224)
+//   block  1000 x 7168 x 7168    81 / 54 / 66 / 89 (224)        2048 x 7168 x 7168    91 / 103 / 124 / 152 (224)
+//   block  1000 x 2048 x 4096    40 / 27 / 19 / 16 (256)        1400 x 2048 x 4096    40 / 27 / 20 / 26 (176)
+//   block  1400 x 3072 x 3072    32 / 22 / 28 / 30 (132)         400 x 1024 x 8192    73 / 47 / 31 / 23 (56)
+//   block  1531 x 7168 x 2048 (168 / 336 / 672 tiles)  26 / 31 / 30        4096 x 4096 x 4096  57 / 62 / 75
+//   pow2   2048 x 4096 x 7168    76 / 51 / 65                   rows   2048 x 1024 x 4096    51 / 33 / 34 / 18
+//   rows, onto c  1024 x 1024 x 4096   59 / 38 / 31 / 19
 static TileShape pick_shape(int64_t M, int64_t N) {
   const int mode = g_small_gemm_mode.load(std::memory_order_relaxed);
-  if (mode != 0) return mode == 1 ? k256x256 : (mode == 2 ? k128x128 : k128x256);
   const int64_t cus = persistent_grid((int64_t)1 << 40);
+  if (mode != 0) return mode == 1 ? k256x256 : (mode == 2 ? k64x128 : (mode == 3 ? k128x256 : k128x128));
+  if (tile_count(M, N, k64x128) <= cus) return k64x128;
   if (tile_count(M, N, k128x128) <= cus) return k128x128;
   if (tile_count(M, N, k128x256) <= cus) return k128x256;
   return k256x256;
@@ -1178,16 +1128,6 @@ static GroupedTiles pick_grouped(int64_t M, int64_t N, int experts) {
   return M / 129 * tiles_n <= cus / 4 ? kLowTiles : kEitherTiles;
 }
 
-// 64 x 128 tiles, where that is still one round (dense, per tensor or by blocks; 256 x 7168 x 7168: 30 us against 41
-// with 128 x 128 tiles, 700 x 1024 x 8192: 32 against 46).
-static bool use_small_kernel(int64_t M, int64_t N) {
-  const int mode = g_small_gemm_mode.load(std::memory_order_relaxed);
-  if (mode == 1 || mode == 3) return false;
-  const int64_t cus = persistent_grid((int64_t)1 << 40);
-  if (mode == 2) return tile_count(M, N, k128x128) < cus;
-  return ((M + kSmallRows - 1) / kSmallRows) * (N / kSmallTile) <= cus;
-}
-
 // Few rows of a (decode): bound by reading b once, which the tile kernels do not reach (gemm_skinny.hip; 8 rows of
 // [7168, 16384]: 60 us with 64 x 128 tiles, 20.6 us; 64 rows: 64 and 26.8 us; 37 rows of [36864, 7168]: 81 us with 256 x 256
 // tiles, 41.6 us), with the same bits.  try_skinny hands the problem over if it is one; otherwise false.
@@ -1205,37 +1145,29 @@ static bool try_skinny(const GemmParams& p, SkinnyMode mode, int out_type, hipSt
   return true;
 }
 
-template <int MODE>
-static int launch_small(const GemmParams& p, int out_type, hipStream_t stream) {
-  dim3 grid((unsigned)((((int64_t)p.M + kSmallRows - 1) / kSmallRows) * (p.N / kSmallTile))), block(kSmallThreads);
-  if (out_type == HPFP8_OUT_F32) gemm_small_kernel<MODE, true><<<grid, block, 0, stream>>>(p);
-  else gemm_small_kernel<MODE, false><<<grid, block, 0, stream>>>(p);
-  return check_launch("gemm (small tiles)");
-}
-
-template <int MODE, int GROUPED, bool SA4, int WM, int NS>
+template <int MODE, int GROUPED, bool SA4, int WM, int NS, int WN>
 static int launch_sa(const GemmParams& p, int out_type, int64_t tiles, hipStream_t stream) {
-  dim3 grid((unsigned)persistent_grid(tiles)), block(128 * WM);
+  dim3 grid((unsigned)persistent_grid(tiles)), block(tile_threads(WM, WN));
   if (out_type == HPFP8_OUT_F32) {
     if constexpr (MODE != kScaleTensor && GROUPED == kDense) {   // (the per-tensor and grouped entry points have no accumulate)
       if (p.accumulate) {
-        gemm_kernel<MODE, GROUPED, true, true, SA4, 0, WM, NS><<<grid, block, 0, stream>>>(p);
+        gemm_kernel<MODE, GROUPED, true, true, SA4, 0, WM, NS, WN><<<grid, block, 0, stream>>>(p);
         return check_launch("gemm");
       }
     }
-    gemm_kernel<MODE, GROUPED, true, false, SA4, 0, WM, NS><<<grid, block, 0, stream>>>(p);
+    gemm_kernel<MODE, GROUPED, true, false, SA4, 0, WM, NS, WN><<<grid, block, 0, stream>>>(p);
   } else {
-    gemm_kernel<MODE, GROUPED, false, false, SA4, 0, WM, NS><<<grid, block, 0, stream>>>(p);
+    gemm_kernel<MODE, GROUPED, false, false, SA4, 0, WM, NS, WN><<<grid, block, 0, stream>>>(p);
   }
   return check_launch("gemm");
 }
 
-template <int MODE, int GROUPED, int WM, int NS>
+template <int MODE, int GROUPED, int WM, int NS, int WN>
 static int launch_shape(const GemmParams& p, int out_type, int64_t tiles, hipStream_t stream) {
-  if constexpr (MODE != kScaleTensor) {
-    if (p.sa_sm == 1) return launch_sa<MODE, GROUPED, true, WM, NS>(p, out_type, tiles, stream);
+  if constexpr (MODE != kScaleTensor && !fetchers(WM)) {      // (fetched to LDS, sa may have any strides)
+    if (p.sa_sm == 1) return launch_sa<MODE, GROUPED, true, WM, NS, WN>(p, out_type, tiles, stream);
   }
-  return launch_sa<MODE, GROUPED, false, WM, NS>(p, out_type, tiles, stream);
+  return launch_sa<MODE, GROUPED, false, WM, NS, WN>(p, out_type, tiles, stream);
 }
 
 template <int MODE, int GROUPED>
@@ -1246,12 +1178,13 @@ static int launch(GemmParams p, int out_type, TileShape shape, hipStream_t strea
   // upper bound on row tiles: every expert may add one partial tile
   if (GROUPED == kGroupedRows) tiles = (p.M / (shape == k256x256 ? 256 : 128) + p.experts) * ((p.N + 255) / 256);
   if constexpr (GROUPED != kGroupedK) {
-    if (shape == k128x256) return launch_shape<MODE, GROUPED, 2, 8>(p, out_type, tiles, stream);
+    if (shape == k128x256) return launch_shape<MODE, GROUPED, 2, 8, 2>(p, out_type, tiles, stream);
   }
   if constexpr (GROUPED == kDense) {
-    if (shape == k128x128) return launch_shape<MODE, GROUPED, 2, 4>(p, out_type, tiles, stream);
+    if (shape == k128x128) return launch_shape<MODE, GROUPED, 2, 4, 2>(p, out_type, tiles, stream);
+    if (shape == k64x128) return launch_shape<MODE, GROUPED, 1, 2, 4>(p, out_type, tiles, stream);
   }
-  return launch_shape<MODE, GROUPED, 4, 8>(p, out_type, tiles, stream);
+  return launch_shape<MODE, GROUPED, 4, 8, 2>(p, out_type, tiles, stream);
 }
 
 template <int MODE>
@@ -1331,7 +1264,6 @@ static int gemm_blockwise_impl(const void* a, int64_t lda, const float* sa, int6
   if (sb_gran == 128) {
     if (try_skinny(p, pow2 ? kSkinnyPow2 : kSkinnyBlock, out_type, (hipStream_t)stream, rc)) return rc;
     if (pow2) return launch<kScalePow2, kDense>(p, out_type, pick_shape(M, N), (hipStream_t)stream);
-    if (!accumulate && use_small_kernel(M, N)) return launch_small<kScaleBlock>(p, out_type, (hipStream_t)stream);
     return launch<kScaleBlock, kDense>(p, out_type, pick_shape(M, N), (hipStream_t)stream);
   }
   // per-row b scales travel to LDS as one contiguous 1 KB piece per k-block
@@ -1396,13 +1328,13 @@ int hpfp8_gemm_blockwise_swiglu_quantize(const void* a, int64_t lda, const float
   const TileShape shape = pick_shape_swiglu(M, 2 * inter);
   const int64_t tiles = tile_count(M, 2 * inter, shape);
   p.tiles = (int)tiles;
-  dim3 grid((unsigned)persistent_grid(tiles)), block(shape == k256x256 ? 512 : 256);
+  dim3 grid((unsigned)persistent_grid(tiles)), block(tile_threads(shape == k256x256 ? 4 : 2, 2));
   hipStream_t st = (hipStream_t)stream;
   const bool sa4 = sa_stride_m == 1;
 #define HPFP8_LAUNCH_EPI(MODE, SA4, EPI) \
   do { \
     if (shape == k256x256) gemm_kernel<MODE, kDense, false, false, SA4, EPI, 4><<<grid, block, 0, st>>>(p); \
-    else gemm_kernel<MODE, kDense, false, false, SA4, EPI, 2><<<grid, block, 0, st>>>(p); \
+    else gemm_kernel<MODE, kDense, false, false, false, EPI, 2><<<grid, block, 0, st>>>(p); \
   } while (0)
   if (pow2) {
     if (sa4) { if (fast) HPFP8_LAUNCH_EPI(kScalePow2, true, 2); else HPFP8_LAUNCH_EPI(kScalePow2, true, 1); }
@@ -1415,7 +1347,7 @@ int hpfp8_gemm_blockwise_swiglu_quantize(const void* a, int64_t lda, const float
   return check_launch(what);
 }
 
-void hpfp8_debug_set_small_gemm(int mode) { g_small_gemm_mode.store(mode >= 1 && mode <= 3 ? mode : 0, std::memory_order_relaxed); }
+void hpfp8_debug_set_small_gemm(int mode) { g_small_gemm_mode.store(mode >= 1 && mode <= 4 ? mode : 0, std::memory_order_relaxed); }
 
 int64_t hpfp8_gemm_few_rows(int64_t K) { return few_rows(K); }
 
@@ -1429,7 +1361,6 @@ int hpfp8_gemm_per_tensor(const void* a, int64_t lda, const float* sa_inv, const
   p.c = c; p.ldc = ldc; p.bias = (const uint16_t*)bias;
   p.M = (int)M; p.N = (int)N; p.K = (int)K;
   if (try_skinny(p, kSkinnyTensor, out_type, (hipStream_t)stream, rc)) return rc;
-  if (use_small_kernel(M, N)) return launch_small<kScaleTensor>(p, out_type, (hipStream_t)stream);
   return launch<kScaleTensor, kDense>(p, out_type, pick_shape(M, N), (hipStream_t)stream);
 }
 

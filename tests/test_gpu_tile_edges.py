@@ -539,3 +539,34 @@ def test_per_tensor_codes_with_their_transpose(gpu, m, k, one_launch, polls, mon
                 assert torch.equal(out[3], ops.column_sum(x))
     finally:
         _lib.load().hpfp8_debug_set_spin_limit(256)
+
+
+@pytest.mark.parametrize("mode", [2, 3, 4])
+@pytest.mark.parametrize("m,n,blocks", [(70, 256, 1), (200, 384, 2), (130, 128, 3), (129, 640, 4), (64, 128, 6), (65, 256, 7), (1300, 2560, 3),
+                                        (2300, 4224, 1)])
+def test_tiles_with_fetching_waves_give_the_bits_of_256_x_256_ones(gpu, mode, m, n, blocks):
+    """Contractions of fewer k-blocks than the rings hold, as many and more; ragged rows and columns; several tiles per workgroup (the last
+    two shapes: 420 and 1188 tiles of 64 x 128, 220 and 594 of 128 x 128, 110 and 306 of 128 x 256); scales of a in both layouts."""
+    from hpfp8 import _lib, ops
+    k = 128 * blocks
+    x, w = _normal((m, k), 1, gpu, outliers=True), _normal((n, k), 2, gpu, 0.05)
+    bias, c0 = _normal((n,), 3, gpu), _normal((m, n), 4, gpu).float()
+    got = {}
+    for hook in (1, mode):
+        _lib.load().hpfp8_debug_set_small_gemm(hook)
+        try:
+            r = got[hook] = []
+            for pow2 in (False, True):
+                a, sa = ops.quantize_1x128(x, kmajor=True, pow2=pow2)
+                for gran, (b, sb) in ((128, ops.quantize_128x128(w, pow2=pow2)), (1, ops.quantize_1x128(w, kmajor=True, pow2=pow2))):
+                    for s in (sa, sa.contiguous()):
+                        r.append(ops.gemm_blockwise(a, s, b, sb, bias=bias, sb_gran=gran, pow2_scales=pow2))
+                        r.append(ops.gemm_blockwise(a, s, b, sb, sb_gran=gran, out=c0.clone(), accumulate=True, pow2_scales=pow2))
+            a, _, sa = ops.quantize_per_tensor(x)
+            b, _, sb = ops.quantize_per_tensor(w)
+            r.append(ops.gemm_per_tensor(a, sa, b, sb, bias=bias))
+            r.append(ops.gemm_per_tensor(a, sa, b, sb, out_dtype=torch.float32))
+        finally:
+            _lib.load().hpfp8_debug_set_small_gemm(0)
+    for one, other in zip(got[1], got[mode]):
+        assert torch.equal(one, other)
