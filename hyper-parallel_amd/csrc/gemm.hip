@@ -88,7 +88,7 @@ struct GemmParams {
   int pow2_out;
   float* q_scale;
   float* q_scale_inv;
-  int choose_cus;         // grouped by rows: launched with both tile heights, the kernel of the better one runs (0: the only one)
+  int choose_cus;         // grouped by rows, tile chosen on the device: the compute units there are
 };
 
 // n / d for uniform values, without the compiler's division (some 30 dependent instructions; a tile lookup has four, and a
@@ -178,37 +178,50 @@ struct ExpertChunk {
 
 // Offsets that decrease or run past the row count (a malformed table) are clamped, so that every address derived from them
 // stays inside a.
-__device__ __forceinline__ void load_experts(ExpertChunk& c, const GemmParams& p, int tile_rows, int tiles_n, int lane) {
+__device__ __forceinline__ void expert_ends(ExpertChunk& c, const GemmParams& p, int lane) {
   int end = c.first + lane < p.experts ? p.offs[c.first + lane] : 0;
   end = wave_scan(end > c.row ? end : c.row, [](int a, int b) { return a > b ? a : b; });
   c.end = end < p.M ? end : p.M;
-  int prev = __shfl_up(c.end, 1);
-  if (lane == 0) prev = c.row;
-  c.tile_end = c.tile + wave_scan((c.end - prev + tile_rows - 1) / tile_rows, [](int a, int b) { return a + b; }) * tiles_n;
+}
+__device__ __forceinline__ int expert_rows(const ExpertChunk& c, int lane) {
+  const int prev = __shfl_up(c.end, 1);
+  return c.end - (lane == 0 ? c.row : prev);
+}
+__device__ __forceinline__ void count_tiles(ExpertChunk& c, int tile_rows, int tiles_n, int lane) {
+  c.tile_end = c.tile + wave_scan((expert_rows(c, lane) + tile_rows - 1) / tile_rows, [](int a, int b) { return a + b; }) * tiles_n;
 }
 __device__ __forceinline__ bool next_experts(ExpertChunk& c, const GemmParams& p, int tile_rows, int tiles_n, int lane) {
   if (c.first + 64 >= p.experts) return false;
   c.first += 64;
   c.row = __builtin_amdgcn_readlane(c.end, 63);
   c.tile = __builtin_amdgcn_readlane(c.tile_end, 63);
-  load_experts(c, p, tile_rows, tiles_n, lane);
+  expert_ends(c, p, lane);
+  count_tiles(c, tile_rows, tiles_n, lane);
   return true;
 }
-__device__ __forceinline__ int grouped_tiles(ExpertChunk& c, const GemmParams& p, int tile_rows, int tiles_n, int lane) {
-  c = ExpertChunk{0, 0, 0, 0, 0};
-  load_experts(c, p, tile_rows, tiles_n, lane);
-  while (next_experts(c, p, tile_rows, tiles_n, lane)) {}
-  return __builtin_amdgcn_readlane(c.tile_end, 63);
-}
 
-// Grouped by rows, launched with both tile heights: whether 128-row tiles are the better ones for the rows that the experts
-// have.  A round of them takes three fifths of one of 256-row tiles.
-__device__ __forceinline__ bool better_is_low(const GemmParams& p, int tiles_n, int lane) {
-  ExpertChunk c;
-  const int low = grouped_tiles(c, p, 128, tiles_n, lane), high = grouped_tiles(c, p, 256, tiles_n, lane);
-  const int low_rounds = (low + p.choose_cus - 1) / p.choose_cus;
-  const int high_rounds = (high + p.choose_cus - 1) / p.choose_cus;
-  return __builtin_amdgcn_readfirstlane(3 * low_rounds <= 5 * high_rounds ? 1 : 0) != 0;
+// Grouped by rows: the rows of the best tile for the rows that the experts have, 64 (x 128 columns), 128 or 256 (x 256).  What
+// counts is the rounds of one tile per compute unit; rounds cost 26 : 50 : 83 (measured, us with 64 / 128 / 256 rows: 8192
+// rows of one expert [4096, 7168], 16 / 4 / 2 rounds 338 / 213 / 183, bound by arithmetic; 2048 rows over 32 of them evenly, 4 / 2 / 2
+// rounds 165 / 168 / 224, bound by reading b; 64 rows of one, one round each 21 / 41 / 66).  c: the first 64 experts.
+__device__ __forceinline__ int grouped_tile_rows(const ExpertChunk& c, const GemmParams& p, int lane) {
+  int low = 0, mid = 0, high = 0;
+  for (ExpertChunk e = c;;) {
+    const int rows = expert_rows(e, lane);
+    const auto sum = [](int a, int b) { return a + b; };
+    low += __builtin_amdgcn_readlane(wave_scan((rows + 63) / 64, sum), 63);
+    mid += __builtin_amdgcn_readlane(wave_scan((rows + 127) / 128, sum), 63);
+    high += __builtin_amdgcn_readlane(wave_scan((rows + 255) / 256, sum), 63);
+    if (e.first + 64 >= p.experts) break;
+    e.first += 64;
+    e.row = __builtin_amdgcn_readlane(e.end, 63);
+    expert_ends(e, p, lane);
+  }
+  const int cus = p.choose_cus, tiles_n = (p.N + 255) / 256;
+  const int64_t low_cost = 26 * (int64_t)quotient(low * ((p.N + 127) / 128) + cus - 1, cus);
+  const int64_t mid_cost = 50 * (int64_t)quotient(mid * tiles_n + cus - 1, cus);
+  const int64_t high_cost = 83 * (int64_t)quotient(high * tiles_n + cus - 1, cus);
+  return low_cost <= mid_cost && low_cost <= high_cost ? 64 : (mid_cost <= high_cost ? 128 : 256);
 }
 
 // WM, NS, WN: WM x WN waves multiply, each 64 rows x NS subtiles of 16 columns.  Tiles of 64 and of 128 rows have four more
@@ -216,14 +229,33 @@ __device__ __forceinline__ bool better_is_low(const GemmParams& p, int tiles_n, 
 __host__ __device__ constexpr bool fetchers(int wm) { return wm <= 2; }
 __host__ __device__ constexpr int tile_threads(int wm, int wn) { return 64 * (wm * wn + (fetchers(wm) ? 4 : 0)); }
 
+__host__ __device__ constexpr bool row_scales(int mode) { return mode == kScaleRow || mode == kScalePow2Row; }
+__host__ __device__ constexpr int tile_stages(int mode, int wm, int tn) {         // k-blocks of b (and, with fetching waves, of a) in LDS
+  return !fetchers(wm) ? b_stages(mode) : (wm == 1 ? 6 : (tn == 256 ? 3 : 4));
+}
+// With fetching waves the scales of a k-block travel with its tiles, into a slot of one part per fetching wave: 256 bytes of sb
+// (the scale of the left or of the right half's block; with per-row scales 64 of the tile's rows) and the upper or the lower 64
+// rows of sa.
+constexpr int kScaleSlot = 2048;
+// One LDS object for everything.  (With a second __shared__ array the compiler tells the two apart
+// with alias scopes, and from then on makes every LDS read wait for all transfers into the array it
+// reads, those to other buffers included: the transfers' latency would be paid in every round.)
+__host__ __device__ constexpr int tile_lds(int mode, int wm, int tn) {
+  const int stages = tile_stages(mode, wm, tn);
+  const int scales = fetchers(wm) ? (mode == kScaleTensor ? 0 : (stages + 1) * kScaleSlot) : (row_scales(mode) ? 3 * 256 * 4 : 0);
+  return (fetchers(wm) ? stages : 2) * 64 * wm * BK + stages * tn * BK + scales;
+}
+
+// group: grouped by rows, the first 64 experts with their ends; then those among which tiles are looked up (tile numbers are
+// asked for in increasing order).
 // SA4: the activation scales have unit stride over rows (the k-block-major layout), so a lane's four
 // of them are one 16-byte load.
 // EPI: 0 = c is the GEMM's result; 1 / 2 = the gate/up projection of a SwiGLU MLP with the activation and its
 // 1x128 quantization as the epilogue (1: exactly specified silu, 2: hardware exponential and reciprocal).  A tile's
 // 256 columns are then the 128 gate columns and the 128 up columns of one scaling group of the activation: the b
 // tile's upper 128 rows come from `inter` rows further down, the two waves that share 64 rows hold gate and up.
-template <int MODE, int GROUPED, bool OUT_F32, bool ACC, bool SA4, int EPI = 0, int WM = 4, int NS = 8, int WN = 2>
-__global__ __launch_bounds__(tile_threads(WM, WN)) void gemm_kernel(const GemmParams p) {
+template <int MODE, int GROUPED, bool OUT_F32, bool ACC, bool SA4, int EPI, int WM, int NS, int WN>
+__device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const lds, ExpertChunk group) {
   constexpr int TM = 64 * WM, TN = 16 * NS * WN;       // the tile
   constexpr int WC = 16 * NS;                          // a wave's columns
   constexpr int kWaves = WM * WN;                      // that multiply
@@ -239,21 +271,13 @@ __global__ __launch_bounds__(tile_threads(WM, WN)) void gemm_kernel(const GemmPa
   static_assert(GROUPED != kGroupedK || (!ACC && (MODE == kScaleRow || MODE == kScalePow2Row)),
                 "grouped along the contraction: the wgrad form");
   static_assert(!kFetchers || GROUPED != kGroupedK, "the fetching waves count k-blocks from 0");
-  constexpr int kBStages = !kFetchers ? b_stages(MODE) : (WM == 1 ? 6 : (TN == 256 ? 3 : 4));
+  constexpr int kBStages = tile_stages(MODE, WM, TN);
   constexpr int kAStages = kFetchers ? kBStages : 2;
-  constexpr bool kRowScales = MODE == kScaleRow || MODE == kScalePow2Row;   // per-row b scales, staged in LDS
+  constexpr bool kRowScales = row_scales(MODE);                             // per-row b scales, staged in LDS
   constexpr bool kPromote = MODE == kScaleBlock || MODE == kScaleRow;       // partial sums scaled by FMAs
   constexpr bool kHwScale = MODE == kScalePow2 || MODE == kScalePow2Row;    // scales applied by the MFMA
   constexpr int kBAhead = kBStages - 1;     // k-blocks between issuing a b transfer and using it
-  // One LDS object for everything.  (With a second __shared__ array the compiler tells the two apart
-  // with alias scopes, and from then on makes every LDS read wait for all transfers into the array it
-  // reads, those to other buffers included: the transfers' latency would be paid in every round.)
-  // kFetchers: the scales of a k-block travel with its tiles, into a slot of one part per fetching wave: 256 bytes of sb (the
-  // scale of the left or of the right half's block; with per-row scales 64 of the tile's rows) and the upper or the lower 64
-  // rows of sa.
-  constexpr int kScaleOps = MODE == kScaleTensor ? 0 : 2, kScaleSlot = 2048, kScaleSlots = kBStages + 1;
-  constexpr int kScaleBytes = kFetchers ? (kScaleOps ? kScaleSlots * kScaleSlot : 0) : (kRowScales ? 3 * 256 * 4 : 0);
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[kAStages * kATile + kBStages * kBTile + kScaleBytes];
+  constexpr int kScaleOps = MODE == kScaleTensor ? 0 : 2, kScaleSlots = kBStages + 1;
   // per-row scales of the b operand for one k-block (wgrad form), three stages of 256 floats: the
   // stage of k-block kb+1 is filled while slower waves may still read that of kb-1
   uint8_t* const scale_lds = lds + kAStages * kATile + kBStages * kBTile;
@@ -275,14 +299,15 @@ __global__ __launch_bounds__(tile_threads(WM, WN)) void gemm_kernel(const GemmPa
   // through that run side by side, so at any moment they work on one rectangle.
   int total_tiles = p.tiles;
   if (GROUPED == kGroupedK) total_tiles = p.experts * p.tiles;
-  ExpertChunk group;       // grouped by rows: the experts among which tiles are looked up (tile numbers are asked for in increasing order)
   if (GROUPED == kGroupedRows) {
-    if (p.choose_cus && better_is_low(p, tiles_n, lane) != (TM == 128)) return;
     // tiles are numbered expert by expert; an expert with no rows has none
-    total_tiles = grouped_tiles(group, p, TM, tiles_n, lane);
+    const ExpertChunk first = group;
+    count_tiles(group, TM, tiles_n, lane);
+    while (next_experts(group, p, TM, tiles_n, lane)) {}
+    total_tiles = __builtin_amdgcn_readlane(group.tile_end, 63);
     if (p.experts > 64) {
-      group = ExpertChunk{0, 0, 0, 0, 0};
-      load_experts(group, p, TM, tiles_n, lane);
+      group = first;
+      count_tiles(group, TM, tiles_n, lane);
     }
   }
   int my_tiles, t_first, t_step;
@@ -1046,6 +1071,28 @@ __global__ __launch_bounds__(tile_threads(WM, WN)) void gemm_kernel(const GemmPa
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
 }
 
+template <int MODE, int GROUPED, bool OUT_F32, bool ACC, bool SA4, int EPI = 0, int WM = 4, int NS = 8, int WN = 2>
+__global__ __launch_bounds__(tile_threads(WM, WN)) void gemm_kernel(const GemmParams p) {
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[tile_lds(MODE, WM, 16 * NS * WN)];
+  ExpertChunk group{0, 0, 0, 0, 0};
+  if (GROUPED == kGroupedRows) expert_ends(group, p, threadIdx.x & 63);
+  gemm_tiles<MODE, GROUPED, OUT_F32, ACC, SA4, EPI, WM, NS, WN>(p, lds, group);
+}
+
+// Grouped by rows, the tile chosen here, where the experts' rows are known.
+template <int MODE, bool OUT_F32, bool SA4>
+__global__ __launch_bounds__(512) void gemm_grouped_kernel(const GemmParams p) {
+  constexpr int kMost = tile_lds(MODE, 4, 256) > tile_lds(MODE, 1, 128) ? tile_lds(MODE, 4, 256) : tile_lds(MODE, 1, 128);
+  static_assert(tile_threads(4, 2) == 512 && tile_threads(2, 2) == 512 && tile_threads(1, 4) == 512 && kMost >= tile_lds(MODE, 2, 256), "");
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[kMost];
+  ExpertChunk group{0, 0, 0, 0, 0};
+  expert_ends(group, p, threadIdx.x & 63);
+  const int rows = grouped_tile_rows(group, p, threadIdx.x & 63);
+  if (rows == 64) gemm_tiles<MODE, kGroupedRows, OUT_F32, false, false, 0, 1, 2, 4>(p, lds, group);
+  else if (rows == 128) gemm_tiles<MODE, kGroupedRows, OUT_F32, false, false, 0, 2, 8, 2>(p, lds, group);
+  else gemm_tiles<MODE, kGroupedRows, OUT_F32, false, SA4, 0, 4, 8, 2>(p, lds, group);
+}
+
 // Test hook.  0: pick_shape and the rules below choose the form; 1: always 256 x 256 tiles; 2: the smallest tile a form has;
 // 3: 128 x 256 and 4: 128 x 128 tiles where a form has them
 static std::atomic<int> g_small_gemm_mode{0};   // (atomic: the test hook may be called from any thread)
@@ -1069,9 +1116,18 @@ static int persistent_grid(int64_t tiles) {
 // The tile of a GEMM: 256 x 256 (8 waves), or 128 x 256, 128 x 128 or 64 x 128 (4 waves that multiply, 4 that fetch).
 enum TileShape { k256x256, k128x256, k128x128, k64x128 };
 
+static int64_t shape_rows(TileShape shape) { return shape == k256x256 ? 256 : (shape == k64x128 ? 64 : 128); }
+static int64_t shape_cols(TileShape shape) { return shape == k128x128 || shape == k64x128 ? 128 : 256; }
+
 static int64_t tile_count(int64_t M, int64_t N, TileShape shape) {
-  const int tm = shape == k256x256 ? 256 : (shape == k64x128 ? 64 : 128), tn = shape == k128x128 || shape == k64x128 ? 128 : 256;
+  const int64_t tm = shape_rows(shape), tn = shape_cols(shape);
   return ((M + tm - 1) / tm) * ((N + tn - 1) / tn);
+}
+
+// Grouped by rows: the most tiles there can be (every expert with rows ends in a partial one).
+static int64_t most_grouped_tiles(int64_t M, int64_t N, int64_t experts, TileShape shape) {
+  const int64_t tm = shape_rows(shape), tn = shape_cols(shape), used = experts < M ? experts : M;
+  return (M + used * (tm - 1)) / tm * ((N + tn - 1) / tn);
 }
 
 // The smallest tile with which the problem is still one round, one tile per compute unit; problems of several rounds
@@ -1103,29 +1159,25 @@ static TileShape pick_shape_swiglu(int64_t M, int64_t N) {
   return tile_count(M, N, k128x256) <= persistent_grid((int64_t)1 << 40) ? k128x256 : k256x256;
 }
 
-// Grouped by rows: every expert ends in a partial tile, which costs as much as a whole one, so with few rows per expert low
-// tiles are better, with many (or the rows of many with one expert) high ones.  The rows of an expert are known on the device
-// only.  Even the largest number of low tiles is one round: low.  Of more than 256 rows per expert on average: high.  Low
-// tiles are at most M / 129 row tiles more than high ones: where that is at most a quarter of a round, low; at that quarter what
-// is lost where they are just one round more (32 experts [2048, 7168], 1024 rows by Zipf's law: 264 / 256 tiles, 137 / 120
-// us) is about what a second launch would cost on every call.  In between both kernels are launched, count both kinds of tiles
-// and one of them returns at once (3 to 5 us).  us with 128 / 256 rows per tile, for rows
-// spread evenly / by Zipf's law / half with one expert / all with one:
-//   32 experts [4096, 7168],   512 rows   187 / 257   167 / 207   209 / 267    49 / 69
-//                             4096 rows   175 / 235   267 / 278   226 / 295   112 / 99
-//                             8192 rows   281 / 234   338 / 366   392 / 320   224 / 187
-//                            16384 rows               606 / 531
-//   8 experts  [4096, 7168],  2048 rows    58 / 81     98 / 78    102 / 79     57 / 76
-//   64 experts [2048, 2048], 16384 rows    95 / 83    111 / 125   132 / 102    76 / 70
-enum GroupedTiles { kLowTiles, kHighTiles, kEitherTiles };
+// Grouped by rows every expert ends in a partial tile, which costs as much as a whole one, so with few rows per expert low
+// tiles are better, with many (or the rows of many with one expert) high ones; the rows of an expert are known on the device
+// only.  Where even the most 64 x 128 tiles there can be are one round: those.  Of more than 256 rows per expert on average and
+// two rounds of 256 x 256 tiles or more: those.  In between the kernel chooses (grouped_tile_rows).  us with 64 / 128 / 256 rows per
+// tile, for rows spread evenly / by Zipf's law / half with one expert / all with one:
+//   32 experts [4096, 7168],   512 rows   163 / 165 / 220   180 / 158 / 212   183 / 208 / 212    25 /  42 /  66
+//                             2048 rows   165 / 168 / 224   234 / 202 / 275   211 / 204 / 280    87 /  54 /  73
+//                             8192 rows   432 / 261 / 235   476 / 312 / 377   445 / 273 / 334   338 / 213 / 183
+//   8 experts  [4096, 7168],   512 rows    37 /  46 /  72    48 /  43 /  68    50 /  43 /  69    25 /  42 /  66
+//   16 experts [1024, 4096],  2048 rows    18 /  28 /  43    28 /  28 /  42    22 /  27 /  42    17 /  27 /  41
+//   64 experts [2048, 2048], 16384 rows   144 /  81 /  76   146 /  97 / 117   145 /  84 / 101   118 /  70 /  63
+enum GroupedTiles { kLowestTiles, kLowTiles, kHighTiles, kChosenTiles };
 
 static GroupedTiles pick_grouped(int64_t M, int64_t N, int experts) {
   const int mode = g_small_gemm_mode.load(std::memory_order_relaxed);
-  if (mode != 0) return mode == 1 ? kHighTiles : kLowTiles;
-  const int64_t cus = persistent_grid((int64_t)1 << 40), tiles_n = (N + 255) / 256;
-  if ((M / 128 + experts) * tiles_n <= cus) return kLowTiles;
-  if (M > (int64_t)256 * experts) return kHighTiles;
-  return M / 129 * tiles_n <= cus / 4 ? kLowTiles : kEitherTiles;
+  if (mode != 0) return mode == 1 ? kHighTiles : (mode == 2 ? kLowestTiles : kLowTiles);
+  const int64_t cus = persistent_grid((int64_t)1 << 40);
+  if (most_grouped_tiles(M, N, experts, k64x128) <= cus) return kLowestTiles;
+  return M > (int64_t)256 * experts && M / 256 * ((N + 255) / 256) >= 2 * cus ? kHighTiles : kChosenTiles;
 }
 
 // Few rows of a (decode): bound by reading b once, which the tile kernels do not reach (gemm_skinny.hip; 8 rows of
@@ -1176,12 +1228,14 @@ static int launch(GemmParams p, int out_type, TileShape shape, hipStream_t strea
   p.tiles = (int)tiles;                        // (grouped by rows: the kernel counts the experts' own tiles)
   if (GROUPED == kGroupedK) tiles *= p.experts;
   // upper bound on row tiles: every expert may add one partial tile
-  if (GROUPED == kGroupedRows) tiles = (p.M / (shape == k256x256 ? 256 : 128) + p.experts) * ((p.N + 255) / 256);
+  if (GROUPED == kGroupedRows) tiles = most_grouped_tiles(p.M, p.N, p.experts, shape);
   if constexpr (GROUPED != kGroupedK) {
     if (shape == k128x256) return launch_shape<MODE, GROUPED, 2, 8, 2>(p, out_type, tiles, stream);
   }
   if constexpr (GROUPED == kDense) {
     if (shape == k128x128) return launch_shape<MODE, GROUPED, 2, 4, 2>(p, out_type, tiles, stream);
+  }
+  if constexpr (GROUPED != kGroupedK) {
     if (shape == k64x128) return launch_shape<MODE, GROUPED, 1, 2, 4>(p, out_type, tiles, stream);
   }
   return launch_shape<MODE, GROUPED, 4, 8, 2>(p, out_type, tiles, stream);
@@ -1190,12 +1244,20 @@ static int launch(GemmParams p, int out_type, TileShape shape, hipStream_t strea
 template <int MODE>
 static int launch_grouped(GemmParams p, int out_type, hipStream_t stream) {
   const GroupedTiles tiles = pick_grouped(p.M, p.N, p.experts);
-  p.choose_cus = tiles == kEitherTiles ? persistent_grid((int64_t)1 << 40) : 0;
-  if (tiles != kHighTiles) {
-    const int rc = launch<MODE, kGroupedRows>(p, out_type, k128x256, stream);
-    if (rc != HPFP8_OK || tiles == kLowTiles) return rc;
+  if (tiles == kLowestTiles) return launch<MODE, kGroupedRows>(p, out_type, k64x128, stream);
+  if (tiles == kLowTiles) return launch<MODE, kGroupedRows>(p, out_type, k128x256, stream);
+  if (tiles == kHighTiles) return launch<MODE, kGroupedRows>(p, out_type, k256x256, stream);
+  p.choose_cus = persistent_grid((int64_t)1 << 40);
+  dim3 grid((unsigned)persistent_grid(most_grouped_tiles(p.M, p.N, p.experts, k64x128))), block(512);
+  const bool sa4 = p.sa_sm == 1;
+  if (out_type == HPFP8_OUT_F32) {
+    if (sa4) gemm_grouped_kernel<MODE, true, true><<<grid, block, 0, stream>>>(p);
+    else gemm_grouped_kernel<MODE, true, false><<<grid, block, 0, stream>>>(p);
+  } else {
+    if (sa4) gemm_grouped_kernel<MODE, false, true><<<grid, block, 0, stream>>>(p);
+    else gemm_grouped_kernel<MODE, false, false><<<grid, block, 0, stream>>>(p);
   }
-  return launch<MODE, kGroupedRows>(p, out_type, k256x256, stream);
+  return check_launch("gemm (grouped)");
 }
 
 static int check_common(const char* what, const void* a, int64_t lda, const void* b, int64_t ldb, const float* sa,

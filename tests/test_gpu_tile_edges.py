@@ -570,3 +570,29 @@ def test_tiles_with_fetching_waves_give_the_bits_of_256_x_256_ones(gpu, mode, m,
             _lib.load().hpfp8_debug_set_small_gemm(0)
     for one, other in zip(got[1], got[mode]):
         assert torch.equal(one, other)
+
+
+@pytest.mark.parametrize("counts", [[5], [0, 64, 0, 65, 1], [300] * 3, [0] * 63 + [200], [3] * 64, [0] * 64 + [129], [1, 0, 2] * 43, [40] * 70,
+                                    [2500, 7, 0, 1]])
+@pytest.mark.parametrize("n", [128, 640])
+def test_grouped_rows_give_the_same_bits_with_every_tile(gpu, counts, n):
+    """The tile that the kernel chooses and each one asked for, rows of an expert around the tiles' heights, experts around a
+    wave's 64; rows past the last offset are left as they are."""
+    from hpfp8 import _lib, ops
+    k, e, m = 384, len(counts), sum(counts)
+    a, sa = ops.quantize_1x128(_normal((m + 3, k), 1, gpu, outliers=True), kmajor=True)
+    b, sb = ops.quantize_128x128(_normal((8 * n, k), 2, gpu, 0.05))
+    pick = torch.arange(e, device=gpu) % 8
+    b, sb = b.view(torch.uint8).view(8, n, k)[pick].view(b.dtype), sb.view(8, n // 128, k // 128)[pick].contiguous()
+    offs = torch.tensor(counts).cumsum(0).to(torch.int32).to(gpu)
+    got = {}
+    for mode in (1, 0, 2, 3):
+        _lib.load().hpfp8_debug_set_small_gemm(mode)
+        try:
+            got[mode] = [ops.gemm_grouped_blockwise(a, s, b, sb, offs)[:m] for s in (sa, sa.contiguous())]
+        finally:
+            _lib.load().hpfp8_debug_set_small_gemm(0)
+        assert torch.equal(got[mode][0], got[1][0]) and torch.equal(got[mode][1], got[1][0])
+    for i, c in enumerate(counts[:6]):
+        rows = slice(int(sum(counts[:i])), int(sum(counts[:i + 1])))
+        assert torch.equal(got[0][0][rows], ops.gemm_blockwise(a[rows], sa[rows], b[i], sb[i]))
