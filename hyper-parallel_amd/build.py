@@ -1,4 +1,5 @@
-"""Builds libhpfp8.so (HIP kernels + C ABI) in-tree with hipcc for gfx950.
+"""Builds libhpfp8.so (HIP kernels + C ABI) in-tree with hipcc for gfx950, and _native.so (the tensor operators' host path, host
+code only) against the installed torch.
 
 Usage: python build.py [--force]
 """
@@ -11,6 +12,8 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "hpfp8", "libhpfp8.so")
+NATIVE = os.path.join(HERE, "hpfp8", "_native.so")
+NATIVE_SOURCE = os.path.join(CSRC, "torch_ops.cpp")
 SOURCES = ["capi.hip", "quantize.hip", "bucket.hip", "grouped.hip", "gemm.hip", "gemm_skinny.hip"]
 HEADERS = ["gemm_skinny.h", "gemm_tile.h", "hpfp8_device.h", "hpfp8_host.h", os.path.join("..", "..", "include", "hpfp8.h")]
 
@@ -29,27 +32,42 @@ def _flags():
     ]
 
 
-def needs_build() -> bool:
-    if not os.path.exists(OUT):
+def _native_command():
+    import sysconfig
+    import torch
+    from torch.utils.cpp_extension import include_paths
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    return (["g++", "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+            + ["-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1"]
+            + [f"-I{d}" for d in include_paths("cuda") + [sysconfig.get_paths()["include"]]]
+            + [NATIVE_SOURCE, "-o", NATIVE, f"-L{lib}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", f"-Wl,-rpath,{lib}"])
+
+
+def _older(out, deps) -> bool:
+    if not os.path.exists(out):
         return True
-    t = os.path.getmtime(OUT)
-    deps = [os.path.join(CSRC, s) for s in SOURCES + HEADERS] + [os.path.abspath(__file__)]
-    return any(os.path.getmtime(d) > t for d in deps)
+    t = os.path.getmtime(out)
+    return any(os.path.getmtime(d) > t for d in deps + [os.path.abspath(__file__)])
+
+
+def needs_build() -> bool:
+    header = os.path.join(CSRC, HEADERS[-1])
+    return _older(OUT, [os.path.join(CSRC, s) for s in SOURCES + HEADERS]) or _older(NATIVE, [NATIVE_SOURCE, header])
 
 
 def build(force: bool = False, verbose: bool = False) -> str:
     if not force and not needs_build():
         return OUT
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
-    cmd = [hipcc] + _flags() + [os.path.join(CSRC, s) for s in SOURCES] + ["-o", OUT]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
-    out = "\n".join(l for l in res.stdout.splitlines() if "packed-fp32-ops" not in l)
-    if res.returncode != 0:
-        raise RuntimeError("hipcc failed:\n" + out)
-    if verbose and out.strip():
-        print(out)
+    for cmd in ([hipcc] + _flags() + [os.path.join(CSRC, s) for s in SOURCES] + ["-o", OUT], _native_command()):
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+        out = "\n".join(l for l in res.stdout.splitlines() if "packed-fp32-ops" not in l)
+        if res.returncode != 0:
+            raise RuntimeError(f"{cmd[0]} failed:\n" + out)
+        if verbose and out.strip():
+            print(out)
     return OUT
 
 

@@ -119,9 +119,25 @@ def load():
     return lib
 
 
+def fail(name: str, rc: int) -> None:
+    msg = load().hpfp8_last_error().decode("utf-8", "replace")
+    raise Hpfp8Error(f"{name} failed ({rc}): {msg}")
+
+
 def call(name: str, *args) -> None:
     lib = _lib if _lib is not None else load()
     rc = getattr(lib, name)(*args)
     if rc != 0:
-        msg = lib.hpfp8_last_error().decode("utf-8", "replace")
-        raise Hpfp8Error(f"{name} failed ({rc}): {msg}")
+        fail(name, rc)
+
+
+def load_native():
+    """The tensor operators' native host path (csrc/torch_ops.cpp), bound to the loaded library."""
+    import torch
+    try:
+        from . import _native
+    except ImportError as e:
+        raise ImportError(f"hpfp8/_native.so is missing or does not fit the installed torch ({e}): run `python "
+                          f"{os.path.join(os.path.dirname(_HERE), 'build.py')}`.") from e
+    _native.bind(load()._handle, fail, torch.nn.Parameter)
+    return _native

@@ -108,39 +108,77 @@ def _empty_batch_grads(ctx, go):
     return dx, dw, db
 
 
+def _forward_blockwise(x, weight, bias, wq, sw, wqt, need_dx, need_dw, pow2):
+    """(y, xt, sxt, wqt, sw): the result and what the gradients asked for will need."""
+    x2 = _flatten(x)
+    # With a weight gradient to come x is read once: its 1x128 codes for this GEMM and its transposed 128x1
+    # codes for wgrad, which are what is kept for backward (1 byte per element instead of the bf16 source).
+    # The 128x1 groups run along the tokens; a ragged token count is filled up with zero rows by the kernel.
+    if need_dw and x2.shape[0] > 0:
+        xq, sx, xt, sxt = _both_forms(x2, pow2=pow2)
+    else:
+        xq, sx = ops.quantize_1x128(x2, kmajor=True, pow2=pow2)
+        xt = sxt = None
+    if wq is None:                          # no prequantized form of the weight was passed in
+        if need_dx:
+            wq, sw, wqt = ops.quantize_128x128(weight, with_transpose=True, pow2=pow2)
+        else:
+            wq, sw = ops.quantize_128x128(weight, pow2=pow2)
+    elif need_dx and wqt is None:
+        wqt = ops.transpose_codes(wq)
+    y = ops.gemm_blockwise(xq, sx, wq, sw, bias=bias, pow2_scales=pow2)
+    return y if x.dim() == 2 else y.reshape(x.shape[:-1] + (weight.shape[0],)), xt, sxt, wqt, sw
+
+
+def _forward_per_tensor(x, weight, bias, wq, sw, need_dx, need_dw):
+    """(y, xt, sx, w, sw, w_transposed): the result and what the gradients asked for will need."""
+    x2 = _flatten(x)
+    m = x2.shape[0]
+    # With one scale per tensor the codes of a transposed tensor are the transposed codes: what a gradient will
+    # need transposed is written beside the codes in the same pass, and kept (1 byte per element).
+    xt = wqt = None
+    if need_dw and m > 0:
+        xq, sx, xt = ops.quantize_per_tensor_t(x2)
+    else:
+        xq, _, sx = ops.quantize_per_tensor(x2)
+    if wq is None:                          # no prequantized form of the weight was passed in
+        if need_dx and m > 0 and weight.shape[0] > 0:
+            wq, sw, wqt = ops.quantize_per_tensor_t(weight)
+        else:
+            wq, _, sw = ops.quantize_per_tensor(weight)
+    y = ops.gemm_per_tensor(xq, sx, wq, sw, bias=bias)
+    return (y if x.dim() == 2 else y.reshape(x.shape[:-1] + (weight.shape[0],)), xt, sx, wqt if wqt is not None else wq, sw,
+            wqt is not None)
+
+
+def _trained(x, weight, bias, wq, sw, wqt, per_tensor, pow2):
+    """The linear with gradients of x and weight to come, as a graph node of csrc/torch_ops.cpp: the steps of the functions
+    below, without the interpreter in backward."""
+    with torch.no_grad():
+        if per_tensor:
+            y, xt, sxt, w, sw, w_transposed = _forward_per_tensor(x, weight, bias, wq, sw, True, True)
+        else:
+            y, xt, sxt, w, sw = _forward_blockwise(x, weight, bias, wq, sw, wqt, True, True, pow2)
+            w_transposed = True
+    return ops._native.linear_node(x, weight, bias, y, xt, sxt, w, sw, per_tensor, pow2, w_transposed)
+
+
 class _Fp8LinearBlockwise(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, bias, wq=None, sw=None, wqt=None, on_main_grad=False, pow2=False, grad_mode=True):
         ctx.main_grad_of = weight if on_main_grad else None
         ctx.pow2 = pow2
-        x2 = _flatten(x)
-        m = x2.shape[0]
         # grad_mode: whether the caller ran with gradients enabled (inside this function they never are).  A
         # Parameter has requires_grad set under torch.no_grad() too; without a backward to come nothing is
         # prepared or kept for it.
         need_dx, need_dw = grad_mode and x.requires_grad, grad_mode and weight.requires_grad
-        # With a weight gradient to come x is read once: its 1x128 codes for this GEMM and its transposed 128x1
-        # codes for wgrad, which are what is kept for backward (1 byte per element instead of the bf16 source).
-        # The 128x1 groups run along the tokens; a ragged token count is filled up with zero rows by the kernel.
-        if need_dw and m > 0:
-            xq, sx, xt, sxt = _both_forms(x2, pow2=pow2)
-        else:
-            xq, sx = ops.quantize_1x128(x2, kmajor=True, pow2=pow2)
-            xt = sxt = None
-        if wq is None:                          # no prequantized form of the weight was passed in
-            if need_dx:
-                wq, sw, wqt = ops.quantize_128x128(weight, with_transpose=True, pow2=pow2)
-            else:
-                wq, sw = ops.quantize_128x128(weight, pow2=pow2)
-        elif need_dx and wqt is None:
-            wqt = ops.transpose_codes(wq)
-        y = ops.gemm_blockwise(xq, sx, wq, sw, bias=bias, pow2_scales=pow2)
+        y, xt, sxt, wqt, sw = _forward_blockwise(x, weight, bias, wq, sw, wqt, need_dx, need_dw, pow2)
         ctx.save_for_backward(xt, sxt, wqt if need_dx else None, sw)
         ctx.x_shape = x.shape
         ctx.w_shape = weight.shape
         ctx.has_bias = bias is not None
         ctx.need = (need_dx, need_dw)
-        return y.reshape(x.shape[:-1] + (weight.shape[0],))
+        return y
 
     @staticmethod
     def backward(ctx, grad_out):
@@ -191,30 +229,15 @@ class _Fp8LinearBlockwise(torch.autograd.Function):
 class _Fp8LinearPerTensor(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, bias, wq=None, sw=None, grad_mode=True):
-        x2 = _flatten(x)
-        m = x2.shape[0]
         # (grad_mode: as in the blockwise form)
         need_dx, need_dw = grad_mode and x.requires_grad, grad_mode and weight.requires_grad
-        # With one scale per tensor the codes of a transposed tensor are the transposed codes: what a gradient will
-        # need transposed is written beside the codes in the same pass, and kept (1 byte per element).
-        xt = wqt = None
-        if need_dw and m > 0:
-            xq, sx, xt = ops.quantize_per_tensor_t(x2)
-        else:
-            xq, _, sx = ops.quantize_per_tensor(x2)
-        if wq is None:                          # no prequantized form of the weight was passed in
-            if need_dx and m > 0 and weight.shape[0] > 0:
-                wq, sw, wqt = ops.quantize_per_tensor_t(weight)
-            else:
-                wq, _, sw = ops.quantize_per_tensor(weight)
-        y = ops.gemm_per_tensor(xq, sx, wq, sw, bias=bias)
-        ctx.w_transposed = wqt is not None
-        ctx.save_for_backward(xt, sx, (wqt if wqt is not None else wq) if need_dx else None, sw)
+        y, xt, sx, w, sw, ctx.w_transposed = _forward_per_tensor(x, weight, bias, wq, sw, need_dx, need_dw)
+        ctx.save_for_backward(xt, sx, w if need_dx else None, sw)
         ctx.x_shape = x.shape
         ctx.w_shape = weight.shape
         ctx.has_bias = bias is not None
         ctx.need = (need_dx, need_dw)
-        return y.reshape(x.shape[:-1] + (weight.shape[0],))
+        return y
 
     @staticmethod
     def backward(ctx, grad_out):
@@ -262,11 +285,10 @@ def fp8_linear(input: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.T
     `weight.main_grad` instead of `weight.grad`: a float32 [out_features, in_features] tensor that the
     first backward creates and every later one adds onto, inside the wgrad GEMM.
     """
-    out = _hand_off(fp8_linear, tuple(t for t in (input, weight, bias) if t is not None), (input, weight, bias),
-                    dict(recipe=recipe, weight_fp8=weight_fp8, apply_grad_on_fp32_main_grad=apply_grad_on_fp32_main_grad),
-                    _FP8_LINEAR_DEFAULTS)
-    if out is not NotImplemented:
-        return out
+    if torch.overrides.has_torch_function((input, weight) if bias is None else (input, weight, bias)):
+        return _hand_off(fp8_linear, tuple(t for t in (input, weight, bias) if t is not None), (input, weight, bias),
+                         dict(recipe=recipe, weight_fp8=weight_fp8, apply_grad_on_fp32_main_grad=apply_grad_on_fp32_main_grad),
+                         _FP8_LINEAR_DEFAULTS)
     if recipe not in RECIPES:
         raise ValueError(f"recipe must be one of {RECIPES}, got {recipe!r}")
     if weight.dim() != 2:
@@ -284,23 +306,24 @@ def fp8_linear(input: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.T
         if mg is not None and (mg.dtype != torch.float32 or tuple(mg.shape) != tuple(weight.shape) or
                                not mg.is_contiguous()):
             raise ValueError("weight.main_grad must be a contiguous float32 tensor of the weight's shape")
+    wq = sw = wqt = None
     if weight_fp8 is not None:
-        if tuple(weight_fp8.codes.shape) != tuple(weight.shape):
+        wq, sw, wqt = weight_fp8.codes, weight_fp8.scale_inv, weight_fp8.codes_t
+        if tuple(wq.shape) != tuple(weight.shape):
             raise ValueError("weight_fp8 does not have the weight's shape")
         if recipe == "per_tensor":
-            if weight_fp8.scale_inv.numel() != 1:
+            if sw.numel() != 1:
                 raise ValueError("weight_fp8 was not quantized with one scale per tensor")
-            return _Fp8LinearPerTensor.apply(input, weight, bias, weight_fp8.codes, weight_fp8.scale_inv, torch.is_grad_enabled())
-        if weight_fp8.scale_inv.dim() != 2:
-            raise ValueError("weight_fp8 was quantized with one scale per tensor")
-        if bool(weight_fp8.pow2) != pow2:
-            raise ValueError("weight_fp8 was quantized for the other blockwise recipe")
-        return _Fp8LinearBlockwise.apply(input, weight, bias, weight_fp8.codes, weight_fp8.scale_inv,
-                                         weight_fp8.codes_t, apply_grad_on_fp32_main_grad, pow2, torch.is_grad_enabled())
-    if recipe != "per_tensor":
-        return _Fp8LinearBlockwise.apply(input, weight, bias, None, None, None, apply_grad_on_fp32_main_grad, pow2,
-                                         torch.is_grad_enabled())
-    return _Fp8LinearPerTensor.apply(input, weight, bias, None, None, torch.is_grad_enabled())
+        else:
+            if sw.dim() != 2:
+                raise ValueError("weight_fp8 was quantized with one scale per tensor")
+            if bool(weight_fp8.pow2) != pow2:
+                raise ValueError("weight_fp8 was quantized for the other blockwise recipe")
+    if not apply_grad_on_fp32_main_grad and ops._native.trains(input, weight, bias):
+        return _trained(input, weight, bias, wq, sw, wqt, recipe == "per_tensor", pow2)
+    if recipe == "per_tensor":
+        return _Fp8LinearPerTensor.apply(input, weight, bias, wq, sw, torch.is_grad_enabled())
+    return _Fp8LinearBlockwise.apply(input, weight, bias, wq, sw, wqt, apply_grad_on_fp32_main_grad, pow2, torch.is_grad_enabled())
 
 
 _FP8_LINEAR_DEFAULTS = dict(recipe="blockwise", weight_fp8=None, apply_grad_on_fp32_main_grad=False)

@@ -27,6 +27,15 @@ _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda de
 _device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
 
 
+_native = _lib.load_native()
+_PLAIN = frozenset((torch.Tensor, torch.nn.Parameter))
+
+
+def _gpu(x) -> bool:
+    """Whether the native form of an operator is to be asked (it returns None for what it does not take)."""
+    return type(x) in _PLAIN and x.is_cuda
+
+
 def _stream() -> int:
     """The handle of the current device's current stream."""
     return _raw_stream(torch.cuda.current_device())
@@ -173,6 +182,13 @@ def quantize_per_tensor_t(x: torch.Tensor, column_sum: bool = False):
     """`quantize_per_tensor` of x[M, K] (K a multiple of 128, any M > 0) with the transposed codes from the same read:
     (codes[M, K], scale_inv, codes_t[K, Mp]), Mp = M rounded up to a multiple of 128, the codes of the rows past M zero.
     With ``column_sum`` a fourth result, the bits of `column_sum(x)`."""
+    if _gpu(x) and x.dim() == 2:
+        tiles = (x.shape[0] + BLOCK - 1) // BLOCK * (x.shape[1] // BLOCK)
+        device = _device()
+        out = _native.quantize_per_tensor_t(x, column_sum, _sync_words(x.device) if 0 < tiles <= _ONE_PASS_TILES else None, device,
+                                            _raw_stream(device))
+        if out is not None:
+            return out
     x = _check_bf16(x, "x")
     if x.dim() != 2 or x.shape[1] % BLOCK or x.numel() == 0:
         raise ValueError("x must be [M, K] with M > 0 and K a positive multiple of 128")
@@ -203,6 +219,11 @@ def quantize_1x128(x: torch.Tensor, want_scale: bool = False, kmajor: bool = Fal
     ``pow2`` (k-block-major layout only; also on the other blockwise quantizers): scale_inv rounded up
     to a power of two, the optional recipe whose GEMMs are ``gemm_blockwise(..., pow2_scales=True)``.
     """
+    if kmajor and not want_scale and _gpu(x):
+        device = _device()
+        out = _native.quantize_1x128(x, pow2, device, _raw_stream(device))
+        if out is not None:
+            return out
     x = _check_bf16(x, "x")
     if x.dim() < 1:
         raise ValueError("x must have at least one dimension")
@@ -234,6 +255,11 @@ def quantize_1x128(x: torch.Tensor, want_scale: bool = False, kmajor: bool = Fal
 
 def quantize_128x128(w: torch.Tensor, with_transpose: bool = False, want_scale: bool = False, pow2: bool = False):
     """w[R, C] -> (codes[R, C], scale_inv[R/128, C/128]) (+ codes_t[C, R]) (+ scale)."""
+    if not want_scale and _gpu(w):
+        device = _device()
+        out = _native.quantize_128x128(w, with_transpose, pow2, device, _raw_stream(device))
+        if out is not None:
+            return out
     w = _check_bf16(w, "w")
     if w.dim() != 2:
         raise ValueError("w must be 2-D")
@@ -421,6 +447,11 @@ def quantize_1x128_and_128x1_t_rows(x: torch.Tensor, pow2: bool = False, column_
     """`quantize_1x128_and_128x1_t` (k-block-major scales) of x[M, K] for any M > 0, from one read of x: the transposed form
     is that of `quantize_128x1_t_rows`, codes_t[K, Mp] and scale_inv_t[K, Mp/128] with Mp = M rounded up to a multiple of
     128; the other results have M rows."""
+    if _gpu(x):
+        device = _device()
+        out = _native.both_forms(x, pow2, column_sum, device, _raw_stream(device))
+        if out is not None:
+            return out
     x = _check_bf16(x, "x")
     if x.dim() != 2 or x.shape[1] % BLOCK or x.shape[0] == 0:
         raise ValueError("x must be [M, K] with M > 0 and K a multiple of 128")
@@ -448,6 +479,11 @@ def quantize_1x128_and_128x1_t(x: torch.Tensor, kmajor: bool = True, pow2: bool 
     With ``column_sum`` (k-block-major scales only) a fifth result: the bf16 sum of x over its rows [K], from the
     same read -- a bias gradient when x is grad_out -- with the bits of `column_sum(x)`.
     """
+    if kmajor and _gpu(x) and x.dim() == 2 and x.shape[0] % BLOCK == 0:
+        device = _device()
+        out = _native.both_forms(x, pow2, column_sum, device, _raw_stream(device))
+        if out is not None:
+            return out
     x = _check_bf16(x, "x")
     if x.dim() != 2:
         raise ValueError("x must be 2-D")
@@ -575,6 +611,15 @@ def gemm_blockwise(a: torch.Tensor, sa: torch.Tensor, b: torch.Tensor, sb: torch
     a[M,K], b[N,K] codes (unit inner stride, any 16-byte-multiple row stride); sa, sb 2-D fp32 views
     (any strides) of scale_inv values.
     """
+    if _gpu(a) and (out_dtype is torch.bfloat16 or out is not None):
+        device = _device()
+        c = _native.gemm_blockwise(a, sa, b, sb, bias, out, sb_gran, accumulate, pow2_scales, device, _raw_stream(device))
+        if c is not None:
+            return c
+    return _gemm_blockwise(a, sa, b, sb, bias, out_dtype, sb_gran, out, accumulate, pow2_scales)
+
+
+def _gemm_blockwise(a, sa, b, sb, bias=None, out_dtype=torch.bfloat16, sb_gran=128, out=None, accumulate=False, pow2_scales=False):
     a = _check_codes_2d(a, "a")
     b = _check_codes_2d(b, "b")
     sa = _check_f32(sa, "sa")
@@ -643,7 +688,7 @@ def gemm_blockwise_swiglu_quantize(a: torch.Tensor, sa: torch.Tensor, b: torch.T
         # A decode step: the GEMM is bound by reading the weight, which its few-rows form does at twice the rate of the
         # 256 x 256 tiles the epilogue belongs to; gate | up is a few megabytes (37 rows of a [36864, 7168] weight: 86 us
         # for the epilogue form, 42 + 5 us for the two launches, the same bits).
-        h = gemm_blockwise(a, sa, b, sb, pow2_scales=pow2_scales)
+        h = _gemm_blockwise(a, sa, b, sb, pow2_scales=pow2_scales)
         if fast:
             _lib.call("hpfp8_swiglu_quantize_1x128_fast_bf16", _ptr(h), m, inter, n, 1, int(pow2_out), _ptr(q), _ptr(s), _ptr(s_inv),
                       None, _stream())
@@ -660,6 +705,11 @@ def gemm_blockwise_swiglu_quantize(a: torch.Tensor, sa: torch.Tensor, b: torch.T
 def gemm_per_tensor(a: torch.Tensor, sa_inv: torch.Tensor, b: torch.Tensor, sb_inv: torch.Tensor,
                     bias: Optional[torch.Tensor] = None, out_dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:
     """c = (a . b^T) * (sa_inv * sb_inv) (+ bias); sa_inv / sb_inv are 0-dim (or 1-element) fp32."""
+    if _gpu(a) and out_dtype is torch.bfloat16:
+        device = _device()
+        c = _native.gemm_per_tensor(a, sa_inv, b, sb_inv, bias, device, _raw_stream(device))
+        if c is not None:
+            return c
     a = _check_codes_2d(a, "a")
     b = _check_codes_2d(b, "b")
     sa_inv = _check_f32(sa_inv, "sa_inv")

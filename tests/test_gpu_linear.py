@@ -788,3 +788,111 @@ def test_grouped_linear_prequantized_weight_and_inference(gpu):
     assert torch.equal(y2[:500], y0.detach()[:500]) and not y2.requires_grad
     with pytest.raises(ValueError):
         hpfp8.fp8_grouped_linear(x, w, offs[:3])
+
+
+@pytest.mark.parametrize("recipe", ["blockwise", "blockwise_pow2", "per_tensor"])
+@pytest.mark.parametrize("shape,n,bias,cached", [((256, 384), 256, True, None), ((1, 128), 128, False, None), ((2, 65, 256), 384, True, "codes_t"),
+                                                 ((200, 1280), 128, False, "codes"), ((384, 2176), 2304, True, "codes")])
+def test_graph_node_equals_the_python_autograd_function(gpu, recipe, shape, n, bias, cached, monkeypatch):
+    """The native node's output and gradients are the Python function's bit for bit: ragged and whole token counts, more dimensions, one
+    and two launches of the per-tensor quantizer, a weight's FP8 form with and without its transposed codes; also with every saved tensor
+    moved to the host and back in another layout; tensors that a hook hands back on the host are refused."""
+    import types
+    import hpfp8
+    from hpfp8 import ops
+    x, w = U.randn_bf16(shape, 1).to(gpu).requires_grad_(True), U.randn_bf16((n, shape[-1]), 2, 0.05).to(gpu).requires_grad_(True)
+    b = U.randn_bf16((n,), 3).to(gpu).requires_grad_(True) if bias else None
+    go = U.randn_bf16(shape[:-1] + (n,), 4, 0.01).to(gpu)
+    f8 = None
+    if cached:
+        f8 = hpfp8.quantize_weight(w.detach(), with_transpose=cached == "codes_t", pow2=recipe == "blockwise_pow2", per_tensor=recipe == "per_tensor")
+
+    def step(pack=None, unpack=None):
+        with torch.autograd.graph.saved_tensors_hooks(pack or (lambda t: t), unpack or (lambda t: t)):
+            y = hpfp8.fp8_linear(x, w, b, recipe=recipe, weight_fp8=f8)
+        return [y.detach(), *torch.autograd.grad(y, [t for t in (x, w, b) if t is not None], go)], y
+
+    got, y = step()
+    assert type(y.grad_fn).__name__ == "CppFunction" and y.shape == shape[:-1] + (n,)
+    moved, _ = step(lambda t: t.cpu().contiguous(), lambda t: t.to(gpu))
+    for one, other in zip(got, moved):
+        assert torch.equal(one, other)
+    with pytest.raises(ValueError):
+        step(lambda t: t.cpu(), lambda t: t)
+    native = types.SimpleNamespace(**{k: getattr(ops._native, k) for k in dir(ops._native) if not k.startswith("__")})
+    native.trains = lambda *a: False
+    monkeypatch.setattr(ops, "_native", native)
+    want, y = step()
+    assert type(y.grad_fn).__name__.startswith("_Fp8Linear")
+    for one, other in zip(got, want):
+        assert one.shape == other.shape and torch.equal(one, other)
+
+
+def test_native_operators_leave_other_calls_to_the_python_form(gpu, monkeypatch):
+    """Strided, padded and integer-typed operands, refused shapes and types: the same results and errors as without the native forms."""
+    import hpfp8
+    from hpfp8 import ops
+    x, w = U.randn_bf16((256, 384), 1).to(gpu), U.randn_bf16((256, 384), 2, 0.05).to(gpu)
+    xq, sx = hpfp8.quantize_1x128(x, kmajor=True)
+    wq, sw = hpfp8.quantize_128x128(w)
+    wr, sr = hpfp8.quantize_1x128(w)                        # row-major per-row scales: copied
+    wide = torch.zeros((256, 400), dtype=torch.bfloat16, device=gpu)
+    calls = [lambda: ops.quantize_1x128(x.t().contiguous().t(), kmajor=True), lambda: ops.quantize_1x128(wide, kmajor=True),
+             lambda: ops.quantize_1x128(wide[:, :384], kmajor=True), lambda: ops.quantize_1x128(x.float(), kmajor=True),
+             lambda: ops.quantize_1x128(x[:0], kmajor=True), lambda: ops.quantize_1x128(x.view(2, 128, 384), kmajor=True),
+             lambda: ops.quantize_1x128(x.cpu(), kmajor=True), lambda: ops.quantize_128x128(x[:200], with_transpose=True),
+             lambda: ops.quantize_1x128_and_128x1_t(x[:200]), lambda: ops.quantize_1x128_and_128x1_t_rows(x[:200], column_sum=True),
+             lambda: ops.quantize_1x128_and_128x1_t(x.view(-1)[1:1 + 128 * 384].view(128, 384)), lambda: ops.quantize_per_tensor_t(x[:0]),
+             lambda: ops.gemm_blockwise(xq.view(torch.uint8), sx, wq, sw), lambda: ops.gemm_blockwise(xq, sx, wr, sr, sb_gran=1),
+             lambda: ops.gemm_blockwise(xq, sx, wq, sw, bias=x[0, :256].float()), lambda: ops.gemm_blockwise(xq, sx, wq, sw[:1]),
+             lambda: ops.gemm_blockwise(xq[:, :256], sx[:, :2], wq[:, :256], sw[:, :2]), lambda: ops.gemm_blockwise(xq, sx.double(), wq, sw),
+             lambda: ops.gemm_blockwise(xq, sx, wq, sw, accumulate=True), lambda: ops.gemm_blockwise(xq[:0], sx[:0], wq, sw),
+             lambda: ops.gemm_blockwise(xq, sx, wq, sw, out=torch.zeros((256, 256), dtype=torch.float32, device=gpu), accumulate=True)]
+
+    def outcome(f):
+        try:
+            r = f()
+        except Exception as e:
+            return type(e), str(e)
+        return [t.contiguous().view(torch.uint8).cpu() if t.dtype == torch.float8_e4m3fn else t.cpu() for t in (r if isinstance(r, tuple) else (r,))]
+
+    got = [outcome(f) for f in calls]
+    monkeypatch.setattr(ops, "_gpu", lambda t: False)
+    for i, f in enumerate(calls):
+        want = outcome(f)
+        if isinstance(want, tuple):
+            assert got[i] == want, i
+        else:
+            assert len(got[i]) == len(want) and all(torch.equal(a, b) for a, b in zip(got[i], want)), i
+
+
+@pytest.mark.parametrize("recipe", ["blockwise", "per_tensor"])
+def test_linear_training_step_replays_from_a_captured_graph(gpu, recipe):
+    import hpfp8
+    if hasattr(torch.autograd.graph, "set_warn_on_accumulate_grad_stream_mismatch"):
+        torch.autograd.graph.set_warn_on_accumulate_grad_stream_mismatch(False)
+    w, b = U.randn_bf16((256, 384), 1, 0.05).to(gpu).requires_grad_(True), U.randn_bf16((256,), 2).to(gpu).requires_grad_(True)
+    go, xs = U.randn_bf16((130, 256), 3, 0.01).to(gpu), [U.randn_bf16((130, 384), 4 + i, 1.0 + i).to(gpu) for i in range(4)]
+    x_static = xs[0].clone().requires_grad_(True)
+
+    def step(x):
+        y = hpfp8.fp8_linear(x, w, b, recipe=recipe)
+        return (y.detach(), *torch.autograd.grad(y, (x, w, b), go))
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(3):
+            step(x_static)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        outs = step(x_static)
+    for x in xs[1:] + xs[:2]:
+        with torch.no_grad():
+            x_static.copy_(x)
+        graph.replay()
+        torch.cuda.synchronize()
+        for one, other in zip(outs, step(x.clone().requires_grad_(True))):
+            assert torch.equal(one, other)
