@@ -728,3 +728,25 @@ def test_column_sum_at_full_size_against_float64(gpu):
     assert bool(((db.double() - ref).abs() <= bound).all())
     sl = go[:, 1280:1536].contiguous()
     assert np.array_equal(U.bits(db[1280:1536]), O.column_sum(U.bits(sl))[2])
+
+
+@pytest.mark.parametrize("entries", [1, 63, 64, 65, 127, 128, 129, 257])
+@pytest.mark.parametrize("shards", [1, 3])
+def test_bucket_tables_around_the_sizes_of_a_search_and_of_a_launch(gpu, entries, shards):
+    """Entries are found one per lane, 64 at a time, and travel 128 to a launch: each entry's codes and scales are those of its own chunk
+    (filled up with zeros to whole groups), and its unpacked values those codes decoded."""
+    import hpfp8
+    sizes = [(7919 * e) % 211 + 1 if e % 5 else 8192 * (e % 3 + 1) + 40 * e for e in range(entries)]
+    grads = [U.randn_bf16((n * shards,), 10 + e, 1.0).to(gpu) for e, n in enumerate(sizes)]
+    bucket = hpfp8.Fp8GradBucket(sizes, shard_size=shards, grad_scale=0.125)
+    q, si = bucket.pack(grads)
+    outs = [torch.empty(n, dtype=torch.bfloat16, device=gpu) for n in sizes]
+    bucket.unpack(q[shards - 1], si[shards - 1], outs)
+    for e, (n, o) in enumerate(zip(sizes, bucket.offsets)):
+        groups = -(-n // 128)
+        flat = torch.zeros((shards, groups * 128), dtype=torch.bfloat16, device=gpu)
+        flat[:, :n] = grads[e].view(shards, n)
+        want, scales = hpfp8.quantize_1x128(flat)
+        assert torch.equal(q[:, o:o + groups * 128].view(torch.uint8), want.view(torch.uint8)), e
+        assert torch.equal(si[:, o // 128:o // 128 + groups], scales), e
+        assert torch.equal(outs[e], hpfp8.dequantize_1x128(want[-1:], scales[-1:], 0.125).view(-1)[:n]), e
