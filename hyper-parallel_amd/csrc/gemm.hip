@@ -15,12 +15,12 @@
 //     chunks XOR-swizzled by row so that both the DMA writes and the ds_read_b128 fragment reads
 //     are bank-conflict free.
 //   * Where a launch would leave compute units idle the tile is smaller: 128 x 256, 128 x 128 or 64 x 128 with four
-//     multiplying waves (wave tiles 64 x 128, 64 x 64 and 64 x 32), the same template (WM, NS, WN) and the same results bit
+//     multiplying waves (wave tiles 64 x 128, 64 x 64 and 64 x 32) or 64 x 64 with two, the same template (WM, NS, WN) and the same results bit
 //     for bit; pick_shape has the rule and the figures.  There a SIMD has one wave that multiplies, which waits whenever a
 //     transfer it issues finds the memory path occupied (78 clocks per transfer while the first k-blocks arrive, 21 later), so
-//     four more waves do the transfers, 3, 4 and 6 k-blocks at a time in LDS, the scales with them.  us, transfers by the
-//     multiplying waves with two buffers of a / by waves of their own: 1000 x 7168 x 7168 62 / 54, 1531 x 2048 x 7168 41 / 33,
-//     500 x 7168 x 16384 106 / 75, by rows 1024 x 1024 x 2048 16.7 / 11.0.  What is left there is what a k-block's transfers
+//     four more waves do the transfers, 3, 4, 6 and 8 k-blocks at a time in LDS, the scales with them.  us, transfers by the
+//     multiplying waves with two buffers of a / by waves of their own: 1000 x 7168 x 7168 62 / 54, 1531 x 2048 x 7168 41 / 31,
+//     500 x 7168 x 16384 106 / 75, by rows 1024 x 1024 x 2048 16.7 / 10.3.  What is left there is what a k-block's transfers
 //     take by themselves (0.54 us for 48 KB, 0.39 for 32 KB, with every compute unit at it) and a first microsecond or three in
 //     which code and the first tiles arrive through cold caches.
 //   * The grid is persistent: one workgroup per CU walks a list of tiles, and the rounds of
@@ -231,7 +231,7 @@ __host__ __device__ constexpr int tile_threads(int wm, int wn) { return 64 * (wm
 
 __host__ __device__ constexpr bool row_scales(int mode) { return mode == kScaleRow || mode == kScalePow2Row; }
 __host__ __device__ constexpr int tile_stages(int mode, int wm, int tn) {         // k-blocks of b (and, with fetching waves, of a) in LDS
-  return !fetchers(wm) ? b_stages(mode) : (wm == 1 ? 6 : (tn == 256 ? 3 : 4));
+  return !fetchers(wm) ? b_stages(mode) : (tn == 256 ? 3 : (wm == 2 ? 4 : (tn == 128 ? 6 : 8)));
 }
 // With fetching waves the scales of a k-block travel with its tiles, into a slot of one part per fetching wave: 256 bytes of sb
 // (the scale of the left or of the right half's block; with per-row scales 64 of the tile's rows) and the upper or the lower 64
@@ -683,7 +683,11 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
   // waiting on LDS at once.  Fragments that cross the round boundary are carried in registers.
   // Rounds follow each other without a gap across tiles: the last rounds of a tile already fetch
   // the first k-blocks of the next one, and its stores drain while the next tile computes.
-  v8i xf[4], wf_n0, wf_n1;
+  // With few subtiles there are not enough of them behind the barrier to cover the activation fragments read one by one
+  // (64 x 128 tiles: 770 clocks a round for 384 of work): they are read right behind it then, into a second set of registers (us,
+  // before / so: block 400 x 1024 x 8192 21.7 / 19.8, 256 x 3072 x 3072 11.6 / 11.1, 1531 x 2048 x 7168 33 / 31).
+  constexpr bool kTwoX = kFetchers && NS <= 4;
+  v8i xf[4], xg[4], wf_n0, wf_n1;
   wf_n0 = frag_read(b_lds + b_frag_off, pc0);
 #pragma unroll
   for (int j = 0; j < 4; ++j) xf[j] = frag_read(lds + a_frag_off + j * 16 * BK, pc0);
@@ -709,7 +713,8 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
   for (int tile = 0; tile < my_tiles; ++tile) {
   if (ACC) load_old_values(T0);
   const int kbn0 = kcount(T0);         // k-blocks of this tile
-  for (int kb = 0; kb < kbn0; ++kb) {
+  // one k-block: its activation fragments are xf; the next one's go to xn
+  auto round = [&](int kb, v8i (&xf)[4], v8i (&xn)[4]) __attribute__((always_inline)) {
     // Where this round's transfers and scale loads go: one k-block ahead (scales, second half of
     // those tiles), two ahead (first half of those tiles, or the whole b tile when it has three
     // buffers).  Only in the last
@@ -808,6 +813,10 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
         if (i == NS - 2) round_sync();
         wf[(i + 2) % 3] = read_ahead(i);
         if (kFetchers && i == NS - 2) read_scales(snext, s_raw);
+        if (kTwoX && i == NS - 2) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) xn[j] = frag_read(anxt + a_frag_off + j * 16 * BK, pc0);
+        }
         if (MODE == kScaleRow && i > 0) sbv[i & 1] = *reinterpret_cast<const v4f*>(sb_row + i * 16);   // used by the FMAs of group i+1
         issue_slot(i);
         __builtin_amdgcn_sched_barrier(0);
@@ -823,7 +832,7 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
               acc[ip][j][r] = __builtin_fmaf(pv, i == 0 ? s_old[j] : s_cur[j], acc[ip][j][r]);
             }
           }
-          if (i == NS - 1) xf[j] = frag_read(anxt + a_frag_off + j * 16 * BK, pc0);
+          if (!kTwoX && i == NS - 1) xn[j] = frag_read(anxt + a_frag_off + j * 16 * BK, pc0);
           __builtin_amdgcn_sched_barrier(0);   // keep this (MFMA, FMAs) group together, in this order
         }
       }
@@ -856,6 +865,10 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
         if (i == NS - 2) round_sync();
         wf[(i + 2) % 3] = read_ahead(i);
         if (kFetchers && i == NS - 2) read_scales(snext, s_raw);
+        if (kTwoX && i == NS - 2) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) xn[j] = frag_read(anxt + a_frag_off + j * 16 * BK, pc0);
+        }
         if (MODE == kScalePow2Row && i < NS - 1) e_bi[(i + 1) & 1] = (int)(__builtin_bit_cast(uint32_t, sb_lane[(i + 1) * 16]) >> 23);
         issue_slot(i);
         __builtin_amdgcn_sched_barrier(0);
@@ -868,7 +881,7 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
                                                                         MODE == kScalePow2 ? e_b : e_bi[i & 1], 0, e_a[j]);
           else
             acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[i % 3], xf[j], acc[i][j], 0, 0, 0, 0, 0, 0);
-          if (i == NS - 1) xf[j] = frag_read(anxt + a_frag_off + j * 16 * BK, pc0);
+          if (!kTwoX && i == NS - 1) xn[j] = frag_read(anxt + a_frag_off + j * 16 * BK, pc0);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -882,6 +895,20 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
     stage ^= 1;
     bbuf = bnext;
     sbuf = snext;
+  };
+  if constexpr (kTwoX) {
+    int kb = 0;
+    for (; kb + 1 < kbn0; kb += 2) {
+      round(kb, xf, xg);
+      round(kb + 1, xg, xf);
+    }
+    if (kb < kbn0) {
+      round(kb, xf, xg);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) xf[j] = xg[j];
+    }
+  } else {
+    for (int kb = 0; kb < kbn0; ++kb) round(kb, xf, xf);
   }
   // ---- the tile is complete: last promotion, then its stores
   if (kCarry) {
@@ -1094,7 +1121,7 @@ __global__ __launch_bounds__(512) void gemm_grouped_kernel(const GemmParams p) {
 }
 
 // Test hook.  0: pick_shape and the rules below choose the form; 1: always 256 x 256 tiles; 2: the smallest tile a form has;
-// 3: 128 x 256 and 4: 128 x 128 tiles where a form has them
+// 3: 128 x 256, 4: 128 x 128 and 5: 64 x 128 tiles where a form has them
 static std::atomic<int> g_small_gemm_mode{0};   // (atomic: the test hook may be called from any thread)
 
 // Workgroups to launch for `tiles` tiles: at most one per CU, a multiple of 8 (one share per XCD) unless there are fewer
@@ -1113,11 +1140,11 @@ static int persistent_grid(int64_t tiles) {
   return (int)(up < most ? up : most);
 }
 
-// The tile of a GEMM: 256 x 256 (8 waves), or 128 x 256, 128 x 128 or 64 x 128 (4 waves that multiply, 4 that fetch).
-enum TileShape { k256x256, k128x256, k128x128, k64x128 };
+// The tile of a GEMM: 256 x 256 (8 waves), 128 x 256, 128 x 128 or 64 x 128 (4 waves that multiply, 4 that fetch) or 64 x 64 (2 and 4).
+enum TileShape { k256x256, k128x256, k128x128, k64x128, k64x64 };
 
-static int64_t shape_rows(TileShape shape) { return shape == k256x256 ? 256 : (shape == k64x128 ? 64 : 128); }
-static int64_t shape_cols(TileShape shape) { return shape == k128x128 || shape == k64x128 ? 128 : 256; }
+static int64_t shape_rows(TileShape shape) { return shape == k256x256 ? 256 : (shape == k64x128 || shape == k64x64 ? 64 : 128); }
+static int64_t shape_cols(TileShape shape) { return shape == k64x64 ? 64 : (shape == k128x128 || shape == k64x128 ? 128 : 256); }
 
 static int64_t tile_count(int64_t M, int64_t N, TileShape shape) {
   const int64_t tm = shape_rows(shape), tn = shape_cols(shape);
@@ -1136,15 +1163,18 @@ static int64_t most_grouped_tiles(int64_t M, int64_t N, int64_t experts, TileSha
 // on the same critical path.  us with 256 x 256 / 128 x 256 / 128 x 128 / 64 x 128 tiles (tiles of the one taken):
 //   block   256 x 7168 x 7168    80 / 53 / 39 / 30 (224)         512 x 7168 x 7168    79 / 52 / 39 / 51 (224)
 //   block  1000 x 7168 x 7168    81 / 54 / 66 / 89 (224)        2048 x 7168 x 7168    91 / 103 / 124 / 152 (224)
-//   block  1000 x 2048 x 4096    40 / 27 / 19 / 16 (256)        1400 x 2048 x 4096    40 / 27 / 20 / 26 (176)
-//   block  1400 x 3072 x 3072    32 / 22 / 28 / 30 (132)         400 x 1024 x 8192    73 / 47 / 31 / 23 (56)
+//   block  1000 x 2048 x 4096    40 / 27 / 18 / 15 (256)        1400 x 2048 x 4096    40 / 27 / 18 / 25 (176)
+//   block  1400 x 3072 x 3072    32 / 22 / 27 / 29 (132)
 //   block  1531 x 7168 x 2048 (168 / 336 / 672 tiles)  26 / 31 / 30        4096 x 4096 x 4096  57 / 62 / 75
-//   pow2   2048 x 4096 x 7168    76 / 51 / 65                   rows   2048 x 1024 x 4096    51 / 33 / 34 / 18
-//   rows, onto c  1024 x 1024 x 4096   59 / 38 / 31 / 19
+//   pow2   2048 x 4096 x 7168    76 / 51 / 65                   rows   2048 x 1024 x 4096    51 / 33 / 33 / 17
+// and with 128 x 128 / 64 x 128 / 64 x 64 (up to 256 of the last)
+//   block   128 x 7168 x 7168    39 / 31 / 23 (224)              400 x 1024 x 8192    29 / 22 / 20 (112)
+//   rows, onto c  1024 x 1024 x 4096   23 / 18 / 16 (256)        tensor  512 x 1024 x 1024    7.3 / 6.7 / 6.0 (128)
 static TileShape pick_shape(int64_t M, int64_t N) {
   const int mode = g_small_gemm_mode.load(std::memory_order_relaxed);
   const int64_t cus = persistent_grid((int64_t)1 << 40);
-  if (mode != 0) return mode == 1 ? k256x256 : (mode == 2 ? k64x128 : (mode == 3 ? k128x256 : k128x128));
+  if (mode != 0) return mode == 1 ? k256x256 : (mode == 2 ? k64x64 : (mode == 3 ? k128x256 : (mode == 4 ? k128x128 : k64x128)));
+  if (tile_count(M, N, k64x64) <= cus) return k64x64;
   if (tile_count(M, N, k64x128) <= cus) return k64x128;
   if (tile_count(M, N, k128x128) <= cus) return k128x128;
   if (tile_count(M, N, k128x256) <= cus) return k128x256;
@@ -1161,7 +1191,7 @@ static TileShape pick_shape_swiglu(int64_t M, int64_t N) {
 
 // Grouped by rows every expert ends in a partial tile, which costs as much as a whole one, so with few rows per expert low
 // tiles are better, with many (or the rows of many with one expert) high ones; the rows of an expert are known on the device
-// only.  Where even the most 64 x 128 tiles there can be are one round: those.  Of more than 256 rows per expert on average and
+// only.  Where even the most 64 x 64 or 64 x 128 tiles there can be are one round: those.  Of more than 256 rows per expert on average and
 // two rounds of 256 x 256 tiles or more: those.  In between the kernel chooses (grouped_tile_rows).  us with 64 / 128 / 256 rows per
 // tile, for rows spread evenly / by Zipf's law / half with one expert / all with one:
 //   32 experts [4096, 7168],   512 rows   163 / 165 / 220   180 / 158 / 212   183 / 208 / 212    25 /  42 /  66
@@ -1170,12 +1200,13 @@ static TileShape pick_shape_swiglu(int64_t M, int64_t N) {
 //   8 experts  [4096, 7168],   512 rows    37 /  46 /  72    48 /  43 /  68    50 /  43 /  69    25 /  42 /  66
 //   16 experts [1024, 4096],  2048 rows    18 /  28 /  43    28 /  28 /  42    22 /  27 /  42    17 /  27 /  41
 //   64 experts [2048, 2048], 16384 rows   144 /  81 /  76   146 /  97 / 117   145 /  84 / 101   118 /  70 /  63
-enum GroupedTiles { kLowestTiles, kLowTiles, kHighTiles, kChosenTiles };
+enum GroupedTiles { kSmallestTiles, kLowestTiles, kLowTiles, kHighTiles, kChosenTiles };
 
 static GroupedTiles pick_grouped(int64_t M, int64_t N, int experts) {
   const int mode = g_small_gemm_mode.load(std::memory_order_relaxed);
-  if (mode != 0) return mode == 1 ? kHighTiles : (mode == 2 ? kLowestTiles : kLowTiles);
+  if (mode != 0) return mode == 1 ? kHighTiles : (mode == 2 ? kSmallestTiles : (mode == 5 ? kLowestTiles : kLowTiles));
   const int64_t cus = persistent_grid((int64_t)1 << 40);
+  if (most_grouped_tiles(M, N, experts, k64x64) <= cus) return kSmallestTiles;
   if (most_grouped_tiles(M, N, experts, k64x128) <= cus) return kLowestTiles;
   return M > (int64_t)256 * experts && M / 256 * ((N + 255) / 256) >= 2 * cus ? kHighTiles : kChosenTiles;
 }
@@ -1237,6 +1268,7 @@ static int launch(GemmParams p, int out_type, TileShape shape, hipStream_t strea
   }
   if constexpr (GROUPED != kGroupedK) {
     if (shape == k64x128) return launch_shape<MODE, GROUPED, 1, 2, 4>(p, out_type, tiles, stream);
+    if (shape == k64x64) return launch_shape<MODE, GROUPED, 1, 2, 2>(p, out_type, tiles, stream);
   }
   return launch_shape<MODE, GROUPED, 4, 8, 2>(p, out_type, tiles, stream);
 }
@@ -1244,6 +1276,7 @@ static int launch(GemmParams p, int out_type, TileShape shape, hipStream_t strea
 template <int MODE>
 static int launch_grouped(GemmParams p, int out_type, hipStream_t stream) {
   const GroupedTiles tiles = pick_grouped(p.M, p.N, p.experts);
+  if (tiles == kSmallestTiles) return launch<MODE, kGroupedRows>(p, out_type, k64x64, stream);
   if (tiles == kLowestTiles) return launch<MODE, kGroupedRows>(p, out_type, k64x128, stream);
   if (tiles == kLowTiles) return launch<MODE, kGroupedRows>(p, out_type, k128x256, stream);
   if (tiles == kHighTiles) return launch<MODE, kGroupedRows>(p, out_type, k256x256, stream);
@@ -1409,7 +1442,7 @@ int hpfp8_gemm_blockwise_swiglu_quantize(const void* a, int64_t lda, const float
   return check_launch(what);
 }
 
-void hpfp8_debug_set_small_gemm(int mode) { g_small_gemm_mode.store(mode >= 1 && mode <= 4 ? mode : 0, std::memory_order_relaxed); }
+void hpfp8_debug_set_small_gemm(int mode) { g_small_gemm_mode.store(mode >= 1 && mode <= 5 ? mode : 0, std::memory_order_relaxed); }
 
 int64_t hpfp8_gemm_few_rows(int64_t K) { return few_rows(K); }
 

@@ -541,12 +541,12 @@ def test_per_tensor_codes_with_their_transpose(gpu, m, k, one_launch, polls, mon
         _lib.load().hpfp8_debug_set_spin_limit(256)
 
 
-@pytest.mark.parametrize("mode", [2, 3, 4])
-@pytest.mark.parametrize("m,n,blocks", [(70, 256, 1), (200, 384, 2), (130, 128, 3), (129, 640, 4), (64, 128, 6), (65, 256, 7), (1300, 2560, 3),
+@pytest.mark.parametrize("mode", [2, 3, 4, 5])
+@pytest.mark.parametrize("m,n,blocks", [(70, 256, 1), (200, 384, 2), (130, 128, 3), (129, 640, 4), (64, 128, 6), (65, 256, 7), (65, 256, 9), (1300, 2560, 3),
                                         (2300, 4224, 1)])
 def test_tiles_with_fetching_waves_give_the_bits_of_256_x_256_ones(gpu, mode, m, n, blocks):
     """Contractions of fewer k-blocks than the rings hold, as many and more; ragged rows and columns; several tiles per workgroup (the last
-    two shapes: 420 and 1188 tiles of 64 x 128, 220 and 594 of 128 x 128, 110 and 306 of 128 x 256); scales of a in both layouts."""
+    two shapes: 840 and 2376 tiles of 64 x 64, 420 and 1188 of 64 x 128, 220 and 594 of 128 x 128, 110 and 306 of 128 x 256); scales of a in both layouts."""
     from hpfp8 import _lib, ops
     k = 128 * blocks
     x, w = _normal((m, k), 1, gpu, outliers=True), _normal((n, k), 2, gpu, 0.05)
@@ -586,7 +586,7 @@ def test_grouped_rows_give_the_same_bits_with_every_tile(gpu, counts, n):
     b, sb = b.view(torch.uint8).view(8, n, k)[pick].view(b.dtype), sb.view(8, n // 128, k // 128)[pick].contiguous()
     offs = torch.tensor(counts).cumsum(0).to(torch.int32).to(gpu)
     got = {}
-    for mode in (1, 0, 2, 3):
+    for mode in (1, 0, 2, 3, 5):
         _lib.load().hpfp8_debug_set_small_gemm(mode)
         try:
             got[mode] = [ops.gemm_grouped_blockwise(a, s, b, sb, offs)[:m] for s in (sa, sa.contiguous())]
