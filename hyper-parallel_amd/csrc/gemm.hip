@@ -264,7 +264,7 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
   constexpr int kATile = TM * BK, kBTile = TN * BK;    // one operand tile in LDS
   constexpr int NA = TM / 8 / kFetchWaves, NB = TN / 8 / kFetchWaves;     // transfers per wave and k-block
   constexpr int kSlice = kBTile / kWaves;              // a wave's part of a b buffer
-  static_assert(EPI == 0 || NS == 8, "SwiGLU epilogue: 128 gate and 128 up columns per tile");
+  static_assert(EPI == 0 || TN == 256, "SwiGLU epilogue: 128 gate and 128 up columns per tile");
   static_assert(EPI == 0 || ((MODE == kScaleBlock || MODE == kScalePow2) && GROUPED == kDense && !OUT_F32 && !ACC),
                 "SwiGLU epilogue: dense block-scaled forward");
   static_assert(!ACC || (OUT_F32 && MODE != kScaleTensor), "accumulating onto c: fp32 output, sums that start from c's values");
@@ -1016,15 +1016,16 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
     }
   };
   if constexpr (EPI != 0) {
-    // SwiGLU epilogue.  Per pass j (16 of the wave's 64 rows) both waves of a pair write their bf16-rounded
-    // results -- gate from the wave with wn = 0, up from its neighbour -- into their staging slices as for a plain
-    // store; after a barrier each wave of the pair takes 8 of the 16 rows, reads gate and up of a row from the two
+    // SwiGLU epilogue.  Per pass j (16 of the wave's 64 rows) the WN waves of a row write their bf16-rounded
+    // results -- gate from the first half of them, up from the second -- into their staging slices as for a plain
+    // store; after a barrier each of them takes its part of the 16 rows, reads gate and up of a row from the
     // slices (16 lanes x 8 columns: one scaling group of the activation), and computes, quantizes and stores
     // the activation exactly as the stand-alone kernel does on a bf16 gate/up tensor.  A second barrier keeps the
     // next pass's writes (and, after the last pass, the next tile's transfers) off slices still being read.
     static_assert(kBStages == 3, "staging rows 0..15 of a wave are contiguous");
-    const uint8_t* gate_s = stg - (wave & 1) * kSlice;
-    const uint8_t* up_s = gate_s + kSlice;
+    constexpr int kLanes = WC / 8;                   // lanes whose columns lie in one slice
+    const uint8_t* gate_s = stg - wn * kSlice + l16e / kLanes * kSlice;
+    const uint8_t* up_s = gate_s + WN / 2 * kSlice;
     const uint32_t stg_we = (uint32_t)(uintptr_t)(lds_ptr_t)(stg + l16e * 256);   // this lane's staging row
     const int gcol = n0 >> 1;                        // first activation column of the tile's scaling group
     const __amdgpu_buffer_rsrc_t rsrc_q = __builtin_amdgcn_make_buffer_rsrc(
@@ -1049,9 +1050,9 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
       }
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
-      for (int it = 0; it < 2; ++it) {
-        const int srow = 8 * wn + 4 * it + ge;                   // staging row: tile row wm * 64 + 4 * srow + j
-        const int soff = srow * 256 + ((l16e ^ srow) * 16);
+      for (int it = 0; it < 4 / WN; ++it) {
+        const int srow = 16 / WN * wn + 4 * it + ge;             // staging row: tile row wm * 64 + 4 * srow + j
+        const int soff = srow * 256 + ((l16e % kLanes ^ srow) * 16);
         const v4i gv = *reinterpret_cast<const v4i*>(gate_s + soff);
         const v4i uv = *reinterpret_cast<const v4i*>(up_s + soff);
         uint4 a;
@@ -1141,9 +1142,9 @@ static int persistent_grid(int64_t tiles) {
 }
 
 // The tile of a GEMM: 256 x 256 (8 waves), 128 x 256, 128 x 128 or 64 x 128 (4 waves that multiply, 4 that fetch) or 64 x 64 (2 and 4).
-enum TileShape { k256x256, k128x256, k128x128, k64x128, k64x64 };
+enum TileShape { k256x256, k128x256, k128x128, k64x128, k64x64, k64x256 /* SwiGLU epilogue */ };
 
-static int64_t shape_rows(TileShape shape) { return shape == k256x256 ? 256 : (shape == k64x128 || shape == k64x64 ? 64 : 128); }
+static int64_t shape_rows(TileShape shape) { return shape == k256x256 ? 256 : (shape == k128x256 || shape == k128x128 ? 128 : 64); }
 static int64_t shape_cols(TileShape shape) { return shape == k64x64 ? 64 : (shape == k128x128 || shape == k64x128 ? 128 : 256); }
 
 static int64_t tile_count(int64_t M, int64_t N, TileShape shape) {
@@ -1158,7 +1159,7 @@ static int64_t most_grouped_tiles(int64_t M, int64_t N, int64_t experts, TileSha
 }
 
 // The smallest tile with which the problem is still one round, one tile per compute unit; problems of several rounds
-// take 256 x 256, which moves the fewest bytes through L2 and LDS per product.  A workgroup's round trip per k-block
+// take 256 x 256, which moves the fewest bytes through L2 and LDS per product, or 128 x 256 (better_low).  A workgroup's round trip per k-block
 // is bound by what its compute unit's vector-memory path and LDS move, so with idle units a smaller tile is less work
 // on the same critical path.  us with 256 x 256 / 128 x 256 / 128 x 128 / 64 x 128 tiles (tiles of the one taken):
 //   block   256 x 7168 x 7168    80 / 53 / 39 / 30 (224)         512 x 7168 x 7168    79 / 52 / 39 / 51 (224)
@@ -1170,6 +1171,16 @@ static int64_t most_grouped_tiles(int64_t M, int64_t N, int64_t experts, TileSha
 // and with 128 x 128 / 64 x 128 / 64 x 64 (up to 256 of the last)
 //   block   128 x 7168 x 7168    39 / 31 / 23 (224)              400 x 1024 x 8192    29 / 22 / 20 (112)
 //   rows, onto c  1024 x 1024 x 4096   23 / 18 / 16 (256)        tensor  512 x 1024 x 1024    7.3 / 6.7 / 6.0 (128)
+// Between 128 x 256 and 256 x 256 tiles beyond one round: a round of the lower ones takes three fifths of one of the others, so they are
+// better where they need three rounds and the others a second one for few tiles.  us with 256 x 256 / 128 x 256:
+//   block  2300 x 8192 x 7168 (288 / 576 tiles) 164 / 141       3000 x 7168 x 7168 (336 / 672) 156 / 146
+//   block  2000 x 14336 x 7168 (448 / 896)      172 / 193       8200 x 8192 x 2048 (1056 / 2080) 134 / 137
+//   rows   4352 x 4096 x 2048 (272 / 544)        61 / 56        pow2  3000 x 7168 x 4096 85 / 78
+static bool better_low(int64_t M, int64_t N, int64_t cus) {
+  const int64_t low = (tile_count(M, N, k128x256) + cus - 1) / cus, high = (tile_count(M, N, k256x256) + cus - 1) / cus;
+  return low == 1 || 3 * low < 5 * high;
+}
+
 static TileShape pick_shape(int64_t M, int64_t N) {
   const int mode = g_small_gemm_mode.load(std::memory_order_relaxed);
   const int64_t cus = persistent_grid((int64_t)1 << 40);
@@ -1177,16 +1188,18 @@ static TileShape pick_shape(int64_t M, int64_t N) {
   if (tile_count(M, N, k64x64) <= cus) return k64x64;
   if (tile_count(M, N, k64x128) <= cus) return k64x128;
   if (tile_count(M, N, k128x128) <= cus) return k128x128;
-  if (tile_count(M, N, k128x256) <= cus) return k128x256;
-  return k256x256;
+  return better_low(M, N, cus) ? k128x256 : k256x256;
 }
 
-// SwiGLU epilogue: a tile's columns are the gate and the up half of one scaling group, 256 in all
-// (500 x 8192 x 4096: 52 us with 64 tiles of 256 rows, 37 with 128 of 128 rows; 1000 x 12288 x 4096, 192 and 384: 62, 81).
+// SwiGLU epilogue: a tile's columns are the gate and the up half of one scaling group, 256 in all.  us with 256 / 128 / 64 rows:
+//   500 x 8192 x 4096 (64 / 128 / 256 tiles)  46 / 31 / 22      1000 x 12288 x 4096 (192 / 384 / 768)  55 / 61 / 62
+//   128 x 8192 x 7168 (32 / 32 / 64)          69 / 44 / 30       400 x 36864 x 7168 (288 / 576 / 1008) 154 / 142 / 136
 static TileShape pick_shape_swiglu(int64_t M, int64_t N) {
   const int mode = g_small_gemm_mode.load(std::memory_order_relaxed);
-  if (mode != 0) return mode == 1 ? k256x256 : k128x256;
-  return tile_count(M, N, k128x256) <= persistent_grid((int64_t)1 << 40) ? k128x256 : k256x256;
+  if (mode != 0) return mode == 1 ? k256x256 : (mode == 2 ? k64x256 : k128x256);
+  const int64_t cus = persistent_grid((int64_t)1 << 40);
+  if (tile_count(M, N, k64x256) <= cus) return k64x256;
+  return better_low(M, N, cus) ? k128x256 : k256x256;
 }
 
 // Grouped by rows every expert ends in a partial tile, which costs as much as a whole one, so with few rows per expert low
@@ -1423,12 +1436,14 @@ int hpfp8_gemm_blockwise_swiglu_quantize(const void* a, int64_t lda, const float
   const TileShape shape = pick_shape_swiglu(M, 2 * inter);
   const int64_t tiles = tile_count(M, 2 * inter, shape);
   p.tiles = (int)tiles;
-  dim3 grid((unsigned)persistent_grid(tiles)), block(tile_threads(shape == k256x256 ? 4 : 2, 2));
+  dim3 grid((unsigned)persistent_grid(tiles)), block(512);
+  static_assert(tile_threads(4, 2) == 512 && tile_threads(2, 2) == 512 && tile_threads(1, 4) == 512, "");
   hipStream_t st = (hipStream_t)stream;
   const bool sa4 = sa_stride_m == 1;
 #define HPFP8_LAUNCH_EPI(MODE, SA4, EPI) \
   do { \
     if (shape == k256x256) gemm_kernel<MODE, kDense, false, false, SA4, EPI, 4><<<grid, block, 0, st>>>(p); \
+    else if (shape == k64x256) gemm_kernel<MODE, kDense, false, false, false, EPI, 1, 4, 4><<<grid, block, 0, st>>>(p); \
     else gemm_kernel<MODE, kDense, false, false, false, EPI, 2><<<grid, block, 0, st>>>(p); \
   } while (0)
   if (pow2) {
