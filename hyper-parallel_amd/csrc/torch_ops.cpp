@@ -458,15 +458,17 @@ struct LinearNode : torch::autograd::Function<LinearNode> {
   }
 };
 
-// (x, weight, bias or None) -> whether linear_node takes them: ordinary tensors that are trained, no mode, trace or transform under
-// way that a Python autograd function would answer in its own way (or refuse).
+// (x, weight, bias, codes, scale_inv, codes_t of the weight; None from the bias on) -> whether linear_node takes them: ordinary tensors,
+// x and weight trained, no mode, trace or transform under way that a Python autograd function would answer in its own way (or refuse).
 PyObject* trains(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  expect(n, 3);
-  const at::Tensor *x, *weight, *bias = nullptr;
+  expect(n, 6);
+  const at::Tensor *x, *weight, *bias = nullptr, *form;
   if (!c10::GradMode::is_enabled() || !THPVariable_Check(args[0]) || !THPVariable_Unpack(args[0]).is_cuda()) Py_RETURN_FALSE;
   const int64_t device = THPVariable_Unpack(args[0]).get_device();
   if (!plain(args[0], device, x) || !plain(args[1], device, weight) || (args[2] != Py_None && !plain(args[2], device, bias))) Py_RETURN_FALSE;
+  for (int i = 3; i < 6; ++i)
+    if (args[i] != Py_None && !plain(args[i], device, form)) Py_RETURN_FALSE;
   const bool ok = x->requires_grad() && weight->requires_grad() && x->dim() >= 2 && x->numel() > 0 && weight->numel() > 0 && no_modes() &&
                   !torch::jit::tracer::isTracing() && !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) &&
                   !x->_fw_grad(0).defined() && !weight->_fw_grad(0).defined() && !(bias && bias->_fw_grad(0).defined());

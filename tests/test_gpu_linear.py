@@ -828,6 +828,24 @@ def test_graph_node_equals_the_python_autograd_function(gpu, recipe, shape, n, b
         assert one.shape == other.shape and torch.equal(one, other)
 
 
+def test_weight_form_of_a_tensor_subclass_is_trained_with_as_before(gpu):
+    """A program's own tensor class among a weight's FP8 form goes to the Python autograd function, which takes it."""
+    import hpfp8
+
+    class Own(torch.Tensor):
+        pass
+
+    x, w = U.randn_bf16((256, 384), 1).to(gpu).requires_grad_(True), U.randn_bf16((256, 384), 2, 0.05).to(gpu).requires_grad_(True)
+    go = U.randn_bf16((256, 256), 3, 0.01).to(gpu)
+    f8 = hpfp8.quantize_weight(w.detach(), with_transpose=True)
+    results = []
+    for form in (f8, f8._replace(scale_inv=f8.scale_inv.as_subclass(Own))):
+        y = hpfp8.fp8_linear(x, w, weight_fp8=form)
+        results.append([y.detach(), *torch.autograd.grad(y, (x, w), go)])
+    for one, other in zip(*results):
+        assert torch.equal(one, other)
+
+
 def test_native_operators_leave_other_calls_to_the_python_form(gpu, monkeypatch):
     """Strided, padded and integer-typed operands, refused shapes and types: the same results and errors as without the native forms."""
     import hpfp8
