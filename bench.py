@@ -430,7 +430,7 @@ def other_configs_compact(dev):
     t_both = _time_rot(lambda i: (quant(i), gemm(i)), n1, iters=200, warm=100)
     res["cfg1_per_tensor"] = {"quantize_x": _gb(x.numel() * 3, t_q), "gemm": _tf(2.0 * 2048 * 1024 * 1024, t_g),
                               "quantize_x_plus_gemm_us": t_both * 1e3,
-                              "note": "launch-bound: two launches (one-pass amax + cast, 128 x 128-tile GEMM), times "
+                              "note": "launch-bound: two launches (one-pass amax + cast, 64 x 128-tile GEMM), times "
                                       "include the launches; buffers rotate over 64 copies"}
     del x, w, xq, wq, q1, c1, x1, xq1
     # cfg 2's layer as an inference MLP block: the gate/up GEMM with SwiGLU + the 1x128 quantizer as its epilogue
