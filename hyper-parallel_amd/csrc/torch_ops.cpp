@@ -39,6 +39,7 @@ struct Library {
 #undef HPFP8_POINTER
 } lib;
 PyObject* fail_function = nullptr;       // fail_function(name, status) raises
+PyObject* backward_function = nullptr;   // backward_function(grad_out, saved tensors, ..., as LinearNode has them) -> (dx, dw, db)
 PyObject* parameter_class = nullptr;
 
 // A tensor without wrappers or modes around it, on the device that kernels are launched on.
@@ -358,24 +359,26 @@ uint32_t* sync_block(const at::Tensor& x, int64_t tiles, hipStream_t stream) {
   return (uint32_t*)t.data_ptr();
 }
 
-[[noreturn]] void raise(const Call& call) {
-  pybind11::gil_scoped_acquire held;
-  failed(call);
+[[noreturn]] void raise_python_error() {       // (with the interpreter's lock held)
   python_error e;
   e.persist();
   throw e;
 }
+[[noreturn]] void raise(const Call& call) {
+  pybind11::gil_scoped_acquire held;
+  failed(call);
+  raise_python_error();
+}
 
 // Saved tensors come back through whatever hooks the program has set, so they are looked at again before a kernel reads them.
-void check_codes(const at::Tensor& t, const at::Tensor& go, int64_t r, int64_t c, const char* what) {
-  TORCH_CHECK_VALUE(t.defined() && t.device() == go.device() && !at::isTensorSubclassLike(t) &&
-                        (t.scalar_type() == at::kFloat8_e4m3fn || t.scalar_type() == at::kByte) && t.dim() == 2 && t.size(0) == r && t.size(1) == c &&
-                        t.stride(1) == 1 && (r == 1 || t.stride(0) % 16 == 0),
-                    what, " must be codes [", r, ", ", c, "] on ", go.device(), " with unit inner stride and a row stride that is a multiple of 16");
+bool codes_again(const at::Tensor& t, const at::Tensor& go, int64_t r, int64_t c) {
+  return t.defined() && t.device() == go.device() && t.layout() == at::kStrided && !at::isTensorSubclassLike(t) &&
+         (t.scalar_type() == at::kFloat8_e4m3fn || t.scalar_type() == at::kByte) && t.dim() == 2 && t.size(0) == r && t.size(1) == c &&
+         t.stride(1) == 1 && (r == 1 || t.stride(0) % 16 == 0);
 }
-void check_floats(const at::Tensor& t, const at::Tensor& go, at::IntArrayRef sizes, const char* what) {
-  TORCH_CHECK_VALUE(t.defined() && t.device() == go.device() && !at::isTensorSubclassLike(t) && t.scalar_type() == at::kFloat && t.sizes() == sizes, what,
-                    " must be float32 ", sizes, " on ", go.device());
+bool floats_again(const at::Tensor& t, const at::Tensor& go, at::IntArrayRef sizes) {
+  return t.defined() && t.device() == go.device() && t.layout() == at::kStrided && !at::isTensorSubclassLike(t) && t.scalar_type() == at::kFloat &&
+         t.sizes() == sizes;
 }
 
 // What forward has made, in Python, for y = x W^T + b with gradients of x and W to come: y, and for backward xt, sxt (per
@@ -398,29 +401,45 @@ struct LinearNode : torch::autograd::Function<LinearNode> {
     return made.y;
   }
 
+  static torch::autograd::variable_list in_python(const at::Tensor& go, const torch::autograd::variable_list& saved,
+                                                  const std::vector<int64_t>& shape, int64_t flags) {
+    pybind11::gil_scoped_acquire held;
+    pybind11::tuple size(shape.size());
+    for (size_t i = 0; i < shape.size(); ++i) size[i] = shape[i];
+    const pybind11::tuple args = pybind11::make_tuple(go, saved[0], saved[1], saved[2], saved[3], size, bool(flags & 1), bool(flags & 2),
+                                                      bool(flags & 4), bool(flags & 8));
+    const auto grads = pybind11::reinterpret_steal<pybind11::object>(PyObject_CallObject(backward_function, args.ptr()));
+    if (!grads) raise_python_error();
+    torch::autograd::variable_list out(4);
+    for (int i = 0; i < 3; ++i) {
+      const pybind11::object g = pybind11::tuple(grads)[i];
+      if (!g.is_none()) out[i] = g.cast<at::Tensor>();
+    }
+    return out;
+  }
+
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads) {
     const auto saved = ctx->get_saved_variables();
     const at::Tensor &xt = saved[0], &sxt = saved[1], &w = saved[2], &sw = saved[3];
     const int64_t flags = ctx->saved_data["flags"].toInt();
     const bool per_tensor = flags & 1, pow2 = flags & 2, has_bias = flags & 4, w_transposed = flags & 8;
     const std::vector<int64_t> shape = ctx->saved_data["shape"].toIntVector();
+    // Under a dispatch mode (the engine carries the program's into its threads), and for anything but ordinary tensors where the kernels
+    // read them, the Python function answers.
+    if (!no_modes() || at::isTensorSubclassLike(grads[0])) return in_python(grads[0], saved, shape, flags);
     at::Tensor go = grads[0];
     if (go.dim() != 2) go = go.reshape({-1, go.size(-1)});
     if (go.scalar_type() != at::kBFloat16) go = go.to(at::kBFloat16);
     go = go.contiguous();
-    TORCH_CHECK_VALUE(go.is_cuda() && !at::isTensorSubclassLike(go), "grad_out must be a plain tensor on the GPU (got device ", go.device(),
-                      "); this path has no CPU fallback");
     const int64_t m = go.size(0), mp = rows_up(m), out = go.size(1), in = shape.back();
-    check_codes(xt, go, in, mp, "the saved x^T");
-    check_codes(w, go, per_tensor && !w_transposed ? out : in, per_tensor && !w_transposed ? in : out, "the saved weight");
-    if (per_tensor) {
-      TORCH_CHECK_VALUE(sxt.numel() == 1 && sw.numel() == 1, "per-tensor scales must have exactly one element");
-      check_floats(sxt, go, sxt.sizes(), "the saved scale");
-      check_floats(sw, go, sw.sizes(), "the weight's scale");
-    } else {
-      check_floats(sxt, go, {in, mp / kBlock}, "the saved scales");
-      check_floats(sw, go, {out / kBlock, in / kBlock}, "the weight's scales");
-    }
+    bool plain = go.is_cuda() && go.layout() == at::kStrided;
+    if (per_tensor)
+      plain = plain && codes_again(xt, go, in, mp) && codes_again(w, go, w_transposed ? in : out, w_transposed ? out : in) &&
+              sxt.numel() == 1 && floats_again(sxt, go, sxt.sizes()) && sw.numel() == 1 && floats_again(sw, go, sw.sizes());
+    else
+      plain = plain && codes_again(xt, go, in, mp) && codes_again(w, go, in, out) && floats_again(sxt, go, {in, mp / kBlock}) &&
+              floats_again(sw, go, {out / kBlock, in / kBlock});
+    if (!plain) return in_python(grads[0], saved, shape, flags);
     const c10::hip::HIPStream current = c10::hip::getCurrentHIPStream(go.get_device());
     void* const stream = current.stream();
     Call call;
@@ -509,9 +528,20 @@ PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// (the Python function that LinearNode's backward calls where it does not apply itself)
+PyObject* bind_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  expect(n, 1);
+  Py_INCREF(args[0]);
+  backward_function = args[0];
+  Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
+}
+
 #define HPFP8_METHOD(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {HPFP8_METHOD(bind), HPFP8_METHOD(quantize_1x128), HPFP8_METHOD(both_forms), HPFP8_METHOD(quantize_128x128),
-                         HPFP8_METHOD(quantize_per_tensor_t), HPFP8_METHOD(gemm_blockwise), HPFP8_METHOD(gemm_per_tensor), HPFP8_METHOD(trains), HPFP8_METHOD(linear_node),
+PyMethodDef methods[] = {HPFP8_METHOD(bind), HPFP8_METHOD(bind_backward), HPFP8_METHOD(quantize_1x128), HPFP8_METHOD(both_forms),
+                         HPFP8_METHOD(quantize_128x128), HPFP8_METHOD(quantize_per_tensor_t), HPFP8_METHOD(gemm_blockwise),
+                         HPFP8_METHOD(gemm_per_tensor), HPFP8_METHOD(trains), HPFP8_METHOD(linear_node),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -20,6 +20,7 @@ Recipes
 """
 from __future__ import annotations
 
+import types
 from typing import NamedTuple, Optional
 
 import torch
@@ -264,6 +265,18 @@ class _Fp8LinearPerTensor(torch.autograd.Function):
         if need_dw:
             dw = ops.gemm_per_tensor(got, sgo, xt, sx)     # (contraction over the tokens, filled up with zero codes)
         return dx, dw, db, None, None, None
+
+
+def _node_backward(grad_out, xt, sxt, w, sw, shape, per_tensor, pow2, has_bias, w_transposed):
+    """(dx, dw, db) of the graph node of csrc/torch_ops.cpp where its own backward does not apply: a dispatch mode is active, or
+    grad_out or a saved tensor has come back as something other than an ordinary tensor."""
+    out_features = grad_out.shape[-1]
+    ctx = types.SimpleNamespace(saved_tensors=(xt, sxt, w, sw), x_shape=torch.Size(shape), w_shape=torch.Size((out_features, shape[-1])),
+                                has_bias=has_bias, need=(True, True), pow2=pow2, w_transposed=w_transposed, main_grad_of=None)
+    return (_Fp8LinearPerTensor if per_tensor else _Fp8LinearBlockwise).backward(ctx, grad_out)[:3]
+
+
+ops._native.bind_backward(_node_backward)
 
 
 def fp8_linear(input: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, *,

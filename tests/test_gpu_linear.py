@@ -828,6 +828,38 @@ def test_graph_node_equals_the_python_autograd_function(gpu, recipe, shape, n, b
         assert one.shape == other.shape and torch.equal(one, other)
 
 
+@pytest.mark.parametrize("recipe", ["blockwise", "blockwise_pow2", "per_tensor"])
+@pytest.mark.parametrize("cached", [False, True])
+def test_backward_under_a_dispatch_mode(gpu, recipe, cached):
+    """A step whose forward has made the native node may run its backward under a dispatch mode (a counter, a tracker, a log): the same
+    gradients, and the mode sees what the Python function allocates."""
+    import hpfp8
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from torch.utils.flop_counter import FlopCounterMode
+
+    class Log(TorchDispatchMode):
+        def __init__(self):
+            super().__init__()
+            self.seen = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    x, w = U.randn_bf16((2, 65, 256), 1).to(gpu).requires_grad_(True), U.randn_bf16((384, 256), 2, 0.05).to(gpu).requires_grad_(True)
+    b, go = U.randn_bf16((384,), 3).to(gpu).requires_grad_(True), U.randn_bf16((2, 65, 384), 4, 0.01).to(gpu)
+    f8 = hpfp8.quantize_weight(w.detach(), pow2=recipe == "blockwise_pow2", per_tensor=recipe == "per_tensor") if cached else None
+    want = torch.autograd.grad(hpfp8.fp8_linear(x, w, b, recipe=recipe, weight_fp8=f8), (x, w, b), go)
+    for mode in (Log(), FlopCounterMode(display=False)):
+        y = hpfp8.fp8_linear(x, w, b, recipe=recipe, weight_fp8=f8)
+        assert type(y.grad_fn).__name__ == "CppFunction"
+        with mode:
+            got = torch.autograd.grad(y, (x, w, b), go)
+        for one, other in zip(got, want):
+            assert torch.equal(one, other)
+        assert not isinstance(mode, Log) or any("empty" in name for name in mode.seen)
+
+
 def test_weight_form_of_a_tensor_subclass_is_trained_with_as_before(gpu):
     """A program's own tensor class among a weight's FP8 form goes to the Python autograd function, which takes it."""
     import hpfp8
