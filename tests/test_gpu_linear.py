@@ -946,3 +946,89 @@ def test_linear_training_step_replays_from_a_captured_graph(gpu, recipe):
         torch.cuda.synchronize()
         for one, other in zip(outs, step(x.clone().requires_grad_(True))):
             assert torch.equal(one, other)
+
+
+@pytest.mark.parametrize("recipe", ["blockwise", "per_tensor"])
+@pytest.mark.parametrize("way", ["mode", "vmap", "grad", "forward_ad", "trace", "batched_backward", "create_graph", "checkpoint", "reentrant",
+                                 "dispatching_grad", "sparse_grad", "detect_anomaly"])
+def test_what_else_torch_does_with_a_step_has_the_python_functions_outcome(gpu, recipe, way, monkeypatch):
+    """Modes, transforms, traces and tensors of other kinds around a linear's forward or backward: values and errors are those that the
+    Python autograd function gives by itself."""
+    import types
+    import hpfp8
+    import torch.autograd.forward_ad as fwAD
+    from hpfp8 import ops
+    from torch.utils.checkpoint import checkpoint
+    from torch.utils._python_dispatch import TorchDispatchMode
+    x, w = U.randn_bf16((256, 256), 1).to(gpu).requires_grad_(True), U.randn_bf16((128, 256), 2, 0.05).to(gpu).requires_grad_(True)
+    go = U.randn_bf16((256, 128), 3, 0.01).to(gpu)
+
+    class Pass(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Dispatching(torch.Tensor):
+        @staticmethod
+        def __new__(cls, t):
+            return torch.Tensor._make_subclass(cls, t)
+
+        @classmethod
+        def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+            raw = lambda a: a.as_subclass(torch.Tensor) if isinstance(a, cls) else a
+            with torch._C._DisableTorchDispatch():
+                return func(*[raw(a) for a in args], **(kwargs or {}))
+
+    def f(a, b):
+        return hpfp8.fp8_linear(a, b, recipe=recipe)
+
+    def step():
+        if way == "mode":
+            with Pass():
+                y = f(x, w)
+            return (y, *torch.autograd.grad(y, (x, w), go))
+        if way == "vmap":
+            return torch.func.vmap(f, in_dims=(0, None))(x.view(2, 128, 256), w)
+        if way == "grad":
+            return torch.func.grad(lambda a: f(a, w).float().sum())(x)
+        if way == "forward_ad":
+            with fwAD.dual_level():
+                return f(fwAD.make_dual(x, torch.ones_like(x)), w)
+        if way == "trace":
+            return torch.jit.trace(f, (x, w), check_trace=False)(x, w)
+        y = checkpoint(f, x, w, use_reentrant=way == "reentrant") if way in ("checkpoint", "reentrant") else f(x, w)
+        if way == "batched_backward":
+            return torch.autograd.grad(y, (x, w), torch.stack((go, go)), is_grads_batched=True)
+        if way == "create_graph":
+            return (y, *torch.autograd.grad(y, (x, w), go, create_graph=True))
+        if way == "dispatching_grad":
+            return torch.autograd.grad(y, (x, w), Dispatching(go))
+        if way == "sparse_grad":
+            return torch.autograd.grad(y, (x, w), go.to_sparse())
+        if way == "detect_anomaly":
+            with torch.autograd.detect_anomaly(check_nan=True):
+                return torch.autograd.grad(y, (x, w), go)
+        return (y, *torch.autograd.grad(y, (x, w), go)) if way != "reentrant" else (y, *_leaf_grads(y, (x, w), go))
+
+    def outcome():
+        try:
+            r = step()
+        except Exception as e:
+            return type(e), str(e).split("\n")[0]
+        return list(r) if isinstance(r, (tuple, list)) else [r]
+
+    def _leaf_grads(y, leaves, go):
+        for t in leaves:
+            t.grad = None
+        y.backward(go)
+        return [t.grad for t in leaves]
+
+    got = outcome()
+    native = types.SimpleNamespace(**{k: getattr(ops._native, k) for k in dir(ops._native) if not k.startswith("__")})
+    native.trains = lambda *a: False
+    monkeypatch.setattr(ops, "_native", native)
+    want = outcome()
+    if isinstance(want, tuple):
+        assert got == want
+    else:
+        assert isinstance(got, list), got
+        assert len(got) == len(want) and all(type(a) is type(b) and a.requires_grad == b.requires_grad and torch.equal(a, b) for a, b in zip(got, want))
