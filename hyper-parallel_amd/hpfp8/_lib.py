@@ -1,6 +1,7 @@
 """ctypes binding of libhpfp8.so (the C ABI declared in include/hpfp8.h).
 
-There is no fallback: if the library is missing, or a call fails, an exception is raised.
+There is no fallback: if the library is missing, or a call fails, an exception is raised.  (The native host path around it,
+_native.so, may be missing: `load_native`.)
 """
 from __future__ import annotations
 
@@ -132,12 +133,15 @@ def call(name: str, *args) -> None:
 
 
 def load_native():
-    """The tensor operators' native host path (csrc/torch_ops.cpp), bound to the loaded library."""
+    """The tensor operators' native host path (csrc/torch_ops.cpp), bound to the loaded library.  Where it is missing or does not load
+    beside the installed torch: None, with a warning; the Python form of each operator launches the same kernels, with more host time."""
+    import warnings
     import torch
     try:
         from . import _native
     except ImportError as e:
-        raise ImportError(f"hpfp8/_native.so is missing or does not fit the installed torch ({e}): run `python "
-                          f"{os.path.join(os.path.dirname(_HERE), 'build.py')}`.") from e
+        warnings.warn(f"hpfp8/_native.so is missing or does not fit ({e}): operators are launched from Python, at twice the host time. "
+                      f"Run `python {os.path.join(os.path.dirname(_HERE), 'build.py')}`.", RuntimeWarning, stacklevel=2)
+        return None
     _native.bind(load()._handle, fail, torch.nn.Parameter)
     return _native

@@ -276,7 +276,8 @@ def _node_backward(grad_out, xt, sxt, w, sw, shape, per_tensor, pow2, has_bias, 
     return (_Fp8LinearPerTensor if per_tensor else _Fp8LinearBlockwise).backward(ctx, grad_out)[:3]
 
 
-ops._native.bind_backward(_node_backward)
+if ops._native is not None:
+    ops._native.bind_backward(_node_backward)
 
 
 def fp8_linear(input: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, *,
@@ -332,7 +333,7 @@ def fp8_linear(input: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.T
                 raise ValueError("weight_fp8 was quantized with one scale per tensor")
             if bool(weight_fp8.pow2) != pow2:
                 raise ValueError("weight_fp8 was quantized for the other blockwise recipe")
-    if not apply_grad_on_fp32_main_grad and ops._native.trains(input, weight, bias, wq, sw, wqt):
+    if not apply_grad_on_fp32_main_grad and ops._native is not None and ops._native.trains(input, weight, bias, wq, sw, wqt):
         return _trained(input, weight, bias, wq, sw, wqt, recipe == "per_tensor", pow2)
     if recipe == "per_tensor":
         return _Fp8LinearPerTensor.apply(input, weight, bias, wq, sw, torch.is_grad_enabled())

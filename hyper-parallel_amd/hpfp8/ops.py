@@ -33,7 +33,7 @@ _PLAIN = frozenset((torch.Tensor, torch.nn.Parameter))
 
 def _gpu(x) -> bool:
     """Whether the native form of an operator is to be asked (it returns None for what it does not take)."""
-    return type(x) in _PLAIN and x.is_cuda
+    return _native is not None and type(x) in _PLAIN and x.is_cuda
 
 
 def _stream() -> int:
