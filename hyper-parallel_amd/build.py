@@ -5,9 +5,11 @@ Usage: python build.py [--force]
 """
 from __future__ import annotations
 
+import importlib.util
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -32,13 +34,19 @@ def _flags():
     ]
 
 
+def _native_tag() -> str:
+    spec = importlib.util.spec_from_file_location("hpfp8_lib", os.path.join(HERE, "hpfp8", "_lib.py"))
+    lib = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(lib)
+    return lib.native_tag()
+
+
 def _native_command():
-    import sysconfig
     import torch
     from torch.utils.cpp_extension import include_paths
     lib = os.path.join(os.path.dirname(torch.__file__), "lib")
     return (["g++", "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
-            + ["-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1"]
+            + ["-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f'-DHPFP8_BUILT_FOR="{_native_tag()}"']
             + [f"-I{d}" for d in include_paths("cuda") + [sysconfig.get_paths()["include"]]]
             + [NATIVE_SOURCE, "-o", NATIVE, f"-L{lib}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", f"-Wl,-rpath,{lib}"])
 
@@ -50,24 +58,40 @@ def _older(out, deps) -> bool:
     return any(os.path.getmtime(d) > t for d in deps + [os.path.abspath(__file__)])
 
 
+def library_stale() -> bool:
+    return _older(OUT, [os.path.join(CSRC, s) for s in SOURCES + HEADERS])
+
+
+def native_stale() -> bool:
+    """Older than its source, or built for another torch or interpreter (the module holds the name of what it was built for)."""
+    if _older(NATIVE, [NATIVE_SOURCE, os.path.join(CSRC, HEADERS[-1])]):
+        return True
+    with open(NATIVE, "rb") as f:
+        return _native_tag().encode() + b"\0" not in f.read()
+
+
 def needs_build() -> bool:
-    header = os.path.join(CSRC, HEADERS[-1])
-    return _older(OUT, [os.path.join(CSRC, s) for s in SOURCES + HEADERS]) or _older(NATIVE, [NATIVE_SOURCE, header])
+    return library_stale() or native_stale()
+
+
+def _run(cmd, verbose: bool) -> None:
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    out = "\n".join(l for l in res.stdout.splitlines() if "packed-fp32-ops" not in l)
+    if res.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed:\n" + out)
+    if verbose and out.strip():
+        print(out)
 
 
 def build(force: bool = False, verbose: bool = False) -> str:
-    if not force and not needs_build():
-        return OUT
-    hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
-    for cmd in ([hipcc] + _flags() + [os.path.join(CSRC, s) for s in SOURCES] + ["-o", OUT], _native_command()):
-        if verbose:
-            print(" ".join(cmd), flush=True)
-        res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
-        out = "\n".join(l for l in res.stdout.splitlines() if "packed-fp32-ops" not in l)
-        if res.returncode != 0:
-            raise RuntimeError(f"{cmd[0]} failed:\n" + out)
-        if verbose and out.strip():
-            print(out)
+    """Each of the two where it is stale (``force``: both); the library first, which the package can do with alone."""
+    if force or library_stale():
+        hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+        _run([hipcc] + _flags() + [os.path.join(CSRC, s) for s in SOURCES] + ["-o", OUT], verbose)
+    if force or native_stale():
+        _run(_native_command(), verbose)
     return OUT
 
 

@@ -528,6 +528,9 @@ PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// -> the torch, C++ ABI and interpreter that this module was built for (hpfp8/_lib.py native_tag)
+PyObject* built_for(PyObject*, PyObject* const*, Py_ssize_t) { return PyUnicode_FromString(HPFP8_BUILT_FOR); }
+
 // (the Python function that LinearNode's backward calls where it does not apply itself)
 PyObject* bind_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -539,7 +542,7 @@ PyObject* bind_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
 }
 
 #define HPFP8_METHOD(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {HPFP8_METHOD(bind), HPFP8_METHOD(bind_backward), HPFP8_METHOD(quantize_1x128), HPFP8_METHOD(both_forms),
+PyMethodDef methods[] = {HPFP8_METHOD(built_for), HPFP8_METHOD(bind), HPFP8_METHOD(bind_backward), HPFP8_METHOD(quantize_1x128), HPFP8_METHOD(both_forms),
                          HPFP8_METHOD(quantize_128x128), HPFP8_METHOD(quantize_per_tensor_t), HPFP8_METHOD(gemm_blockwise),
                          HPFP8_METHOD(gemm_per_tensor), HPFP8_METHOD(trains), HPFP8_METHOD(linear_node),
                          {nullptr, nullptr, 0, nullptr}};

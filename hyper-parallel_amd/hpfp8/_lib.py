@@ -132,13 +132,23 @@ def call(name: str, *args) -> None:
         fail(name, rc)
 
 
+def native_tag() -> str:
+    """What _native.so is built against: a module built for another torch or interpreter may load and then misread their classes."""
+    import sys
+    import torch
+    return f"torch {torch.__version__}, C++ ABI {int(torch._C._GLIBCXX_USE_CXX11_ABI)}, {sys.implementation.cache_tag}"
+
+
 def load_native():
-    """The tensor operators' native host path (csrc/torch_ops.cpp), bound to the loaded library.  Where it is missing or does not load
-    beside the installed torch: None, with a warning; the Python form of each operator launches the same kernels, with more host time."""
+    """The tensor operators' native host path (csrc/torch_ops.cpp), bound to the loaded library.  Where it is missing or was built for
+    another torch: None, with a warning; the Python form of each operator launches the same kernels, with more host time."""
     import warnings
     import torch
     try:
         from . import _native
+        made_for = getattr(_native, "built_for", lambda: "an unnamed torch")()
+        if made_for != native_tag():
+            raise ImportError(f"it was built for {made_for}, this is {native_tag()}")
     except ImportError as e:
         warnings.warn(f"hpfp8/_native.so is missing or does not fit ({e}): operators are launched from Python, at twice the host time. "
                       f"Run `python {os.path.join(os.path.dirname(_HERE), 'build.py')}`.", RuntimeWarning, stacklevel=2)

@@ -21,6 +21,27 @@ def test_package_is_imported_without_the_native_host_path():
     assert r.stdout.split() == ["False", "128"]
 
 
+def test_a_module_built_for_another_torch_is_stale_and_not_used(monkeypatch):
+    """Its classes might be laid out otherwise: the build makes it again (and not the library), the package goes without it."""
+    import importlib.util
+    from hpfp8 import _lib
+    spec = importlib.util.spec_from_file_location("hpfp8_build", os.path.join(PKG, "build.py"))
+    build = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(build)
+    monkeypatch.setattr(build, "_older", lambda out, deps: False)
+    assert not build.native_stale() and not build.needs_build()
+    monkeypatch.setattr(build, "_native_tag", lambda: "torch 2.1")
+    assert build.native_stale() and build.needs_build() and not build.library_stale()
+    ran = []
+    monkeypatch.setattr(build, "_run", lambda cmd, verbose: ran.append(cmd[0]))
+    build.build()
+    assert ran == ["g++"]
+    assert _lib.load_native() is not None
+    monkeypatch.setattr(_lib, "native_tag", lambda: "torch 2.1")
+    with pytest.warns(RuntimeWarning, match="built for torch"):
+        assert _lib.load_native() is None
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("recipe", ["blockwise", "blockwise_pow2", "per_tensor"])
 def test_step_without_the_native_host_path_has_the_same_bits(gpu, recipe, monkeypatch):
