@@ -616,10 +616,6 @@ def gemm_blockwise(a: torch.Tensor, sa: torch.Tensor, b: torch.Tensor, sb: torch
         c = _native.gemm_blockwise(a, sa, b, sb, bias, out, sb_gran, accumulate, pow2_scales, device, _raw_stream(device))
         if c is not None:
             return c
-    return _gemm_blockwise(a, sa, b, sb, bias, out_dtype, sb_gran, out, accumulate, pow2_scales)
-
-
-def _gemm_blockwise(a, sa, b, sb, bias=None, out_dtype=torch.bfloat16, sb_gran=128, out=None, accumulate=False, pow2_scales=False):
     a = _check_codes_2d(a, "a")
     b = _check_codes_2d(b, "b")
     sa = _check_f32(sa, "sa")
@@ -686,9 +682,9 @@ def gemm_blockwise_swiglu_quantize(a: torch.Tensor, sa: torch.Tensor, b: torch.T
     # (a weight that spans 2 GiB or more is left to the fused call, which refuses it at every row count)
     if 0 < m <= _lib.load().hpfp8_gemm_few_rows(k) and n * _ld(b) < 0x7FFFF000:
         # A decode step: the GEMM is bound by reading the weight, which its few-rows form does at twice the rate of the
-        # 256 x 256 tiles the epilogue belongs to; gate | up is a few megabytes (37 rows of a [36864, 7168] weight: 86 us
+        # tiles the epilogue belongs to; gate | up is a few megabytes (37 rows of a [36864, 7168] weight: 86 us
         # for the epilogue form, 42 + 5 us for the two launches, the same bits).
-        h = _gemm_blockwise(a, sa, b, sb, pow2_scales=pow2_scales)
+        h = gemm_blockwise(a, sa, b, sb, pow2_scales=pow2_scales)
         if fast:
             _lib.call("hpfp8_swiglu_quantize_1x128_fast_bf16", _ptr(h), m, inter, n, 1, int(pow2_out), _ptr(q), _ptr(s), _ptr(s_inv),
                       None, _stream())

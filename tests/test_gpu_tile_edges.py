@@ -232,8 +232,9 @@ def test_swiglu_operator_takes_two_launches_where_the_gemm_takes_few_rows(gpu, m
     k, inter = 2048, 128
     a, sa = ops.quantize_1x128(_normal((m, k), 1, gpu), kmajor=True)
     b, sb = ops.quantize_128x128(_normal((2 * inter, k), 2, gpu, 0.05))
-    names, call = [], _lib.call
+    names, call, gemm = [], _lib.call, ops.gemm_blockwise
     monkeypatch.setattr(_lib, "call", lambda name, *args: (names.append(name), call(name, *args))[1])
+    monkeypatch.setattr(ops, "gemm_blockwise", lambda *args, **kw: (names.append("gemm_blockwise"), gemm(*args, **kw))[1])
     _lib.load().hpfp8_debug_set_small_gemm(mode)
     try:
         few = m <= _lib.load().hpfp8_gemm_few_rows(k)
@@ -241,7 +242,7 @@ def test_swiglu_operator_takes_two_launches_where_the_gemm_takes_few_rows(gpu, m
     finally:
         _lib.load().hpfp8_debug_set_small_gemm(0)
     assert few == (m == 64 and mode == 0)
-    assert names == (["hpfp8_gemm_blockwise", "hpfp8_swiglu_quantize_1x128_bf16"] if few else ["hpfp8_gemm_blockwise_swiglu_quantize"])
+    assert names == (["gemm_blockwise", "hpfp8_swiglu_quantize_1x128_bf16"] if few else ["hpfp8_gemm_blockwise_swiglu_quantize"])
 
 
 @pytest.mark.parametrize("m", [1, 64, 65])
