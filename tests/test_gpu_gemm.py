@@ -22,8 +22,8 @@ TOL_BF16 = 3e-3          # bf16 output: one rounding (2^-9 relative per element)
 
 @pytest.fixture(autouse=True, params=["large tiles only", "default rule"])
 def gemm_kernel_choice(request):
-    """Most shapes here have few tiles, which the library would hand to its small-tile kernel: every test of this
-    module runs once with that kernel switched off (so the 256 x 256-tile kernel sees the small, ragged and edge
+    """Most shapes here have few tiles, for which the library would take small ones: every test of this
+    module runs once with those switched off (so the 256 x 256 tiles see the small, ragged and edge
     cases too) and once under the default rule."""
     from hpfp8 import _lib
     lib = _lib.load()
@@ -720,11 +720,9 @@ def small_gemm_mode():
 @pytest.mark.parametrize("shape", [(2048, 1024, 1024), (1, 128, 128), (130, 384, 256), (64, 2304, 512), (257, 128, 1152),
                                    (1000, 640, 384), (2048, 2304, 256), (4100, 1024, 384)])
 def test_small_tile_kernel_equals_the_large_tile_kernel_and_the_oracle(gpu, shape, small_gemm_mode):
-    """The small-tile kernel (problems with few tiles: BASELINE configuration 1, decode-sized M) does the same
-    arithmetic in the same order as the 256 x 256-tile kernel: identical bits for the block and the per-tensor
-    form, fp32 and bf16 output, with and without bias, ragged M; and the fp32 output agrees with the oracle as the
-    large kernel's does.  Mode 2 is that kernel (64 x 128 tiles) where 128 x 128 tiles would be fewer than the 256
-    compute units (the first six shapes) and 128 x 128 tiles of the large kernel otherwise (288 and 264 of them)."""
+    """The small tiles (64 x 64, 128 x 128 and 64 x 128, asked for one after the other: what problems with few tiles take) do the same
+    arithmetic in the same order as 256 x 256 ones: identical bits for the block and the per-tensor form, fp32 and bf16 output, with and
+    without bias, ragged M; and the fp32 output agrees with the oracle as that of the large tiles does."""
     import hpfp8
     m, n, k = shape
     x = U.randn_bf16((m, k), 40 + m, 1.0, 0.001, 30.0).to(gpu)
@@ -735,15 +733,16 @@ def test_small_tile_kernel_equals_the_large_tile_kernel_and_the_oracle(gpu, shap
     xt, _, sxt = hpfp8.quantize_per_tensor(x)
     wt, _, swt = hpfp8.quantize_per_tensor(w)
     out = {}
-    for mode in (1, 2):
+    for mode in (1, 2, 4, 5):
         small_gemm_mode(mode)
         out[mode] = [hpfp8.gemm_blockwise(xq, sx, wq, sw, out_dtype=torch.float32),
                      hpfp8.gemm_blockwise(xq, sx, wq, sw, bias=bias),
                      hpfp8.gemm_per_tensor(xt, sxt, wt, swt, out_dtype=torch.float32),
                      hpfp8.gemm_per_tensor(xt, sxt, wt, swt, bias=bias)]
-    for big, small in zip(out[1], out[2]):
-        assert torch.equal(big.view(torch.int32) if big.dtype == torch.float32 else big.view(torch.int16),
-                           small.view(torch.int32) if small.dtype == torch.float32 else small.view(torch.int16))
+    for mode in (2, 4, 5):
+        for big, small in zip(out[1], out[mode]):
+            assert torch.equal(big.view(torch.int32) if big.dtype == torch.float32 else big.view(torch.int16),
+                               small.view(torch.int32) if small.dtype == torch.float32 else small.view(torch.int16))
     if m * n * k <= 2048 * 1024 * 1024:
         want, _ = O.gemm_blockwise(U.codes(xq), U.f32(sx), U.codes(wq), U.f32(sw))
         assert rel(U.f32(out[2][0]), want) < TOL_F32
@@ -755,9 +754,9 @@ def test_small_tile_kernel_equals_the_large_tile_kernel_and_the_oracle(gpu, shap
 
 
 def test_small_problems_select_the_small_tile_kernel(gpu, small_gemm_mode):
-    """Under the default rule configuration 1 (32 large tiles) runs the small-tile kernel and configuration 2 does
-    not; observable through the hook: forcing either kernel gives the same bits, so only timing can tell -- here
-    the rule itself is checked through identical results in all three modes on a small and a larger problem."""
+    """Under the default rule a problem of 32 large tiles takes small ones and one of 128 need not; forcing either gives the same
+    bits, so only timing can tell -- here the rule is checked through identical results under it, with large tiles and with the
+    smallest on a small and a larger problem."""
     import hpfp8
     for m, n, k in ((2048, 1024, 1024), (1024, 8192, 256)):
         x = U.randn_bf16((m, k), 50, 1.0).to(gpu)

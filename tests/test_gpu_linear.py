@@ -792,10 +792,11 @@ def test_grouped_linear_prequantized_weight_and_inference(gpu):
 
 @pytest.mark.parametrize("recipe", ["blockwise", "blockwise_pow2", "per_tensor"])
 @pytest.mark.parametrize("shape,n,bias,cached", [((256, 384), 256, True, None), ((1, 128), 128, False, None), ((2, 65, 256), 384, True, "codes_t"),
-                                                 ((200, 1280), 128, False, "codes"), ((384, 2176), 2304, True, "codes")])
+                                                 ((200, 1280), 128, False, "codes"), ((384, 2176), 2304, True, "codes"),
+                                                 ((2048, 2048), 2048, True, None), ((2050, 2304), 2304, True, None)])
 def test_graph_node_equals_the_python_autograd_function(gpu, recipe, shape, n, bias, cached, monkeypatch):
     """The native node's output and gradients are the Python function's bit for bit: ragged and whole token counts, more dimensions, one
-    and two launches of the per-tensor quantizer, a weight's FP8 form with and without its transposed codes; also with every saved tensor
+    (up to 256 tiles, the first of the last two shapes) and two launches of the per-tensor quantizer (the last), a weight's FP8 form with and without its transposed codes; also with every saved tensor
     moved to the host and back in another layout; tensors that a hook hands back on the host are refused."""
     import types
     import hpfp8

@@ -324,14 +324,15 @@ def test_gemm_tiles_are_exact_on_integer_inputs(gpu, m, n, k):
 
 @pytest.mark.parametrize("m,n,k", [(1, 128, 128), (127, 384, 256), (129, 640, 640), (300, 2432, 384), (1000, 1152, 1152)])
 def test_every_tile_shape_gives_the_same_bits(gpu, m, n, k):
-    """256 x 256, 128 x 256, 128 x 128 and 64 x 128 tiles, asked for one after the other (so whatever the number of compute
-    units) on random values: all scale forms, output types, bias, accumulation, the SwiGLU epilogue and experts."""
+    """256 x 256, 64 x 64 (64 x 256 for the SwiGLU epilogue), 128 x 256, 128 x 128 and 64 x 128 tiles, asked for one after the other (so
+    whatever the number of compute units; a form that lacks one takes the next larger) on random values: all scale forms, output types,
+    bias, accumulation, the SwiGLU epilogue and experts."""
     from hpfp8 import _lib, ops
     x, w = _normal((m, k), 1, gpu, outliers=True), _normal((2 * n, k), 2, gpu, 0.05)
     bias, c0 = _normal((n,), 3, gpu), _normal((m, n), 4, gpu).float()
     rows = torch.tensor([m // 3, 0, m - m // 3]).cumsum(0).to(torch.int32).to(gpu)
     out = {}
-    for mode in (1, 2, 3):
+    for mode in (1, 2, 3, 4, 5):
         _lib.load().hpfp8_debug_set_small_gemm(mode)
         try:
             r = out[mode] = []
@@ -343,20 +344,22 @@ def test_every_tile_shape_gives_the_same_bits(gpu, m, n, k):
                 r.append(ops.gemm_blockwise(a, sa, b1, sb1, pow2_scales=pow2, out_dtype=torch.float32))
                 r.append(ops.gemm_blockwise(a, sa.contiguous(), b1, sb1, bias=bias, pow2_scales=pow2))
                 r.append(ops.gemm_blockwise(a, sa, br, sr, sb_gran=1, pow2_scales=pow2))
+                r.append(ops.gemm_blockwise(a, sa.contiguous(), br, sr, sb_gran=1, pow2_scales=pow2, out_dtype=torch.float32))
                 for gran, bb, ss in ((128, b1, sb1), (1, br, sr)):
                     r.append(ops.gemm_blockwise(a, sa, bb, ss, sb_gran=gran, out=c0.clone(), accumulate=True, pow2_scales=pow2))
                 r += ops.gemm_blockwise_swiglu_quantize(a, sa, b, sb, fast=pow2, pow2_scales=pow2, pow2_out=pow2, want_scale=True)
                 stack = b.view(2, n, k), sb.view(2, n // 128, k // 128)
                 experts = [torch.cat((t, t[:1])) if t.dtype == torch.float32 else torch.cat((t.view(torch.uint8), t[:1].view(torch.uint8)))
                            for t in stack]
-                r.append(ops.gemm_grouped_blockwise(a, sa, *experts, rows, pow2_scales=pow2))
+                for dtype in (torch.bfloat16, torch.float32):
+                    r.append(ops.gemm_grouped_blockwise(a, sa, *experts, rows, pow2_scales=pow2, out_dtype=dtype))
             a, _, sa = ops.quantize_per_tensor(x)
             b, _, sb = ops.quantize_per_tensor(w[:n])
             r.append(ops.gemm_per_tensor(a, sa, b, sb, out_dtype=torch.float32))
             r.append(ops.gemm_per_tensor(a, sa, b, sb, bias=bias))
         finally:
             _lib.load().hpfp8_debug_set_small_gemm(0)
-    for mode in (2, 3):
+    for mode in (2, 3, 4, 5):
         for got, want in zip(out[mode], out[1]):
             assert torch.equal(got.view(torch.uint8) if got.dtype == torch.float8_e4m3fn else got,
                                want.view(torch.uint8) if want.dtype == torch.float8_e4m3fn else want)
@@ -597,3 +600,34 @@ def test_grouped_rows_give_the_same_bits_with_every_tile(gpu, counts, n):
     for i, c in enumerate(counts[:6]):
         rows = slice(int(sum(counts[:i])), int(sum(counts[:i + 1])))
         assert torch.equal(got[0][0][rows], ops.gemm_blockwise(a[rows], sa[rows], b[i], sb[i]))
+
+
+def _chosen_rows(counts, n, cus=256):
+    """The height that grouped_tile_rows (csrc/gemm.hip) chooses for these rows of the experts."""
+    tiles = {tm: sum(-(-c // tm) for c in counts) * -(-n // tn) for tm, tn in ((64, 128), (128, 256), (256, 256))}
+    cost = {tm: w * -(-tiles[tm] // cus) for tm, w in ((64, 26), (128, 50), (256, 83))}
+    return min(cost, key=lambda tm: (cost[tm], tm))
+
+
+@pytest.mark.parametrize("rows,counts", [(64, [70] + [0] * 31), (128, [64] * 31 + [61]), (256, [7900] + [0] * 30 + [100])])
+@pytest.mark.parametrize("pow2", [False, True])
+def test_grouped_kernel_that_chooses_its_tile_has_the_bits_of_one_that_does_not(gpu, rows, counts, pow2):
+    """Each of the three forms inside the kernel that chooses, reached through the default rule: both output types, scales of a in both
+    layouts."""
+    from hpfp8 import _lib, ops
+    n, k, e, m = 4096, 256, len(counts), sum(counts)
+    assert torch.cuda.get_device_properties(0).multi_processor_count != 256 or _chosen_rows(counts, n) == rows
+    a, sa = ops.quantize_1x128(_normal((m, k), 1, gpu, outliers=True), kmajor=True, pow2=pow2)
+    b, sb = ops.quantize_128x128(_normal((e * n, k), 2, gpu, 0.05), pow2=pow2)
+    b, sb = b.view(e, n, k), sb.view(e, n // 128, k // 128)
+    offs = torch.tensor(counts).cumsum(0).to(torch.int32).to(gpu)
+    got = {}
+    for mode in (1, 0):
+        _lib.load().hpfp8_debug_set_small_gemm(mode)
+        try:
+            got[mode] = [ops.gemm_grouped_blockwise(a, s, b, sb, offs, out_dtype=dtype, pow2_scales=pow2)
+                         for s in (sa, sa.contiguous()) for dtype in (torch.bfloat16, torch.float32)]
+        finally:
+            _lib.load().hpfp8_debug_set_small_gemm(0)
+    for one, other in zip(got[0], got[1]):
+        assert torch.equal(one, other)
