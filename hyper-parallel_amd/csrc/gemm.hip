@@ -92,8 +92,12 @@ struct GemmParams {
 };
 
 // n / d for uniform values, without the compiler's division (some 30 dependent instructions; a tile lookup has four, and a
-// workgroup does nothing else before its first transfers)
+// workgroup does nothing else before its first transfers).  The reciprocal is not kept across a tile's products: hoisted out of
+// the loop over tiles it took a vector register that 256 x 256 forms do not have, and came back from scratch memory behind a wait
+// for every transfer under way.
 __device__ __forceinline__ int quotient(int n, int d) {
+  d = __builtin_amdgcn_readfirstlane(d);
+  asm volatile("" : "+s"(d));
   if (n >= (1 << 22)) return n / d;
   int q = (int)((float)n * __builtin_amdgcn_rcpf((float)d));      // n and d exact in fp32, rcp within one ulp: off by one at most
   const int rest = n - q * d;
