@@ -88,7 +88,7 @@ struct GemmParams {
   int pow2_out;
   float* q_scale;
   float* q_scale_inv;
-  int choose_cus;         // grouped by rows, tile chosen on the device: the compute units there are
+  int choose_cus;         // grouped by rows, tile chosen on the device: the compute units there are (test hook: minus the rows asked for)
 };
 
 // n / d for uniform values, without the compiler's division (some 30 dependent instructions; a tile lookup has four, and a
@@ -1119,7 +1119,7 @@ __global__ __launch_bounds__(512) void gemm_grouped_kernel(const GemmParams p) {
   __shared__ __attribute__((aligned(1024))) uint8_t lds[kMost];
   ExpertChunk group{0, 0, 0, 0, 0};
   expert_ends(group, p, threadIdx.x & 63);
-  const int rows = grouped_tile_rows(group, p, threadIdx.x & 63);
+  const int rows = p.choose_cus < 0 ? -p.choose_cus : grouped_tile_rows(group, p, threadIdx.x & 63);
   if (rows == 64) gemm_tiles<MODE, kGroupedRows, OUT_F32, false, false, 0, 1, 2, 4>(p, lds, group);
   else if (rows == 128) gemm_tiles<MODE, kGroupedRows, OUT_F32, false, false, 0, 2, 8, 2>(p, lds, group);
   else gemm_tiles<MODE, kGroupedRows, OUT_F32, false, SA4, 0, 4, 8, 2>(p, lds, group);
@@ -1217,7 +1217,7 @@ static TileShape pick_shape_swiglu(int64_t M, int64_t N) {
 //   8 experts  [4096, 7168],   512 rows    37 /  46 /  72    48 /  43 /  68    50 /  43 /  69    25 /  42 /  66
 //   16 experts [1024, 4096],  2048 rows    18 /  28 /  43    28 /  28 /  42    22 /  27 /  42    17 /  27 /  41
 //   64 experts [2048, 2048], 16384 rows   144 /  81 /  76   146 /  97 / 117   145 /  84 / 101   118 /  70 /  63
-enum GroupedTiles { kSmallestTiles, kLowestTiles, kLowTiles, kHighTiles, kChosenTiles };
+enum GroupedTiles { kSmallestTiles, kLowestTiles, kHighTiles, kChosenTiles, kLowTiles /* test hook: as chosen */ };
 
 static GroupedTiles pick_grouped(int64_t M, int64_t N, int experts) {
   const int mode = g_small_gemm_mode.load(std::memory_order_relaxed);
@@ -1264,10 +1264,11 @@ static int launch_sa(const GemmParams& p, int out_type, int64_t tiles, hipStream
 
 template <int MODE, int GROUPED, int WM, int NS, int WN>
 static int launch_shape(const GemmParams& p, int out_type, int64_t tiles, hipStream_t stream) {
+  if constexpr (GROUPED == kGroupedK) return launch_sa<MODE, GROUPED, true, WM, NS, WN>(p, out_type, tiles, stream);   // (sa_sm = 1)
   if constexpr (MODE != kScaleTensor && !fetchers(WM)) {      // (fetched to LDS, sa may have any strides)
     if (p.sa_sm == 1) return launch_sa<MODE, GROUPED, true, WM, NS, WN>(p, out_type, tiles, stream);
   }
-  return launch_sa<MODE, GROUPED, false, WM, NS, WN>(p, out_type, tiles, stream);
+  if constexpr (GROUPED != kGroupedK) return launch_sa<MODE, GROUPED, false, WM, NS, WN>(p, out_type, tiles, stream);
 }
 
 template <int MODE, int GROUPED>
@@ -1277,10 +1278,8 @@ static int launch(GemmParams p, int out_type, TileShape shape, hipStream_t strea
   if (GROUPED == kGroupedK) tiles *= p.experts;
   // upper bound on row tiles: every expert may add one partial tile
   if (GROUPED == kGroupedRows) tiles = most_grouped_tiles(p.M, p.N, p.experts, shape);
-  if constexpr (GROUPED != kGroupedK) {
-    if (shape == k128x256) return launch_shape<MODE, GROUPED, 2, 8, 2>(p, out_type, tiles, stream);
-  }
   if constexpr (GROUPED == kDense) {
+    if (shape == k128x256) return launch_shape<MODE, GROUPED, 2, 8, 2>(p, out_type, tiles, stream);
     if (shape == k128x128) return launch_shape<MODE, GROUPED, 2, 4, 2>(p, out_type, tiles, stream);
   }
   if constexpr (GROUPED != kGroupedK) {
@@ -1295,9 +1294,8 @@ static int launch_grouped(GemmParams p, int out_type, hipStream_t stream) {
   const GroupedTiles tiles = pick_grouped(p.M, p.N, p.experts);
   if (tiles == kSmallestTiles) return launch<MODE, kGroupedRows>(p, out_type, k64x64, stream);
   if (tiles == kLowestTiles) return launch<MODE, kGroupedRows>(p, out_type, k64x128, stream);
-  if (tiles == kLowTiles) return launch<MODE, kGroupedRows>(p, out_type, k128x256, stream);
   if (tiles == kHighTiles) return launch<MODE, kGroupedRows>(p, out_type, k256x256, stream);
-  p.choose_cus = persistent_grid((int64_t)1 << 40);
+  p.choose_cus = tiles == kLowTiles ? -128 : persistent_grid((int64_t)1 << 40);
   dim3 grid((unsigned)persistent_grid(most_grouped_tiles(p.M, p.N, p.experts, k64x128))), block(512);
   const bool sa4 = p.sa_sm == 1;
   if (out_type == HPFP8_OUT_F32) {
