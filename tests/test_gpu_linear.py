@@ -951,7 +951,7 @@ def test_linear_training_step_replays_from_a_captured_graph(gpu, recipe):
 
 @pytest.mark.parametrize("recipe", ["blockwise", "per_tensor"])
 @pytest.mark.parametrize("way", ["mode", "vmap", "grad", "forward_ad", "trace", "batched_backward", "create_graph", "checkpoint", "reentrant",
-                                 "dispatching_grad", "sparse_grad", "detect_anomaly"])
+                                 "dispatching_grad", "sparse_grad", "detect_anomaly", "in_place", "in_place_3d", "twice", "retained", "other_stream", "hooks"])
 def test_what_else_torch_does_with_a_step_has_the_python_functions_outcome(gpu, recipe, way, monkeypatch):
     """Modes, transforms, traces and tensors of other kinds around a linear's forward or backward: values and errors are those that the
     Python autograd function gives by itself."""
@@ -1005,6 +1005,22 @@ def test_what_else_torch_does_with_a_step_has_the_python_functions_outcome(gpu, 
             return torch.autograd.grad(y, (x, w), Dispatching(go))
         if way == "sparse_grad":
             return torch.autograd.grad(y, (x, w), go.to_sparse())
+        if way.startswith("in_place"):
+            y = f(x.view(2, 128, 256) if way == "in_place_3d" else x, w)
+            y += 1
+            return (y, *torch.autograd.grad(y, (x, w), go.view(y.shape)))
+        if way in ("twice", "retained"):
+            torch.autograd.grad(y, (x, w), go, retain_graph=way == "retained")
+        if way == "other_stream":
+            side = torch.cuda.Stream()
+            side.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(side):
+                y = f(x, w)
+            torch.cuda.current_stream().wait_stream(side)
+            y.record_stream(torch.cuda.current_stream())
+        if way == "hooks":
+            y.register_hook(lambda g: g * 2)
+            y.grad_fn.register_hook(lambda grads_in, grads_out: tuple(None if g is None else g * 2 for g in grads_in))
         if way == "detect_anomaly":
             with torch.autograd.detect_anomaly(check_nan=True):
                 return torch.autograd.grad(y, (x, w), go)
@@ -1014,7 +1030,7 @@ def test_what_else_torch_does_with_a_step_has_the_python_functions_outcome(gpu, 
         try:
             r = step()
         except Exception as e:
-            return type(e), str(e).split("\n")[0]
+            return type(e), str(e).split("\n")[0].split(" is a view")[-1]       # (that message names the node, before these words)
         return list(r) if isinstance(r, (tuple, list)) else [r]
 
     def _leaf_grads(y, leaves, go):
