@@ -19,10 +19,12 @@
 //     for bit; pick_shape has the rule and the figures.  There a SIMD has one wave that multiplies, which waits whenever a
 //     transfer it issues finds the memory path occupied (78 clocks per transfer while the first k-blocks arrive, 21 later), so
 //     four more waves do the transfers, 3, 4, 6 and 8 k-blocks at a time in LDS, the scales with them.  us, transfers by the
-//     multiplying waves with two buffers of a / by waves of their own: 1000 x 7168 x 7168 62 / 54, 1531 x 2048 x 7168 41 / 31,
-//     500 x 7168 x 16384 106 / 75, by rows 1024 x 1024 x 2048 16.7 / 10.3.  What is left there is what a k-block's transfers
-//     take by themselves (0.54 us for 48 KB, 0.39 for 32 KB, with every compute unit at it) and a first microsecond or three in
-//     which code and the first tiles arrive through cold caches.
+//     multiplying waves with two buffers of a / by waves of their own: 1000 x 7168 x 7168 62 / 54, 1531 x 2048 x 7168 41 / 33,
+//     500 x 7168 x 16384 106 / 75, by rows 1024 x 1024 x 2048 16.7 / 11.0.  A k-block of one round of these tiles over 7168
+//     columns takes 0.83, 0.60, 0.44 and 0.31 us with a weight from HBM (0.76, 0.47, 0.30, 0.22 with one that stays in the
+//     caches), of 128 x 256, 128 x 128, 64 x 128 and 64 x 64; its transfers by themselves 0.54 and 0.39 in the first two.  With
+//     power-of-two scales, without promotion, it takes as long from HBM (0.84, 0.59, 0.44, 0.31), so what multiplies is not what
+//     is waited for there.  A launch's first microsecond or three are code and first tiles arriving through cold caches.
 //   * The grid is persistent: one workgroup per CU walks a list of tiles, and the rounds of
 //     consecutive tiles follow each other without a gap.  Each XCD (own L2) owns a contiguous run
 //     of tile numbers.

@@ -681,9 +681,9 @@ def gemm_blockwise_swiglu_quantize(a: torch.Tensor, sa: torch.Tensor, b: torch.T
     s = torch.empty_like(s_inv) if want_scale else None
     # (a weight that spans 2 GiB or more is left to the fused call, which refuses it at every row count)
     if 0 < m <= _lib.load().hpfp8_gemm_few_rows(k) and n * _ld(b) < 0x7FFFF000:
-        # A decode step: the GEMM is bound by reading the weight, which its few-rows form does at twice the rate of the
-        # tiles the epilogue belongs to; gate | up is a few megabytes (37 rows of a [36864, 7168] weight: 86 us
-        # for the epilogue form, 42 + 5 us for the two launches, the same bits).
+        # A decode step: the GEMM is bound by reading the weight, which its few-rows form does faster than the tiles the
+        # epilogue belongs to; gate | up is a few megabytes (weight [36864, 7168], epilogue form / the two launches, the same bits:
+        # 37 rows 61 / 48 us, 64 rows 62 / 50).
         h = gemm_blockwise(a, sa, b, sb, pow2_scales=pow2_scales)
         if fast:
             _lib.call("hpfp8_swiglu_quantize_1x128_fast_bf16", _ptr(h), m, inter, n, 1, int(pow2_out), _ptr(q), _ptr(s), _ptr(s_inv),

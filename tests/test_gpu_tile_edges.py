@@ -393,8 +393,8 @@ def test_grouped_tiles_are_exact_on_integer_inputs(gpu, counts, n, k):
                                             (1024, 4, 16384)])
 @pytest.mark.parametrize("spread", ["even", "zipf", "half", "two", "one", "none"])
 def test_grouped_gemm_leaves_the_tile_height_to_the_device(gpu, rows, experts, n, spread):
-    """Row counts at which the host cannot know which tile height is better and both kernels are launched (and the first
-    beyond them, and some at which it knows): every row is computed, by one of them, with the bits of either."""
+    """Row counts at which the host cannot know which tile is better and the kernel chooses (and some at which it knows): every row is
+    computed, with the bits of 256 x 256 tiles."""
     from hpfp8 import _lib, ops
     k = 256
     counts = {"even": [rows // experts] * experts, "zipf": [int(rows / 4 / (i + 1)) for i in range(experts)],
