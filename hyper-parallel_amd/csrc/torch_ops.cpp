@@ -432,14 +432,14 @@ struct LinearNode : torch::autograd::Function<LinearNode> {
     if (go.scalar_type() != at::kBFloat16) go = go.to(at::kBFloat16);
     go = go.contiguous();
     const int64_t m = go.size(0), mp = rows_up(m), out = go.size(1), in = shape.back();
-    bool plain = go.is_cuda() && go.layout() == at::kStrided;
+    bool as_made = go.is_cuda() && go.layout() == at::kStrided;
     if (per_tensor)
-      plain = plain && codes_again(xt, go, in, mp) && codes_again(w, go, w_transposed ? in : out, w_transposed ? out : in) &&
-              sxt.numel() == 1 && floats_again(sxt, go, sxt.sizes()) && sw.numel() == 1 && floats_again(sw, go, sw.sizes());
+      as_made = as_made && codes_again(xt, go, in, mp) && codes_again(w, go, w_transposed ? in : out, w_transposed ? out : in) &&
+                sxt.numel() == 1 && floats_again(sxt, go, sxt.sizes()) && sw.numel() == 1 && floats_again(sw, go, sw.sizes());
     else
-      plain = plain && codes_again(xt, go, in, mp) && codes_again(w, go, in, out) && floats_again(sxt, go, {in, mp / kBlock}) &&
-              floats_again(sw, go, {out / kBlock, in / kBlock});
-    if (!plain) return in_python(grads[0], saved, shape, flags);
+      as_made = as_made && codes_again(xt, go, in, mp) && codes_again(w, go, in, out) && floats_again(sxt, go, {in, mp / kBlock}) &&
+                floats_again(sw, go, {out / kBlock, in / kBlock});
+    if (!as_made) return in_python(grads[0], saved, shape, flags);
     const c10::hip::HIPStream current = c10::hip::getCurrentHIPStream(go.get_device());
     void* const stream = current.stream();
     Call call;
