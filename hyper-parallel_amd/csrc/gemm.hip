@@ -922,8 +922,12 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
     for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[NS - 1][j][r] = __builtin_fmaf(part_c[j][r], s_old[j], acc[NS - 1][j][r]);
+    // (the next tile's first round adds these zeros times the scales kept: also where those are not finite)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) part_c[j] = zero;
+    for (int j = 0; j < 4; ++j) {
+      part_c[j] = zero;
+      s_old[j] = 0.f;
+    }
   }
   // The wave's 64 x 128 results go out 16 rows at a time (pass j: rows 4 s + j, s = 0..15, of the wave's
   // 64, the a tile's rows being permuted in LDS) through its own 4 KB slice of the b buffer

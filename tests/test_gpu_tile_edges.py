@@ -631,3 +631,24 @@ def test_grouped_kernel_that_chooses_its_tile_has_the_bits_of_one_that_does_not(
             _lib.load().hpfp8_debug_set_small_gemm(0)
     for one, other in zip(got[0], got[1]):
         assert torch.equal(one, other)
+
+
+@pytest.mark.parametrize("mode,m,n", [(1, 2304, 8704), (2, 640, 2048), (3, 1152, 8704), (4, 1152, 4352), (5, 640, 4352)])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_scales_that_are_not_finite_stay_with_their_tile(gpu, mode, m, n, value):
+    """Several tiles per compute unit with every tile shape: a NaN or an infinity among the scales of a tile's last k-block makes its own
+    rows (columns) NaN or infinite, and none of the tile that the same waves compute next."""
+    from hpfp8 import _lib, ops
+    k = 256
+    x, w = _normal((m, k), 1, gpu), _normal((n, k), 2, gpu)
+    a, sa = ops.quantize_1x128(x, kmajor=True)
+    bad = torch.tensor([3, 21, 40, 63], device=gpu)
+    sa[bad, -1] = value
+    _lib.load().hpfp8_debug_set_small_gemm(mode)
+    try:
+        for b, sb, gran in ((*ops.quantize_128x128(w), 128), (*ops.quantize_1x128(w, kmajor=True), 1)):
+            c = ops.gemm_blockwise(a, sa, b, sb, sb_gran=gran)
+            assert torch.equal((~c.isfinite()).any(1).nonzero().flatten(), bad)
+            assert not bool(c[bad].isfinite().any())
+    finally:
+        _lib.load().hpfp8_debug_set_small_gemm(0)
