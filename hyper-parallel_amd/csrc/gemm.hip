@@ -475,9 +475,11 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
   int sb_soff = 0;             // block form: byte offset of the b tile's scale row
   const int sa_kstep = (int)p.sa_sk * 4, sb_kstep = (int)p.sb_sk * 4;
   auto scale_target = [&](const TileInfo& ti) {
+    int lane_s = lane;
+    asm volatile("" : "+v"(lane_s));    // (keeps what the offsets are made of out of the registers held through the rounds)
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int r = ti.row0 + wm * 64 + l16 * 4 + j;
+      const int r = ti.row0 + wm * 64 + (lane_s & 15) * 4 + j;
       // (SA4 does not clamp: words past the end of the array read as zero, and rows past M are never stored)
       sa_voff[j] = SA4 ? (uint32_t)r * 4u : (uint32_t)(r < p.M ? r : p.M - 1) * (uint32_t)((int)p.sa_sm * 4);
     }
