@@ -52,7 +52,7 @@ constexpr int BM = 256, BN = 256;
 // LDS: two buffers for the a tile, then kBStages buffers for the b tile.  The b operand is the one
 // that streams from HBM (each weight panel is used by one XCD only), so where LDS allows it gets a
 // third buffer and its transfers run two k-blocks ahead; a's re-reads come from the Infinity Cache.
-__host__ __device__ constexpr int b_stages(int mode) { return (mode == 2 || mode == 4) /* per-row b scales: LDS also holds them */ ? 2 : 3; }
+__host__ __device__ constexpr int b_stages(int mode) { return mode == 4 /* LDS also holds per-row b scales */ ? 2 : 3; }
 constexpr int kRectTiles = 32;              // tiles of the rectangle one XCD (32 CUs) works on at a time
 
 // kScalePow2: scales laid out as for kScaleBlock but every one a power of two; the matrix instruction
@@ -248,8 +248,28 @@ constexpr int kScaleSlot = 2048;
 // reads, those to other buffers included: the transfers' latency would be paid in every round.)
 __host__ __device__ constexpr int tile_lds(int mode, int wm, int tn) {
   const int stages = tile_stages(mode, wm, tn);
-  const int scales = fetchers(wm) ? (mode == kScaleTensor ? 0 : (stages + 1) * kScaleSlot) : (row_scales(mode) ? 3 * 256 * 4 : 0);
+  const int scales = fetchers(wm) ? (mode == kScaleTensor ? 0 : (stages + 1) * kScaleSlot) : (mode == kScalePow2Row ? 3 * 256 * 4 : 0);
   return (fetchers(wm) ? stages : 2) * 64 * wm * BK + stages * tn * BK + scales;
+}
+
+// Per-row scales on both operands: the four products sb * sa that a lane needs for one 16 x 16 subtile, in the layout of the
+// subtile's sums (rows of b 4 g + r, r = 0..3, and row of a l16, for lane 16 g + l16), as the outer products of one small matrix
+// instruction: 16 blocks of 4 x 4, block l / 4 of lane l.  Its b rows are those of block `sub` of the four blocks that share
+// g, so one register holds the b scales of four subtiles: lane l that of row 16 ((l / 4) % 4) + 4 (l / 16) + l % 4.
+// A promotion is then one FMA per element as with a scale per block of b, where a multiplication by the b scale ahead of it made
+// this form bound by instruction issue (a matrix instruction takes about 15 of a SIMD's issue cycles, a vector instruction 4: 47
+// per group of one and eight against 32 of matrix pipe).  The four of a subtile are issued back to back: 43 cycles a group, where
+// one in front of each large matrix instruction makes it 51.  us before / so: 7168 x 16384 x 4096 466 / 437 (one by one 469),
+// 36864 x 7168 x 4096 1064 / 997, 2048 x 7168 x 1536 28.2 / 27.6, 1400 x 3072 x 4096 33.1 / 29.5, 1024 x 1024 x 4096 13.5 / 12.4.
+__device__ __forceinline__ int scale_row(int lane) { return ((lane >> 2) & 3) * 16 + (lane >> 4) * 4 + (lane & 3); }
+__device__ __forceinline__ v4f scale_products(float sb, float sa, int sub) {
+  const v4f zero = {0.f, 0.f, 0.f, 0.f};
+  switch (sub) {       // (a literal in the instruction; sub is known when the loops are unrolled)
+    case 0: return __builtin_amdgcn_mfma_f32_4x4x1f32(sb, sa, zero, 2, 0, 0);
+    case 1: return __builtin_amdgcn_mfma_f32_4x4x1f32(sb, sa, zero, 2, 1, 0);
+    case 2: return __builtin_amdgcn_mfma_f32_4x4x1f32(sb, sa, zero, 2, 2, 0);
+    default: return __builtin_amdgcn_mfma_f32_4x4x1f32(sb, sa, zero, 2, 3, 0);
+  }
 }
 
 // group: grouped by rows, the first 64 experts with their ends; then those among which tiles are looked up (tile numbers are
@@ -279,12 +299,14 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
   static_assert(!kFetchers || GROUPED != kGroupedK, "the fetching waves count k-blocks from 0");
   constexpr int kBStages = tile_stages(MODE, WM, TN);
   constexpr int kAStages = kFetchers ? kBStages : 2;
-  constexpr bool kRowScales = row_scales(MODE);                             // per-row b scales, staged in LDS
+  constexpr bool kRowScales = row_scales(MODE);                             // per-row b scales
+  constexpr bool kStagedScales = MODE == kScalePow2Row && !kFetchers;       // staged in LDS by the multiplying waves
+  constexpr int kScaleRegs = (NS + 3) / 4;                                  // kScaleRow: registers of them, four subtiles each
   constexpr bool kPromote = MODE == kScaleBlock || MODE == kScaleRow;       // partial sums scaled by FMAs
   constexpr bool kHwScale = MODE == kScalePow2 || MODE == kScalePow2Row;    // scales applied by the MFMA
   constexpr int kBAhead = kBStages - 1;     // k-blocks between issuing a b transfer and using it
   constexpr int kScaleOps = MODE == kScaleTensor ? 0 : 2, kScaleSlots = kBStages + 1;
-  // per-row scales of the b operand for one k-block (wgrad form), three stages of 256 floats: the
+  // per-row scales of the b operand for one k-block (wgrad form, powers of two), three stages of 256 floats: the
   // stage of k-block kb+1 is filled while slower waves may still read that of kb-1
   uint8_t* const scale_lds = lds + kAStages * kATile + kBStages * kBTile;
   float* const sb_lds = reinterpret_cast<float*>(scale_lds);
@@ -346,7 +368,7 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
       const int t = t_first + k * t_step;
       int tm, tn;
       if (GROUPED == kGroupedK) {
-        const int i = t / p.tiles;
+        const int i = quotient(t, p.tiles);
         expert = p.layout[4 * p.experts + i];
         kb0 = p.layout[4 * expert + 2];
         kbn = p.layout[4 * expert + 3];
@@ -425,12 +447,12 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
     const int chunk = (lane & 7) ^ row_swizzle(r);
     b_off[i] = (uint32_t)(EPI && r >= 128 ? r - 128 + p.inter : r) * (uint32_t)p.ldb + chunk * 16;
   }
-  // wgrad form: the 256 per-row scales of the b tile for one k-block are one more 1 KB transfer
+  // kStagedScales: the 256 per-row scales of the b tile for one k-block are one more 1 KB transfer
   // (wave 0), possible because that scale array is k-block-major (unit stride over rows).
   const __amdgpu_buffer_rsrc_t rsrc_sb = __builtin_amdgcn_make_buffer_rsrc(
       (void*)p.sb, 0, kRowScales ? (int)((((int64_t)kblocks - 1) * p.sb_sk + N) * 4) : 0, 0x00020000);
   auto issue_sb_load = [&](const TileInfo& ti, int kb, int stage) {      // kb counted inside the tile's own contraction
-    if (kRowScales && wave == 0)
+    if (kStagedScales && wave == 0)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_sb, (lds_ptr_t)(sb_lds + stage * 256), 16,
                                                (uint32_t)(ti.n0 + lane * 4) * 4u,
                                                (int)(((GROUPED == kGroupedK ? ti.kb0 : 0) + kb) * p.sb_sk * 4), 0, 0);
@@ -458,9 +480,13 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
   // ---- fragment addressing
   const int wn = wave % WN, wm = wave / WN;
   const int l16 = lane & 15, g = lane >> 4;
-  const int pc0 = (2 * g) ^ row_swizzle(l16);
-  const int a_frag_off = (wm * 64 + l16) * BK;               // + j * 16 rows
-  const int b_frag_off = (wn * WC + l16) * BK;               // + i * 16 rows, inside a b buffer
+  // A lane's two chunks of a fragment lie equally far behind the fragment's first row in both operands.  256 x 256 tiles keep these
+  // two offsets (opaque: taken apart again, the parts would take two registers more) and the rest of an address is scalar.
+  const int l16_row = l16 * BK;
+  int frag_lo = (kFetchers ? 0 : l16_row) + ((2 * g) ^ row_swizzle(l16)) * 16, frag_hi = frag_lo ^ 16;
+  if (!kFetchers) asm volatile("" : "+v"(frag_lo), "+v"(frag_hi));
+  const int a_frag = wm * 64 * BK + (kFetchers ? l16_row : 0);                           // + j * 16 rows
+  const int b_frag = wn * WC * BK + (kFetchers ? l16_row : 0);                           // + i * 16 rows, inside a b buffer
 
   // ---- scales.  Raw values for one k-block are loaded at the top of the round before it and only
   // combined (sa * sb) at its end, so nothing waits on global memory in between.
@@ -473,6 +499,7 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
   const __amdgpu_buffer_rsrc_t rsrc_sbb = __builtin_amdgcn_make_buffer_rsrc((void*)p.sb, 0, p.sb_bytes, 0x00020000);
   uint32_t sa_voff[4];         // byte offset of this lane's four rows in sa (SA4: [0] covers all four)
   int sb_soff = 0;             // block form: byte offset of the b tile's scale row
+  uint32_t sb_voff = 0;        // kScaleRow: byte offset of this lane's column of the b tile in sb
   const int sa_kstep = (int)p.sa_sk * 4, sb_kstep = (int)p.sb_sk * 4;
   auto scale_target = [&](const TileInfo& ti) {
     int lane_s = lane;
@@ -483,11 +510,17 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
       // (SA4 does not clamp: words past the end of the array read as zero, and rows past M are never stored)
       sa_voff[j] = SA4 ? (uint32_t)r * 4u : (uint32_t)(r < p.M ? r : p.M - 1) * (uint32_t)((int)p.sa_sm * 4);
     }
+    if (MODE == kScaleRow) sb_voff = (uint32_t)(ti.n0 + wn * WC + scale_row(lane_s)) * 4u;      // (past N: columns that are not stored)
     int nblk_idx = EPI ? (ti.n0 >> 8) + wn * (p.inter >> 7) : (ti.n0 + wn * WC) >> 7;
     if (nblk_idx > (N >> 7) - 1) nblk_idx = (N >> 7) - 1;
     sb_soff = ((GROUPED == kGroupedRows ? ti.expert * (int)p.sb_se : 0) + nblk_idx * (int)p.sb_sn) * 4;
   };
-  auto load_scales = [&](int kb, float raw[5]) {
+  auto load_scales = [&](int kb, float raw[6]) {
+    if (MODE == kScaleRow) {
+#pragma unroll
+      for (int h = 0; h < kScaleRegs; ++h)
+        raw[4 + h] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc_sb, sb_voff + h * 256, kb * sb_kstep, 0));
+    }
     if (MODE == kScaleBlock || MODE == kScalePow2)
       raw[4] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc_sbb, 0, sb_soff + kb * sb_kstep, 0));
     if (MODE != kScaleTensor) {
@@ -579,9 +612,14 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
       return;
     }
   }
-  auto read_scales = [&](int slot, float raw[5]) {      // (kFetchers)
+  auto read_scales = [&](int slot, float raw[6]) {      // (kFetchers)
     if (MODE == kScaleTensor) return;
     const uint8_t* const src = scale_lds + slot * kScaleSlot + (wm * 2 + wn * 2 / WN) * 256;
+    if (MODE == kScaleRow) {
+#pragma unroll
+      for (int h = 0; h < kScaleRegs; ++h)
+        raw[4 + h] = *reinterpret_cast<const float*>(scale_lds + slot * kScaleSlot + (wn * WC + h * 64 + scale_row(lane)) * 4);
+    }
     const v4f four = *reinterpret_cast<const v4f*>(src + 1024 + l16 * 16);
 #pragma unroll
     for (int j = 0; j < 4; ++j) raw[j] = four[j];
@@ -590,7 +628,12 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
   // kScalePow2: the exponent fields of the scales of the current k-block, which are their E8M0 codes:
   // e_a[j] for the activation rows j * 16 + l16 of this lane, e_b for the weight block
   int e_a[4] = {127, 127, 127, 127}, e_b = 127;
-  auto combine_scales = [&](const float raw[5], float s[4]) {
+  float sb_cur[2] = {1.f, 1.f};       // kScaleRow
+  auto combine_scales = [&](const float raw[6], float s[4]) {
+    if (MODE == kScaleRow) {
+#pragma unroll
+      for (int h = 0; h < kScaleRegs; ++h) sb_cur[h] = raw[4 + h];
+    }
 #pragma unroll
     for (int j = 0; j < 4; ++j) s[j] = MODE == kScaleBlock ? raw[j] * raw[4] : raw[j];
     if (kHwScale) {
@@ -637,7 +680,7 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
 
   // ---- prologue: k-block 0 of both operands, k-block 1 of b where it has three buffers, and the
   // first half of k-block 1 of a (and of b where it has two buffers)
-  float s_cur[4] = {1.f, 1.f, 1.f, 1.f}, s_raw[5] = {1.f, 1.f, 1.f, 1.f, 1.f};
+  float s_cur[4] = {1.f, 1.f, 1.f, 1.f}, s_raw[6] = {1.f, 1.f, 1.f, 1.f, 1.f, 1.f};
   // (k-block numbers passed to transfers and scale loads are absolute: grouped along the contraction, a tile's
   // own k-blocks start at its expert's first block kb0; otherwise kb0 is 0)
   auto kfirst = [](const TileInfo& ti) { return GROUPED == kGroupedK ? ti.kb0 : 0; };
@@ -696,17 +739,17 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
   // before / so: block 400 x 1024 x 8192 21.7 / 19.8, 256 x 3072 x 3072 11.6 / 11.1, 1531 x 2048 x 7168 33 / 31).
   constexpr bool kTwoX = kFetchers && NS <= 4;
   v8i xf[4], xg[4], wf_n0, wf_n1;
-  wf_n0 = frag_read(b_lds + b_frag_off, pc0);
+  wf_n0 = frag_read(b_lds + b_frag, frag_lo, frag_hi);
 #pragma unroll
-  for (int j = 0; j < 4; ++j) xf[j] = frag_read(lds + a_frag_off + j * 16 * BK, pc0);
-  wf_n1 = frag_read(b_lds + b_frag_off + 16 * BK, pc0);
+  for (int j = 0; j < 4; ++j) xf[j] = frag_read(lds + a_frag + j * 16 * BK, frag_lo, frag_hi);
+  wf_n1 = frag_read(b_lds + b_frag + 16 * BK, frag_lo, frag_hi);
 
-  constexpr bool kCarry = MODE == kScaleBlock;   // promote subtile 7 inside the next round's first group
   v4f part_c[4] = {zero, zero, zero, zero};
   float s_old[4] = {0.f, 0.f, 0.f, 0.f};
+  v4f s_of[4] = {zero, zero, zero, zero};          // kScaleRow: products of scales for the subtile that is promoted
   int stage = 0;                       // a buffer holding the current k-block
   int bbuf = 0;                        // b buffer holding the current k-block
-  int sbuf = 0;                        // scale stage (wgrad form) holding the current k-block
+  int sbuf = 0;                        // scale stage (kStagedScales) or slot (kFetchers) holding the current k-block
   // transfer targets (ordinal in the tile list) and their buffer resources
   int ord_1 = 0, ord_2 = 0;
   TileInfo tile_1 = T0;
@@ -762,7 +805,7 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
     // rounds ahead at 2..5; after the barrier the first half of the a tile after next, into the
     // buffer whose fragments every wave has just left behind.  One transfer per subtile: a burst
     // would queue up in the texture path ahead of the LDS reads.
-    // With two b buffers (wgrad form) the b tile has to land within one round like the a tile, so
+    // With two b buffers (kStagedScales) the b tile has to land within one round like the a tile, so
     // both go out in the four subtiles that follow the barrier, one transfer of each per subtile.
     auto issue_slot = [&](int i) {
       if (kFetchers) return;
@@ -797,8 +840,8 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
     };
     // weight fragment of subtile i + 2 (the first two of the next round once past the barrier)
     auto read_ahead = [&](int i) {
-      return i + 2 < NS ? frag_read(bcur + b_frag_off + (i + 2) * 16 * BK, pc0)
-                       : frag_read(bnxt + b_frag_off + (i + 2 - NS) * 16 * BK, pc0);
+      return i + 2 < NS ? frag_read(bcur + b_frag + (i + 2) * 16 * BK, frag_lo, frag_hi)
+                       : frag_read(bnxt + b_frag + (i + 2 - NS) * 16 * BK, frag_lo, frag_hi);
     };
     if (kPromote) {
       // Software pipeline over the 8 n-subtiles: the matrix instructions of subtile i are issued
@@ -810,11 +853,6 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
       wf[1] = wf_n1;
 #pragma unroll
       for (int j = 0; j < 4; ++j) part[1][j] = part_c[j];
-      // wgrad form: the four per-row b scales of subtile i for this lane's four n
-      const float* sb_row = sb_lds + sbuf * kSbSlot + wn * WC + g * 4;
-      v4f sbv[2];
-      if (MODE == kScaleRow) sbv[0] = *reinterpret_cast<const v4f*>(sb_row);
-      if (MODE == kScaleRow && !kFetchers) issue_sb_load(tile_1, kb1_rel, snext);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int i = 0; i < NS; ++i) {
@@ -823,39 +861,32 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
         if (kFetchers && i == NS - 2) read_scales(snext, s_raw);
         if (kTwoX && i == NS - 2) {
 #pragma unroll
-          for (int j = 0; j < 4; ++j) xn[j] = frag_read(anxt + a_frag_off + j * 16 * BK, pc0);
+          for (int j = 0; j < 4; ++j) xn[j] = frag_read(anxt + a_frag + j * 16 * BK, frag_lo, frag_hi);
         }
-        if (MODE == kScaleRow && i > 0) sbv[i & 1] = *reinterpret_cast<const v4f*>(sb_row + i * 16);   // used by the FMAs of group i+1
         issue_slot(i);
         __builtin_amdgcn_sched_barrier(0);
+        if (MODE == kScaleRow && i > 0) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) s_of[j] = scale_products(sb_cur[(i - 1) / 4], s_cur[j], (i - 1) % 4);
+          __builtin_amdgcn_sched_barrier(0);
+        }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           part[i & 1][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[i % 3], xf[j], zero, 0, 0, 0, 0, 0, 0);
-          if (i > 0 || kCarry) {
-            const int ip = (i + NS - 1) % NS;     // subtile being promoted; for i = 0 the last one of the previous round
+          if (MODE == kScaleRow) __builtin_amdgcn_sched_barrier(0);
+          const int ip = (i + NS - 1) % NS;     // subtile being promoted; for i = 0 the last one of the previous round
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              float pv = part[(i - 1) & 1][j][r];
-              if (MODE == kScaleRow) pv *= sbv[(i - 1) & 1][r];
-              acc[ip][j][r] = __builtin_fmaf(pv, i == 0 ? s_old[j] : s_cur[j], acc[ip][j][r]);
-            }
-          }
-          if (!kTwoX && i == NS - 1) xn[j] = frag_read(anxt + a_frag_off + j * 16 * BK, pc0);
+          for (int r = 0; r < 4; ++r)
+            acc[ip][j][r] = __builtin_fmaf(part[(i - 1) & 1][j][r], MODE == kScaleRow ? s_of[j][r] : (i == 0 ? s_old[j] : s_cur[j]),
+                                           acc[ip][j][r]);
+          if (!kTwoX && i == NS - 1) xn[j] = frag_read(anxt + a_frag + j * 16 * BK, frag_lo, frag_hi);
           __builtin_amdgcn_sched_barrier(0);   // keep this (MFMA, FMAs) group together, in this order
         }
       }
-      if (kCarry) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) part_c[j] = part[1][j];
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            float pv = part[1][j][r];
-            if (MODE == kScaleRow) pv *= sbv[1][r];
-            acc[NS - 1][j][r] = __builtin_fmaf(pv, s_cur[j], acc[NS - 1][j][r]);
-          }
+      for (int j = 0; j < 4; ++j) {
+        part_c[j] = part[1][j];
+        if (MODE == kScaleRow) s_of[j] = scale_products(sb_cur[kScaleRegs - 1], s_cur[j], (NS - 1) % 4);
       }
       wf_n0 = wf[NS % 3];
       wf_n1 = wf[(NS + 1) % 3];
@@ -864,10 +895,10 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
       wf[0] = wf_n0;
       wf[1] = wf_n1;
       // per-row b scales: this lane's row of subtile i is row i * 16 + l16 of the wave's 128
-      const float* sb_lane = sb_lds + sbuf * kSbSlot + wn * WC + l16;
+      const float* sb_own = sb_lds + sbuf * kSbSlot + wn * WC + l16;
       int e_bi[2] = {127, 127};
-      if (MODE == kScalePow2Row) e_bi[0] = (int)(__builtin_bit_cast(uint32_t, sb_lane[0]) >> 23);
-      if (MODE == kScalePow2Row && !kFetchers) issue_sb_load(tile_1, kb1_rel, snext);
+      if (MODE == kScalePow2Row) e_bi[0] = (int)(__builtin_bit_cast(uint32_t, sb_own[0]) >> 23);
+      if (kStagedScales) issue_sb_load(tile_1, kb1_rel, snext);
 #pragma unroll
       for (int i = 0; i < NS; ++i) {
         if (i == NS - 2) round_sync();
@@ -875,9 +906,9 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
         if (kFetchers && i == NS - 2) read_scales(snext, s_raw);
         if (kTwoX && i == NS - 2) {
 #pragma unroll
-          for (int j = 0; j < 4; ++j) xn[j] = frag_read(anxt + a_frag_off + j * 16 * BK, pc0);
+          for (int j = 0; j < 4; ++j) xn[j] = frag_read(anxt + a_frag + j * 16 * BK, frag_lo, frag_hi);
         }
-        if (MODE == kScalePow2Row && i < NS - 1) e_bi[(i + 1) & 1] = (int)(__builtin_bit_cast(uint32_t, sb_lane[(i + 1) * 16]) >> 23);
+        if (MODE == kScalePow2Row && i < NS - 1) e_bi[(i + 1) & 1] = (int)(__builtin_bit_cast(uint32_t, sb_own[(i + 1) * 16]) >> 23);
         issue_slot(i);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -889,7 +920,7 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
                                                                         MODE == kScalePow2 ? e_b : e_bi[i & 1], 0, e_a[j]);
           else
             acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[i % 3], xf[j], acc[i][j], 0, 0, 0, 0, 0, 0);
-          if (!kTwoX && i == NS - 1) xn[j] = frag_read(anxt + a_frag_off + j * 16 * BK, pc0);
+          if (!kTwoX && i == NS - 1) xn[j] = frag_read(anxt + a_frag + j * 16 * BK, frag_lo, frag_hi);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -919,16 +950,20 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
     for (int kb = 0; kb < kbn0; ++kb) round(kb, xf, xf);
   }
   // ---- the tile is complete: last promotion, then its stores
-  if (kCarry) {
+  if (kPromote) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 4; ++j) {
+      v4f s = {s_old[j], s_old[j], s_old[j], s_old[j]};
+      if (MODE == kScaleRow) s = s_of[j];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) acc[NS - 1][j][r] = __builtin_fmaf(part_c[j][r], s_old[j], acc[NS - 1][j][r]);
+      for (int r = 0; r < 4; ++r) acc[NS - 1][j][r] = __builtin_fmaf(part_c[j][r], s[r], acc[NS - 1][j][r]);
+    }
     // (the next tile's first round adds these zeros times the scales kept: also where those are not finite)
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       part_c[j] = zero;
       s_old[j] = 0.f;
+      s_of[j] = zero;
     }
   }
   // The wave's 64 x 128 results go out 16 rows at a time (pass j: rows 4 s + j, s = 0..15, of the wave's

@@ -23,14 +23,15 @@ __device__ __forceinline__ v4i lds_read16(const uint8_t* p) {
   return *reinterpret_cast<const v4i*>(p);
 }
 
-__device__ __forceinline__ v8i frag_read(const uint8_t* row_base, int pc0) {
-  v4i lo = lds_read16(row_base + pc0 * 16);
-  v4i hi = lds_read16(row_base + (pc0 ^ 1) * 16);
+__device__ __forceinline__ v8i frag_read(const uint8_t* first, int lo_off, int hi_off) {
+  v4i lo = lds_read16(first + lo_off);
+  v4i hi = lds_read16(first + hi_off);
   v8i r;
   r[0] = lo[0]; r[1] = lo[1]; r[2] = lo[2]; r[3] = lo[3];
   r[4] = hi[0]; r[5] = hi[1]; r[6] = hi[2]; r[7] = hi[3];
   return r;
 }
+__device__ __forceinline__ v8i frag_read(const uint8_t* row_base, int pc0) { return frag_read(row_base, pc0 * 16, (pc0 ^ 1) * 16); }
 
 // two floats -> two bf16 in one word (a low, b high): one v_cvt_pk_bf16_f32 (converted one by one, each
 // value costs a conversion, a shift and an or)

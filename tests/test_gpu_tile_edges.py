@@ -652,3 +652,27 @@ def test_scales_that_are_not_finite_stay_with_their_tile(gpu, mode, m, n, value)
             assert not bool(c[bad].isfinite().any())
     finally:
         _lib.load().hpfp8_debug_set_small_gemm(0)
+
+
+@pytest.mark.parametrize("mode,m,n", [(1, 300, 640), (2, 65, 256), (3, 129, 384), (4, 130, 384), (5, 65, 640), (1, 2305, 8704), (2, 1100, 1152)])
+@pytest.mark.parametrize("k", [128, 384])
+def test_per_row_scales_on_both_operands_are_those_of_their_rows_and_blocks(gpu, mode, m, n, k):
+    """Scales with full mantissas, another in every row and k-block, on integer codes: the sum of a k-block is an exact integer below 2^12, so
+    with one k-block c is that integer times the fp32 product of the two scales, rounded once; with more of them each adds at most
+    its own rounding, 2^-24 of the sum so far."""
+    from hpfp8 import _lib, ops
+    a, b, kb = _ints((m, k), 1, gpu), _ints((n, k), 2, gpu), k // 128
+    g = torch.Generator(device="cpu").manual_seed(3)
+    sa, sb = ((torch.rand((kb, r), generator=g) + 0.5).to(gpu).t() for r in (m, n))
+    part = torch.stack([a.double()[:, i * 128:(i + 1) * 128] @ b.double()[:, i * 128:(i + 1) * 128].t() for i in range(kb)])
+    scale = torch.stack([sa[:, i:i + 1] * sb[:, i] for i in range(kb)])
+    _lib.load().hpfp8_debug_set_small_gemm(mode)
+    try:
+        for s in (sa, sa.contiguous()):
+            c = ops.gemm_blockwise(a, s, b, sb, sb_gran=1, out_dtype=torch.float32)
+            if kb == 1:
+                assert torch.equal(c, part[0].float() * scale[0])
+            terms = part * scale.double()
+            assert bool(((c.double() - terms.sum(0)).abs() <= kb * 2.0 ** -23 * terms.abs().sum(0)).all())
+    finally:
+        _lib.load().hpfp8_debug_set_small_gemm(0)
