@@ -1278,6 +1278,11 @@ static int64_t few_rows(int64_t K) {        // the most rows that count as few
   return K >= kSkinnyMinK && g_small_gemm_mode.load(std::memory_order_relaxed) == 0 ? kSkinnyMaxRows : 0;
 }
 
+// Below this contraction a fused epilogue on tiles is still the better choice with few rows than the few-rows form and a launch
+// behind it: what those save on the GPU (weight [8192, 1024], 8 rows 11.6 -> 9.0 us; [36864, 512], 64 rows 9.9 -> 13.5) the second
+// call costs on the host (15 -> 25 us).
+constexpr int64_t kEpilogueMaxK = 2048;
+
 static bool try_skinny(const GemmParams& p, SkinnyMode mode, int out_type, hipStream_t stream, int& rc) {
   if (p.accumulate || p.M > few_rows(p.K)) return false;
   SkinnyParams q{};
@@ -1504,7 +1509,7 @@ int hpfp8_gemm_blockwise_swiglu_quantize(const void* a, int64_t lda, const float
 
 void hpfp8_debug_set_small_gemm(int mode) { g_small_gemm_mode.store(mode >= 1 && mode <= 5 ? mode : 0, std::memory_order_relaxed); }
 
-int64_t hpfp8_gemm_few_rows(int64_t K) { return few_rows(K); }
+int64_t hpfp8_gemm_few_rows(int64_t K) { return K >= kEpilogueMaxK ? few_rows(K) : 0; }
 
 int hpfp8_gemm_per_tensor(const void* a, int64_t lda, const float* sa_inv, const void* b, int64_t ldb,
                           const float* sb_inv, int64_t M, int64_t N, int64_t K, const void* bias, void* c,

@@ -27,9 +27,10 @@ struct SkinnyParams {
 
 constexpr int kSkinnyMaxRows = 64;        // four fragments of 16 rows; one row more takes tiles (64 rows of [7168, 16384]: 27 us here,
                                           // 64 us with the 64 x 128 tiles that 65 rows take)
-// Contractions from here on.  Measured, 16 rows of [4096, K] with tiles / here: K = 256 4.9 / 4.9 us, 512 5.6 / 5.3, 1024 7.2 /
-// 5.1, 1920 10.1 / 5.1; of [36864, 512] 10.3 / 6.4: below 512 there is nothing to gain, from 512 to here there would be.
-constexpr int kSkinnyMinK = 2048;
+// Contractions from here on.  Measured, us with tiles / here: 8 rows of [1024, 1024] 6.2 / 3.4, of [4096, 1536] 9.0 / 4.5, 24 rows of
+// [16384, 1920] 10.2 / 8.1, 64 rows of [36864, 512] 9.2 / 8.7; over 5 row counts up to 64, 6 widths from 1024 to 36864 and 4
+// contractions from 512 to 1920 a third less on average and nowhere more.  Shorter ones: 16 rows of [4096, 256] 4.9 / 4.9.
+constexpr int kSkinnyMinK = 512;
 
 int launch_skinny(const SkinnyParams& p, SkinnyMode mode, int cus, hipStream_t stream);
 

@@ -47,7 +47,7 @@ def _dequantized(q, s, rows, cols=128):
 
 
 @pytest.mark.parametrize("m", [1, 16, 17, 32, 33, 48, 49, 64, 65])
-@pytest.mark.parametrize("n,k", [(128, 128), (256, 640), (1152, 1152), (33024, 384), (384, 2048), (256, 2432), (33024, 2048)])
+@pytest.mark.parametrize("n,k", [(128, 128), (256, 640), (1152, 1152), (33024, 384), (384, 512), (1152, 896), (384, 2048), (256, 2432), (33024, 2048)])
 def test_gemm_with_few_rows_is_exact_on_integer_inputs(gpu, m, n, k):
     """Every row-fragment count of the few-rows GEMM and the first row count beyond it; contractions on both sides of the
     shortest it takes, k-blocks that divide into its stages and that do not; fewer runs of columns than compute units and
@@ -70,8 +70,9 @@ def test_gemm_with_few_rows_is_exact_on_integer_inputs(gpu, m, n, k):
 
 # (n, k) of the few-rows form: with the row counts below every number of fragments per workgroup (1, 2, 3, 4, 6 and 9 on 256
 # compute units) in one run and in several, last runs that are partly missing, stages of two, four and eight k-blocks that
-# divide the contraction and that do not
-FEW_ROWS_SHAPES = [(128, 2048), (1152, 2432), (8320, 2176), (12160, 2304), (16384, 2432), (24704, 2176), (36736, 2432), (38400, 2176)]
+# divide the contraction and that do not, or that are longer than it
+FEW_ROWS_SHAPES = [(128, 2048), (1152, 2432), (8320, 2176), (12160, 2304), (16384, 2432), (24704, 2176), (36736, 2432), (38400, 2176),
+                   (1152, 512), (8320, 640), (24704, 1024), (33024, 1920)]
 
 
 def _normal(shape, seed, gpu, std=1.0, outliers=False):
