@@ -134,6 +134,7 @@ struct TileInfo {
   int n0;              // first row of b / column of c
   int expert;
   int kb0, kbn;        // grouped along the contraction: first k-block of the tile's expert and how many (>= 1)
+  bool b_once;         // (fetching waves) no other tile reads these rows of b
 };
 
 // Position `d` k-blocks after k-block kb of the current tile (which has k0 k-blocks, the next one k1, every
@@ -157,6 +158,7 @@ __device__ __forceinline__ TileInfo pick_tile(int q, TileInfo t0, TileInfo t1, T
   r.expert = q == 2 ? t2.expert : (q == 1 ? t1.expert : t0.expert);
   r.kb0 = q == 2 ? t2.kb0 : (q == 1 ? t1.kb0 : t0.kb0);
   r.kbn = q == 2 ? t2.kbn : (q == 1 ? t1.kbn : t0.kbn);
+  r.b_once = false;      // (the fetching waves look their tiles up)
   return r;
 }
 
@@ -228,6 +230,11 @@ __device__ __forceinline__ int grouped_tile_rows(const ExpertChunk& c, const Gem
   const int64_t mid_cost = 50 * (int64_t)quotient(mid * tiles_n + cus - 1, cus);
   const int64_t high_cost = 83 * (int64_t)quotient(high * tiles_n + cus - 1, cus);
   return low_cost <= mid_cost && low_cost <= high_cost ? 64 : (mid_cost <= high_cost ? 128 : 256);
+}
+
+// one wave's transfer of 8 rows x 128 bytes to LDS, as data read once
+__device__ __forceinline__ void stream_1k(__amdgpu_buffer_rsrc_t rs, uint8_t* dst, uint32_t lane_off, int off) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)dst, 16, lane_off, off, 0, 2);
 }
 
 // WM, NS, WN: WM x WN waves multiply, each 64 rows x NS subtiles of 16 columns.  Tiles of 64 and of 128 rows have four more
@@ -363,7 +370,7 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
   if (my_tiles == 0) return;
   const int n_pad = tiles_n * TN;
   auto lookup = [&](int k, TileInfo& ti) {
-    int row0 = p.M, row_end = p.M, n0 = n_pad, expert = 0, kb0 = 0, kbn = GROUPED == kGroupedK ? 1 : kblocks;
+    int row0 = p.M, row_end = p.M, n0 = n_pad, expert = 0, kb0 = 0, kbn = GROUPED == kGroupedK ? 1 : kblocks, row_tiles = 0;
     if (k < my_tiles) {
       const int t = t_first + k * t_step;
       int tm, tn;
@@ -382,6 +389,7 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
         if (l < 64) {
           const int end = __builtin_amdgcn_readlane(group.end, l), prev = l ? __builtin_amdgcn_readlane(group.end, l - 1) : group.row;
           const int cnt = (end - prev + TM - 1) / TM;
+          row_tiles = cnt;
           rect_map(t - (__builtin_amdgcn_readlane(group.tile_end, l) - cnt * tiles_n), cnt, tiles_n, tm, tn);
           expert = group.first + l;
           row0 = prev + tm * TM;
@@ -390,7 +398,8 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
           n0 = tn * TN;
         }
       } else {
-        rect_map(t, (p.M + TM - 1) / TM, tiles_n, tm, tn);
+        row_tiles = (p.M + TM - 1) / TM;
+        rect_map(t, row_tiles, tiles_n, tm, tn);
         row0 = tm * TM;
         row_end = row0 + TM < p.M ? row0 + TM : p.M;
         n0 = tn * TN;
@@ -404,20 +413,23 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
     ti.expert = __builtin_amdgcn_readfirstlane(expert);
     ti.kb0 = __builtin_amdgcn_readfirstlane(kb0);
     ti.kbn = __builtin_amdgcn_readfirstlane(kbn);
+    ti.b_once = __builtin_amdgcn_readfirstlane(row_tiles) == 1;
   };
   // ---- global -> LDS tile DMA.  One wave instruction moves 8 rows x 128 B (lane i -> LDS slot
   // i); the lane picks the 16-byte global chunk whose swizzled home is its slot.  The buffer
   // resource of a transfer starts at the tile's first row and ends with the tensor, so lane
   // offsets do not depend on the tile and rows past the end of the tensor read as zero.
-  // (The resource runs on to the end of the tensor rather than to the end of the tile: transfers
-  // through a resource that only just covers the rows they touch were measured markedly slower.  Rows
-  // of a between the end of a ragged tile and the end of the tensor are read but never stored.)
+  // (The resource runs on to the end of the tensor rather than to the end of the tile: dense, transfers
+  // through a resource that only just covers the rows they touch were measured markedly slower.  Grouped by rows, where most of a
+  // tile may be rows of other experts that are not stored, it ends with the tile's own: us with resources that end with the tensor /
+  // with the tile 64 rows of 8 experts [4096, 7168] 39.1 / 36.3, 1024 of 32 [2048, 7168] 107 / 98, 8192 of 32 [4096, 7168] 313 / 299, 131072
+  // 3239 / 3212.)
   auto span_bytes = [&](int64_t rows, int64_t ld) {     // up to the end of the last row's K codes
     const int64_t bytes = rows > 0 ? (rows - 1) * ld + K : 0;
     return (int)(bytes < (int64_t)0x7FFFF000 ? bytes : (int64_t)0x7FFFF000);   // 256 rows always fit (host check)
   };
   auto rsrc_a_of = [&](const TileInfo& ti) {
-    const int rows = ti.row_end > ti.row0 ? p.M - ti.row0 : 0;
+    const int rows = ti.row_end > ti.row0 ? (GROUPED == kGroupedRows ? ti.row_end : p.M) - ti.row0 : 0;
     return __builtin_amdgcn_make_buffer_rsrc((void*)(p.a + (int64_t)ti.row0 * p.lda), 0, span_bytes(rows, p.lda),
                                              0x00020000);
   };
@@ -475,6 +487,12 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
   };
   auto issue_b = [&](const __amdgpu_buffer_rsrc_t& rs, int buf, int kb, int sub) {
     transfer(rs, b_off[sub], b_lds + buf * kBTile + wave * (NB * 1024), kb, sub);
+  };
+  // Rows of b that one tile alone reads are streamed: they stay in no cache, which leaves those to a's rows (us, grouped by rows,
+  // before / so: 512 rows of 32 experts [4096, 7168] by Zipf's law 158 / 137, 64 of 8 36.3 / 33.1, 1024 of 32 [2048, 7168] 98 / 92; where
+  // several tiles share them it would cost: 8192 of 32 [4096, 7168] 299 / 310).
+  auto stream_b = [&](const __amdgpu_buffer_rsrc_t& rs, int buf, int kb, int sub) {
+    stream_1k(rs, b_lds + buf * kBTile + wave * (NB * 1024) + sub * 1024, b_off[sub], kb * BK);
   };
 
   // ---- fragment addressing
@@ -545,9 +563,11 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
       __amdgpu_buffer_rsrc_t ra, rb;
       uint32_t sa_off, sb_off = 0;
       int sb_first = 0;
+      bool b_once = false;
       auto enter = [&](const TileInfo& ti) {
         ra = rsrc_a_of(ti);
         rb = rsrc_b_of(ti);
+        b_once = ti.b_once;
         const int row = ti.row0 + (wave >> 1) * 64 + lane;       // (rows past M repeat the last one's scale: they are not stored)
         sa_off = (uint32_t)(row < p.M ? row : p.M - 1) * (uint32_t)((int)p.sa_sm * 4);
         if (kRowScales) {
@@ -563,8 +583,13 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
         for (int sub = 0; sub < NA; ++sub) issue_a(ra, buf, f_kb, sub);
       };
       auto fetch_rest = [&]() {
+        if (b_once) {
 #pragma unroll
-        for (int sub = 0; sub < NB; ++sub) issue_b(rb, buf, f_kb, sub);
+          for (int sub = 0; sub < NB; ++sub) stream_b(rb, buf, f_kb, sub);
+        } else {
+#pragma unroll
+          for (int sub = 0; sub < NB; ++sub) issue_b(rb, buf, f_kb, sub);
+        }
         if (kScaleOps) {
           uint8_t* const dst = scale_lds + slot * kScaleSlot + wave * 256;
           __builtin_amdgcn_raw_ptr_buffer_load_lds(kRowScales ? rsrc_sb : rsrc_sbb, (lds_ptr_t)dst, 4, sb_off,
@@ -1254,12 +1279,12 @@ static TileShape pick_shape_swiglu(int64_t M, int64_t N) {
 // only.  Where even the most 64 x 64 or 64 x 128 tiles there can be are one round: those.  Of more than 256 rows per expert on average and
 // two rounds of 256 x 256 tiles or more: those.  In between the kernel chooses (grouped_tile_rows).  us with 64 / 128 / 256 rows per
 // tile, for rows spread evenly / by Zipf's law / half with one expert / all with one:
-//   32 experts [4096, 7168],   512 rows   163 / 165 / 220   180 / 158 / 212   183 / 208 / 212    25 /  42 /  66
-//                             2048 rows   165 / 168 / 224   234 / 202 / 275   211 / 204 / 280    87 /  54 /  73
-//                             8192 rows   432 / 261 / 235   476 / 312 / 377   445 / 273 / 334   338 / 213 / 183
-//   8 experts  [4096, 7168],   512 rows    37 /  46 /  72    48 /  43 /  68    50 /  43 /  69    25 /  42 /  66
-//   16 experts [1024, 4096],  2048 rows    18 /  28 /  43    28 /  28 /  42    22 /  27 /  42    17 /  27 /  41
-//   64 experts [2048, 2048], 16384 rows   144 /  81 /  76   146 /  97 / 117   145 /  84 / 101   118 /  70 /  63
+//   32 experts [4096, 7168],   512 rows   140 / 139 / 196   155 / 140 / 193   159 / 179 / 197    24 /  44 /  65
+//                             2048 rows   159 / 151 / 211   199 / 179 / 249   190 / 179 / 261    85 /  58 /  77
+//                             8192 rows   445 / 257 / 234   455 / 298 / 356   509 / 343 / 305   337 / 214 / 183
+//   8 experts  [4096, 7168],   512 rows    41 /  57 /  81    54 /  56 /  81    59 /  54 /  84    24 /  43 /  65
+//   16 experts [1024, 4096],  2048 rows    23 /  33 /  48    31 /  32 /  47    32 /  31 /  48    16 /  27 /  40
+//   64 experts [2048, 2048], 16384 rows   156 /  87 /  79   155 /  96 / 122   167 / 115 / 106   115 /  70 /  63
 enum GroupedTiles { kSmallestTiles, kLowestTiles, kHighTiles, kChosenTiles, kLowTiles /* test hook: as chosen */ };
 
 static GroupedTiles pick_grouped(int64_t M, int64_t N, int experts) {
