@@ -6,6 +6,9 @@
 // refused calls among them: the Python form of the operator then runs as if this one were not there, and copies, pads or raises.
 // Host time of a call, us, Python form / here: quantize_1x128 10.5 / 5.3, both forms 15.9 / 7.8, with the bias gradient 24.4 / 12.1,
 // 128 x 128 with the transposed codes 12.7 / 6.4, gemm_blockwise 12.2 / 4.9.
+// What a program calls many times for little work goes in one call: a layer in inference, operators one by one / here, linear 16 / 11,
+// per tensor 23 / 11.5, the MLP block 30 to 35 / 16 to 20, the grouped linear 23 / 12; the forward of a training step, per tensor 26 / 18;
+// the gradient bucket there and back, 72 gradients, 67 / 15.
 #include <ATen/ATen.h>
 #include <ATen/TensorSubclassLikeUtils.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
@@ -32,7 +35,10 @@ constexpr int64_t kBlock = 128;
   X(hpfp8_quantize_1x128_kmajor_bf16) X(hpfp8_quantize_1x128_kmajor_pow2_bf16) X(hpfp8_quantize_1x128_and_128x1_t_bf16) \
   X(hpfp8_quantize_1x128_and_128x1_t_pow2_bf16) X(hpfp8_quantize_128x1_t_colsum_bf16) X(hpfp8_quantize_rows_128x1_t_bf16) \
   X(hpfp8_column_sum_finish) X(hpfp8_quantize_128x128_bf16) X(hpfp8_quantize_128x128_pow2_bf16) \
-  X(hpfp8_quantize_per_tensor_t_bf16) X(hpfp8_transpose_codes) X(hpfp8_gemm_blockwise) X(hpfp8_gemm_blockwise_pow2) X(hpfp8_gemm_per_tensor)
+  X(hpfp8_quantize_per_tensor_t_bf16) X(hpfp8_transpose_codes) X(hpfp8_gemm_blockwise) X(hpfp8_gemm_blockwise_pow2) X(hpfp8_gemm_per_tensor) \
+  X(hpfp8_quantize_per_tensor_sync_bf16) X(hpfp8_gemm_few_rows) X(hpfp8_gemm_blockwise_swiglu_quantize) X(hpfp8_swiglu_quantize_1x128_bf16) \
+  X(hpfp8_swiglu_quantize_1x128_pow2_bf16) X(hpfp8_swiglu_quantize_1x128_fast_bf16) X(hpfp8_gemm_grouped_blockwise) \
+  X(hpfp8_bucket_pack_quantize_bf16) X(hpfp8_bucket_unpack_dequantize_bf16)
 struct Library {
 #define HPFP8_POINTER(name) decltype(&::name) name = nullptr;
   HPFP8_FUNCTIONS(HPFP8_POINTER)
@@ -128,6 +134,17 @@ void expect(Py_ssize_t got, Py_ssize_t want) {
   TORCH_CHECK_TYPE(got == want, "expected ", want, " arguments, got ", got);
 }
 
+struct Rows {
+  at::Tensor q, s;        // codes, scale_inv stored k-block-major
+};
+// the 1x128 form of m rows of k values
+Rows make_rows(const at::Tensor& x, int64_t m, int64_t k, bool pow2, void* stream, Call& call) {
+  Rows r{new_codes(x, m, k), new_floats_t(x, m, k / kBlock)};
+  if (pow2) HPFP8_CALL(call, hpfp8_quantize_1x128_kmajor_pow2_bf16, x.data_ptr(), m, k, r.q.data_ptr(), nullptr, f32(r.s), stream);
+  else HPFP8_CALL(call, hpfp8_quantize_1x128_kmajor_bf16, x.data_ptr(), m, k, r.q.data_ptr(), nullptr, f32(r.s), stream);
+  return r;
+}
+
 // (x, pow2, device, stream) -> (codes, scale_inv), k-block-major scales
 PyObject* quantize_1x128(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -136,17 +153,13 @@ PyObject* quantize_1x128(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const bool pow2 = truth(args[1]);
   const at::Tensor* x;
   if (!source_2d(args[0], w.device, x) || !no_modes()) Py_RETURN_NONE;
-  at::Tensor q, s;
+  Rows r;
   Call call;
   {
     pybind11::gil_scoped_release free;
-    const int64_t m = x->size(0), k = x->size(1);
-    q = new_codes(*x, m, k);
-    s = new_floats_t(*x, m, k / kBlock);
-    if (pow2) HPFP8_CALL(call, hpfp8_quantize_1x128_kmajor_pow2_bf16, x->data_ptr(), m, k, q.data_ptr(), nullptr, f32(s), w.stream);
-    else HPFP8_CALL(call, hpfp8_quantize_1x128_kmajor_bf16, x->data_ptr(), m, k, q.data_ptr(), nullptr, f32(s), w.stream);
+    r = make_rows(*x, x->size(0), x->size(1), pow2, w.stream, call);
   }
-  return call.ok() ? tuple_of(std::move(q), std::move(s)) : failed(call);
+  return call.ok() ? tuple_of(std::move(r.q), std::move(r.s)) : failed(call);
   END_HANDLE_TH_ERRORS
 }
 
@@ -348,9 +361,9 @@ PyObject* gemm_per_tensor(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
 // ------------------------------------------------------------------------------------------------
 // One block per device and stream for the one-launch per-tensor quantizer, as ops._sync_words keeps (which has the rule: zero
 // between calls, never two launches at once, none while a graph is captured).
-uint32_t* sync_block(const at::Tensor& x, int64_t tiles, hipStream_t stream) {
-  constexpr int64_t kOnePassTiles = 256;
-  if (tiles > kOnePassTiles || c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return nullptr;
+constexpr int64_t kOnePassTiles = 256, kOnePassValues = (int64_t)1 << 22;
+uint32_t* sync_block(const at::Tensor& x, bool one_pass, hipStream_t stream) {
+  if (!one_pass || c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return nullptr;
   static std::mutex lock;
   static auto* const blocks = new std::map<std::pair<int64_t, hipStream_t>, at::Tensor>;      // (never destroyed: the device may go first)
   std::lock_guard<std::mutex> guard(lock);
@@ -445,7 +458,7 @@ struct LinearNode : torch::autograd::Function<LinearNode> {
     Call call;
     at::Tensor dx, dw, db;
     if (per_tensor) {
-      Forms f = make_per_tensor(go, has_bias, sync_block(go, mp / kBlock * (out / kBlock), current.stream()), stream, call);
+      Forms f = make_per_tensor(go, has_bias, sync_block(go, mp / kBlock * (out / kBlock) <= kOnePassTiles, current.stream()), stream, call);
       if (!call.ok()) raise(call);
       at::Tensor wt = w;
       if (!w_transposed) {
@@ -509,6 +522,311 @@ PyObject* linear_node(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// ------------------------------------------------------------------------------------------------
+// inference: a layer's steps in one call
+// ------------------------------------------------------------------------------------------------
+// A layer's input: bf16 [..., K > 0, a multiple of 128], contiguous, with rows.
+bool layer_input(PyObject* o, int64_t device, const at::Tensor*& t) {
+  return plain(o, device, t) && t->scalar_type() == at::kBFloat16 && t->dim() >= 1 && t->numel() > 0 && t->size(-1) % kBlock == 0 &&
+         t->is_contiguous();
+}
+// Whether a call on these (None among them) is one without a graph, trace or transform, which a Python autograd function would answer
+// in its own way.
+bool without_graph(PyObject* const* tensors, int n) {
+  if (!no_modes() || torch::jit::tracer::isTracing() || c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode))
+    return false;
+  const bool grad = c10::GradMode::is_enabled();
+  for (int i = 0; i < n; ++i) {
+    if (tensors[i] == Py_None) continue;
+    if (!THPVariable_Check(tensors[i])) return false;
+    const at::Tensor& t = THPVariable_Unpack(tensors[i]);
+    if (at::isTensorSubclassLike(t) || (grad && t.requires_grad()) || t._fw_grad(0).defined()) return false;
+  }
+  return true;
+}
+at::Tensor new_rows_like(const at::Tensor& x, int64_t n) {
+  std::vector<int64_t> shape = x.sizes().vec();
+  shape.back() = n;
+  return at::empty(shape, x.options().requires_grad(false));
+}
+bool weight_form(PyObject* codes, PyObject* scale_inv, int64_t device, const at::Tensor*& q, const at::Tensor*& s) {
+  return codes_2d(codes, device, q) && floats(scale_inv, device, s) && q->size(0) % kBlock == 0 && s->dim() == 2 &&
+         s->size(0) == q->size(0) / kBlock && s->size(1) == q->size(1) / kBlock;
+}
+// c[m rows, n] = rows . weight^T (+ bias); c of any shape with n as its last, contiguous
+void multiply_rows(const Rows& r, const at::Tensor& w, const at::Tensor& sw, const void* bias, const at::Tensor& c, bool pow2, void* stream, Call& call) {
+  const int64_t m = r.q.size(0), k = r.q.size(1), n = w.size(0);
+  if (pow2)
+    HPFP8_CALL(call, hpfp8_gemm_blockwise_pow2, r.q.data_ptr(), k, f32(r.s), r.s.stride(0), r.s.stride(1), w.data_ptr(), row_stride(w), f32(sw),
+               sw.stride(0), sw.stride(1), (int)kBlock, m, n, k, bias, c.data_ptr(), n, HPFP8_OUT_BF16, 0, stream);
+  else
+    HPFP8_CALL(call, hpfp8_gemm_blockwise, r.q.data_ptr(), k, f32(r.s), r.s.stride(0), r.s.stride(1), w.data_ptr(), row_stride(w), f32(sw),
+               sw.stride(0), sw.stride(1), (int)kBlock, m, n, k, bias, c.data_ptr(), n, HPFP8_OUT_BF16, 0, stream);
+}
+
+// (x, weight, bias or None, the weight's codes, scale_inv, codes_t or None each, per_tensor, pow2, device, stream) -> y with its place in
+// the graph: forward of what `trains` has taken (hpfp8/linear.py _trained) in one call.  A blockwise weight that has no FP8 form yet is
+// left to the operators one by one (quantizing it dominates such a step).
+PyObject* linear_train(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  expect(n_args, 10);
+  const Where at_ = where(args, n_args);
+  const bool per_tensor = truth(args[6]), pow2 = truth(args[7]);
+  const at::Tensor *x, *weight, *bias, *wq = nullptr, *sw = nullptr, *wqt = nullptr;
+  if (!layer_input(args[0], at_.device, x) || x->dim() < 2 || !source_2d(args[1], at_.device, weight)) Py_RETURN_NONE;
+  const int64_t k = x->size(-1), m = x->numel() / k, n = weight->size(0);
+  if (weight->size(1) != k || n % kBlock || !bias_of(args[2], at_.device, n, bias) || (args[3] == Py_None && !per_tensor)) Py_RETURN_NONE;
+  if (args[3] != Py_None) {
+    if (!codes_2d(args[3], at_.device, wq) || wq->size(0) != n || wq->size(1) != k || !floats(args[4], at_.device, sw)) Py_RETURN_NONE;
+    if (per_tensor ? sw->numel() != 1 : (sw->dim() != 2 || sw->size(0) != n / kBlock || sw->size(1) != k / kBlock)) Py_RETURN_NONE;
+    if (!per_tensor && args[5] != Py_None && (!codes_2d(args[5], at_.device, wqt) || wqt->size(0) != k || wqt->size(1) != n)) Py_RETURN_NONE;
+  }
+  Made made{{}, {}, {}, {}, {}, per_tensor, pow2, bias != nullptr, true};
+  Call call;
+  {
+    pybind11::gil_scoped_release free;
+    at::NoGradGuard no_grad;
+    void* const stream = at_.stream;
+    const at::Tensor x2 = x->dim() == 2 ? *x : x->view({m, k});
+    auto transposed = [&](const at::Tensor& codes) {
+      at::Tensor t = new_codes_t(codes, k, n);
+      HPFP8_CALL(call, hpfp8_transpose_codes, codes.data_ptr(), n, k, row_stride(codes), t.data_ptr(), t.stride(0), stream);
+      return t;
+    };
+    Forms fx, fw;
+    if (per_tensor) {
+      const int64_t tiles = rows_up(m) / kBlock * (k / kBlock);
+      fx = make_per_tensor(x2, false, sync_block(x2, tiles <= kOnePassTiles, (hipStream_t)stream), stream, call);
+      if (call.ok() && !wq) fw = make_per_tensor(*weight, false, sync_block(*weight, n / kBlock * (k / kBlock) <= kOnePassTiles, (hipStream_t)stream), stream, call);
+      made.w_transposed = !wq;
+      made.w = wq ? *wq : fw.qt;
+      made.sw = wq ? *sw : fw.s;
+      made.xt = fx.qt;
+      made.sxt = fx.s;
+      if (call.ok()) made.y = multiply_per_tensor(fx.q, fx.s, wq ? *wq : fw.q, made.sw, bias ? bias->data_ptr() : nullptr, stream, call);
+    } else {
+      fx = make_both(x2, pow2, false, stream, call);
+      if (call.ok()) {
+        made.w = wqt ? *wqt : transposed(*wq);
+        made.sw = *sw;
+      }
+      made.xt = fx.qt;
+      made.sxt = fx.st;
+      if (call.ok()) {
+        made.y = at::empty({m, n}, x->options().requires_grad(false));
+        multiply_blockwise(fx.q, fx.s, *wq, made.sw, made.sw.stride(0), made.sw.stride(1), bias ? bias->data_ptr() : nullptr, made.y, kBlock,
+                           false, pow2, stream, call);
+      }
+    }
+    if (call.ok() && x->dim() != 2) {
+      std::vector<int64_t> shape = x->sizes().vec();
+      shape.back() = n;
+      made.y = made.y.view(shape);
+    }
+  }
+  if (!call.ok()) return failed(call);
+  return THPVariable_Wrap(LinearNode::apply(*x, *weight, bias ? std::optional<at::Tensor>(*bias) : std::nullopt, made));
+  END_HANDLE_TH_ERRORS
+}
+
+// (x, weight, bias or None, codes, scale_inv, per_tensor, pow2, device, stream) -> y
+PyObject* linear_infer(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  expect(n_args, 9);
+  const Where at_ = where(args, n_args);
+  const bool per_tensor = truth(args[5]), pow2 = truth(args[6]);
+  const at::Tensor *x, *w, *sw, *bias;
+  if (!without_graph(args, 3) || !layer_input(args[0], at_.device, x) || !codes_2d(args[3], at_.device, w) || !floats(args[4], at_.device, sw))
+    Py_RETURN_NONE;
+  const int64_t k = x->size(-1), m = x->numel() / k, n = w->size(0);
+  if (w->size(1) != k || n % kBlock || !bias_of(args[2], at_.device, n, bias)) Py_RETURN_NONE;
+  if (per_tensor ? sw->numel() != 1 : !weight_form(args[3], args[4], at_.device, w, sw)) Py_RETURN_NONE;
+  at::Tensor y;
+  Call call;
+  bool taken = true;
+  {
+    pybind11::gil_scoped_release free;
+    const void* const b = bias ? bias->data_ptr() : nullptr;
+    if (per_tensor) {
+      uint32_t* const sync = sync_block(*x, x->numel() <= kOnePassValues, (hipStream_t)at_.stream);
+      taken = sync != nullptr;       // (larger ones, and all under capture, take two launches: the Python form)
+      if (taken) {
+        const at::Tensor q = new_codes(*x, m, k), s = at::empty({}, x->options().dtype(at::kFloat).requires_grad(false));
+        HPFP8_CALL(call, hpfp8_quantize_per_tensor_sync_bf16, x->data_ptr(), x->numel(), q.data_ptr(), nullptr, nullptr, f32(s), sync, at_.stream);
+        if (call.ok()) {
+          y = new_rows_like(*x, n);
+          HPFP8_CALL(call, hpfp8_gemm_per_tensor, q.data_ptr(), k, f32(s), w->data_ptr(), row_stride(*w), f32(*sw), m, n, k, b, y.data_ptr(), n,
+                     HPFP8_OUT_BF16, at_.stream);
+        }
+      }
+    } else {
+      const Rows r = make_rows(*x, m, k, pow2, at_.stream, call);
+      if (call.ok()) {
+        y = new_rows_like(*x, n);
+        multiply_rows(r, *w, *sw, b, y, pow2, at_.stream, call);
+      }
+    }
+  }
+  if (!taken) Py_RETURN_NONE;
+  return call.ok() ? THPVariable_Wrap(std::move(y)) : failed(call);
+  END_HANDLE_TH_ERRORS
+}
+
+// (x, gate/up codes, scale_inv, pow2, down codes, scale_inv, pow2, fast, device, stream) -> y
+PyObject* swiglu_mlp_infer(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  expect(n_args, 10);
+  const Where at_ = where(args, n_args);
+  const bool pow2 = truth(args[3]), pow2_down = truth(args[6]), fast = truth(args[7]);
+  const at::Tensor *x, *gu, *sgu, *dn, *sdn;
+  if (!no_modes() || !layer_input(args[0], at_.device, x) || !weight_form(args[1], args[2], at_.device, gu, sgu) ||
+      !weight_form(args[4], args[5], at_.device, dn, sdn))
+    Py_RETURN_NONE;
+  const int64_t k = x->size(-1), m = x->numel() / k, n = gu->size(0), inter = n / 2;
+  if (gu->size(1) != k || n % (2 * kBlock) || dn->size(1) != inter) Py_RETURN_NONE;
+  at::Tensor y;
+  Call call;
+  {
+    pybind11::gil_scoped_release free;
+    const Rows r = make_rows(*x, m, k, pow2, at_.stream, call);
+    Rows a;
+    if (call.ok()) {
+      a = Rows{new_codes(*x, m, inter), new_floats_t(*x, m, inter / kBlock)};
+      // (ops.gemm_blockwise_swiglu_quantize has the reason for the two forms)
+      if (m <= lib.hpfp8_gemm_few_rows(k) && n * row_stride(*gu) < 0x7FFFF000) {
+        const at::Tensor h = at::empty({m, n}, x->options().requires_grad(false));
+        multiply_rows(r, *gu, *sgu, nullptr, h, pow2, at_.stream, call);
+        if (call.ok()) {
+          if (fast)
+            HPFP8_CALL(call, hpfp8_swiglu_quantize_1x128_fast_bf16, h.data_ptr(), m, inter, n, 1, pow2_down, a.q.data_ptr(), nullptr, f32(a.s), nullptr, at_.stream);
+          else if (pow2_down)
+            HPFP8_CALL(call, hpfp8_swiglu_quantize_1x128_pow2_bf16, h.data_ptr(), m, inter, n, 1, a.q.data_ptr(), nullptr, f32(a.s), nullptr, at_.stream);
+          else
+            HPFP8_CALL(call, hpfp8_swiglu_quantize_1x128_bf16, h.data_ptr(), m, inter, n, 1, a.q.data_ptr(), nullptr, f32(a.s), nullptr, at_.stream);
+        }
+      } else {
+        HPFP8_CALL(call, hpfp8_gemm_blockwise_swiglu_quantize, r.q.data_ptr(), k, f32(r.s), r.s.stride(0), r.s.stride(1), gu->data_ptr(), row_stride(*gu),
+                   f32(*sgu), sgu->stride(0), sgu->stride(1), m, inter, k, fast, pow2, pow2_down, a.q.data_ptr(), inter, nullptr, f32(a.s), at_.stream);
+      }
+    }
+    if (call.ok()) {
+      y = new_rows_like(*x, dn->size(0));
+      multiply_rows(a, *dn, *sdn, nullptr, y, pow2_down, at_.stream, call);
+    }
+  }
+  return call.ok() ? THPVariable_Wrap(std::move(y)) : failed(call);
+  END_HANDLE_TH_ERRORS
+}
+
+// (x, weight, offs, codes, scale_inv, device, stream) -> y
+PyObject* grouped_infer(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  expect(n_args, 7);
+  const Where at_ = where(args, n_args);
+  const at::Tensor *x, *offs, *w, *sw;
+  if (!without_graph(args, 3) || !layer_input(args[0], at_.device, x) || x->dim() != 2 || !plain(args[2], at_.device, offs) || !plain(args[3], at_.device, w) ||
+      !floats(args[4], at_.device, sw))
+    Py_RETURN_NONE;
+  const int64_t m = x->size(0), k = x->size(1);
+  if (w->dim() != 3 || w->scalar_type() != at::kFloat8_e4m3fn || !w->is_contiguous() || w->size(2) != k || w->size(1) % kBlock || w->numel() == 0 ||
+      offs->scalar_type() != at::kInt || offs->dim() != 1 || !offs->is_contiguous() || offs->size(0) != w->size(0) || !sw->is_contiguous() ||
+      sw->sizes() != at::IntArrayRef({w->size(0), w->size(1) / kBlock, k / kBlock}))
+    Py_RETURN_NONE;
+  at::Tensor y;
+  Call call;
+  {
+    pybind11::gil_scoped_release free;
+    const Rows r = make_rows(*x, m, k, false, at_.stream, call);
+    if (call.ok()) {
+      const int64_t n = w->size(1);
+      y = new_rows_like(*x, n);
+      HPFP8_CALL(call, hpfp8_gemm_grouped_blockwise, r.q.data_ptr(), k, f32(r.s), r.s.stride(0), r.s.stride(1), w->data_ptr(), f32(*sw),
+                 offs->data_ptr<int32_t>(), (int)w->size(0), m, n, k, y.data_ptr(), n, HPFP8_OUT_BF16, at_.stream);
+    }
+  }
+  return call.ok() ? THPVariable_Wrap(std::move(y)) : failed(call);
+  END_HANDLE_TH_ERRORS
+}
+
+// ------------------------------------------------------------------------------------------------
+// the gradient bucket
+// ------------------------------------------------------------------------------------------------
+// A table of int64 (an array of ctypes, held by the bucket) while a call lasts.
+struct Table {
+  Py_buffer view{};
+  bool held;
+  Table(PyObject* o, int64_t count) : held(PyObject_GetBuffer(o, &view, PyBUF_SIMPLE) == 0) {
+    if (!held) throw python_error();
+    TORCH_CHECK_TYPE(view.len >= count * 8, "a table of ", count, " entries expected");
+  }
+  ~Table() {
+    if (held) PyBuffer_Release(&view);
+  }
+  Table(const Table&) = delete;
+  const int64_t* data() const { return (const int64_t*)view.buf; }
+};
+// The addresses of a list or tuple of contiguous bf16 tensors of numels[i] * times elements; nothing where one is anything else.
+bool gradients(PyObject* o, int64_t device, const int64_t* numels, int64_t count, int64_t times, std::vector<void*>& ptrs) {
+  if (!(PyList_CheckExact(o) || PyTuple_CheckExact(o)) || PySequence_Fast_GET_SIZE(o) != count) return false;
+  ptrs.resize(count);
+  for (int64_t i = 0; i < count; ++i) {
+    const at::Tensor* t;
+    if (!plain(PySequence_Fast_GET_ITEM(o, i), device, t) || t->scalar_type() != at::kBFloat16 || !t->is_contiguous() || t->numel() != numels[i] * times)
+      return false;
+    ptrs[i] = t->data_ptr();
+  }
+  return true;
+}
+
+// (gradients, numels, offsets, count, shards, row_elems, device, stream) -> (codes, scale_inv)
+PyObject* bucket_pack(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  expect(n_args, 8);
+  const Where at_ = where(args, n_args);
+  const int64_t count = PyLong_AsLongLong(args[3]), shards = PyLong_AsLongLong(args[4]), row = PyLong_AsLongLong(args[5]);
+  if (PyErr_Occurred()) throw python_error();
+  if (count <= 0 || !no_modes()) Py_RETURN_NONE;
+  const Table numels(args[1], count), offsets(args[2], count);
+  std::vector<void*> ptrs;
+  if (!gradients(args[0], at_.device, numels.data(), count, shards, ptrs)) Py_RETURN_NONE;
+  const at::TensorOptions options = THPVariable_Unpack(PySequence_Fast_GET_ITEM(args[0], 0)).options().requires_grad(false);
+  const at::Tensor q = at::empty({shards, row}, options.dtype(at::kFloat8_e4m3fn)), s = at::empty({shards, row / kBlock}, options.dtype(at::kFloat));
+  Call call;
+  {
+    pybind11::gil_scoped_release free;
+    HPFP8_CALL(call, hpfp8_bucket_pack_quantize_bf16, ptrs.data(), numels.data(), offsets.data(), (int)count, (int)shards, row, q.data_ptr(), nullptr,
+               f32(s), at_.stream);
+  }
+  return call.ok() ? tuple_of(q, s) : failed(call);
+  END_HANDLE_TH_ERRORS
+}
+
+// (codes_row, scale_inv_row, outs, numels, offsets, count, row_elems, grad_scale, device, stream) -> whether it was done
+PyObject* bucket_unpack(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  expect(n_args, 10);
+  const Where at_ = where(args, n_args);
+  const int64_t count = PyLong_AsLongLong(args[5]), row = PyLong_AsLongLong(args[6]);
+  const double grad_scale = PyFloat_AsDouble(args[7]);
+  if (PyErr_Occurred()) throw python_error();
+  const at::Tensor *q, *s;
+  if (count <= 0 || !no_modes() || !plain(args[0], at_.device, q) || !floats(args[1], at_.device, s) || q->scalar_type() != at::kFloat8_e4m3fn ||
+      q->numel() != row || s->numel() != row / kBlock || !q->is_contiguous() || !s->is_contiguous())
+    Py_RETURN_FALSE;
+  const Table numels(args[3], count), offsets(args[4], count);
+  std::vector<void*> ptrs;
+  if (!gradients(args[2], at_.device, numels.data(), count, 1, ptrs)) Py_RETURN_FALSE;
+  Call call;
+  {
+    pybind11::gil_scoped_release free;
+    HPFP8_CALL(call, hpfp8_bucket_unpack_dequantize_bf16, ptrs.data(), numels.data(), offsets.data(), (int)count, row, q->data_ptr(), f32(*s),
+               (float)grad_scale, at_.stream);
+  }
+  if (!call.ok()) return failed(call);
+  Py_RETURN_TRUE;
+  END_HANDLE_TH_ERRORS
+}
+
 // (handle of the loaded library, function that raises for a name and a status, torch.nn.Parameter)
 PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -544,7 +862,8 @@ PyObject* bind_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
 #define HPFP8_METHOD(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {HPFP8_METHOD(built_for), HPFP8_METHOD(bind), HPFP8_METHOD(bind_backward), HPFP8_METHOD(quantize_1x128), HPFP8_METHOD(both_forms),
                          HPFP8_METHOD(quantize_128x128), HPFP8_METHOD(quantize_per_tensor_t), HPFP8_METHOD(gemm_blockwise),
-                         HPFP8_METHOD(gemm_per_tensor), HPFP8_METHOD(trains), HPFP8_METHOD(linear_node),
+                         HPFP8_METHOD(gemm_per_tensor), HPFP8_METHOD(trains), HPFP8_METHOD(linear_node), HPFP8_METHOD(linear_train), HPFP8_METHOD(linear_infer),
+                         HPFP8_METHOD(swiglu_mlp_infer), HPFP8_METHOD(grouped_infer), HPFP8_METHOD(bucket_pack), HPFP8_METHOD(bucket_unpack),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

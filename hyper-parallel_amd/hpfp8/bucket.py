@@ -79,6 +79,12 @@ class Fp8GradBucket:
     def pack(self, grads: Sequence[torch.Tensor]):
         """_copy_grad_to_unsharded_buffer + cast: gradients (each shard_size * numels[e] elements) ->
         (codes [shard_size, row_elems] e4m3, scale_inv [shard_size, row_elems / 128] fp32)."""
+        if ops._native is not None:
+            device = ops._device()
+            out = ops._native.bucket_pack(grads, self._numels_c, self._offsets_c, len(self.numels), self.shard_size, self.row_elems, device,
+                                          ops._raw_stream(device))
+            if out is not None:
+                return out
         ptrs = self._ptr_table(grads, [n * self.shard_size for n in self.numels])    # (checks: all on the current GPU)
         dev = torch.device("cuda", torch.cuda.current_device())
         q = torch.empty((self.shard_size, self.row_elems), dtype=ops.FP8, device=dev)
@@ -91,6 +97,11 @@ class Fp8GradBucket:
     def unpack(self, codes_row: torch.Tensor, scale_inv_row: torch.Tensor, outs: Sequence[torch.Tensor]):
         """_set_grad_data: one reduced row (codes [row_elems], scale_inv [row_elems / 128]) -> outs[e]
         (bf16, numels[e] elements each), times grad_scale after the cast back."""
+        if ops._native is not None:
+            device = ops._device()
+            if ops._native.bucket_unpack(codes_row, scale_inv_row, outs, self._numels_c, self._offsets_c, len(self.numels), self.row_elems,
+                                         self.grad_scale, device, ops._raw_stream(device)):
+                return list(outs)
         if codes_row.numel() != self.row_elems or scale_inv_row.numel() != self.row_elems // ops.BLOCK:
             raise ValueError("row does not have this bucket's size")
         if codes_row.dtype != ops.FP8 or scale_inv_row.dtype != torch.float32 or \

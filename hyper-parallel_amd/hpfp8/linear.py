@@ -334,7 +334,14 @@ def fp8_linear(input: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.T
             if bool(weight_fp8.pow2) != pow2:
                 raise ValueError("weight_fp8 was quantized for the other blockwise recipe")
     if not apply_grad_on_fp32_main_grad and ops._native is not None and ops._native.trains(input, weight, bias, wq, sw, wqt):
-        return _trained(input, weight, bias, wq, sw, wqt, recipe == "per_tensor", pow2)
+        device = ops._device()
+        y = ops._native.linear_train(input, weight, bias, wq, sw, wqt, recipe == "per_tensor", pow2, device, ops._raw_stream(device))
+        return _trained(input, weight, bias, wq, sw, wqt, recipe == "per_tensor", pow2) if y is None else y
+    if wq is not None and ops._gpu(input):
+        device = ops._device()
+        y = ops._native.linear_infer(input, weight, bias, wq, sw, recipe == "per_tensor", pow2, device, ops._raw_stream(device))
+        if y is not None:
+            return y
     if recipe == "per_tensor":
         return _Fp8LinearPerTensor.apply(input, weight, bias, wq, sw, torch.is_grad_enabled())
     return _Fp8LinearBlockwise.apply(input, weight, bias, wq, sw, wqt, apply_grad_on_fp32_main_grad, pow2, torch.is_grad_enabled())
@@ -544,6 +551,11 @@ def fp8_grouped_linear(input: torch.Tensor, weight: torch.Tensor, offs: torch.Te
     if weight_fp8 is not None:
         if tuple(weight_fp8.codes.shape) != tuple(weight.shape) or weight_fp8.scale_inv.dim() != 3 or weight_fp8.pow2:
             raise ValueError("weight_fp8 must be the blockwise form of this weight (quantize_grouped_weight)")
+        if ops._gpu(input):
+            device = ops._device()
+            y = ops._native.grouped_infer(input, weight, offs, weight_fp8.codes, weight_fp8.scale_inv, device, ops._raw_stream(device))
+            if y is not None:
+                return y
         return _Fp8GroupedLinear.apply(input, weight, offs, weight_fp8.codes, weight_fp8.scale_inv, weight_fp8.codes_t,
                                        torch.is_grad_enabled())
     return _Fp8GroupedLinear.apply(input, weight, offs, None, None, None, torch.is_grad_enabled())
@@ -692,6 +704,12 @@ def fp8_swiglu_mlp(input: torch.Tensor, w_gate_up, w_down, *, fast: bool = True,
     inter = gu.codes.shape[0] // 2
     if gu.codes.shape[0] % (2 * ops.BLOCK) or dn.codes.shape[1] != inter:
         raise ValueError("w_gate_up must be [2I, K] with I a multiple of 128 and w_down [N, I]")
+    if ops._gpu(input):
+        device = ops._device()
+        y = ops._native.swiglu_mlp_infer(input, gu.codes, gu.scale_inv, gu.pow2, dn.codes, dn.scale_inv, dn.pow2, fast, device,
+                                         ops._raw_stream(device))
+        if y is not None:
+            return y
     with torch.no_grad():
         x2 = _flatten(input)
         xq, sx = ops.quantize_1x128(x2, kmajor=True, pow2=gu.pow2)

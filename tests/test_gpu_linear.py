@@ -1049,3 +1049,103 @@ def test_what_else_torch_does_with_a_step_has_the_python_functions_outcome(gpu, 
     else:
         assert isinstance(got, list), got
         assert len(got) == len(want) and all(type(a) is type(b) and a.requires_grad == b.requires_grad and torch.equal(a, b) for a, b in zip(got, want))
+
+
+def _with_and_without_native(run, monkeypatch):
+    """What a call gives through the native host path and as the Python form: results, or the type of the error."""
+    from hpfp8 import ops
+    assert ops._native is not None
+
+    def outcome():
+        try:
+            r = run()
+            return [t.clone() if torch.is_tensor(t) else t for t in (r if isinstance(r, (list, tuple)) else [r])]
+        except Exception as e:      # noqa: BLE001
+            return type(e)
+    got = outcome()
+    with monkeypatch.context() as m:
+        m.setattr(ops, "_native", None)
+        want = outcome()
+    return got, want
+
+
+def _same(got, want):
+    if isinstance(want, type):
+        return got is want
+    return len(got) == len(want) and all(a.shape == b.shape and a.dtype == b.dtype and a.requires_grad == b.requires_grad and
+                                         torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8)) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("recipe", ["blockwise", "blockwise_pow2", "per_tensor"])
+@pytest.mark.parametrize("shape", [(256,), (1, 256), (37, 256), (3, 5, 256), (200, 2048), (0, 256), (4, 128)])
+@pytest.mark.parametrize("how", ["plain", "strided", "trained input", "trained weight, no_grad", "offset", "no bias"])
+def test_a_layer_in_inference_has_the_python_forms_outcome(gpu, recipe, shape, how, monkeypatch):
+    """Inputs of any rank, empty ones and wrong widths, strides, an address between two vectors, tensors that would need a graph: what the
+    one native call takes has the bits of the operators one by one, and what it leaves to them their results and errors."""
+    import hpfp8
+    g = torch.Generator(device="cpu").manual_seed(0)
+    k = 2048 if shape[-1] == 2048 else 256
+    x = torch.randn(shape, generator=g).bfloat16().to(gpu)
+    w = torch.nn.Parameter(torch.randn((384, k), generator=g).bfloat16().to(gpu), requires_grad=how == "trained weight, no_grad")
+    b = None if how == "no bias" else torch.randn(384, generator=g).bfloat16().to(gpu)
+    f8 = hpfp8.quantize_weight(w.detach(), with_transpose=False, pow2=recipe == "blockwise_pow2", per_tensor=recipe == "per_tensor")
+    if how == "strided":
+        x = torch.stack([x, x], dim=-1)[..., 0]
+    elif how == "offset":
+        x = torch.cat([x.flatten()[:1], x.flatten()])[1:].view(shape)
+    elif how == "trained input":
+        x.requires_grad_(True)
+    with torch.set_grad_enabled(how != "trained weight, no_grad"):
+        got, want = _with_and_without_native(lambda: hpfp8.fp8_linear(x, w, b, recipe=recipe, weight_fp8=f8), monkeypatch)
+    assert _same(got, want)
+
+
+@pytest.mark.parametrize("shape,inter", [((1, 256), 128), ((37, 2048), 384), ((64, 2176), 128), ((65, 2048), 256), ((2, 3, 256), 256), ((0, 256), 128), ((3, 384), 128)])
+@pytest.mark.parametrize("fast", [True, False])
+@pytest.mark.parametrize("pow2", [(False, False), (True, False), (False, True)])
+def test_an_mlp_block_in_inference_has_the_python_forms_outcome(gpu, shape, inter, fast, pow2, monkeypatch):
+    import hpfp8
+    g = torch.Generator(device="cpu").manual_seed(0)
+    k = 256 if shape[-1] == 384 else shape[-1]
+    x = torch.randn(shape, generator=g).bfloat16().to(gpu)
+    gu = hpfp8.quantize_weight((torch.randn((2 * inter, k), generator=g) * 0.1).bfloat16().to(gpu), with_transpose=False, pow2=pow2[0])
+    dn = hpfp8.quantize_weight((torch.randn((256, inter), generator=g) * 0.1).bfloat16().to(gpu), with_transpose=False, pow2=pow2[1])
+    got, want = _with_and_without_native(lambda: hpfp8.fp8_swiglu_mlp(x, gu, dn, fast=fast), monkeypatch)
+    assert _same(got, want)
+
+
+@pytest.mark.parametrize("rows", [[3, 0, 130, 1], [0, 0, 0, 0], [64, 64, 64, 64]])
+@pytest.mark.parametrize("offs_type", [torch.int32, torch.int64])
+def test_a_grouped_layer_in_inference_has_the_python_forms_outcome(gpu, rows, offs_type, monkeypatch):
+    import hpfp8
+    g = torch.Generator(device="cpu").manual_seed(0)
+    x = torch.randn((sum(rows), 256), generator=g).bfloat16().to(gpu)
+    w = torch.randn((4, 384, 256), generator=g).bfloat16().to(gpu)
+    offs = torch.tensor(rows).cumsum(0).to(offs_type).to(gpu)
+    f8 = hpfp8.quantize_grouped_weight(w, with_transpose=False)
+    got, want = _with_and_without_native(lambda: hpfp8.fp8_grouped_linear(x, w, offs, weight_fp8=f8), monkeypatch)
+    assert _same(got, want)
+
+
+@pytest.mark.parametrize("numels,shards", [([128], 1), ([1, 129, 4096], 4), ([7, 300] * 70, 2)])
+@pytest.mark.parametrize("wrong", [None, "a tuple", "type", "size", "strided", "count", "a generator"])
+def test_the_bucket_has_the_python_forms_outcome(gpu, numels, shards, wrong, monkeypatch):
+    import hpfp8
+    g = torch.Generator(device="cpu").manual_seed(0)
+    bucket = hpfp8.Fp8GradBucket(numels, shard_size=shards, grad_scale=0.5)
+    grads = [torch.randn(n * shards, generator=g).bfloat16().to(gpu) for n in numels]
+    outs = [torch.zeros(n, dtype=torch.bfloat16, device=gpu) for n in numels]
+    if wrong == "type":
+        grads[-1], outs[-1] = grads[-1].float(), outs[-1].float()
+    elif wrong == "size":
+        grads[-1], outs[-1] = torch.cat([grads[-1], grads[-1]]), torch.cat([outs[-1], outs[-1]])
+    elif wrong == "strided" and numels[-1] > 1:
+        grads[-1], outs[-1] = torch.stack([grads[-1], grads[-1]], 1)[:, 0], torch.stack([outs[-1], outs[-1]], 1)[:, 0]
+    elif wrong == "count":
+        grads, outs = grads + grads[:1], outs + outs[:1]
+    given = (lambda t: tuple(t)) if wrong == "a tuple" else ((lambda t: (v for v in t)) if wrong == "a generator" else (lambda t: t))
+    got, want = _with_and_without_native(lambda: bucket.pack(given(grads)), monkeypatch)
+    assert _same(got, want)
+    if not isinstance(want, type):
+        got, want = _with_and_without_native(lambda: bucket.unpack(want[0].view(torch.uint8)[0].view(torch.float8_e4m3fn), want[1][0], given(outs)), monkeypatch)
+        assert _same(got, want)
