@@ -1536,6 +1536,31 @@ void hpfp8_debug_set_small_gemm(int mode) { g_small_gemm_mode.store(mode >= 1 &&
 
 int64_t hpfp8_gemm_few_rows(int64_t K) { return K >= kEpilogueMaxK ? few_rows(K) : 0; }
 
+// Up to 8 rows are quantized inside the product (gemm_skinny.hip has the figures).  With few runs of columns and a long contraction
+// every compute unit's chain of k-blocks is longer than in two launches and what those cost more is less: us, 8 rows, two / one
+// [1024, 10240] 11.0 / 10.1, [1024, 12288] 11.6 / 11.4 (1 row 10.4 / 10.9), [2048, 16384] 13.6 / 14.2, [4096, 16384] 16.2 / 14.4.
+int64_t hpfp8_linear_few_rows(int64_t N, int64_t K) {
+  if (K > 10240 && 4 * (N / 16) <= 3 * (int64_t)persistent_grid((int64_t)1 << 40)) return 0;
+  return few_rows(K) > kSkinnyMaxRowsBf16 ? kSkinnyMaxRowsBf16 : few_rows(K);
+}
+
+int hpfp8_linear_few_rows_bf16(const void* x, const void* b, int64_t ldb, const float* sb, int64_t sb_stride_n, int64_t sb_stride_k,
+                               int64_t M, int64_t N, int64_t K, int pow2, const void* bias, void* c, int64_t ldc, int out_type,
+                               hpfp8_stream_t stream) {
+  const char* what = "linear_few_rows";
+  HPFP8_REQUIRE(pow2 == 0 || pow2 == 1, HPFP8_ERR_ARG, "%s: pow2 must be 0 or 1", what);
+  HPFP8_REQUIRE(M <= kSkinnyMaxRowsBf16, HPFP8_ERR_SHAPE, "%s: more than %d rows", what, kSkinnyMaxRowsBf16);
+  int rc = check_common(what, x, 2 * K, b, ldb, sb, sb, M, N, K, bias, c, ldc, out_type, 0);
+  if (rc <= 0) return rc;
+  rc = check_scale_span(what, N / kBlock, K / BK, sb_stride_n, sb_stride_k, "sb");
+  if (rc <= 0) return rc;
+  SkinnyParams p{};
+  p.a = (const uint8_t*)x; p.lda = 2 * K; p.b = (const uint8_t*)b; p.ldb = ldb; p.sb = sb; p.sb_sn = sb_stride_n; p.sb_sk = sb_stride_k;
+  p.sb_bytes = (int)(((N / kBlock - 1) * sb_stride_n + (K / BK - 1) * sb_stride_k + 1) * 4);
+  p.bias = (const uint16_t*)bias; p.c = c; p.ldc = ldc; p.M = (int)M; p.N = (int)N; p.K = (int)K; p.out_f32 = out_type == HPFP8_OUT_F32;
+  return launch_skinny_rows_bf16(p, pow2 != 0, persistent_grid((int64_t)1 << 40), (hipStream_t)stream);
+}
+
 int hpfp8_gemm_per_tensor(const void* a, int64_t lda, const float* sa_inv, const void* b, int64_t ldb,
                           const float* sb_inv, int64_t M, int64_t N, int64_t K, const void* bias, void* c,
                           int64_t ldc, int out_type, hpfp8_stream_t stream) {

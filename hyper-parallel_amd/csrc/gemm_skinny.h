@@ -34,4 +34,8 @@ constexpr int kSkinnyMinK = 512;
 
 int launch_skinny(const SkinnyParams& p, SkinnyMode mode, int cus, hipStream_t stream);
 
+// a is bf16 (lda bytes between its rows), quantized 1x128 in the kernel; M <= kSkinnyMaxRowsBf16.  sa is not read.
+constexpr int kSkinnyMaxRowsBf16 = 8;
+int launch_skinny_rows_bf16(const SkinnyParams& p, bool pow2, int cus, hipStream_t stream);
+
 }  // namespace hpfp8

@@ -22,6 +22,12 @@
 // Measured (weights rotating beyond the Infinity Cache): 8 rows of [7168, 16384] 20.6 us (5.7 TB/s), of [36864, 7168] 39.5
 // us (6.7 TB/s); 37 rows of the latter 41.6, 64 rows 44.0.  64 rows of [7168, 16384] 26.8 us: a's rows are then two
 // thirds of what passes a compute unit's vector-memory path.
+// QUANT, up to 8 rows: a is the bf16 source.  Its quantizer would be a launch of 3.5 us that reads what fits in a corner of one XCD's
+// L2; here every workgroup quantizes all of it, k-block by k-block as it arrives, in waves of their own (a k-block of a stage each, while
+// the stage before is multiplied), for 1 KB more per k-block on the vector-memory path.  That leaves no room for wider forms than 3
+// fragments; with the multiplying waves quantizing as well the two chains add up ([7168, 16384] 25.4 us).  us, 8 rows, quantizer and
+// product / this: [7168, 16384] 23.3 / 21.5, [36864, 7168] 41.4 / 38.8, [7168, 7168] 12.4 / 11.3, [16384, 16384] 45.2 / 42.9,
+// [10240, 5120] 13.2 / 11.1, [4096, 1536] 6.5 / 4.9, [1024, 1024] 5.4 / 3.8, 1 row alike; hpfp8_linear_few_rows has the exceptions.
 // Transfers past the end go through an empty resource (with no scalar offset: out of range in any lane): they fetch
 // nothing, write zeros and keep the number of operations in flight constant, which is what the waits count.
 #include "gemm_skinny.h"
@@ -32,15 +38,17 @@
 namespace hpfp8 {
 
 constexpr int kSkinnyWaves = 4;                         // so many fetch, so many multiply
-constexpr int kSkinnyThreads = 2 * kSkinnyWaves * 64;
 // ME: 8-row pieces of a, one transfer each (M <= 8 ME); F: 16-column fragments of a workgroup.
 // A stage: KS k-blocks, each b's rows, a's rows, the scales of a's rows (64) and of the fragments.
-constexpr int skinny_kstep(int me, int f) { return 2 * f + me <= 6 ? 8 : (2 * f + me <= 12 ? 4 : 2); }
+// QUANT: a comes as bf16, 8 rows of it in two transfers (ME = 2), and is quantized here.
+constexpr int skinny_kstep(int me, int f, bool quant = false) { return quant ? (f == 1 ? 8 : 4) : (2 * f + me <= 6 ? 8 : (2 * f + me <= 12 ? 4 : 2)); }
+// (QUANT: one wave more per k-block of a stage)
+constexpr int skinny_threads(int f, bool quant) { return (2 * kSkinnyWaves + (quant ? skinny_kstep(2, f, true) : 0)) * 64; }
 constexpr int skinny_block_bytes(int me, int f) { return (2 * f + me) * 1024 + 512; }
-constexpr int skinny_stage_bytes(int me, int f) { return skinny_kstep(me, f) * skinny_block_bytes(me, f); }
+constexpr int skinny_stage_bytes(int me, int f, bool quant = false) { return skinny_kstep(me, f, quant) * skinny_block_bytes(me, f); }
 constexpr int kSkinnySpare = 1024;       // behind the ring: where a transfer without a piece of its own goes
-constexpr int skinny_stages(int me, int f) {
-  const int fit = (160 * 1024 - kSkinnySpare) / skinny_stage_bytes(me, f);
+constexpr int skinny_stages(int me, int f, bool quant = false) {
+  const int fit = (160 * 1024 - kSkinnySpare) / skinny_stage_bytes(me, f, quant);
   return fit > 8 ? 8 : fit;
 }
 
@@ -60,13 +68,35 @@ __device__ __forceinline__ void transfer_256(__amdgpu_buffer_rsrc_t rs, uint8_t*
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)dst, 4, lane_off, off, 0, 0);
 }
 
+// One k-block of 8 rows, bf16 [8][128] in LDS -> its codes, in the image of an operand tile, over the first half of them, and its
+// scales: quant_1x128_kmajor_kernel's arithmetic.  One wave does it, so every lane has read before one writes.  Lane 8 r + p has
+// the values 8 p .. and 64 + 8 p .. of row r (odd rows the latter first, so that two rows read from different banks).
+__device__ __forceinline__ void quantize_k_block(uint8_t* rows, float* scales, int lane, int pow2) {
+  const int r = lane >> 3, p = lane & 7;
+  const int part[2] = {p + (r & 1) * 8, p + 8 - (r & 1) * 8};
+  uint4 v[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) v[i] = *reinterpret_cast<const uint4*>(rows + r * 256 + part[i] * 16);
+  uint32_t m = umax(mag8(v[0]), mag8(v[1]));
+  m = umax(m, dpp_u32<kDppQuadXor1>(m));
+  m = umax(m, dpp_u32<kDppQuadXor2>(m));
+  m = umax(m, dpp_u32<kDppRowHalfMirror>(m));
+  float scale, scale_inv;
+  scales_from_amax(__uint_as_float(m << 16), scale, scale_inv, pow2);
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    *reinterpret_cast<uint2*>(rows + r * BK + ((part[i] >> 1) ^ row_swizzle(r)) * 16 + (part[i] & 1) * 8) = cvt8<false>(v[i], scale);
+  if (p == 0) scales[r] = scale_inv;
+}
+
 // (Rows of a fragment past the last piece hold what lies behind it in the LDS: a row of the product depends on its own
 // row of a alone, and rows past M are not stored.)
-template <int MODE, int ME, int F>
-__global__ __launch_bounds__(kSkinnyThreads) void gemm_skinny_kernel(const SkinnyParams p, int units) {
+template <int MODE, int ME, int F, bool QUANT = false>
+__global__ __launch_bounds__(skinny_threads(F, QUANT)) void gemm_skinny_kernel(const SkinnyParams p, int units) {
+  static_assert(!QUANT || (ME == 2 && MODE != kSkinnyTensor), "eight rows of bf16, scales of their own");
   constexpr int MF = (ME + 1) / 2;                              // 16-row fragments of a
-  constexpr int KS = skinny_kstep(ME, F), U = skinny_stages(ME, F);
-  constexpr int kBlockBytes = skinny_block_bytes(ME, F), kStage = skinny_stage_bytes(ME, F);
+  constexpr int KS = skinny_kstep(ME, F, QUANT), U = skinny_stages(ME, F, QUANT);
+  constexpr int kBlockBytes = skinny_block_bytes(ME, F), kStage = skinny_stage_bytes(ME, F, QUANT);
   constexpr int kA = 2 * F * 1024, kScales = (2 * F + ME) * 1024;     // a's rows and the scales inside a k-block's bytes
   constexpr int kCols = 16 * F;
   __shared__ __attribute__((aligned(1024))) uint8_t lds[U * kStage + kSkinnySpare];
@@ -85,9 +115,11 @@ __global__ __launch_bounds__(kSkinnyThreads) void gemm_skinny_kernel(const Skinn
     constexpr int KW = KS > kSkinnyWaves ? KS / kSkinnyWaves : 1;       // k-blocks a wave fetches per stage
     constexpr int W = KS < kSkinnyWaves ? kSkinnyWaves / KS : 1;        // waves that fetch one k-block together
     constexpr int NBP = (2 * F + W - 1) / W, NAP = (ME + W - 1) / W;    // a wave's transfers of b and of a per k-block
-    constexpr int kScaleOps = MODE == kSkinnyTensor ? 0 : (W == 1 ? 2 : 1);
-    constexpr int kLeft = (U - 2) * KW * (NBP + NAP + kScaleOps);       // in flight behind the oldest stage
-    static_assert(U >= 3 && kLeft <= 63, "the wait counter holds 63");
+    constexpr int kScaleOps = MODE == kSkinnyTensor ? 0 : (W == 1 && !QUANT ? 2 : 1);
+    constexpr int kStageOps = KW * (NBP + NAP + kScaleOps);
+    constexpr int kLeft = (U - (QUANT ? 3 : 2)) * kStageOps;            // in flight behind the oldest stage that has to be there
+    static_assert(U >= 3 && kLeft <= 63 && (U - 2) * kStageOps <= 63, "the wait counter holds 63");
+    static_assert(!QUANT || (W == 1 && U >= 4), "a stage is quantized while the one before is multiplied");
     static_assert(W <= 2, "every wave of a k-block has scales to fetch");
     const int h = wave % W, kb0 = wave / W * KW;
     uint32_t b_off[NBP], a_off[NAP];
@@ -99,11 +131,12 @@ __global__ __launch_bounds__(kSkinnyThreads) void gemm_skinny_kernel(const Skinn
 #pragma unroll
     for (int i = 0; i < NAP; ++i) {                             // (rows past M lie past the end of the resource)
       const int r = (i * W + h) * 8 + (lane >> 3);
-      a_off[i] = (uint32_t)r * (uint32_t)p.lda + ((lane & 7) ^ row_swizzle(r)) * 16;
+      a_off[i] = QUANT ? (uint32_t)(i * 4 + (lane >> 4)) * (uint32_t)p.lda + (lane & 15) * 16       // 4 rows x 256 bytes
+                       : (uint32_t)r * (uint32_t)p.lda + ((lane & 7) ^ row_swizzle(r)) * 16;
     }
     const uint32_t sa_off = (uint32_t)(lane < p.M ? lane : p.M - 1) * (uint32_t)p.sa_sm * 4u;
-    const int a_bytes = (int)((p.M - 1) * p.lda + p.K);
-    const int sa_bytes = MODE == kSkinnyTensor ? 0 : (int)(((p.M - 1) * p.sa_sm + (kblocks - 1) * p.sa_sk + 1) * 4);
+    const int a_bytes = (int)((p.M - 1) * p.lda + (QUANT ? 2 * p.K : p.K));
+    const int sa_bytes = MODE == kSkinnyTensor || QUANT ? 0 : (int)(((p.M - 1) * p.sa_sm + (kblocks - 1) * p.sa_sk + 1) * 4);
     const int sa_step = (int)p.sa_sk * 4, sb_step = (int)p.sb_sk * 4;
     int unit = first, kb = kb0, slot = 0;                       // the next stage to fetch
     const uint8_t* b0;
@@ -133,12 +166,12 @@ __global__ __launch_bounds__(kSkinnyThreads) void gemm_skinny_kernel(const Skinn
         for (int i = 0; i < NAP; ++i) {
           const bool in = ME % W == 0 || i * W + h < ME;
           const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)p.a, 0, ok && in ? a_bytes : 0, 0x00020000);
-          transfer_1k<false>(ra, in ? dst + kA + (i * W + h) * 1024 : lds + U * kStage, a_off[i], in ? off : 0);
+          transfer_1k<false>(ra, in ? dst + kA + (i * W + h) * 1024 : lds + U * kStage, a_off[i], in ? (QUANT ? 2 * off : off) : 0);
         }
         if (MODE != kSkinnyTensor) {
           const __amdgpu_buffer_rsrc_t rsa = __builtin_amdgcn_make_buffer_rsrc((void*)p.sa, 0, ok ? sa_bytes : 0, 0x00020000);
           const __amdgpu_buffer_rsrc_t rsb = __builtin_amdgcn_make_buffer_rsrc((void*)p.sb, 0, ok ? p.sb_bytes : 0, 0x00020000);
-          if (h == 0) transfer_256(rsa, dst + kScales, sa_off, ok ? (kb + j) * sa_step : 0);
+          if (h == 0 && !QUANT) transfer_256(rsa, dst + kScales, sa_off, ok ? (kb + j) * sa_step : 0);
           if (h == W - 1) transfer_256(rsb, dst + kScales + 256, sb_off, ok ? (kb + j) * sb_step : 0);
         }
       }
@@ -151,14 +184,41 @@ __global__ __launch_bounds__(kSkinnyThreads) void gemm_skinny_kernel(const Skinn
       }
     };
     for (int u = 0; u < U - 1; ++u) fetch();
+    if (QUANT) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((U - 2) * kStageOps) : "memory");     // the first stage has landed
     for (int u = first; u < units; u += step)
       for (int t = 0; t < stages; ++t) {
-        // own transfers of this stage have landed; then everyone's, and the stage before has been read
+        // own transfers of this stage (QUANT: of the next one) have landed; then everyone's, and the stage before has been read
         asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kLeft) : "memory");
         fetch();
       }
     __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the empty transfers still write to this workgroup's LDS
     return;
+  }
+
+  auto sync = [&]() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // the stage is there; the one before has been read
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  if (QUANT) {
+    sync();
+    if (wave >= 2 * kSkinnyWaves) {
+      // ---- quantizing: a k-block of the next stage, while this one is multiplied.  (Past the last stage zeros: the empty transfers
+      // have written them.)
+      int slot = 0;
+      auto quantize = [&]() {
+        uint8_t* const src = lds + slot * kStage + (wave - 2 * kSkinnyWaves) * kBlockBytes;
+        quantize_k_block(src + kA, reinterpret_cast<float*>(src + kScales), lane, MODE == kSkinnyPow2);
+        slot = slot + 1 == U ? 0 : slot + 1;
+      };
+      quantize();
+      for (int u = first; u < units; u += step)
+        for (int t = 0; t < stages; ++t) {
+          sync();
+          quantize();
+        }
+      return;
+    }
   }
 
   // ---- multiplying.  WF waves along the fragments of b, WJ along those of a; FW x JW results per wave (the last ones of
@@ -218,9 +278,7 @@ __global__ __launch_bounds__(kSkinnyThreads) void gemm_skinny_kernel(const Skinn
   int slot = 0;
   for (int unit = first; unit < units; unit += step) {
     for (int t = 0; t < stages; ++t) {
-      __builtin_amdgcn_sched_barrier(0);
-      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // the stage is there; the one before has been read
-      __builtin_amdgcn_sched_barrier(0);
+      sync();
       if (active) {
         const uint8_t* const src = lds + slot * kStage;
         if ((t + 1) * KS <= kblocks) {
@@ -263,14 +321,15 @@ __global__ __launch_bounds__(kSkinnyThreads) void gemm_skinny_kernel(const Skinn
 // vector-memory path (1.4 : 1 per KB), and 1.4 times that where a stage is fewer than four k-blocks; taken is the form whose
 // runs cost least, the narrowest of equals.  Over 10 widths from 4096 to 36864, 4 contractions from 4096 to 16384 and 5 row
 // counts this is 0.7 % slower on average than the best of the six forms of each, 14 % at most (24 rows of [18432, 7168]).
-static int skinny_fragments(int64_t N, int me, int cus) {
+static int skinny_fragments(int64_t N, int me, int cus, bool quant = false) {
   const int forms[] = {1, 2, 3, 4, 6, 9};
   int best = 0;
   int64_t best_cost = 0;
   for (int f : forms) {
+    if (quant && f > 3) break;
     const int64_t units = (N / 16 + f - 1) / f, runs = (units + cus - 1) / cus;
     const int64_t run = 14 * 2 * f > 10 * (2 * f + me) ? 14 * 2 * f : 10 * (2 * f + me);
-    const int64_t cost = runs * run * (skinny_kstep(me, f) >= 4 ? 10 : 14);
+    const int64_t cost = runs * run * (skinny_kstep(me, f, quant) >= 4 ? 10 : 14);
     if (!best || cost < best_cost) {
       best = f;
       best_cost = cost;
@@ -279,10 +338,10 @@ static int skinny_fragments(int64_t N, int me, int cus) {
   return best;
 }
 
-template <int MODE, int ME, int F>
+template <int MODE, int ME, int F, bool QUANT = false>
 static void launch_skinny_form(const SkinnyParams& p, int cus, hipStream_t stream) {
   const int units = (p.N / 16 + F - 1) / F;
-  gemm_skinny_kernel<MODE, ME, F><<<dim3((unsigned)(units < cus ? units : cus)), dim3(kSkinnyThreads), 0, stream>>>(p, units);
+  gemm_skinny_kernel<MODE, ME, F, QUANT><<<dim3((unsigned)(units < cus ? units : cus)), dim3(skinny_threads(F, QUANT)), 0, stream>>>(p, units);
 }
 
 template <int MODE, int ME>
@@ -317,6 +376,21 @@ int launch_skinny(const SkinnyParams& p, SkinnyMode mode, int cus, hipStream_t s
   else if (mode == kSkinnyPow2) launch_skinny_rows<kSkinnyPow2>(p, cus, stream);
   else launch_skinny_rows<kSkinnyBlock>(p, cus, stream);
   return check_launch("gemm (few rows)");
+}
+
+template <int MODE>
+static void launch_skinny_bf16(const SkinnyParams& p, int cus, hipStream_t stream) {
+  switch (skinny_fragments(p.N, 2, cus, true)) {
+    case 1: launch_skinny_form<MODE, 2, 1, true>(p, cus, stream); break;
+    case 2: launch_skinny_form<MODE, 2, 2, true>(p, cus, stream); break;
+    default: launch_skinny_form<MODE, 2, 3, true>(p, cus, stream); break;
+  }
+}
+
+int launch_skinny_rows_bf16(const SkinnyParams& p, bool pow2, int cus, hipStream_t stream) {
+  if (pow2) launch_skinny_bf16<kSkinnyPow2>(p, cus, stream);
+  else launch_skinny_bf16<kSkinnyBlock>(p, cus, stream);
+  return check_launch("linear (few rows)");
 }
 
 }  // namespace hpfp8

@@ -36,7 +36,7 @@ constexpr int64_t kBlock = 128;
   X(hpfp8_quantize_1x128_and_128x1_t_pow2_bf16) X(hpfp8_quantize_128x1_t_colsum_bf16) X(hpfp8_quantize_rows_128x1_t_bf16) \
   X(hpfp8_column_sum_finish) X(hpfp8_quantize_128x128_bf16) X(hpfp8_quantize_128x128_pow2_bf16) \
   X(hpfp8_quantize_per_tensor_t_bf16) X(hpfp8_transpose_codes) X(hpfp8_gemm_blockwise) X(hpfp8_gemm_blockwise_pow2) X(hpfp8_gemm_per_tensor) \
-  X(hpfp8_quantize_per_tensor_sync_bf16) X(hpfp8_gemm_few_rows) X(hpfp8_gemm_blockwise_swiglu_quantize) X(hpfp8_swiglu_quantize_1x128_bf16) \
+  X(hpfp8_quantize_per_tensor_sync_bf16) X(hpfp8_gemm_few_rows) X(hpfp8_linear_few_rows) X(hpfp8_linear_few_rows_bf16) X(hpfp8_gemm_blockwise_swiglu_quantize) X(hpfp8_swiglu_quantize_1x128_bf16) \
   X(hpfp8_swiglu_quantize_1x128_pow2_bf16) X(hpfp8_swiglu_quantize_1x128_fast_bf16) X(hpfp8_gemm_grouped_blockwise) \
   X(hpfp8_bucket_pack_quantize_bf16) X(hpfp8_bucket_unpack_dequantize_bf16)
 struct Library {
@@ -564,6 +564,18 @@ void multiply_rows(const Rows& r, const at::Tensor& w, const at::Tensor& sw, con
                sw.stride(0), sw.stride(1), (int)kBlock, m, n, k, bias, c.data_ptr(), n, HPFP8_OUT_BF16, 0, stream);
 }
 
+// c = x . weight^T (+ bias) of m rows of bf16, quantized here or, where that is the better form, inside the product.
+void multiply_source(const at::Tensor& x, int64_t m, int64_t k, const at::Tensor& w, const at::Tensor& sw, const void* bias, const at::Tensor& c, bool pow2,
+                     void* stream, Call& call) {
+  if (m <= lib.hpfp8_linear_few_rows(w.size(0), k) && (uintptr_t)x.data_ptr() % 16 == 0) {
+    HPFP8_CALL(call, hpfp8_linear_few_rows_bf16, x.data_ptr(), w.data_ptr(), row_stride(w), f32(sw), sw.stride(0), sw.stride(1), m, w.size(0), k, pow2,
+               bias, c.data_ptr(), w.size(0), HPFP8_OUT_BF16, stream);
+    return;
+  }
+  const Rows r = make_rows(x, m, k, pow2, stream, call);
+  if (call.ok()) multiply_rows(r, w, sw, bias, c, pow2, stream, call);
+}
+
 // (x, weight, bias or None, the weight's codes, scale_inv, codes_t or None each, per_tensor, pow2, device, stream) -> y with its place in
 // the graph: forward of what `trains` has taken (hpfp8/linear.py _trained) in one call.  A blockwise weight that has no FP8 form yet is
 // left to the operators one by one (quantizing it dominates such a step).
@@ -660,11 +672,8 @@ PyObject* linear_infer(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
         }
       }
     } else {
-      const Rows r = make_rows(*x, m, k, pow2, at_.stream, call);
-      if (call.ok()) {
-        y = new_rows_like(*x, n);
-        multiply_rows(r, *w, *sw, b, y, pow2, at_.stream, call);
-      }
+      y = new_rows_like(*x, n);
+      multiply_source(*x, m, k, *w, *sw, b, y, pow2, at_.stream, call);
     }
   }
   if (!taken) Py_RETURN_NONE;
@@ -688,14 +697,15 @@ PyObject* swiglu_mlp_infer(PyObject*, PyObject* const* args, Py_ssize_t n_args) 
   Call call;
   {
     pybind11::gil_scoped_release free;
-    const Rows r = make_rows(*x, m, k, pow2, at_.stream, call);
-    Rows a;
+    // (ops.gemm_blockwise_swiglu_quantize has the reason for the two forms)
+    const bool two_steps = m <= lib.hpfp8_gemm_few_rows(k) && n * row_stride(*gu) < 0x7FFFF000;
+    Rows r, a;
+    if (!two_steps) r = make_rows(*x, m, k, pow2, at_.stream, call);
     if (call.ok()) {
       a = Rows{new_codes(*x, m, inter), new_floats_t(*x, m, inter / kBlock)};
-      // (ops.gemm_blockwise_swiglu_quantize has the reason for the two forms)
-      if (m <= lib.hpfp8_gemm_few_rows(k) && n * row_stride(*gu) < 0x7FFFF000) {
+      if (two_steps) {
         const at::Tensor h = at::empty({m, n}, x->options().requires_grad(false));
-        multiply_rows(r, *gu, *sgu, nullptr, h, pow2, at_.stream, call);
+        multiply_source(*x, m, k, *gu, *sgu, nullptr, h, pow2, at_.stream, call);
         if (call.ok()) {
           if (fast)
             HPFP8_CALL(call, hpfp8_swiglu_quantize_1x128_fast_bf16, h.data_ptr(), m, inter, n, 1, pow2_down, a.q.data_ptr(), nullptr, f32(a.s), nullptr, at_.stream);

@@ -63,6 +63,7 @@ SIGNATURES = {
                                   _vp, _i64, _int, _int, _vp],
     "hpfp8_gemm_blockwise_swiglu_quantize": [_vp, _i64, _vp, _i64, _i64, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _i64,
                                              _int, _int, _int, _vp, _i64, _vp, _vp, _vp],
+    "hpfp8_linear_few_rows_bf16": [_vp, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _i64, _int, _vp, _vp, _i64, _int, _vp],
     "hpfp8_gemm_per_tensor": [_vp, _i64, _vp, _vp, _i64, _vp, _i64, _i64, _i64, _vp, _vp, _i64, _int, _vp],
     "hpfp8_gemm_grouped_blockwise": [_vp, _i64, _vp, _i64, _i64, _vp, _vp, _vp, _int, _i64, _i64, _i64, _vp, _i64,
                                      _int, _vp],
@@ -80,6 +81,7 @@ SIZE_FUNCTIONS = {
     "hpfp8_grouped_padded_rows": [_int, _i64],
     "hpfp8_grouped_layout_words": [_int, _i64],
     "hpfp8_gemm_few_rows": [_i64],
+    "hpfp8_linear_few_rows": [_i64, _i64],
 }
 
 OUT_BF16, OUT_F32 = 0, 1

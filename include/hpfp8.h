@@ -378,7 +378,7 @@ int hpfp8_gemm_per_tensor(const void* a, int64_t lda, const float* sa_inv, const
 
 /* Forms of the GEMMs.  They take the smallest output tile with which a problem is still one tile per compute unit (64 x 64, 64 x 128,
  * 128 x 128, 128 x 256), and otherwise 256 x 256 or, where those would leave most of a second round idle, 128 x 256; the forms grouped by rows take 64 x 64, 64 x 128, 128 x 256 or 256 x 256 ones, which
- * the kernel chooses where the host cannot know.  With at most 64 rows and K >= 2048
+ * the kernel chooses where the host cannot know.  With at most 64 rows and K >= 512
  * hpfp8_gemm_per_tensor and hpfp8_gemm_blockwise[_pow2] with sb_gran = 128 (no accumulate) take a form that reads b once at
  * the memory's rate.  Same arithmetic in the same order in all of them: an element of c has the same bits in each, so it
  * depends neither on the number of rows nor on where b's rows stand (a column shard).  Test hook, not part of the path: mode
@@ -391,6 +391,15 @@ void hpfp8_debug_set_small_gemm(int mode);
  * hpfp8_gemm_per_tensor have for decode steps is worth more than a fused call at contraction K (0: none): a caller that can choose
  * between a fused call and one of these followed by another launch asks here. */
 int64_t hpfp8_gemm_few_rows(int64_t K);
+
+/* quantize_1x128 (power-of-two scales with pow2) of x and hpfp8_gemm_blockwise[_pow2] (sb_gran = 128, no accumulate) in one launch, with
+ * their bits, for at most 8 rows: x[M, K] is contiguous bf16, 16-byte aligned, and its codes and scales stay in the kernel.  The other
+ * arguments are those of hpfp8_gemm_blockwise.  hpfp8_linear_few_rows: the rows up to which that is the form to take with b[N, K]
+ * (0: two launches are as fast). */
+int hpfp8_linear_few_rows_bf16(const void* x, const void* b, int64_t ldb, const float* sb, int64_t sb_stride_n, int64_t sb_stride_k,
+                               int64_t M, int64_t N, int64_t K, int pow2, const void* bias, void* c, int64_t ldc, int out_type,
+                               hpfp8_stream_t stream);
+int64_t hpfp8_linear_few_rows(int64_t N, int64_t K);
 
 /* MoE grouped form (one rank's local experts; no counterpart in the reference, whose expert
  * parallelism is unimplemented): rows of a[total_m, K] (row stride lda) are sorted by expert; offs[e] (int32,

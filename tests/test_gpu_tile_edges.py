@@ -171,6 +171,34 @@ def test_gemm_with_few_rows_keeps_nan_and_infinity_to_their_rows(gpu, m, pow2):
         assert torch.equal(got[keep], clean[keep])
 
 
+@pytest.mark.parametrize("m", [1, 2, 7, 8])
+@pytest.mark.parametrize("n,k", [(128, 128), (256, 512), (1152, 640), (4096, 2432), (7168, 4096), (8320, 1152), (36864, 512)])
+def test_rows_quantized_inside_the_few_rows_product_have_the_bits_of_the_two_launches(gpu, m, n, k):
+    """1, 2 and 3 fragments of columns per workgroup, one run of them and several, k-blocks that fill the last stage and that do not;
+    a row of zeros, one below the smallest scale, and a NaN and an infinity that stay in their row."""
+    from hpfp8 import _lib, ops
+    x, w = _normal((m, k), 1, gpu, outliers=True), _normal((n, k), 2, gpu, 0.02)
+    bias = _normal((n,), 3, gpu)
+    if m > 2:
+        x[1] = 0.0
+        x[2] *= 2.0 ** -60
+    x_bad = x.clone()
+    x_bad[-1, 5], x_bad[-1, k - 1] = float("nan"), float("inf")
+    for pow2 in (False, True):
+        b, sb = ops.quantize_128x128(w, pow2=pow2)
+        for src in (x, x_bad):
+            q, s = ops.quantize_1x128(src, kmajor=True, pow2=pow2)
+            for dtype, with_bias in ((torch.bfloat16, bias), (torch.float32, None)):
+                want = ops.gemm_blockwise(q, s, b, sb, bias=with_bias, pow2_scales=pow2, out_dtype=dtype)
+                c = torch.full((m + 1, n + 8), 7.0, dtype=dtype, device=gpu)
+                _lib.call("hpfp8_linear_few_rows_bf16", src.data_ptr(), b.data_ptr(), b.stride(0), sb.data_ptr(), sb.stride(0), sb.stride(1),
+                          m, n, k, pow2, None if with_bias is None else with_bias.data_ptr(), c.data_ptr(), c.stride(0),
+                          _lib.OUT_F32 if dtype == torch.float32 else _lib.OUT_BF16, ops._stream())
+                assert torch.equal(c[:m, :n].nan_to_num(3.0), want.nan_to_num(3.0))
+                assert torch.equal(c[:m, :n].isnan(), want.isnan())
+                assert bool((c[:m, n:] == 7.0).all()) and bool((c[m] == 7.0).all())
+
+
 def test_gemm_with_few_rows_and_power_of_two_scales_whose_product_is_out_of_range(gpu):
     """Two scales of 2^80: their product is no fp32 number, but a product of codes that is zero stays zero."""
     from hpfp8 import ops
