@@ -281,6 +281,7 @@ __device__ __forceinline__ v4f scale_products(float sb, float sa, int sub) {
 
 // group: grouped by rows, the first 64 experts with their ends; then those among which tiles are looked up (tile numbers are
 // asked for in increasing order).
+// pid, nwg: this workgroup among those that share the tile list.
 // SA4: the activation scales have unit stride over rows (the k-block-major layout), so a lane's four
 // of them are one 16-byte load.
 // EPI: 0 = c is the GEMM's result; 1 / 2 = the gate/up projection of a SwiGLU MLP with the activation and its
@@ -288,7 +289,7 @@ __device__ __forceinline__ v4f scale_products(float sb, float sa, int sub) {
 // 256 columns are then the 128 gate columns and the 128 up columns of one scaling group of the activation: the b
 // tile's upper 128 rows come from `inter` rows further down, the two waves that share 64 rows hold gate and up.
 template <int MODE, int GROUPED, bool OUT_F32, bool ACC, bool SA4, int EPI, int WM, int NS, int WN>
-__device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const lds, ExpertChunk group) {
+__device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const lds, ExpertChunk group, const int pid, const int nwg) {
   constexpr int TM = 64 * WM, TN = 16 * NS * WN;       // the tile
   constexpr int WC = 16 * NS;                          // a wave's columns
   constexpr int kWaves = WM * WN;                      // that multiply
@@ -347,7 +348,6 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
   }
   int my_tiles, t_first, t_step;
   {
-    const int nwg = gridDim.x, pid = blockIdx.x;
     // (the host launches a multiple of 8 workgroups, or fewer than 8)
     const bool few = nwg < kXcds;
     const int xcd = few ? pid : pid % kXcds, slot = few ? 0 : pid / kXcds;
@@ -1176,7 +1176,7 @@ __global__ __launch_bounds__(tile_threads(WM, WN)) void gemm_kernel(const GemmPa
   __shared__ __attribute__((aligned(1024))) uint8_t lds[tile_lds(MODE, WM, 16 * NS * WN)];
   ExpertChunk group{0, 0, 0, 0, 0};
   if (GROUPED == kGroupedRows) expert_ends(group, p, threadIdx.x & 63);
-  gemm_tiles<MODE, GROUPED, OUT_F32, ACC, SA4, EPI, WM, NS, WN>(p, lds, group);
+  gemm_tiles<MODE, GROUPED, OUT_F32, ACC, SA4, EPI, WM, NS, WN>(p, lds, group, blockIdx.x, gridDim.x);
 }
 
 // Grouped by rows, the tile chosen here, where the experts' rows are known.
@@ -1188,9 +1188,59 @@ __global__ __launch_bounds__(512) void gemm_grouped_kernel(const GemmParams p) {
   ExpertChunk group{0, 0, 0, 0, 0};
   expert_ends(group, p, threadIdx.x & 63);
   const int rows = p.choose_cus < 0 ? -p.choose_cus : grouped_tile_rows(group, p, threadIdx.x & 63);
-  if (rows == 64) gemm_tiles<MODE, kGroupedRows, OUT_F32, false, false, 0, 1, 2, 4>(p, lds, group);
-  else if (rows == 128) gemm_tiles<MODE, kGroupedRows, OUT_F32, false, false, 0, 2, 8, 2>(p, lds, group);
-  else gemm_tiles<MODE, kGroupedRows, OUT_F32, false, SA4, 0, 4, 8, 2>(p, lds, group);
+  if (rows == 64) gemm_tiles<MODE, kGroupedRows, OUT_F32, false, false, 0, 1, 2, 4>(p, lds, group, blockIdx.x, gridDim.x);
+  else if (rows == 128) gemm_tiles<MODE, kGroupedRows, OUT_F32, false, false, 0, 2, 8, 2>(p, lds, group, blockIdx.x, gridDim.x);
+  else gemm_tiles<MODE, kGroupedRows, OUT_F32, false, SA4, 0, 4, 8, 2>(p, lds, group, blockIdx.x, gridDim.x);
+}
+
+// Backward of a linear: both products, and the column sums that are its bias gradient, in one launch.
+//   * One after the other each product ends in a round of tiles that fills some compute units, and with the few tiles of a small batch
+//     that may be its only one; together the second product's tiles start wherever the first one's have ended.  One tile per workgroup,
+//     longer tiles first, and the hardware deals them out as compute units come free (a tile's workgroup has the compute unit's LDS to
+//     itself); pick_backward has the rule and the figures.
+//   * Any of four tile shapes for either product, chosen by the host.
+struct BackwardParams {
+  GemmParams gemm[2];          // 0: grad_out . W, block scales; 1: grad_out^T . x, per-row scales
+  int shape[2];                // TileShape
+  int first[2], wgs[2];        // each product's workgroups (a multiple of 8 apart: the XCD is the workgroup's number modulo 8)
+  int sums_first;              // from here on: column sums, 512 a workgroup
+  const float* part;
+  int blocks;
+  uint16_t* sums;
+};
+
+enum TileShape { k256x256, k128x256, k128x128, k64x128, k64x64, k64x256 /* SwiGLU epilogue */ };
+
+template <int MODE>
+__device__ __forceinline__ void backward_tile(const GemmParams& p, int shape, int pid, int nwg, uint8_t* lds) {
+  const ExpertChunk none{0, 0, 0, 0, 0};
+  if (shape == k256x256) gemm_tiles<MODE, kDense, false, false, MODE != kScaleTensor, 0, 4, 8, 2>(p, lds, none, pid, nwg);
+  else if (shape == k128x256) gemm_tiles<MODE, kDense, false, false, false, 0, 2, 8, 2>(p, lds, none, pid, nwg);
+  else if (shape == k128x128) gemm_tiles<MODE, kDense, false, false, false, 0, 2, 4, 2>(p, lds, none, pid, nwg);
+  else gemm_tiles<MODE, kDense, false, false, false, 0, 1, 2, 4>(p, lds, none, pid, nwg);
+}
+constexpr int backward_lds(int mode) {
+  int most = 0;
+  const int of[] = {tile_lds(mode, 4, 256), tile_lds(mode, 2, 256), tile_lds(mode, 2, 128), tile_lds(mode, 1, 128)};
+  for (int v : of) most = v > most ? v : most;
+  return most;
+}
+
+template <int MODE, int MODE_W>
+__global__ __launch_bounds__(512) void gemm_backward_kernel(const BackwardParams q) {
+  static_assert(tile_threads(4, 2) == 512 && tile_threads(2, 2) == 512 && tile_threads(1, 4) == 512, "");
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[backward_lds(MODE) > backward_lds(MODE_W) ? backward_lds(MODE) : backward_lds(MODE_W)];
+  const int wg = blockIdx.x;
+  if (wg >= q.sums_first) {
+    const int col = (wg - q.sums_first) * 512 + threadIdx.x;
+    if (col < q.gemm[1].M) q.sums[col] = __builtin_bit_cast(uint16_t, (__bf16)column_sum_in_block_order(q.part, q.blocks, q.gemm[1].M, col));
+    return;
+  }
+  const int one = wg >= q.first[1] && wg < q.first[1] + q.wgs[1];
+  const int pid = wg - q.first[one];
+  if (pid < 0 || pid >= q.wgs[one]) return;       // (behind a first product of fewer than 8 workgroups)
+  if (one) backward_tile<MODE_W>(q.gemm[1], q.shape[1], pid, q.wgs[1], lds);
+  else backward_tile<MODE>(q.gemm[0], q.shape[0], pid, q.wgs[0], lds);
 }
 
 // Test hook.  0: pick_shape and the rules below choose the form; 1: always 256 x 256 tiles; 2: the smallest tile a form has;
@@ -1214,8 +1264,6 @@ static int persistent_grid(int64_t tiles) {
 }
 
 // The tile of a GEMM: 256 x 256 (8 waves), 128 x 256, 128 x 128 or 64 x 128 (4 waves that multiply, 4 that fetch) or 64 x 64 (2 and 4).
-enum TileShape { k256x256, k128x256, k128x128, k64x128, k64x64, k64x256 /* SwiGLU epilogue */ };
-
 static int64_t shape_rows(TileShape shape) { return shape == k256x256 ? 256 : (shape == k128x256 || shape == k128x128 ? 128 : 64); }
 static int64_t shape_cols(TileShape shape) { return shape == k64x64 ? 64 : (shape == k128x128 || shape == k64x128 ? 128 : 256); }
 
@@ -1296,12 +1344,81 @@ static GroupedTiles pick_grouped(int64_t M, int64_t N, int experts) {
   return M > (int64_t)256 * experts && M / 256 * ((N + 255) / 256) >= 2 * cus ? kHighTiles : kChosenTiles;
 }
 
-// Few rows of a (decode): bound by reading b once, which the tile kernels do not reach (gemm_skinny.hip; 8 rows of
-// [7168, 16384]: 60 us with 64 x 128 tiles, 20.6 us; 64 rows: 64 and 26.8 us; 37 rows of [36864, 7168]: 81 us with 256 x 256
-// tiles, 41.6 us), with the same bits.  try_skinny hands the problem over if it is one; otherwise false.
 static int64_t few_rows(int64_t K) {        // the most rows that count as few
   return K >= kSkinnyMinK && g_small_gemm_mode.load(std::memory_order_relaxed) == 0 ? kSkinnyMaxRows : 0;
 }
+
+// Both products of a linear's backward in one launch (gemm_backward_kernel) where that is shorter by more than a thirty-second: the time
+// at which the last tile ends when the longer ones are dealt out first, for any of four shapes each, against the rounds of two launches
+// and what lies between them.  A tile's time is that of its k-blocks in a full round and, for its first k-block and its stores, about
+// what a launch of one such tile takes (ns).  us in three launches / in one, tokens x outputs x inputs:
+//   block  1531 x 2048 x 7168     57 / 51       1400 x 4096 x 4096   61 / 53       2048 x 1024 x 1024  17.7 / 10.3
+//   block   256 x 1024 x 1024   13.4 / 7.5       512 x 4096 x 4096   32 / 25       8192 x 1024 x 1024  39.3 / 31.5
+//   block  4096 x 7168 x 7168    391 / 364      5000 x 5120 x 13824  659 / 633     3000 x 7168 x 2048   100 / 93
+//   pow2    750 x 2432 x 3840   28.3 / 17.9     tensor  2048 x 1024 x 1024  15.5 / 9.4     1024 x 4096 x 2048  26.5 / 18.9
+// Whole rounds, and many of them, are as fast one after the other: 4096 x 7168 x 16384 806 / 806 to 818.
+static int64_t tile_time(TileShape shape, int64_t kblocks) {
+  switch (shape) {
+    case k256x256: return 5000 + 1300 * kblocks;
+    case k128x256: return 3500 + 900 * kblocks;
+    case k128x128: return 2500 + 600 * kblocks;
+    case k64x128: return 2000 + 440 * kblocks;
+    default: return 2000 + 310 * kblocks;
+  }
+}
+constexpr int64_t kLaunchTime = 3000;
+
+// t1 tiles of d1 each, then t2 tiles of d2 <= d1, each to the compute unit that is free first
+static int64_t dealt_out(int64_t t1, int64_t d1, int64_t t2, int64_t d2, int64_t cus) {
+  const int64_t rounds = t1 / cus, rest = t1 % cus, low = rounds * d1, high = low + (rest ? d1 : 0);
+  auto room = [&](int64_t t) { return (t >= high ? rest * ((t - high) / d2) : 0) + (cus - rest) * ((t - low) / d2); };
+  int64_t j_low = high > low ? (high - low + d2 - 1) / d2 : 0, j_high = 0;
+  for (int64_t t = high;;) {
+    if (room(t) >= t2) return t;
+    const int64_t a = low + j_low * d2, b = high + j_high * d2;
+    t = a < b ? a : b;
+    if (a <= t) ++j_low;
+    if (b <= t) ++j_high;
+  }
+}
+
+static bool pick_backward(int64_t M, int64_t N, int64_t K, int64_t padded, int launches, TileShape shape[2]) {
+  const int mode = g_small_gemm_mode.load(std::memory_order_relaxed);
+  const TileShape shapes[] = {k256x256, k128x256, k128x128, k64x128};
+  if (mode != 0) {                       // (test hook: that shape for both)
+    if (mode == 2) return false;
+    shape[0] = shape[1] = mode == 1 ? k256x256 : (mode == 3 ? k128x256 : (mode == 4 ? k128x128 : k64x128));
+    return true;
+  }
+  if (M <= few_rows(N)) return false;
+  const int64_t cus = persistent_grid((int64_t)1 << 40);
+  const int64_t kb[2] = {N / BK, padded / BK}, rows[2] = {M, N};
+  int64_t apart = (launches - 1) * kLaunchTime;
+  for (int i = 0; i < 2; ++i) {
+    const TileShape s = pick_shape(rows[i], K);
+    apart += tile_time(s, (tile_count(rows[i], K, s) + cus - 1) / cus * kb[i]);      // (a workgroup's tiles follow each other without a gap)
+  }
+  int64_t best = INT64_MAX, best_end = 0;
+  for (TileShape s0 : shapes)
+    for (TileShape s1 : shapes) {
+      const int64_t t[2] = {tile_count(rows[0], K, s0), tile_count(rows[1], K, s1)};
+      const int64_t d[2] = {tile_time(s0, kb[0]), tile_time(s1, kb[1])};
+      const int longer = d[1] > d[0] ? 1 : 0;
+      const int64_t end = dealt_out(t[longer], d[longer], t[1 - longer], d[1 - longer], cus);
+      const int64_t cost = end + (t[0] * d[0] + t[1] * d[1]) / (8 * cus);       // (of forms that end together the one with less to move)
+      if (cost < best) {
+        best = cost;
+        best_end = end;
+        shape[0] = s0;
+        shape[1] = s1;
+      }
+    }
+  return best_end < apart - apart / 32;
+}
+
+// Few rows of a (decode): bound by reading b once, which the tile kernels do not reach (gemm_skinny.hip; 8 rows of
+// [7168, 16384]: 60 us with 64 x 128 tiles, 20.6 us; 64 rows: 64 and 26.8 us; 37 rows of [36864, 7168]: 81 us with 256 x 256
+// tiles, 41.6 us), with the same bits.  try_skinny hands the problem over if it is one; otherwise false.
 
 // Below this contraction a fused epilogue on tiles is still the better choice with few rows than the few-rows form and a launch
 // behind it: what those save on the GPU (weight [8192, 1024], 8 rows 11.6 -> 9.0 us; [36864, 512], 64 rows 9.9 -> 13.5) the second
@@ -1427,14 +1544,14 @@ using namespace hpfp8;
 
 extern "C" {
 
-static int gemm_blockwise_impl(const void* a, int64_t lda, const float* sa, int64_t sa_stride_m, int64_t sa_stride_k,
-                               const void* b, int64_t ldb, const float* sb, int64_t sb_stride_n, int64_t sb_stride_k,
-                               int sb_gran, int64_t M, int64_t N, int64_t K, const void* bias, void* c,
-                               int64_t ldc, int out_type, int accumulate, bool pow2, hpfp8_stream_t stream) {
+// checks and kernel arguments of a product with block scales or (sb_gran 1) per-row scales; 1: there is something to launch
+static int blockwise_params(const void* a, int64_t lda, const float* sa, int64_t sa_stride_m, int64_t sa_stride_k,
+                            const void* b, int64_t ldb, const float* sb, int64_t sb_stride_n, int64_t sb_stride_k,
+                            int sb_gran, int64_t M, int64_t N, int64_t K, const void* bias, void* c,
+                            int64_t ldc, int out_type, int accumulate, GemmParams& p) {
   HPFP8_REQUIRE(sb_gran == 1 || sb_gran == 128, HPFP8_ERR_ARG, "gemm_blockwise: sb_gran must be 1 or 128");
   int rc = check_common("gemm_blockwise", a, lda, b, ldb, sa, sb, M, N, K, bias, c, ldc, out_type, accumulate);
   if (rc <= 0) return rc;
-  GemmParams p{};
   p.a = (const uint8_t*)a; p.b = (const uint8_t*)b; p.sa = sa; p.sb = sb; p.lda = lda; p.ldb = ldb;
   p.sa_sm = sa_stride_m; p.sa_sk = sa_stride_k; p.sb_sn = sb_stride_n; p.sb_sk = sb_stride_k;
   rc = check_scale_span("gemm_blockwise", M, K / BK, sa_stride_m, sa_stride_k, "sa");
@@ -1444,11 +1561,7 @@ static int gemm_blockwise_impl(const void* a, int64_t lda, const float* sa, int6
   p.sb_bytes = (int)(((N / kBlock - 1) * sb_stride_n + (K / BK - 1) * sb_stride_k + 1) * 4);
   p.c = c; p.ldc = ldc; p.bias = (const uint16_t*)bias;
   p.M = (int)M; p.N = (int)N; p.K = (int)K; p.accumulate = accumulate;
-  if (sb_gran == 128) {
-    if (try_skinny(p, pow2 ? kSkinnyPow2 : kSkinnyBlock, out_type, (hipStream_t)stream, rc)) return rc;
-    if (pow2) return launch<kScalePow2, kDense>(p, out_type, pick_shape(M, N), (hipStream_t)stream);
-    return launch<kScaleBlock, kDense>(p, out_type, pick_shape(M, N), (hipStream_t)stream);
-  }
+  if (sb_gran == 128) return 1;
   // per-row b scales travel to LDS as one contiguous 1 KB piece per k-block
   if (K == BK) sb_stride_k = N;     // a single k-block: the stride between k-blocks is never used
   p.sb_sk = sb_stride_k;
@@ -1457,8 +1570,45 @@ static int gemm_blockwise_impl(const void* a, int64_t lda, const float* sa, int6
                 "16-byte aligned rows)");
   HPFP8_REQUIRE(((K / BK - 1) * sb_stride_k + N) * 4 < (int64_t)0x7FFFFFFF, HPFP8_ERR_SHAPE,
                 "gemm_blockwise: b scale array too large");
-  if (pow2) return launch<kScalePow2Row, kDense>(p, out_type, pick_shape(M, N), (hipStream_t)stream);
-  return launch<kScaleRow, kDense>(p, out_type, pick_shape(M, N), (hipStream_t)stream);
+  return 1;
+}
+
+static int launch_blockwise(const GemmParams& p, int sb_gran, int out_type, bool pow2, hipStream_t stream) {
+  const TileShape shape = pick_shape(p.M, p.N);
+  int rc;
+  if (sb_gran == 128) {
+    if (try_skinny(p, pow2 ? kSkinnyPow2 : kSkinnyBlock, out_type, stream, rc)) return rc;
+    if (pow2) return launch<kScalePow2, kDense>(p, out_type, shape, stream);
+    return launch<kScaleBlock, kDense>(p, out_type, shape, stream);
+  }
+  if (pow2) return launch<kScalePow2Row, kDense>(p, out_type, shape, stream);
+  return launch<kScaleRow, kDense>(p, out_type, shape, stream);
+}
+
+static int per_tensor_params(const void* a, int64_t lda, const float* sa_inv, const void* b, int64_t ldb, const float* sb_inv, int64_t M,
+                             int64_t N, int64_t K, const void* bias, void* c, int64_t ldc, int out_type, GemmParams& p) {
+  int rc = check_common("gemm_per_tensor", a, lda, b, ldb, sa_inv, sb_inv, M, N, K, bias, c, ldc, out_type, 0);
+  if (rc <= 0) return rc;
+  p.a = (const uint8_t*)a; p.b = (const uint8_t*)b; p.sa = sa_inv; p.sb = sb_inv; p.lda = lda; p.ldb = ldb;
+  p.c = c; p.ldc = ldc; p.bias = (const uint16_t*)bias;
+  p.M = (int)M; p.N = (int)N; p.K = (int)K;
+  return 1;
+}
+
+static int launch_per_tensor(const GemmParams& p, int out_type, hipStream_t stream) {
+  int rc;
+  if (try_skinny(p, kSkinnyTensor, out_type, stream, rc)) return rc;
+  return launch<kScaleTensor, kDense>(p, out_type, pick_shape(p.M, p.N), stream);
+}
+
+static int gemm_blockwise_impl(const void* a, int64_t lda, const float* sa, int64_t sa_stride_m, int64_t sa_stride_k,
+                               const void* b, int64_t ldb, const float* sb, int64_t sb_stride_n, int64_t sb_stride_k,
+                               int sb_gran, int64_t M, int64_t N, int64_t K, const void* bias, void* c,
+                               int64_t ldc, int out_type, int accumulate, bool pow2, hpfp8_stream_t stream) {
+  GemmParams p{};
+  const int rc = blockwise_params(a, lda, sa, sa_stride_m, sa_stride_k, b, ldb, sb, sb_stride_n, sb_stride_k, sb_gran, M, N, K, bias, c, ldc,
+                                  out_type, accumulate, p);
+  return rc <= 0 ? rc : launch_blockwise(p, sb_gran, out_type, pow2, (hipStream_t)stream);
 }
 
 int hpfp8_gemm_blockwise(const void* a, int64_t lda, const float* sa, int64_t sa_stride_m, int64_t sa_stride_k,
@@ -1564,14 +1714,65 @@ int hpfp8_linear_few_rows_bf16(const void* x, const void* b, int64_t ldb, const 
 int hpfp8_gemm_per_tensor(const void* a, int64_t lda, const float* sa_inv, const void* b, int64_t ldb,
                           const float* sb_inv, int64_t M, int64_t N, int64_t K, const void* bias, void* c,
                           int64_t ldc, int out_type, hpfp8_stream_t stream) {
-  int rc = check_common("gemm_per_tensor", a, lda, b, ldb, sa_inv, sb_inv, M, N, K, bias, c, ldc, out_type, 0);
-  if (rc <= 0) return rc;
   GemmParams p{};
-  p.a = (const uint8_t*)a; p.b = (const uint8_t*)b; p.sa = sa_inv; p.sb = sb_inv; p.lda = lda; p.ldb = ldb;
-  p.c = c; p.ldc = ldc; p.bias = (const uint16_t*)bias;
-  p.M = (int)M; p.N = (int)N; p.K = (int)K;
-  if (try_skinny(p, kSkinnyTensor, out_type, (hipStream_t)stream, rc)) return rc;
-  return launch<kScaleTensor, kDense>(p, out_type, pick_shape(M, N), (hipStream_t)stream);
+  const int rc = per_tensor_params(a, lda, sa_inv, b, ldb, sb_inv, M, N, K, bias, c, ldc, out_type, p);
+  return rc <= 0 ? rc : launch_per_tensor(p, out_type, (hipStream_t)stream);
+}
+
+int hpfp8_linear_backward(const hpfp8_operand* go, const hpfp8_operand* wt, const hpfp8_operand* go_t, const hpfp8_operand* xt, int64_t M,
+                          int64_t N, int64_t K, void* dx, void* dw, const float* partial, void* db, int recipe, hpfp8_stream_t stream) {
+  const char* what = "linear_backward";
+  HPFP8_REQUIRE(go && wt && go_t && xt && (db == nullptr || partial != nullptr), HPFP8_ERR_ARG, "%s: null argument", what);
+  HPFP8_REQUIRE(recipe >= HPFP8_BLOCKWISE && recipe <= HPFP8_PER_TENSOR, HPFP8_ERR_ARG, "%s: bad recipe", what);
+  HPFP8_REQUIRE(M > 0 && N > 0 && K > 0, HPFP8_ERR_SHAPE, "%s: bad shape", what);
+  const int64_t padded = (M + kBlock - 1) / kBlock * kBlock;
+  hipStream_t st = (hipStream_t)stream;
+  BackwardParams q{};
+  int rc[2];
+  if (recipe == HPFP8_PER_TENSOR) {
+    rc[0] = per_tensor_params(go->codes, go->ld, go->scale_inv, wt->codes, wt->ld, wt->scale_inv, M, K, N, nullptr, dx, K, HPFP8_OUT_BF16, q.gemm[0]);
+    if (rc[0] < 0) return rc[0];
+    rc[1] = per_tensor_params(go_t->codes, go_t->ld, go_t->scale_inv, xt->codes, xt->ld, xt->scale_inv, N, K, padded, nullptr, dw, K, HPFP8_OUT_BF16,
+                              q.gemm[1]);
+  } else {
+    rc[0] = blockwise_params(go->codes, go->ld, go->scale_inv, go->stride_r, go->stride_k, wt->codes, wt->ld, wt->scale_inv, wt->stride_r,
+                             wt->stride_k, 128, M, K, N, nullptr, dx, K, HPFP8_OUT_BF16, 0, q.gemm[0]);
+    if (rc[0] < 0) return rc[0];
+    rc[1] = blockwise_params(go_t->codes, go_t->ld, go_t->scale_inv, go_t->stride_r, go_t->stride_k, xt->codes, xt->ld, xt->scale_inv, xt->stride_r,
+                             xt->stride_k, 1, N, K, padded, nullptr, dw, K, HPFP8_OUT_BF16, 0, q.gemm[1]);
+  }
+  if (rc[1] < 0) return rc[1];
+  TileShape shape[2];
+  const bool k_major = recipe == HPFP8_PER_TENSOR || (go->stride_r == 1 && go_t->stride_r == 1);
+  if (k_major && pick_backward(M, N, K, padded, db ? 3 : 2, shape)) {
+    const int64_t tiles[2] = {tile_count(M, K, shape[0]), tile_count(N, K, shape[1])};
+    const int64_t kblocks[2] = {N / BK, padded / BK};
+    const int longer = tile_time(shape[1], kblocks[1]) > tile_time(shape[0], kblocks[0]) ? 1 : 0;
+    for (int i = 0; i < 2; ++i) {
+      q.gemm[i].tiles = (int)tiles[i];
+      q.shape[i] = shape[i];
+      q.wgs[i] = (int)(tiles[i] < kXcds ? tiles[i] : (tiles[i] + kXcds - 1) / kXcds * kXcds);
+    }
+    const int second = (q.wgs[longer] + kXcds - 1) / kXcds * kXcds;
+    q.first[longer] = 0;
+    q.first[1 - longer] = second;
+    q.sums_first = second + q.wgs[1 - longer];
+    q.part = partial;
+    q.blocks = (int)(padded / kBlock);
+    q.sums = (uint16_t*)db;
+    const dim3 grid((unsigned)(q.sums_first + (db ? (N + 511) / 512 : 0))), block(512);
+    if (recipe == HPFP8_PER_TENSOR) gemm_backward_kernel<kScaleTensor, kScaleTensor><<<grid, block, 0, st>>>(q);
+    else if (recipe == HPFP8_BLOCKWISE_POW2) gemm_backward_kernel<kScalePow2, kScalePow2Row><<<grid, block, 0, st>>>(q);
+    else gemm_backward_kernel<kScaleBlock, kScaleRow><<<grid, block, 0, st>>>(q);
+    return check_launch(what);
+  }
+  int status = HPFP8_OK;
+  if (db) status = hpfp8_column_sum_finish(partial, padded / kBlock, N, db, nullptr, stream);
+  for (int i = 0; i < 2 && status == HPFP8_OK; ++i) {
+    if (recipe == HPFP8_PER_TENSOR) status = launch_per_tensor(q.gemm[i], HPFP8_OUT_BF16, st);
+    else status = launch_blockwise(q.gemm[i], i == 0 ? 128 : 1, HPFP8_OUT_BF16, recipe == HPFP8_BLOCKWISE_POW2, st);
+  }
+  return status;
 }
 
 static int gemm_grouped_impl(const void* a, int64_t lda, const float* sa, int64_t sa_stride_m, int64_t sa_stride_k,

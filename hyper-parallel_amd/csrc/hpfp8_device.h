@@ -131,6 +131,21 @@ __device__ __forceinline__ uint2 cvt8(const uint4& v, float scale) {
   return r;
 }
 
+// ((0 + part[0][col]) + part[1][col]) + ... in block order
+__device__ __forceinline__ float column_sum_in_block_order(const float* __restrict__ part, int blocks, int k, int col) {
+  float s = 0.f;
+  int b = 0;
+  for (; b + 16 <= blocks; b += 16) {      // sixteen loads in flight, added in block order (the order is the contract)
+    float v[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) v[u] = part[(int64_t)(b + u) * k + col];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) s += v[u];
+  }
+  for (; b < blocks; ++b) s += part[(int64_t)b * k + col];
+  return s;
+}
+
 // ---- SwiGLU arithmetic (shared by the quantizers and the GEMM epilogue) ----
 // exp(t), t clamped to [-86, 89], from IEEE fp32 operations only (no fused multiply-add, no hardware
 // exp), so that the CPU restatement reproduces it bit for bit: k = rint(t * log2 e),

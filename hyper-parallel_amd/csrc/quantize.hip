@@ -1064,16 +1064,7 @@ __global__ __launch_bounds__(64) void column_sum_finish_kernel(const float* __re
                                                                uint16_t* __restrict__ out_bf16, float* __restrict__ out_f32) {
   const int col = blockIdx.x * 64 + threadIdx.x;
   if (col >= k) return;
-  float s = 0.f;
-  int b = 0;
-  for (; b + 16 <= blocks; b += 16) {      // sixteen loads in flight, added in block order (the order is the contract)
-    float v[16];
-#pragma unroll
-    for (int u = 0; u < 16; ++u) v[u] = part[(int64_t)(b + u) * k + col];
-#pragma unroll
-    for (int u = 0; u < 16; ++u) s += v[u];
-  }
-  for (; b < blocks; ++b) s += part[(int64_t)b * k + col];
+  const float s = column_sum_in_block_order(part, blocks, k, col);
   if (out_f32) out_f32[col] = s;
   if (out_bf16) out_bf16[col] = __builtin_bit_cast(uint16_t, (__bf16)s);
 }

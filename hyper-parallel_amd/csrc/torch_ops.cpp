@@ -36,7 +36,7 @@ constexpr int64_t kBlock = 128;
   X(hpfp8_quantize_1x128_and_128x1_t_pow2_bf16) X(hpfp8_quantize_128x1_t_colsum_bf16) X(hpfp8_quantize_rows_128x1_t_bf16) \
   X(hpfp8_column_sum_finish) X(hpfp8_quantize_128x128_bf16) X(hpfp8_quantize_128x128_pow2_bf16) \
   X(hpfp8_quantize_per_tensor_t_bf16) X(hpfp8_transpose_codes) X(hpfp8_gemm_blockwise) X(hpfp8_gemm_blockwise_pow2) X(hpfp8_gemm_per_tensor) \
-  X(hpfp8_quantize_per_tensor_sync_bf16) X(hpfp8_gemm_few_rows) X(hpfp8_linear_few_rows) X(hpfp8_linear_few_rows_bf16) X(hpfp8_gemm_blockwise_swiglu_quantize) X(hpfp8_swiglu_quantize_1x128_bf16) \
+  X(hpfp8_quantize_per_tensor_sync_bf16) X(hpfp8_gemm_few_rows) X(hpfp8_linear_few_rows) X(hpfp8_linear_few_rows_bf16) X(hpfp8_linear_backward) X(hpfp8_gemm_blockwise_swiglu_quantize) X(hpfp8_swiglu_quantize_1x128_bf16) \
   X(hpfp8_swiglu_quantize_1x128_pow2_bf16) X(hpfp8_swiglu_quantize_1x128_fast_bf16) X(hpfp8_gemm_grouped_blockwise) \
   X(hpfp8_bucket_pack_quantize_bf16) X(hpfp8_bucket_unpack_dequantize_bf16)
 struct Library {
@@ -166,15 +166,16 @@ PyObject* quantize_1x128(PyObject*, PyObject* const* args, Py_ssize_t n) {
 // Both operand forms of x from one read of it, and the sum over its rows; any number of rows.
 struct Forms {
   at::Tensor q, s, qt, st, total;        // (per tensor: s is the one scale, st undefined)
+  at::Tensor part;                       // the sum's parts, where it is left to linear_backward
 };
-Forms make_both(const at::Tensor& x, bool pow2, bool column_sum, void* stream, Call& call) {
+Forms make_both(const at::Tensor& x, bool pow2, bool column_sum, void* stream, Call& call, bool finish = true) {
   const int64_t m = x.size(0), k = x.size(1), mp = rows_up(m);
   Forms f;
   f.q = new_codes(x, m, k);
   f.qt = new_codes_t(x, k, mp);
   f.s = new_floats_t(x, m, k / kBlock);
   f.st = new_floats_t(x, k, mp / kBlock);
-  at::Tensor part;
+  at::Tensor& part = f.part;
   if (column_sum) part = new_floats(x, mp / kBlock, k);
   void *const src = x.data_ptr(), *const q = f.q.data_ptr(), *const qt = f.qt.data_ptr();
   const int64_t ld = f.qt.stride(0);
@@ -186,27 +187,27 @@ Forms make_both(const at::Tensor& x, bool pow2, bool column_sum, void* stream, C
     HPFP8_CALL(call, hpfp8_quantize_1x128_and_128x1_t_pow2_bf16, src, m, k, 1, q, nullptr, f32(f.s), qt, ld, nullptr, f32(f.st), stream);
   else
     HPFP8_CALL(call, hpfp8_quantize_1x128_and_128x1_t_bf16, src, m, k, 1, q, nullptr, f32(f.s), qt, ld, nullptr, f32(f.st), stream);
-  if (column_sum && call.ok()) {
-    f.total = at::empty({k}, x.options());
+  if (column_sum) f.total = at::empty({k}, x.options());
+  if (column_sum && finish && call.ok()) {
     HPFP8_CALL(call, hpfp8_column_sum_finish, f32(part), mp / kBlock, k, f.total.data_ptr(), nullptr, stream);
   }
   return f;
 }
 
 // The same with one scale; sync: the block through which the one-launch form's grid agrees on the maximum, or null.
-Forms make_per_tensor(const at::Tensor& x, bool column_sum, uint32_t* sync, void* stream, Call& call) {
+Forms make_per_tensor(const at::Tensor& x, bool column_sum, uint32_t* sync, void* stream, Call& call, bool finish = true) {
   const int64_t m = x.size(0), k = x.size(1), mp = rows_up(m);
   Forms f;
   f.q = new_codes(x, m, k);
   f.qt = new_codes_t(x, k, mp);
   f.s = at::empty({}, x.options().dtype(at::kFloat));
-  at::Tensor part, amax;
+  at::Tensor &part = f.part, amax;
   if (column_sum) part = new_floats(x, mp / kBlock, k);
   if (!sync) amax = at::empty({}, x.options().dtype(at::kFloat));
   HPFP8_CALL(call, hpfp8_quantize_per_tensor_t_bf16, x.data_ptr(), m, k, f.q.data_ptr(), f.qt.data_ptr(), f.qt.stride(0),
              sync ? nullptr : f32(amax), nullptr, f32(f.s), sync, column_sum ? f32(part) : nullptr, stream);
-  if (column_sum && call.ok()) {
-    f.total = at::empty({k}, x.options());
+  if (column_sum) f.total = at::empty({k}, x.options());
+  if (column_sum && finish && call.ok()) {
     HPFP8_CALL(call, hpfp8_column_sum_finish, f32(part), mp / kBlock, k, f.total.data_ptr(), nullptr, stream);
   }
   return f;
@@ -394,6 +395,11 @@ bool floats_again(const at::Tensor& t, const at::Tensor& go, at::IntArrayRef siz
          t.sizes() == sizes;
 }
 
+hpfp8_operand operand(const at::Tensor& codes, const at::Tensor& scale_inv) {
+  const bool one = scale_inv.dim() != 2;
+  return {codes.data_ptr(), row_stride(codes), f32(scale_inv), one ? 0 : scale_inv.stride(0), one ? 0 : scale_inv.stride(1)};
+}
+
 // What forward has made, in Python, for y = x W^T + b with gradients of x and W to come: y, and for backward xt, sxt (per
 // tensor: the one scale), the weight's transposed codes (per tensor with a cached weight: its codes), sw.
 struct Made {
@@ -458,7 +464,7 @@ struct LinearNode : torch::autograd::Function<LinearNode> {
     Call call;
     at::Tensor dx, dw, db;
     if (per_tensor) {
-      Forms f = make_per_tensor(go, has_bias, sync_block(go, mp / kBlock * (out / kBlock) <= kOnePassTiles, current.stream()), stream, call);
+      Forms f = make_per_tensor(go, has_bias, sync_block(go, mp / kBlock * (out / kBlock) <= kOnePassTiles, current.stream()), stream, call, false);
       if (!call.ok()) raise(call);
       at::Tensor wt = w;
       if (!w_transposed) {
@@ -466,22 +472,25 @@ struct LinearNode : torch::autograd::Function<LinearNode> {
         HPFP8_CALL(call, hpfp8_transpose_codes, w.data_ptr(), w.size(0), w.size(1), row_stride(w), wt.data_ptr(), wt.stride(0), stream);
         if (!call.ok()) raise(call);
       }
-      dx = multiply_per_tensor(f.q, f.s, wt, sw, nullptr, stream, call);
-      if (!call.ok()) raise(call);
-      dw = multiply_per_tensor(f.qt, f.s, xt, sxt, nullptr, stream, call);
+      dx = at::empty({m, in}, go.options());
+      dw = at::empty({out, in}, go.options());
+      const hpfp8_operand a = operand(f.q, f.s), b = operand(wt, sw), at = operand(f.qt, f.s), bt = operand(xt, sxt);
+      HPFP8_CALL(call, hpfp8_linear_backward, &a, &b, &at, &bt, m, out, in, dx.data_ptr(), dw.data_ptr(), has_bias ? f32(f.part) : nullptr,
+                 has_bias ? f.total.data_ptr() : nullptr, HPFP8_PER_TENSOR, stream);
       db = std::move(f.total);
     } else {
-      Forms f = make_both(go, pow2, has_bias, stream, call);
+      Forms f = make_both(go, pow2, has_bias, stream, call, false);
       if (!call.ok()) raise(call);
       // dx[M, K] = go[M, N] . W[N, K]: b operand = W^T codes [K, N], its 128x128 scales W's with the two strides swapped
       dx = at::empty({m, in}, go.options());
-      multiply_blockwise(f.q, f.s, w, sw, sw.stride(1), sw.stride(0), nullptr, dx, kBlock, false, pow2, stream, call);
-      if (!call.ok()) raise(call);
       // dW[N, K] = go^T[N, M] . x[M, K]: contraction over the tokens
       dw = at::empty({out, in}, go.options());
       at::Tensor scales = sxt;           // per row, in the kernel's layout
       if (!row_scales_fit(scales)) scales = scales.t().contiguous().t();
-      multiply_blockwise(f.qt, f.st, xt, scales, scales.stride(0), scales.stride(1), nullptr, dw, 1, false, pow2, stream, call);
+      const hpfp8_operand a = operand(f.q, f.s), b{w.data_ptr(), row_stride(w), f32(sw), sw.stride(1), sw.stride(0)};
+      const hpfp8_operand at = operand(f.qt, f.st), bt = operand(xt, scales);
+      HPFP8_CALL(call, hpfp8_linear_backward, &a, &b, &at, &bt, m, out, in, dx.data_ptr(), dw.data_ptr(), has_bias ? f32(f.part) : nullptr,
+                 has_bias ? f.total.data_ptr() : nullptr, pow2 ? HPFP8_BLOCKWISE_POW2 : HPFP8_BLOCKWISE, stream);
       db = std::move(f.total);
     }
     if (!call.ok()) raise(call);

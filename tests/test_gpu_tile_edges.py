@@ -705,3 +705,48 @@ def test_per_row_scales_on_both_operands_are_those_of_their_rows_and_blocks(gpu,
             assert bool(((c.double() - terms.sum(0)).abs() <= kb * 2.0 ** -23 * terms.abs().sum(0)).all())
     finally:
         _lib.load().hpfp8_debug_set_small_gemm(0)
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 128, 128), (100, 128, 384), (256, 128, 256), (129, 256, 256), (65, 1024, 128), (300, 1024, 640), (1531, 2048, 1152), (2048, 1152, 2176)])
+@pytest.mark.parametrize("recipe", [0, 1, 2])
+def test_both_products_of_a_backward_in_one_launch_have_the_bits_of_two(gpu, m, n, k, recipe):
+    """Every tile shape for both products (the sizes end inside tiles of each), the rule's own choice, and the launches one by one; fewer
+    tiles than XCDs, and more than one per compute unit."""
+    import ctypes
+    from hpfp8 import _lib, ops
+
+    class Operand(ctypes.Structure):
+        _fields_ = [("codes", ctypes.c_void_p), ("ld", ctypes.c_int64), ("scale_inv", ctypes.c_void_p), ("stride_r", ctypes.c_int64),
+                    ("stride_k", ctypes.c_int64)]
+
+        def __init__(self, codes, s):
+            strides = s.stride() if s.dim() == 2 else (0, 0)
+            super().__init__(codes.data_ptr(), codes.stride(0), s.data_ptr(), *strides)
+
+    go, x, w = _normal((m, n), 1, gpu, outliers=True), _normal((m, k), 2, gpu, outliers=True), _normal((n, k), 3, gpu, 0.02)
+    blocks = (m + 127) // 128
+    part = torch.randn((blocks, n), generator=torch.Generator("cpu").manual_seed(4)).to(gpu)
+    db = torch.empty(n, dtype=torch.bfloat16, device=gpu)
+    _lib.call("hpfp8_column_sum_finish", part.data_ptr(), blocks, n, db.data_ptr(), None, ops._stream())
+    if recipe == 2:
+        (g, sg, gt), (_, sx, xt), (_, sw, wt) = (ops.quantize_per_tensor_t(t)[:3] for t in (go, x, w))
+        sgt = sg
+        want = [ops.gemm_per_tensor(g, sg, wt, sw), ops.gemm_per_tensor(gt, sg, xt, sx), db]
+    else:
+        g, sg, gt, sgt = ops.quantize_1x128_and_128x1_t_rows(go, pow2=recipe == 1)
+        _, _, xt, sx = ops.quantize_1x128_and_128x1_t_rows(x, pow2=recipe == 1)
+        _, sw, wt = ops.quantize_128x128(w, with_transpose=True, pow2=recipe == 1)
+        sw = sw.t()
+        want = [ops.gemm_blockwise(g, sg, wt, sw, pow2_scales=recipe == 1), ops.gemm_blockwise(gt, sgt, xt, sx, sb_gran=1, pow2_scales=recipe == 1), db]
+    operands = [Operand(g, sg), Operand(wt, sw), Operand(gt, sgt), Operand(xt, sx)]
+    for mode in (0, 1, 2, 3, 4, 5):
+        got = [torch.full(s, 7.0, dtype=torch.bfloat16, device=gpu) for s in ((m + 1, k), (n + 1, k), (n + 8,))]
+        _lib.load().hpfp8_debug_set_small_gemm(mode)
+        try:
+            _lib.call("hpfp8_linear_backward", *(ctypes.addressof(o) for o in operands), m, n, k, got[0].data_ptr(), got[1].data_ptr(),
+                      part.data_ptr(), got[2].data_ptr(), recipe, ops._stream())
+        finally:
+            _lib.load().hpfp8_debug_set_small_gemm(0)
+        for a, b, rows in zip(got, want, (m, n, n)):
+            assert torch.equal(a[:rows], b)
+            assert bool((a[rows:] == 7.0).all())
