@@ -1211,13 +1211,14 @@ struct BackwardParams {
 
 enum TileShape { k256x256, k128x256, k128x128, k64x128, k64x64, k64x256 /* SwiGLU epilogue */ };
 
-template <int MODE>
+// ACC: added onto fp32
+template <int MODE, bool ACC = false>
 __device__ __forceinline__ void backward_tile(const GemmParams& p, int shape, int pid, int nwg, uint8_t* lds) {
   const ExpertChunk none{0, 0, 0, 0, 0};
-  if (shape == k256x256) gemm_tiles<MODE, kDense, false, false, MODE != kScaleTensor, 0, 4, 8, 2>(p, lds, none, pid, nwg);
-  else if (shape == k128x256) gemm_tiles<MODE, kDense, false, false, false, 0, 2, 8, 2>(p, lds, none, pid, nwg);
-  else if (shape == k128x128) gemm_tiles<MODE, kDense, false, false, false, 0, 2, 4, 2>(p, lds, none, pid, nwg);
-  else gemm_tiles<MODE, kDense, false, false, false, 0, 1, 2, 4>(p, lds, none, pid, nwg);
+  if (shape == k256x256) gemm_tiles<MODE, kDense, ACC, ACC, MODE != kScaleTensor, 0, 4, 8, 2>(p, lds, none, pid, nwg);
+  else if (shape == k128x256) gemm_tiles<MODE, kDense, ACC, ACC, false, 0, 2, 8, 2>(p, lds, none, pid, nwg);
+  else if (shape == k128x128) gemm_tiles<MODE, kDense, ACC, ACC, false, 0, 2, 4, 2>(p, lds, none, pid, nwg);
+  else gemm_tiles<MODE, kDense, ACC, ACC, false, 0, 1, 2, 4>(p, lds, none, pid, nwg);
 }
 constexpr int backward_lds(int mode) {
   int most = 0;
@@ -1226,7 +1227,7 @@ constexpr int backward_lds(int mode) {
   return most;
 }
 
-template <int MODE, int MODE_W>
+template <int MODE, int MODE_W, bool ACC = false>
 __global__ __launch_bounds__(512) void gemm_backward_kernel(const BackwardParams q) {
   static_assert(tile_threads(4, 2) == 512 && tile_threads(2, 2) == 512 && tile_threads(1, 4) == 512, "");
   __shared__ __attribute__((aligned(1024))) uint8_t lds[backward_lds(MODE) > backward_lds(MODE_W) ? backward_lds(MODE) : backward_lds(MODE_W)];
@@ -1239,7 +1240,7 @@ __global__ __launch_bounds__(512) void gemm_backward_kernel(const BackwardParams
   const int one = wg >= q.first[1] && wg < q.first[1] + q.wgs[1];
   const int pid = wg - q.first[one];
   if (pid < 0 || pid >= q.wgs[one]) return;       // (behind a first product of fewer than 8 workgroups)
-  if (one) backward_tile<MODE_W>(q.gemm[1], q.shape[1], pid, q.wgs[1], lds);
+  if (one) backward_tile<MODE_W, ACC>(q.gemm[1], q.shape[1], pid, q.wgs[1], lds);
   else backward_tile<MODE>(q.gemm[0], q.shape[0], pid, q.wgs[0], lds);
 }
 
@@ -1356,7 +1357,10 @@ static int64_t few_rows(int64_t K) {        // the most rows that count as few
 //   block   256 x 1024 x 1024   13.4 / 7.5       512 x 4096 x 4096   32 / 25       8192 x 1024 x 1024  39.3 / 31.5
 //   block  4096 x 7168 x 7168    391 / 364      5000 x 5120 x 13824  659 / 633     3000 x 7168 x 2048   100 / 93
 //   pow2    750 x 2432 x 3840   28.3 / 17.9     tensor  2048 x 1024 x 1024  15.5 / 9.4     1024 x 4096 x 2048  26.5 / 18.9
-// Whole rounds, and many of them, are as fast one after the other: 4096 x 7168 x 16384 806 / 806 to 818.
+// Whole rounds, and many of them, are as fast one after the other: 4096 x 7168 x 16384 806 / 806 to 818.  Added onto fp32 a tile also waits for its
+// old values, all tiles of a round at once where they are a launch of their own (two launches / one): block 4096 x 7168 x 7168 448 / 400,
+// 2048 x 7168 x 4096 149 / 131, 1006 x 9472 x 3456 135 / 100, pow2 2048 x 7168 x 4096 137 / 124; without that time in the model pow2 2048 x
+// 7168 x 4096 stayed with two launches, and block 300 x 1024 x 16384 took 49.9 in one where two take 42.6.
 static int64_t tile_time(TileShape shape, int64_t kblocks) {
   switch (shape) {
     case k256x256: return 5000 + 1300 * kblocks;
@@ -1367,6 +1371,7 @@ static int64_t tile_time(TileShape shape, int64_t kblocks) {
   }
 }
 constexpr int64_t kLaunchTime = 3000;
+static int64_t accumulate_time(TileShape shape) { return 10000 * shape_rows(shape) * shape_cols(shape) / (256 * 256); }      // fp32 read and written
 
 // t1 tiles of d1 each, then t2 tiles of d2 <= d1, each to the compute unit that is free first
 static int64_t dealt_out(int64_t t1, int64_t d1, int64_t t2, int64_t d2, int64_t cus) {
@@ -1382,7 +1387,7 @@ static int64_t dealt_out(int64_t t1, int64_t d1, int64_t t2, int64_t d2, int64_t
   }
 }
 
-static bool pick_backward(int64_t M, int64_t N, int64_t K, int64_t padded, int launches, TileShape shape[2]) {
+static bool pick_backward(int64_t M, int64_t N, int64_t K, int64_t padded, int launches, bool accumulate, TileShape shape[2]) {
   const int mode = g_small_gemm_mode.load(std::memory_order_relaxed);
   const TileShape shapes[] = {k256x256, k128x256, k128x128, k64x128};
   if (mode != 0) {                       // (test hook: that shape for both)
@@ -1396,13 +1401,14 @@ static bool pick_backward(int64_t M, int64_t N, int64_t K, int64_t padded, int l
   int64_t apart = (launches - 1) * kLaunchTime;
   for (int i = 0; i < 2; ++i) {
     const TileShape s = pick_shape(rows[i], K);
-    apart += tile_time(s, (tile_count(rows[i], K, s) + cus - 1) / cus * kb[i]);      // (a workgroup's tiles follow each other without a gap)
+    const int64_t rounds = (tile_count(rows[i], K, s) + cus - 1) / cus;
+    apart += tile_time(s, rounds * kb[i]) + (i && accumulate ? rounds * accumulate_time(s) : 0);      // (its tiles follow each other without a gap)
   }
   int64_t best = INT64_MAX, best_end = 0;
   for (TileShape s0 : shapes)
     for (TileShape s1 : shapes) {
       const int64_t t[2] = {tile_count(rows[0], K, s0), tile_count(rows[1], K, s1)};
-      const int64_t d[2] = {tile_time(s0, kb[0]), tile_time(s1, kb[1])};
+      const int64_t d[2] = {tile_time(s0, kb[0]), tile_time(s1, kb[1]) + (accumulate ? accumulate_time(s1) : 0)};
       const int longer = d[1] > d[0] ? 1 : 0;
       const int64_t end = dealt_out(t[longer], d[longer], t[1 - longer], d[1 - longer], cus);
       const int64_t cost = end + (t[0] * d[0] + t[1] * d[1]) / (8 * cus);       // (of forms that end together the one with less to move)
@@ -1720,11 +1726,14 @@ int hpfp8_gemm_per_tensor(const void* a, int64_t lda, const float* sa_inv, const
 }
 
 int hpfp8_linear_backward(const hpfp8_operand* go, const hpfp8_operand* wt, const hpfp8_operand* go_t, const hpfp8_operand* xt, int64_t M,
-                          int64_t N, int64_t K, void* dx, void* dw, const float* partial, void* db, int recipe, hpfp8_stream_t stream) {
+                          int64_t N, int64_t K, void* dx, void* dw, int accumulate, const float* partial, void* db, int recipe,
+                          hpfp8_stream_t stream) {
   const char* what = "linear_backward";
   HPFP8_REQUIRE(go && wt && go_t && xt && (db == nullptr || partial != nullptr), HPFP8_ERR_ARG, "%s: null argument", what);
   HPFP8_REQUIRE(recipe >= HPFP8_BLOCKWISE && recipe <= HPFP8_PER_TENSOR, HPFP8_ERR_ARG, "%s: bad recipe", what);
   HPFP8_REQUIRE(M > 0 && N > 0 && K > 0, HPFP8_ERR_SHAPE, "%s: bad shape", what);
+  HPFP8_REQUIRE(!accumulate || recipe != HPFP8_PER_TENSOR, HPFP8_ERR_ARG, "%s: accumulate is of the blockwise recipes", what);
+  const int out_w = accumulate ? HPFP8_OUT_F32 : HPFP8_OUT_BF16;
   const int64_t padded = (M + kBlock - 1) / kBlock * kBlock;
   hipStream_t st = (hipStream_t)stream;
   BackwardParams q{};
@@ -1739,15 +1748,15 @@ int hpfp8_linear_backward(const hpfp8_operand* go, const hpfp8_operand* wt, cons
                              wt->stride_k, 128, M, K, N, nullptr, dx, K, HPFP8_OUT_BF16, 0, q.gemm[0]);
     if (rc[0] < 0) return rc[0];
     rc[1] = blockwise_params(go_t->codes, go_t->ld, go_t->scale_inv, go_t->stride_r, go_t->stride_k, xt->codes, xt->ld, xt->scale_inv, xt->stride_r,
-                             xt->stride_k, 1, N, K, padded, nullptr, dw, K, HPFP8_OUT_BF16, 0, q.gemm[1]);
+                             xt->stride_k, 1, N, K, padded, nullptr, dw, K, out_w, accumulate ? 1 : 0, q.gemm[1]);
   }
   if (rc[1] < 0) return rc[1];
   TileShape shape[2];
   const bool k_major = recipe == HPFP8_PER_TENSOR || (go->stride_r == 1 && go_t->stride_r == 1);
-  if (k_major && pick_backward(M, N, K, padded, db ? 3 : 2, shape)) {
+  if (k_major && pick_backward(M, N, K, padded, db ? 3 : 2, accumulate != 0, shape)) {
     const int64_t tiles[2] = {tile_count(M, K, shape[0]), tile_count(N, K, shape[1])};
     const int64_t kblocks[2] = {N / BK, padded / BK};
-    const int longer = tile_time(shape[1], kblocks[1]) > tile_time(shape[0], kblocks[0]) ? 1 : 0;
+    const int longer = tile_time(shape[1], kblocks[1]) + (accumulate ? accumulate_time(shape[1]) : 0) > tile_time(shape[0], kblocks[0]) ? 1 : 0;
     for (int i = 0; i < 2; ++i) {
       q.gemm[i].tiles = (int)tiles[i];
       q.shape[i] = shape[i];
@@ -1762,7 +1771,9 @@ int hpfp8_linear_backward(const hpfp8_operand* go, const hpfp8_operand* wt, cons
     q.sums = (uint16_t*)db;
     const dim3 grid((unsigned)(q.sums_first + (db ? (N + 511) / 512 : 0))), block(512);
     if (recipe == HPFP8_PER_TENSOR) gemm_backward_kernel<kScaleTensor, kScaleTensor><<<grid, block, 0, st>>>(q);
+    else if (recipe == HPFP8_BLOCKWISE_POW2 && accumulate) gemm_backward_kernel<kScalePow2, kScalePow2Row, true><<<grid, block, 0, st>>>(q);
     else if (recipe == HPFP8_BLOCKWISE_POW2) gemm_backward_kernel<kScalePow2, kScalePow2Row><<<grid, block, 0, st>>>(q);
+    else if (accumulate) gemm_backward_kernel<kScaleBlock, kScaleRow, true><<<grid, block, 0, st>>>(q);
     else gemm_backward_kernel<kScaleBlock, kScaleRow><<<grid, block, 0, st>>>(q);
     return check_launch(what);
   }
@@ -1770,7 +1781,7 @@ int hpfp8_linear_backward(const hpfp8_operand* go, const hpfp8_operand* wt, cons
   if (db) status = hpfp8_column_sum_finish(partial, padded / kBlock, N, db, nullptr, stream);
   for (int i = 0; i < 2 && status == HPFP8_OK; ++i) {
     if (recipe == HPFP8_PER_TENSOR) status = launch_per_tensor(q.gemm[i], HPFP8_OUT_BF16, st);
-    else status = launch_blockwise(q.gemm[i], i == 0 ? 128 : 1, HPFP8_OUT_BF16, recipe == HPFP8_BLOCKWISE_POW2, st);
+    else status = launch_blockwise(q.gemm[i], i == 0 ? 128 : 1, i == 0 ? HPFP8_OUT_BF16 : out_w, recipe == HPFP8_BLOCKWISE_POW2, st);
   }
   return status;
 }

@@ -400,6 +400,40 @@ hpfp8_operand operand(const at::Tensor& codes, const at::Tensor& scale_inv) {
   return {codes.data_ptr(), row_stride(codes), f32(scale_inv), one ? 0 : scale_inv.stride(0), one ? 0 : scale_inv.stride(1)};
 }
 
+// (go, sgo, wt, swt, go_t, sgo_t, xt, sxt, main gradient or None, pow2, device, stream) -> (dx, dw): both products of a blockwise backward;
+// swt the weight's scales [K / 128, N / 128], main gradient: fp32 [N, K] that dw is added onto (and is then the same tensor).
+PyObject* linear_backward(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  expect(n_args, 12);
+  const Where at_ = where(args, n_args);
+  const bool pow2 = truth(args[9]);
+  const at::Tensor *q[4], *s[4], *given = nullptr;
+  for (int i = 0; i < 4; ++i)
+    if (!codes_2d(args[2 * i], at_.device, q[i]) || !floats(args[2 * i + 1], at_.device, s[i]) || s[i]->dim() != 2) Py_RETURN_NONE;
+  const int64_t m = q[0]->size(0), n = q[0]->size(1), k = q[1]->size(0), mp = rows_up(m);
+  const int64_t rows[] = {m, k / kBlock, n, k}, blocks[] = {n / kBlock, n / kBlock, mp / kBlock, mp / kBlock};
+  for (int i = 0; i < 4; ++i)
+    if (s[i]->size(0) != rows[i] || s[i]->size(1) != blocks[i]) Py_RETURN_NONE;
+  if (k % kBlock || q[1]->size(1) != n || q[2]->size(0) != n || q[2]->size(1) != mp || q[3]->size(0) != k || q[3]->size(1) != mp || !row_scales_fit(*s[3]) ||
+      !no_modes())
+    Py_RETURN_NONE;
+  if (args[8] != Py_None && (!plain(args[8], at_.device, given) || given->scalar_type() != at::kFloat || given->dim() != 2 || given->size(0) != n ||
+                             given->size(1) != k || !given->is_contiguous()))
+    Py_RETURN_NONE;
+  at::Tensor dx, dw;
+  Call call;
+  {
+    pybind11::gil_scoped_release free;
+    dx = at::empty({m, k}, q[0]->options().dtype(at::kBFloat16));
+    dw = given ? *given : at::empty({n, k}, dx.options());
+    const hpfp8_operand a = operand(*q[0], *s[0]), b = operand(*q[1], *s[1]), at = operand(*q[2], *s[2]), bt = operand(*q[3], *s[3]);
+    HPFP8_CALL(call, hpfp8_linear_backward, &a, &b, &at, &bt, m, n, k, dx.data_ptr(), dw.data_ptr(), given != nullptr, nullptr, nullptr,
+               pow2 ? HPFP8_BLOCKWISE_POW2 : HPFP8_BLOCKWISE, at_.stream);
+  }
+  return call.ok() ? tuple_of(std::move(dx), std::move(dw)) : failed(call);
+  END_HANDLE_TH_ERRORS
+}
+
 // What forward has made, in Python, for y = x W^T + b with gradients of x and W to come: y, and for backward xt, sxt (per
 // tensor: the one scale), the weight's transposed codes (per tensor with a cached weight: its codes), sw.
 struct Made {
@@ -475,7 +509,7 @@ struct LinearNode : torch::autograd::Function<LinearNode> {
       dx = at::empty({m, in}, go.options());
       dw = at::empty({out, in}, go.options());
       const hpfp8_operand a = operand(f.q, f.s), b = operand(wt, sw), at = operand(f.qt, f.s), bt = operand(xt, sxt);
-      HPFP8_CALL(call, hpfp8_linear_backward, &a, &b, &at, &bt, m, out, in, dx.data_ptr(), dw.data_ptr(), has_bias ? f32(f.part) : nullptr,
+      HPFP8_CALL(call, hpfp8_linear_backward, &a, &b, &at, &bt, m, out, in, dx.data_ptr(), dw.data_ptr(), 0, has_bias ? f32(f.part) : nullptr,
                  has_bias ? f.total.data_ptr() : nullptr, HPFP8_PER_TENSOR, stream);
       db = std::move(f.total);
     } else {
@@ -489,7 +523,7 @@ struct LinearNode : torch::autograd::Function<LinearNode> {
       if (!row_scales_fit(scales)) scales = scales.t().contiguous().t();
       const hpfp8_operand a = operand(f.q, f.s), b{w.data_ptr(), row_stride(w), f32(sw), sw.stride(1), sw.stride(0)};
       const hpfp8_operand at = operand(f.qt, f.st), bt = operand(xt, scales);
-      HPFP8_CALL(call, hpfp8_linear_backward, &a, &b, &at, &bt, m, out, in, dx.data_ptr(), dw.data_ptr(), has_bias ? f32(f.part) : nullptr,
+      HPFP8_CALL(call, hpfp8_linear_backward, &a, &b, &at, &bt, m, out, in, dx.data_ptr(), dw.data_ptr(), 0, has_bias ? f32(f.part) : nullptr,
                  has_bias ? f.total.data_ptr() : nullptr, pow2 ? HPFP8_BLOCKWISE_POW2 : HPFP8_BLOCKWISE, stream);
       db = std::move(f.total);
     }
@@ -881,7 +915,7 @@ PyObject* bind_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
 #define HPFP8_METHOD(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {HPFP8_METHOD(built_for), HPFP8_METHOD(bind), HPFP8_METHOD(bind_backward), HPFP8_METHOD(quantize_1x128), HPFP8_METHOD(both_forms),
                          HPFP8_METHOD(quantize_128x128), HPFP8_METHOD(quantize_per_tensor_t), HPFP8_METHOD(gemm_blockwise),
-                         HPFP8_METHOD(gemm_per_tensor), HPFP8_METHOD(trains), HPFP8_METHOD(linear_node), HPFP8_METHOD(linear_train), HPFP8_METHOD(linear_infer),
+                         HPFP8_METHOD(gemm_per_tensor), HPFP8_METHOD(trains), HPFP8_METHOD(linear_node), HPFP8_METHOD(linear_train), HPFP8_METHOD(linear_infer), HPFP8_METHOD(linear_backward),
                          HPFP8_METHOD(swiglu_mlp_infer), HPFP8_METHOD(grouped_infer), HPFP8_METHOD(bucket_pack), HPFP8_METHOD(bucket_unpack),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -207,23 +207,27 @@ class _Fp8LinearBlockwise(torch.autograd.Function):
                 got, sgot = ops.quantize_128x1_t_rows(_for_weight_gradient_alone(go), pow2=pow2)
             if ctx.has_bias:
                 db = ops.column_sum(go)
+        param = ctx.main_grad_of
+        main_grad = None if param is None else getattr(param, "main_grad", None)
+        if need_dx and need_dw and (param is None or main_grad is not None):
+            dx, dw = ops.linear_backward(goq, sgo, wqt, sw.t(), got, sgot, xt, sxt, main_grad=main_grad, pow2=pow2)
+            return dx.reshape(ctx.x_shape), dw if param is None else None, db, None, None, None, None, None, None
         if need_dx:
             # dx[M,K] = go[M,N] . W[N,K]: contraction over N, b operand = W^T codes [K,N] whose
             # 128x128 scales are W's with the two strides swapped.
             dx = ops.gemm_blockwise(goq, sgo, wqt, sw.t(), pow2_scales=pow2).reshape(ctx.x_shape)
         if need_dw:
             # dW[N,K] = go^T[N,M] . x[M,K]: contraction over tokens, both operands 1x128 along M
-            param = ctx.main_grad_of
             if param is None:
                 dw = ops.gemm_blockwise(got, sgot, xt, sxt, sb_gran=1, pow2_scales=pow2)
-            elif getattr(param, "main_grad", None) is None:
+            elif main_grad is None:
                 # the fp32 main gradient of hyper_parallel/platform/torch/fully_shard/param.py:134-167: the
                 # first weight gradient creates it, later ones are added onto it by the GEMM itself, and
                 # .grad stays empty
                 param.main_grad = ops.gemm_blockwise(got, sgot, xt, sxt, sb_gran=1, out_dtype=torch.float32,
                                                      pow2_scales=pow2)
             else:
-                ops.gemm_blockwise(got, sgot, xt, sxt, sb_gran=1, out=param.main_grad, accumulate=True, pow2_scales=pow2)
+                ops.gemm_blockwise(got, sgot, xt, sxt, sb_gran=1, out=main_grad, accumulate=True, pow2_scales=pow2)
         return dx, dw, db, None, None, None, None, None, None
 
 
@@ -652,12 +656,12 @@ class _Fp8SwiGLUMLPBlock(torch.autograd.Function):
         if go.dtype != torch.bfloat16:
             go = go.to(torch.bfloat16)
         goq, sgo, got, sgot = _both_forms(go)
-        dw_down = ops.gemm_blockwise(got, sgot, at, sat, sb_gran=1)
-        dact = ops.gemm_blockwise(goq, sgo, dqt, ds.t())
+        dact, dw_down = ops.linear_backward(goq, sgo, dqt, ds.t(), got, sgot, at, sat)
         dhq, sdh, dht, sdht = ops.swiglu_backward_quantize_1x128_and_128x1_t_rows(h, dact)
-        dx = ops.gemm_blockwise(dhq, sdh, gqt, gs.t()).reshape(ctx.x_shape) if ctx.need_dx else None
-        dw_gate_up = ops.gemm_blockwise(dht, sdht, xt, sxt, sb_gran=1)
-        return dx, dw_gate_up, dw_down, None, None, None
+        if not ctx.need_dx:
+            return None, ops.gemm_blockwise(dht, sdht, xt, sxt, sb_gran=1), dw_down, None, None, None
+        dx, dw_gate_up = ops.linear_backward(dhq, sdh, gqt, gs.t(), dht, sdht, xt, sxt)
+        return dx.reshape(ctx.x_shape), dw_gate_up, dw_down, None, None, None
 
 
 def fp8_swiglu_mlp(input: torch.Tensor, w_gate_up, w_down, *, fast: bool = True,

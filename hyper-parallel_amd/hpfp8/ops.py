@@ -655,6 +655,19 @@ def gemm_blockwise(a: torch.Tensor, sa: torch.Tensor, b: torch.Tensor, sb: torch
     return out
 
 
+def linear_backward(goq, sgo, wqt, swt, got, sgot, xt, sxt, *, main_grad: Optional[torch.Tensor] = None, pow2: bool = False):
+    """Both products of a blockwise linear's backward, which are one launch where that is faster: dx[M, K] = go . w in bf16, from
+    go's codes and the weight's transposed codes [K, N] with scales swt [K/128, N/128], and dw[N, K] = go^T . x from the 128x1 forms
+    -- in bf16, or added onto ``main_grad`` (float32), which is then returned.  The bits are those of `gemm_blockwise`."""
+    if _gpu(goq):
+        device = _device()
+        out = _native.linear_backward(goq, sgo, wqt, swt, got, sgot, xt, sxt, main_grad, pow2, device, _raw_stream(device))
+        if out is not None:
+            return out
+    dx = gemm_blockwise(goq, sgo, wqt, swt, pow2_scales=pow2)
+    return dx, gemm_blockwise(got, sgot, xt, sxt, sb_gran=1, pow2_scales=pow2, out=main_grad, accumulate=main_grad is not None)
+
+
 def gemm_blockwise_swiglu_quantize(a: torch.Tensor, sa: torch.Tensor, b: torch.Tensor, sb: torch.Tensor, *,
                                    fast: bool = False, pow2_scales: bool = False, pow2_out: bool = False,
                                    want_scale: bool = False):

@@ -411,13 +411,15 @@ typedef struct {
 } hpfp8_operand;
 enum { HPFP8_BLOCKWISE = 0, HPFP8_BLOCKWISE_POW2 = 1, HPFP8_PER_TENSOR = 2 };
 
-/* Backward of y[M, N] = x[M, K] . w[N, K]^T + bias: dx[M, K] = go . w and dw[N, K] = go^T . x (bf16, contiguous) and, with db, the bias
+/* Backward of y[M, N] = x[M, K] . w[N, K]^T + bias: dx[M, K] = go . w and dw[N, K] = go^T . x (contiguous; bf16, dw fp32 and added
+ * onto what it holds with accumulate, blockwise recipes only) and, with db, the bias
  * gradient, bf16[N], from the quantizer's column sums (partial, as hpfp8_column_sum_finish takes them).  go: [M, N] codes with 1x128
  * scales; wt: [K, N] codes, scales of 128x128 blocks; go_t: [N, Mp] and xt: [K, Mp], 128x1 scales, Mp = M rounded up to 128, zeros
  * behind M.  The same bits as hpfp8_gemm_blockwise[_pow2] / hpfp8_gemm_per_tensor and hpfp8_column_sum_finish, in one launch where that is
  * faster than three (k-block-major scales of go and go_t), otherwise in those. */
 int hpfp8_linear_backward(const hpfp8_operand* go, const hpfp8_operand* wt, const hpfp8_operand* go_t, const hpfp8_operand* xt, int64_t M,
-                          int64_t N, int64_t K, void* dx, void* dw, const float* partial, void* db, int recipe, hpfp8_stream_t stream);
+                          int64_t N, int64_t K, void* dx, void* dw, int accumulate, const float* partial, void* db, int recipe,
+                          hpfp8_stream_t stream);
 
 /* MoE grouped form (one rank's local experts; no counterpart in the reference, whose expert
  * parallelism is unimplemented): rows of a[total_m, K] (row stride lda) are sorted by expert; offs[e] (int32,

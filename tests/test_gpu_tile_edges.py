@@ -739,12 +739,20 @@ def test_both_products_of_a_backward_in_one_launch_have_the_bits_of_two(gpu, m, 
         sw = sw.t()
         want = [ops.gemm_blockwise(g, sg, wt, sw, pow2_scales=recipe == 1), ops.gemm_blockwise(gt, sgt, xt, sx, sb_gran=1, pow2_scales=recipe == 1), db]
     operands = [Operand(g, sg), Operand(wt, sw), Operand(gt, sgt), Operand(xt, sx)]
+    if recipe != 2:
+        old = torch.randn((n, k), generator=torch.Generator("cpu").manual_seed(5)).to(gpu)
+        summed = ops.gemm_blockwise(gt, sgt, xt, sx, sb_gran=1, pow2_scales=recipe == 1, out=old.clone(), accumulate=True)
     for mode in (0, 1, 2, 3, 4, 5):
         got = [torch.full(s, 7.0, dtype=torch.bfloat16, device=gpu) for s in ((m + 1, k), (n + 1, k), (n + 8,))]
         _lib.load().hpfp8_debug_set_small_gemm(mode)
         try:
-            _lib.call("hpfp8_linear_backward", *(ctypes.addressof(o) for o in operands), m, n, k, got[0].data_ptr(), got[1].data_ptr(),
+            _lib.call("hpfp8_linear_backward", *(ctypes.addressof(o) for o in operands), m, n, k, got[0].data_ptr(), got[1].data_ptr(), 0,
                       part.data_ptr(), got[2].data_ptr(), recipe, ops._stream())
+            if recipe != 2:
+                onto = [torch.full_like(got[0], 7.0), old.clone()]
+                _lib.call("hpfp8_linear_backward", *(ctypes.addressof(o) for o in operands), m, n, k, onto[0].data_ptr(), onto[1].data_ptr(), 1,
+                          None, None, recipe, ops._stream())
+                assert torch.equal(onto[0][:m], want[0]) and torch.equal(onto[1], summed)
         finally:
             _lib.load().hpfp8_debug_set_small_gemm(0)
         for a, b, rows in zip(got, want, (m, n, n)):
