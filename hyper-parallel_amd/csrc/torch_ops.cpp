@@ -36,7 +36,7 @@ constexpr int64_t kBlock = 128;
   X(hpfp8_quantize_1x128_and_128x1_t_pow2_bf16) X(hpfp8_quantize_128x1_t_colsum_bf16) X(hpfp8_quantize_rows_128x1_t_bf16) \
   X(hpfp8_column_sum_finish) X(hpfp8_quantize_128x128_bf16) X(hpfp8_quantize_128x128_pow2_bf16) \
   X(hpfp8_quantize_per_tensor_t_bf16) X(hpfp8_transpose_codes) X(hpfp8_gemm_blockwise) X(hpfp8_gemm_blockwise_pow2) X(hpfp8_gemm_per_tensor) \
-  X(hpfp8_quantize_per_tensor_sync_bf16) X(hpfp8_gemm_few_rows) X(hpfp8_linear_few_rows) X(hpfp8_linear_few_rows_bf16) X(hpfp8_linear_backward) X(hpfp8_gemm_blockwise_swiglu_quantize) X(hpfp8_swiglu_quantize_1x128_bf16) \
+  X(hpfp8_quantize_per_tensor_sync_bf16) X(hpfp8_gemm_few_rows) X(hpfp8_linear_few_rows) X(hpfp8_linear_few_rows_bf16) X(hpfp8_linear_backward) X(hpfp8_quantize_two_per_tensor_t_bf16) X(hpfp8_gemm_blockwise_swiglu_quantize) X(hpfp8_swiglu_quantize_1x128_bf16) \
   X(hpfp8_swiglu_quantize_1x128_pow2_bf16) X(hpfp8_swiglu_quantize_1x128_fast_bf16) X(hpfp8_gemm_grouped_blockwise) \
   X(hpfp8_bucket_pack_quantize_bf16) X(hpfp8_bucket_unpack_dequantize_bf16)
 struct Library {
@@ -369,7 +369,7 @@ uint32_t* sync_block(const at::Tensor& x, bool one_pass, hipStream_t stream) {
   static auto* const blocks = new std::map<std::pair<int64_t, hipStream_t>, at::Tensor>;      // (never destroyed: the device may go first)
   std::lock_guard<std::mutex> guard(lock);
   at::Tensor& t = (*blocks)[{x.get_device(), stream}];
-  if (!t.defined()) t = at::zeros({128}, x.options().dtype(at::kInt));
+  if (!t.defined()) t = at::zeros({256}, x.options().dtype(at::kInt));       // (512 bytes; two tensors at once: the other 512 too)
   return (uint32_t*)t.data_ptr();
 }
 
@@ -651,8 +651,21 @@ PyObject* linear_train(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     Forms fx, fw;
     if (per_tensor) {
       const int64_t tiles = rows_up(m) / kBlock * (k / kBlock);
-      fx = make_per_tensor(x2, false, sync_block(x2, tiles <= kOnePassTiles, (hipStream_t)stream), stream, call);
-      if (call.ok() && !wq) fw = make_per_tensor(*weight, false, sync_block(*weight, n / kBlock * (k / kBlock) <= kOnePassTiles, (hipStream_t)stream), stream, call);
+      const int64_t w_tiles = n / kBlock * (k / kBlock);
+      uint32_t* const sync = sync_block(x2, tiles <= kOnePassTiles, (hipStream_t)stream);
+      if (sync && !wq && w_tiles <= kOnePassTiles) {
+        for (Forms* f : {&fx, &fw}) {
+          const int64_t rows = f == &fx ? m : n;
+          f->q = new_codes(x2, rows, k);
+          f->qt = new_codes_t(x2, k, rows_up(rows));
+          f->s = at::empty({}, x2.options().dtype(at::kFloat).requires_grad(false));
+        }
+        HPFP8_CALL(call, hpfp8_quantize_two_per_tensor_t_bf16, x2.data_ptr(), m, k, fx.q.data_ptr(), fx.qt.data_ptr(), fx.qt.stride(0), f32(fx.s),
+                   weight->data_ptr(), n, fw.q.data_ptr(), fw.qt.data_ptr(), fw.qt.stride(0), f32(fw.s), sync, stream);
+      } else {
+        fx = make_per_tensor(x2, false, sync, stream, call);
+      }
+      if (call.ok() && !wq && !fw.q.defined()) fw = make_per_tensor(*weight, false, sync_block(*weight, w_tiles <= kOnePassTiles, (hipStream_t)stream), stream, call);
       made.w_transposed = !wq;
       made.w = wq ? *wq : fw.qt;
       made.sw = wq ? *sw : fw.s;

@@ -64,6 +64,7 @@ SIGNATURES = {
     "hpfp8_gemm_blockwise_swiglu_quantize": [_vp, _i64, _vp, _i64, _i64, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _i64,
                                              _int, _int, _int, _vp, _i64, _vp, _vp, _vp],
     "hpfp8_linear_few_rows_bf16": [_vp, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _i64, _int, _vp, _vp, _i64, _int, _vp],
+    "hpfp8_quantize_two_per_tensor_t_bf16": [_vp, _i64, _i64, _vp, _vp, _i64, _vp, _vp, _i64, _vp, _vp, _i64, _vp, _vp, _vp],
     "hpfp8_linear_backward": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp, _int, _vp, _vp, _int, _vp],
     "hpfp8_gemm_per_tensor": [_vp, _i64, _vp, _vp, _i64, _vp, _i64, _i64, _i64, _vp, _vp, _i64, _int, _vp],
     "hpfp8_gemm_grouped_blockwise": [_vp, _i64, _vp, _i64, _i64, _vp, _vp, _vp, _int, _i64, _i64, _i64, _vp, _i64,

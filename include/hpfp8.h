@@ -248,6 +248,12 @@ int hpfp8_swiglu_backward_quantize_1x128_and_128x1_t_bf16(const void* h, int64_t
 int hpfp8_quantize_per_tensor_t_bf16(const void* x, int64_t m, int64_t k, void* q, void* q_t, int64_t ld_t, float* amax,
                                      float* scale, float* scale_inv, uint32_t* sync, float* colsum_partial, hpfp8_stream_t stream);
 
+/* hpfp8_quantize_per_tensor_t_bf16 of x[m, k] and of w[n, k], each with its own scale, in one launch, for up to 256 tiles of 128x128
+ * each; the same bits.  sync: 1024 bytes (256-byte aligned), kept as that function's 512. */
+int hpfp8_quantize_two_per_tensor_t_bf16(const void* x, int64_t m, int64_t k, void* q, void* q_t, int64_t ld_t, float* scale_inv, const void* w,
+                                         int64_t n, void* wq, void* wq_t, int64_t ld_wt, float* w_scale_inv, uint32_t* sync,
+                                         hpfp8_stream_t stream);
+
 /* The three dual quantizers above (k-block-major scales, scale_inv only) for any number of rows m.  The 128x1 groups run
  * down the rows; the last one of a ragged m is filled up with zero rows: q_t [k, mb * 128] (row stride ld_t >= mb * 128)
  * and scale_inv_t [mb, k] with mb = ceil(m / 128) are those of the source with zero rows appended, q [m, k] and scale_inv

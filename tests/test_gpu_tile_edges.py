@@ -758,3 +758,27 @@ def test_both_products_of_a_backward_in_one_launch_have_the_bits_of_two(gpu, m, 
         for a, b, rows in zip(got, want, (m, n, n)):
             assert torch.equal(a[:rows], b)
             assert bool((a[rows:] == 7.0).all())
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 128, 128), (300, 128, 384), (2048, 1024, 1024), (128, 4096, 1024), (1025, 256, 2048), (8192, 512, 512)])
+@pytest.mark.parametrize("spins", [256, 0])
+def test_two_tensors_quantized_in_one_launch_have_the_bits_of_two(gpu, m, n, k, spins):
+    """One, two and four tiles per workgroup, the fewest and the most workgroups per tensor, and workgroups that never see the others'
+    maximum and find it by themselves; three times over the same words, which have to be zero again in between."""
+    from hpfp8 import _lib, ops
+    x, w = _normal((m, k), 1, gpu, outliers=True), _normal((n, k), 2, gpu, 0.02)
+    (q, s, qt), (wq, sw, wqt) = ops.quantize_per_tensor_t(x), ops.quantize_per_tensor_t(w)
+    sync = torch.zeros(256, dtype=torch.int32, device=gpu)
+    _lib.load().hpfp8_debug_set_spin_limit(spins)
+    try:
+        for _ in range(3):
+            got = [torch.zeros_like(q), torch.empty(k, qt.stride(0), dtype=torch.float8_e4m3fn, device=gpu).zero_(), torch.zeros_like(s),
+                   torch.zeros_like(wq), torch.empty(k, wqt.stride(0), dtype=torch.float8_e4m3fn, device=gpu).zero_(), torch.zeros_like(sw)]
+            _lib.call("hpfp8_quantize_two_per_tensor_t_bf16", x.data_ptr(), m, k, got[0].data_ptr(), got[1].data_ptr(), qt.stride(0), got[2].data_ptr(),
+                      w.data_ptr(), n, got[3].data_ptr(), got[4].data_ptr(), wqt.stride(0), got[5].data_ptr(), sync.data_ptr(), ops._stream())
+            for a, b in zip(got, (q, qt, s, wq, wqt, sw)):
+                a = a[:, :b.shape[1]] if b.dim() == 2 else a
+                assert torch.equal(a.contiguous().view(torch.uint8) if b.dim() == 2 else a, b.contiguous().view(torch.uint8) if b.dim() == 2 else b)
+            assert int(sync.count_nonzero()) == 0
+    finally:
+        _lib.load().hpfp8_debug_set_spin_limit(256)
