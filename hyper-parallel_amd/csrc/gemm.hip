@@ -1706,7 +1706,8 @@ int hpfp8_linear_few_rows_bf16(const void* x, const void* b, int64_t ldb, const 
   const char* what = "linear_few_rows";
   HPFP8_REQUIRE(pow2 == 0 || pow2 == 1, HPFP8_ERR_ARG, "%s: pow2 must be 0 or 1", what);
   HPFP8_REQUIRE(M <= kSkinnyMaxRowsBf16, HPFP8_ERR_SHAPE, "%s: more than %d rows", what, kSkinnyMaxRowsBf16);
-  int rc = check_common(what, x, 2 * K, b, ldb, sb, sb, M, N, K, bias, c, ldc, out_type, 0);
+  // (rows of x as long as those of the codes that the two launches would make: 8 rows of bf16 are addressed here, not 256)
+  int rc = check_common(what, x, K, b, ldb, sb, sb, M, N, K, bias, c, ldc, out_type, 0);
   if (rc <= 0) return rc;
   rc = check_scale_span(what, N / kBlock, K / BK, sb_stride_n, sb_stride_k, "sb");
   if (rc <= 0) return rc;

@@ -199,6 +199,20 @@ def test_rows_quantized_inside_the_few_rows_product_have_the_bits_of_the_two_lau
                 assert bool((c[:m, n:] == 7.0).all()) and bool((c[m] == 7.0).all())
 
 
+def test_rows_quantized_inside_the_few_rows_product_may_be_as_long_as_those_of_codes(gpu):
+    """The limit on a row is the product's, 8 MiB of codes; the same row of bf16 is twice as many bytes."""
+    from hpfp8 import _lib, ops
+    m, n, k = 8, 128, (1 << 22) + 128
+    x, w = _normal((m, k), 1, gpu), _normal((n, k), 2, gpu, 0.02)
+    b, sb = ops.quantize_128x128(w)
+    q, s = ops.quantize_1x128(x, kmajor=True)
+    want = ops.gemm_blockwise(q, s, b, sb)
+    c = torch.zeros((m, n), dtype=torch.bfloat16, device=gpu)
+    _lib.call("hpfp8_linear_few_rows_bf16", x.data_ptr(), b.data_ptr(), b.stride(0), sb.data_ptr(), sb.stride(0), sb.stride(1), m, n, k, False,
+              None, c.data_ptr(), c.stride(0), _lib.OUT_BF16, ops._stream())
+    assert torch.equal(c, want)
+
+
 def test_gemm_with_few_rows_and_power_of_two_scales_whose_product_is_out_of_range(gpu):
     """Two scales of 2^80: their product is no fp32 number, but a product of codes that is zero stays zero."""
     from hpfp8 import ops
