@@ -79,7 +79,7 @@ class Fp8GradBucket:
     def pack(self, grads: Sequence[torch.Tensor]):
         """_copy_grad_to_unsharded_buffer + cast: gradients (each shard_size * numels[e] elements) ->
         (codes [shard_size, row_elems] e4m3, scale_inv [shard_size, row_elems / 128] fp32)."""
-        if ops._native is not None:
+        if type(grads) in (list, tuple) and grads and ops._gpu(grads[0]):
             device = ops._device()
             out = ops._native.bucket_pack(grads, self._numels_c, self._offsets_c, len(self.numels), self.shard_size, self.row_elems, device,
                                           ops._raw_stream(device))
@@ -97,7 +97,7 @@ class Fp8GradBucket:
     def unpack(self, codes_row: torch.Tensor, scale_inv_row: torch.Tensor, outs: Sequence[torch.Tensor]):
         """_set_grad_data: one reduced row (codes [row_elems], scale_inv [row_elems / 128]) -> outs[e]
         (bf16, numels[e] elements each), times grad_scale after the cast back."""
-        if ops._native is not None:
+        if ops._gpu(codes_row):
             device = ops._device()
             if ops._native.bucket_unpack(codes_row, scale_inv_row, outs, self._numels_c, self._offsets_c, len(self.numels), self.row_elems,
                                          self.grad_scale, device, ops._raw_stream(device)):

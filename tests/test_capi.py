@@ -102,6 +102,24 @@ def test_argument_errors_of_the_fused_and_one_launch_entry_points():
     assert sy(p + 2, 1024, p, None, None, p, p, None) == -3
 
 
+def test_the_bucket_says_what_is_wrong_with_its_arguments_before_it_asks_for_a_gpu():
+    import torch
+    import hpfp8
+    bucket = hpfp8.Fp8GradBucket([100, 200], shard_size=2)
+    grad = torch.zeros(200, dtype=torch.bfloat16)
+    row, scales = torch.zeros(bucket.row_elems, dtype=torch.float8_e4m3fn), torch.zeros(bucket.row_elems // 128)
+    with pytest.raises(ValueError, match="expected 2 tensors, got 1"):
+        bucket.pack([grad])
+    with pytest.raises(ValueError, match="expected 2 tensors, got 0"):
+        bucket.pack([])
+    with pytest.raises(ValueError, match="this bucket's size"):
+        bucket.unpack(row[128:], scales, [grad, grad])
+    with pytest.raises(TypeError, match="float8_e4m3fn"):
+        bucket.unpack(row.float(), scales, [grad, grad])
+    with pytest.raises(ValueError, match="must live on the GPU"):
+        bucket.unpack(row, scales, [grad, grad])
+
+
 def test_python_wrappers_reject_cpu_tensors_and_bad_shapes():
     import torch
     import hpfp8
