@@ -90,6 +90,7 @@ struct GemmParams {
   int pow2_out;
   float* q_scale;
   float* q_scale_inv;
+  int stream_b;           // rows of b that one tile alone reads are not kept in the caches (streams_b)
   int choose_cus;         // grouped by rows, tile chosen on the device: the compute units there are (test hook: minus the rows asked for)
 };
 
@@ -134,7 +135,7 @@ struct TileInfo {
   int n0;              // first row of b / column of c
   int expert;
   int kb0, kbn;        // grouped along the contraction: first k-block of the tile's expert and how many (>= 1)
-  bool b_once;         // (fetching waves) no other tile reads these rows of b
+  bool b_once;         // (fetching waves) no other tile reads these rows of b, and they are not kept in the caches
 };
 
 // Position `d` k-blocks after k-block kb of the current tile (which has k0 k-blocks, the next one k1, every
@@ -413,7 +414,7 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
     ti.expert = __builtin_amdgcn_readfirstlane(expert);
     ti.kb0 = __builtin_amdgcn_readfirstlane(kb0);
     ti.kbn = __builtin_amdgcn_readfirstlane(kbn);
-    ti.b_once = __builtin_amdgcn_readfirstlane(row_tiles) == 1;
+    ti.b_once = p.stream_b && __builtin_amdgcn_readfirstlane(row_tiles) == 1;
   };
   // ---- global -> LDS tile DMA.  One wave instruction moves 8 rows x 128 B (lane i -> LDS slot
   // i); the lane picks the 16-byte global chunk whose swizzled home is its slot.  The buffer
@@ -488,9 +489,9 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
   auto issue_b = [&](const __amdgpu_buffer_rsrc_t& rs, int buf, int kb, int sub) {
     transfer(rs, b_off[sub], b_lds + buf * kBTile + wave * (NB * 1024), kb, sub);
   };
-  // Rows of b that one tile alone reads are streamed: they stay in no cache, which leaves those to a's rows (us, grouped by rows,
-  // before / so: 512 rows of 32 experts [4096, 7168] by Zipf's law 158 / 137, 64 of 8 36.3 / 33.1, 1024 of 32 [2048, 7168] 98 / 92; where
-  // several tiles share them it would cost: 8192 of 32 [4096, 7168] 299 / 310).
+  // Rows of b that one tile alone reads are streamed where b does not fit the Infinity Cache (streams_b has the figures): they stay in
+  // no cache, which leaves those to a's rows.  Where several tiles share them it would cost: 8192 rows of 32 experts [4096, 7168]
+  // 299 / 310 us.
   auto stream_b = [&](const __amdgpu_buffer_rsrc_t& rs, int buf, int kb, int sub) {
     stream_1k(rs, b_lds + buf * kBTile + wave * (NB * 1024) + sub * 1024, b_off[sub], kb * BK);
   };
@@ -1441,6 +1442,21 @@ static bool try_skinny(const GemmParams& p, SkinnyMode mode, int out_type, hipSt
   return true;
 }
 
+// Whether rows of b that only one tile reads are streamed past the caches: where those of all experts that can have rows are more than the
+// Infinity Cache holds, so that none of them would be there when the next call comes.  A smaller b may still be there, and streamed it
+// never is.  us kept / streamed, with one b for every call (and with two or more in turn):
+//   65 rows of    [18432, 7168] (126 MiB)  26.6 / 32.8  (35.7 / 33.8)     [32768, 8192] (256)  43.2 / 56.6  (62.1 / 56.7)
+//                 [40960, 7168] (280)      58.2 / 56.8  (61.6 / 57.3)     [49152, 8192] (384)  77.1 / 70.7  (85.6 / 79.3)
+//   128 rows of   [18432, 7168]            27.3 / 39.3  (42.5 / 40.8)     [65536, 8192] (512)   128 / 120   (128 / 120)
+//   16 rows each of 6 experts [4096, 7168] (168)  28.7 / 30.9  (34.4 / 30.9)     9 (252)  43.7 / 52.7  (57.2 / 52.6)
+//                            10 (280)             55.4 / 54.3  (59.0 / 54.6)    16 (448)  83.2 / 72.0  (83.0 / 72.6)
+//                            24 (672)              121 / 106    (122 / 107)
+//   512 rows of 32 experts (896), evenly 159 / 140, by Zipf's law 175 / 157; of 8 (224) evenly 36.7 / 39.4 (44.5 / 39.9), by Zipf's law 43.2 / 56.6
+static int streams_b(int64_t M, int64_t N, int64_t K, int64_t experts) {
+  constexpr int64_t kInfinityCache = (int64_t)256 << 20;
+  return (experts < M ? experts : M) * N * K > kInfinityCache;
+}
+
 template <int MODE, int GROUPED, bool SA4, int WM, int NS, int WN>
 static int launch_sa(const GemmParams& p, int out_type, int64_t tiles, hipStream_t stream) {
   dim3 grid((unsigned)persistent_grid(tiles)), block(tile_threads(WM, WN));
@@ -1471,6 +1487,7 @@ template <int MODE, int GROUPED>
 static int launch(GemmParams p, int out_type, TileShape shape, hipStream_t stream) {
   int64_t tiles = tile_count(p.M, p.N, shape);
   p.tiles = (int)tiles;                        // (grouped by rows: the kernel counts the experts' own tiles)
+  p.stream_b = streams_b(p.M, p.N, p.K, GROUPED == kGroupedRows ? p.experts : 1);
   if (GROUPED == kGroupedK) tiles *= p.experts;
   // upper bound on row tiles: every expert may add one partial tile
   if (GROUPED == kGroupedRows) tiles = most_grouped_tiles(p.M, p.N, p.experts, shape);
@@ -1491,6 +1508,7 @@ static int launch_grouped(GemmParams p, int out_type, hipStream_t stream) {
   if (tiles == kSmallestTiles) return launch<MODE, kGroupedRows>(p, out_type, k64x64, stream);
   if (tiles == kLowestTiles) return launch<MODE, kGroupedRows>(p, out_type, k64x128, stream);
   if (tiles == kHighTiles) return launch<MODE, kGroupedRows>(p, out_type, k256x256, stream);
+  p.stream_b = streams_b(p.M, p.N, p.K, p.experts);
   p.choose_cus = tiles == kLowTiles ? -128 : persistent_grid((int64_t)1 << 40);
   dim3 grid((unsigned)persistent_grid(most_grouped_tiles(p.M, p.N, p.experts, k64x128))), block(512);
   const bool sa4 = p.sa_sm == 1;
@@ -1667,6 +1685,7 @@ int hpfp8_gemm_blockwise_swiglu_quantize(const void* a, int64_t lda, const float
   const TileShape shape = pick_shape_swiglu(M, 2 * inter);
   const int64_t tiles = tile_count(M, 2 * inter, shape);
   p.tiles = (int)tiles;
+  p.stream_b = streams_b(p.M, p.N, p.K, 1);
   dim3 grid((unsigned)persistent_grid(tiles)), block(512);
   static_assert(tile_threads(4, 2) == 512 && tile_threads(2, 2) == 512 && tile_threads(1, 4) == 512, "");
   hipStream_t st = (hipStream_t)stream;
@@ -1760,6 +1779,7 @@ int hpfp8_linear_backward(const hpfp8_operand* go, const hpfp8_operand* wt, cons
     const int longer = tile_time(shape[1], kblocks[1]) + (accumulate ? accumulate_time(shape[1]) : 0) > tile_time(shape[0], kblocks[0]) ? 1 : 0;
     for (int i = 0; i < 2; ++i) {
       q.gemm[i].tiles = (int)tiles[i];
+      q.gemm[i].stream_b = streams_b(q.gemm[i].M, q.gemm[i].N, q.gemm[i].K, 1);
       q.shape[i] = shape[i];
       q.wgs[i] = (int)(tiles[i] < kXcds ? tiles[i] : (tiles[i] + kXcds - 1) / kXcds * kXcds);
     }

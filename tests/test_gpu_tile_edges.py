@@ -796,3 +796,56 @@ def test_two_tensors_quantized_in_one_launch_have_the_bits_of_two(gpu, m, n, k, 
             assert int(sync.count_nonzero()) == 0
     finally:
         _lib.load().hpfp8_debug_set_spin_limit(256)
+
+
+@pytest.mark.parametrize("grouped", [False, True])
+def test_a_weight_that_stays_in_the_caches_is_read_from_them(gpu, grouped):
+    """Streamed past them, one weight used again and again would take as long as several in turn that do not fit together (measured: 97 %
+    of it dense, 100 % grouped; kept 68 % and 70 %)."""
+    from hpfp8 import ops
+    m, k = (512, 7168) if grouped else (128, 7168)
+    n = 8 * 4096 if grouped else 18432
+    a, sa = ops.quantize_1x128(_normal((m, k), 1, gpu), kmajor=True)
+    weights = [ops.quantize_128x128(_normal((n, k), seed, gpu, 0.02)) for seed in range(4)]
+    sizes = [188, 94, 63, 47, 37, 31, 27, 25]
+    offs = torch.tensor(sizes, device=gpu).cumsum(0).int()
+
+    def product(b, sb):
+        if grouped:
+            return ops.gemm_grouped_blockwise(a, sa, b.view(8, 4096, k), sb.view(8, 32, k // 128), offs)
+        return ops.gemm_blockwise(a, sa, b, sb)
+
+    def fastest(of):
+        times = []
+        for _ in range(7):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            for i in range(4):
+                product(*of[i % len(of)])
+            start.record()
+            for i in range(20):
+                product(*of[i % len(of)])
+            end.record()
+            end.synchronize()
+            times.append(start.elapsed_time(end))
+        return min(times)
+
+    assert fastest(weights[:1]) < 0.85 * fastest(weights)
+
+
+def test_products_whose_weight_is_streamed_past_the_caches_have_the_bits_of_those_that_keep_it(gpu):
+    """Weights larger than the Infinity Cache with rows that one low tile reads alone: dense, with the SwiGLU epilogue and grouped by rows
+    (experts with none, one tile's and several tiles' rows); 256 x 256 tiles stream nothing."""
+    from hpfp8 import ops
+    k, n, experts = 7168, 10 * 4096, 10
+    b, sb = ops.quantize_128x128(_normal((n, k), 2, gpu, 0.02))
+    for m in (65, 128, 129):
+        a, sa = ops.quantize_1x128(_normal((m, k), 1, gpu), kmajor=True)
+        got, want = _both_tiles(lambda: ops.gemm_blockwise(a, sa, b, sb))
+        assert torch.equal(got, want)
+        (gq, gs), (wq, ws) = _both_tiles(lambda: ops.gemm_blockwise_swiglu_quantize(a, sa, b, sb, fast=True)[:2])
+        assert torch.equal(gq.view(torch.uint8), wq.view(torch.uint8)) and torch.equal(gs, ws)
+    for sizes in ([1, 0, 64, 65, 128, 129, 7, 300, 16, 2], [10] * 10):
+        a, sa = ops.quantize_1x128(_normal((sum(sizes), k), 1, gpu), kmajor=True)
+        offs = torch.tensor(sizes, device=gpu).cumsum(0).int()
+        got, want = _both_tiles(lambda: ops.gemm_grouped_blockwise(a, sa, b.view(experts, 4096, k), sb.view(experts, 32, k // 128), offs))
+        assert torch.equal(got, want)
