@@ -269,6 +269,8 @@ __host__ __device__ constexpr int tile_lds(int mode, int wm, int tn) {
 // per group of one and eight against 32 of matrix pipe).  The four of a subtile are issued back to back: 43 cycles a group, where
 // one in front of each large matrix instruction makes it 51.  us before / so: 7168 x 16384 x 4096 466 / 437 (one by one 469),
 // 36864 x 7168 x 4096 1064 / 997, 2048 x 7168 x 1536 28.2 / 27.6, 1400 x 3072 x 4096 33.1 / 29.5, 1024 x 1024 x 4096 13.5 / 12.4.
+// (The instruction keeps subnormal products, and the scales are multiplied first as in the block form: a pair whose product overflows
+// gives NaN for a sum of 0, where multiplied one after the other it gave 0.)
 __device__ __forceinline__ int scale_row(int lane) { return ((lane >> 2) & 3) * 16 + (lane >> 4) * 4 + (lane & 3); }
 __device__ __forceinline__ v4f scale_products(float sb, float sa, int sub) {
   const v4f zero = {0.f, 0.f, 0.f, 0.f};

@@ -328,7 +328,10 @@ int hpfp8_bucket_unpack_dequantize_bf16(void* const* grads, const int64_t* numel
  *
  * a[M, K] and b[N, K] are E4M3 codes with K contiguous and row strides lda / ldb bytes (>= K,
  * multiples of 16); K, N multiples of 128; fp32 accumulation, k-blocks ascending; one rounding to
- * bf16 at the end (or fp32 output).
+ * bf16 at the end (or fp32 output).  sa * sb is formed first, rounded to fp32 (subnormal products are kept), for either
+ * sb_gran: a pair of scales whose product fp32 cannot hold gives an infinity, and NaN for an inner sum of 0.  (Those of the
+ * quantizers lie above 2.2e-15, so no product of two underflows; one overflows where two groups' largest magnitudes multiply to
+ * more than 6.8e43.)
  *   sa(m, kb) = sa[m * sa_stride_m + kb * sa_stride_k]
  *   sb(n, kb) = sb[(n / sb_gran) * sb_stride_n + kb * sb_stride_k],  sb_gran = 128 or 1
  * Uses:  forward  a = x codes (1x128),  b = W codes (128x128),            sb_gran = 128

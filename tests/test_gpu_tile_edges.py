@@ -849,3 +849,30 @@ def test_products_whose_weight_is_streamed_past_the_caches_have_the_bits_of_thos
         offs = torch.tensor(sizes, device=gpu).cumsum(0).int()
         got, want = _both_tiles(lambda: ops.gemm_grouped_blockwise(a, sa, b.view(experts, 4096, k), sb.view(experts, 32, k // 128), offs))
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("tiles", [0, 1, 3, 4, 5])
+@pytest.mark.parametrize("gran", [1, 128])
+def test_the_product_of_two_scales_is_formed_first_and_rounded_to_fp32(gpu, gran, tiles):
+    """part * (sa * sb), the oracle's order, at both ends of the range: a product below the smallest normal number keeps the bits that a
+    subnormal one has, and one that overflows is infinite for every element it scales (times a zero sum: NaN), and for no other."""
+    from hpfp8 import _lib, ops
+    m, n, k = 256, 256, 384
+    a, b = _ints((m, k), 1, gpu), _ints((n, k), 2, gpu)
+    a.view(torch.uint8)[5, 128:256] = 0
+    sa, sb = torch.ones((k // 128, m), device=gpu), torch.ones((k // 128, n // gran), device=gpu)
+    sa[0], sb[0] = 1.25 * 2.0 ** -70, 1.625 * 2.0 ** -76        # 16.25 * 2^-149: rounded to the subnormal number 16 * 2^-149
+    sa[2], sb[2] = 2.0 ** -100, 2.0 ** -40                      # (with it every sum is a whole number of 2^-149 below 2^24 of them)
+    sa[1] = 0.0
+    sa[1, 3:8], sb[1, 1] = 2.0 ** 100, 2.0 ** 100
+    part = [a.float()[:, i * 128:(i + 1) * 128].cpu() @ b.float()[:, i * 128:(i + 1) * 128].cpu().t() for i in range(k // 128)]
+    want = torch.zeros((m, n))
+    for i, p in enumerate(part):
+        want = torch.addcmul(want.double(), p.double(), torch.outer(sa[i].cpu(), sb[i].cpu().repeat_interleave(gran)).double()).float()
+    _lib.load().hpfp8_debug_set_small_gemm(tiles)
+    try:
+        got = ops.gemm_blockwise(a, sa.t(), b, sb.t() if gran == 1 else sb.t().contiguous(), sb_gran=gran, out_dtype=torch.float32).cpu()
+    finally:
+        _lib.load().hpfp8_debug_set_small_gemm(0)
+    assert bool(want[5].isnan().any()) and bool(want[3].isinf().any()) and bool(want[8].isfinite().all())
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(0.0, 1.0, -1.0), want.nan_to_num(0.0, 1.0, -1.0))
