@@ -1051,29 +1051,42 @@ def test_what_else_torch_does_with_a_step_has_the_python_functions_outcome(gpu, 
         assert len(got) == len(want) and all(type(a) is type(b) and a.requires_grad == b.requires_grad and torch.equal(a, b) for a, b in zip(got, want))
 
 
-def _with_and_without_native(run, monkeypatch):
-    """What a call gives through the native host path and as the Python form: results, or the type of the error."""
+def _with_and_without_native(run, entry, monkeypatch):
+    """What a call gives through the native host path and as the Python form, results or the error, and what the native entry point of that
+    name answered: "taken", "left" to the Python form, or "raised"; None where it was not asked."""
+    import types
     from hpfp8 import ops
     assert ops._native is not None
+    answers = [None]
+
+    def asked(*args, answer=getattr(ops._native, entry)):
+        answers.append("raised")
+        r = answer(*args)
+        answers[-1] = "left" if r is None or r is False else "taken"
+        return r
 
     def outcome():
         try:
             r = run()
             return [t.clone() if torch.is_tensor(t) else t for t in (r if isinstance(r, (list, tuple)) else [r])]
         except Exception as e:      # noqa: BLE001
-            return type(e)
-    got = outcome()
+            return type(e), str(e)
+    watched = types.SimpleNamespace(**{k: getattr(ops._native, k) for k in dir(ops._native) if not k.startswith("__")})
+    setattr(watched, entry, asked)
     with monkeypatch.context() as m:
+        m.setattr(ops, "_native", watched)
+        got = outcome()
         m.setattr(ops, "_native", None)
         want = outcome()
-    return got, want
+    return got, want, answers[-1]
 
 
 def _same(got, want):
-    if isinstance(want, type):
-        return got is want
-    return len(got) == len(want) and all(a.shape == b.shape and a.dtype == b.dtype and a.requires_grad == b.requires_grad and
-                                         torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8)) for a, b in zip(got, want))
+    if isinstance(want, tuple):
+        return got == want
+    return isinstance(got, list) and len(got) == len(want) and all(
+        a.shape == b.shape and a.dtype == b.dtype and a.requires_grad == b.requires_grad and
+        torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8)) for a, b in zip(got, want))
 
 
 @pytest.mark.parametrize("recipe", ["blockwise", "blockwise_pow2", "per_tensor"])
@@ -1096,8 +1109,14 @@ def test_a_layer_in_inference_has_the_python_forms_outcome(gpu, recipe, shape, h
     elif how == "trained input":
         x.requires_grad_(True)
     with torch.set_grad_enabled(how != "trained weight, no_grad"):
-        got, want = _with_and_without_native(lambda: hpfp8.fp8_linear(x, w, b, recipe=recipe, weight_fp8=f8), monkeypatch)
+        got, want, answer = _with_and_without_native(lambda: hpfp8.fp8_linear(x, w, b, recipe=recipe, weight_fp8=f8), "linear_infer", monkeypatch)
     assert _same(got, want)
+    if shape[-1] != k:
+        assert answer is None and want[0] is ValueError
+    elif how == "offset" and x.numel():
+        assert answer == "raised" and want[0] is hpfp8._lib.Hpfp8Error
+    else:
+        assert isinstance(want, list) and answer == ("left" if how in ("strided", "trained input") or not x.numel() else "taken")
 
 
 @pytest.mark.parametrize("shape,inter", [((1, 256), 128), ((37, 2048), 384), ((64, 2176), 128), ((65, 2048), 256), ((2, 3, 256), 256), ((0, 256), 128), ((3, 384), 128)])
@@ -1110,8 +1129,12 @@ def test_an_mlp_block_in_inference_has_the_python_forms_outcome(gpu, shape, inte
     x = torch.randn(shape, generator=g).bfloat16().to(gpu)
     gu = hpfp8.quantize_weight((torch.randn((2 * inter, k), generator=g) * 0.1).bfloat16().to(gpu), with_transpose=False, pow2=pow2[0])
     dn = hpfp8.quantize_weight((torch.randn((256, inter), generator=g) * 0.1).bfloat16().to(gpu), with_transpose=False, pow2=pow2[1])
-    got, want = _with_and_without_native(lambda: hpfp8.fp8_swiglu_mlp(x, gu, dn, fast=fast), monkeypatch)
+    got, want, answer = _with_and_without_native(lambda: hpfp8.fp8_swiglu_mlp(x, gu, dn, fast=fast), "swiglu_mlp_infer", monkeypatch)
     assert _same(got, want)
+    if shape[-1] != k:
+        assert answer == "left" and want[0] is ValueError
+    else:
+        assert isinstance(want, list) and answer == ("taken" if x.numel() else "left")
 
 
 @pytest.mark.parametrize("rows", [[3, 0, 130, 1], [0, 0, 0, 0], [64, 64, 64, 64]])
@@ -1123,8 +1146,12 @@ def test_a_grouped_layer_in_inference_has_the_python_forms_outcome(gpu, rows, of
     w = torch.randn((4, 384, 256), generator=g).bfloat16().to(gpu)
     offs = torch.tensor(rows).cumsum(0).to(offs_type).to(gpu)
     f8 = hpfp8.quantize_grouped_weight(w, with_transpose=False)
-    got, want = _with_and_without_native(lambda: hpfp8.fp8_grouped_linear(x, w, offs, weight_fp8=f8), monkeypatch)
+    got, want, answer = _with_and_without_native(lambda: hpfp8.fp8_grouped_linear(x, w, offs, weight_fp8=f8), "grouped_infer", monkeypatch)
     assert _same(got, want)
+    if offs_type is torch.int64:
+        assert answer == "left" and want[0] is TypeError
+    else:
+        assert isinstance(want, list) and answer == ("taken" if x.numel() else "left")
 
 
 @pytest.mark.parametrize("numels,shards", [([128], 1), ([1, 129, 4096], 4), ([7, 300] * 70, 2)])
@@ -1144,8 +1171,13 @@ def test_the_bucket_has_the_python_forms_outcome(gpu, numels, shards, wrong, mon
     elif wrong == "count":
         grads, outs = grads + grads[:1], outs + outs[:1]
     given = (lambda t: tuple(t)) if wrong == "a tuple" else ((lambda t: (v for v in t)) if wrong == "a generator" else (lambda t: t))
-    got, want = _with_and_without_native(lambda: bucket.pack(given(grads)), monkeypatch)
-    assert _same(got, want)
-    if not isinstance(want, type):
-        got, want = _with_and_without_native(lambda: bucket.unpack(want[0].view(torch.uint8)[0].view(torch.float8_e4m3fn), want[1][0], given(outs)), monkeypatch)
+    error = {"type": TypeError, "size": ValueError, "count": ValueError, "a generator": TypeError, "strided": TypeError if numels[-1] > 1 else None}.get(wrong)
+    packed = bucket.pack([torch.randn(n * shards, generator=g).bfloat16().to(gpu) for n in numels])
+    for call, entry in ((lambda: bucket.pack(given(grads)), "bucket_pack"),
+                        (lambda: bucket.unpack(packed[0].view(torch.uint8)[0].view(torch.float8_e4m3fn), packed[1][0], given(outs)), "bucket_unpack")):
+        got, want, answer = _with_and_without_native(call, entry, monkeypatch)
         assert _same(got, want)
+        if error is None:
+            assert isinstance(want, list) and answer == "taken"
+        else:
+            assert want[0] is error and answer == (None if wrong == "a generator" and entry == "bucket_pack" else "left")
