@@ -762,6 +762,13 @@ def test_both_products_of_a_backward_in_one_launch_have_the_bits_of_two(gpu, m, 
         try:
             _lib.call("hpfp8_linear_backward", *(ctypes.addressof(o) for o in operands), m, n, k, got[0].data_ptr(), got[1].data_ptr(), 0,
                       part.data_ptr(), got[2].data_ptr(), recipe, ops._stream())
+            if recipe != 2 and mode < 2:        # (scales that are not k-block-major: the launches one by one)
+                sg_rows, sgt_rows = sg.contiguous(), sgt.contiguous()
+                rows = [Operand(g, sg_rows), operands[1], Operand(gt, sgt_rows), operands[3]]
+                apart = [torch.full_like(t, 7.0) for t in got]
+                _lib.call("hpfp8_linear_backward", *(ctypes.addressof(o) for o in rows), m, n, k, apart[0].data_ptr(), apart[1].data_ptr(), 0,
+                          part.data_ptr(), apart[2].data_ptr(), recipe, ops._stream())
+                assert all(torch.equal(a[:len(b)], b) for a, b in zip(apart, want))
             if recipe != 2:
                 onto = [torch.full_like(got[0], 7.0), old.clone()]
                 _lib.call("hpfp8_linear_backward", *(ctypes.addressof(o) for o in operands), m, n, k, onto[0].data_ptr(), onto[1].data_ptr(), 1,
