@@ -90,7 +90,6 @@ struct GemmParams {
   int pow2_out;
   float* q_scale;
   float* q_scale_inv;
-  int stream_b;           // rows of b that one tile alone reads are not kept in the caches (streams_b)
   int choose_cus;         // grouped by rows, tile chosen on the device: the compute units there are (test hook: minus the rows asked for)
 };
 
@@ -135,7 +134,7 @@ struct TileInfo {
   int n0;              // first row of b / column of c
   int expert;
   int kb0, kbn;        // grouped along the contraction: first k-block of the tile's expert and how many (>= 1)
-  bool b_once;         // (fetching waves) no other tile reads these rows of b, and they are not kept in the caches
+  bool b_once;         // (grouped by rows, fetching waves) no other tile reads these rows of b, and they are not kept in the caches
 };
 
 // Position `d` k-blocks after k-block kb of the current tile (which has k0 k-blocks, the next one k1, every
@@ -232,6 +231,17 @@ __device__ __forceinline__ int grouped_tile_rows(const ExpertChunk& c, const Gem
   const int64_t high_cost = 83 * (int64_t)quotient(high * tiles_n + cus - 1, cus);
   return low_cost <= mid_cost && low_cost <= high_cost ? 64 : (mid_cost <= high_cost ? 128 : 256);
 }
+
+// Grouped by rows, rows of b that one tile alone reads are streamed past the caches where the experts with rows have more than the
+// Infinity Cache (256 MiB) holds, so that little of them would be there when the next call comes; fewer may still be there, and
+// streamed they never are.  us kept / streamed, with one b for every call (with two or more in turn), 16 rows each of experts [4096, 7168]:
+//    6 (168 MiB)  28.7 / 30.9  (34.4 / 30.9)     9 (252)  43.7 / 52.7  (57.2 / 52.6)    10 (280)  55.4 / 54.3  (59.0 / 54.6)
+//   16 (448)      83.2 / 72.0  (83.0 / 72.6)    24 (672)   121 / 106    (122 / 107)
+// 512 rows of 32 (896) evenly 159 / 140, by Zipf's law 175 / 157; of 8 (224) evenly 36.7 / 39.4 (44.5 / 39.9), by Zipf's law 43.2 / 56.6.
+// Over 1000 sizes from 180 to 460 MiB and from 1 to 100 rows per expert streaming takes 1.03 times as long on average (1.16 at most)
+// from 260 to 280 MiB, 0.96 (1.06) to 300, and 0.91 (never more than 1) beyond.  (Dense products do not stream: their kernels are shorter by
+// a quarter of a microsecond without it, which is 6 to 8 % of the smallest.)
+constexpr int64_t kStreamFrom = (int64_t)300 << 20;
 
 // one wave's transfer of 8 rows x 128 bytes to LDS, as data read once
 __device__ __forceinline__ void stream_1k(__amdgpu_buffer_rsrc_t rs, uint8_t* dst, uint32_t lane_off, int off) {
@@ -336,13 +346,17 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
   // numbered so that consecutive numbers cover rectangles of 32 tiles (rect_map), each XCD (workgroup ids
   // congruent mod 8, own L2) owns a contiguous run of numbers, and the workgroups of an XCD walk
   // through that run side by side, so at any moment they work on one rectangle.
+  bool stream_b = false;               // grouped by rows: rows of b that one tile alone reads go past the caches
   int total_tiles = p.tiles;
   if (GROUPED == kGroupedK) total_tiles = p.experts * p.tiles;
   if (GROUPED == kGroupedRows) {
     // tiles are numbered expert by expert; an expert with no rows has none
     const ExpertChunk first = group;
     count_tiles(group, TM, tiles_n, lane);
-    while (next_experts(group, p, TM, tiles_n, lane)) {}
+    auto with_rows = [&]() { return __builtin_popcountll(__ballot(expert_rows(group, lane) != 0)); };
+    int used = kFetchers ? with_rows() : 0;
+    while (next_experts(group, p, TM, tiles_n, lane)) used += kFetchers ? with_rows() : 0;
+    stream_b = kFetchers && (int64_t)used * N * K > kStreamFrom;
     total_tiles = __builtin_amdgcn_readlane(group.tile_end, 63);
     if (p.experts > 64) {
       group = first;
@@ -401,8 +415,7 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
           n0 = tn * TN;
         }
       } else {
-        row_tiles = (p.M + TM - 1) / TM;
-        rect_map(t, row_tiles, tiles_n, tm, tn);
+        rect_map(t, (p.M + TM - 1) / TM, tiles_n, tm, tn);
         row0 = tm * TM;
         row_end = row0 + TM < p.M ? row0 + TM : p.M;
         n0 = tn * TN;
@@ -416,7 +429,7 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
     ti.expert = __builtin_amdgcn_readfirstlane(expert);
     ti.kb0 = __builtin_amdgcn_readfirstlane(kb0);
     ti.kbn = __builtin_amdgcn_readfirstlane(kbn);
-    ti.b_once = p.stream_b && __builtin_amdgcn_readfirstlane(row_tiles) == 1;
+    ti.b_once = stream_b && __builtin_amdgcn_readfirstlane(row_tiles) == 1;
   };
   // ---- global -> LDS tile DMA.  One wave instruction moves 8 rows x 128 B (lane i -> LDS slot
   // i); the lane picks the 16-byte global chunk whose swizzled home is its slot.  The buffer
@@ -491,10 +504,9 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
   auto issue_b = [&](const __amdgpu_buffer_rsrc_t& rs, int buf, int kb, int sub) {
     transfer(rs, b_off[sub], b_lds + buf * kBTile + wave * (NB * 1024), kb, sub);
   };
-  // Rows of b that one tile alone reads are streamed where b does not fit the Infinity Cache (streams_b has the figures): they stay in
-  // no cache, which leaves those to a's rows.  Where several tiles share them it would cost: 8192 rows of 32 experts [4096, 7168]
-  // 299 / 310 us.
-  auto stream_b = [&](const __amdgpu_buffer_rsrc_t& rs, int buf, int kb, int sub) {
+  // Rows of b that one tile alone reads are streamed (b_once): they stay in no cache, which leaves those to a's rows.  Where several tiles
+  // share them it would cost: 8192 rows of 32 experts [4096, 7168] 299 / 310 us.
+  auto issue_stream_b = [&](const __amdgpu_buffer_rsrc_t& rs, int buf, int kb, int sub) {
     stream_1k(rs, b_lds + buf * kBTile + wave * (NB * 1024) + sub * 1024, b_off[sub], kb * BK);
   };
 
@@ -588,7 +600,7 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
       auto fetch_rest = [&]() {
         if (b_once) {
 #pragma unroll
-          for (int sub = 0; sub < NB; ++sub) stream_b(rb, buf, f_kb, sub);
+          for (int sub = 0; sub < NB; ++sub) issue_stream_b(rb, buf, f_kb, sub);
         } else {
 #pragma unroll
           for (int sub = 0; sub < NB; ++sub) issue_b(rb, buf, f_kb, sub);
@@ -1444,21 +1456,6 @@ static bool try_skinny(const GemmParams& p, SkinnyMode mode, int out_type, hipSt
   return true;
 }
 
-// Whether rows of b that only one tile reads are streamed past the caches: where those of all experts that can have rows are more than the
-// Infinity Cache holds, so that none of them would be there when the next call comes.  A smaller b may still be there, and streamed it
-// never is.  us kept / streamed, with one b for every call (and with two or more in turn):
-//   65 rows of    [18432, 7168] (126 MiB)  26.6 / 32.8  (35.7 / 33.8)     [32768, 8192] (256)  43.2 / 56.6  (62.1 / 56.7)
-//                 [40960, 7168] (280)      58.2 / 56.8  (61.6 / 57.3)     [49152, 8192] (384)  77.1 / 70.7  (85.6 / 79.3)
-//   128 rows of   [18432, 7168]            27.3 / 39.3  (42.5 / 40.8)     [65536, 8192] (512)   128 / 120   (128 / 120)
-//   16 rows each of 6 experts [4096, 7168] (168)  28.7 / 30.9  (34.4 / 30.9)     9 (252)  43.7 / 52.7  (57.2 / 52.6)
-//                            10 (280)             55.4 / 54.3  (59.0 / 54.6)    16 (448)  83.2 / 72.0  (83.0 / 72.6)
-//                            24 (672)              121 / 106    (122 / 107)
-//   512 rows of 32 experts (896), evenly 159 / 140, by Zipf's law 175 / 157; of 8 (224) evenly 36.7 / 39.4 (44.5 / 39.9), by Zipf's law 43.2 / 56.6
-static int streams_b(int64_t M, int64_t N, int64_t K, int64_t experts) {
-  constexpr int64_t kInfinityCache = (int64_t)256 << 20;
-  return (experts < M ? experts : M) * N * K > kInfinityCache;
-}
-
 template <int MODE, int GROUPED, bool SA4, int WM, int NS, int WN>
 static int launch_sa(const GemmParams& p, int out_type, int64_t tiles, hipStream_t stream) {
   dim3 grid((unsigned)persistent_grid(tiles)), block(tile_threads(WM, WN));
@@ -1489,7 +1486,6 @@ template <int MODE, int GROUPED>
 static int launch(GemmParams p, int out_type, TileShape shape, hipStream_t stream) {
   int64_t tiles = tile_count(p.M, p.N, shape);
   p.tiles = (int)tiles;                        // (grouped by rows: the kernel counts the experts' own tiles)
-  p.stream_b = streams_b(p.M, p.N, p.K, GROUPED == kGroupedRows ? p.experts : 1);
   if (GROUPED == kGroupedK) tiles *= p.experts;
   // upper bound on row tiles: every expert may add one partial tile
   if (GROUPED == kGroupedRows) tiles = most_grouped_tiles(p.M, p.N, p.experts, shape);
@@ -1510,7 +1506,6 @@ static int launch_grouped(GemmParams p, int out_type, hipStream_t stream) {
   if (tiles == kSmallestTiles) return launch<MODE, kGroupedRows>(p, out_type, k64x64, stream);
   if (tiles == kLowestTiles) return launch<MODE, kGroupedRows>(p, out_type, k64x128, stream);
   if (tiles == kHighTiles) return launch<MODE, kGroupedRows>(p, out_type, k256x256, stream);
-  p.stream_b = streams_b(p.M, p.N, p.K, p.experts);
   p.choose_cus = tiles == kLowTiles ? -128 : persistent_grid((int64_t)1 << 40);
   dim3 grid((unsigned)persistent_grid(most_grouped_tiles(p.M, p.N, p.experts, k64x128))), block(512);
   const bool sa4 = p.sa_sm == 1;
@@ -1687,7 +1682,6 @@ int hpfp8_gemm_blockwise_swiglu_quantize(const void* a, int64_t lda, const float
   const TileShape shape = pick_shape_swiglu(M, 2 * inter);
   const int64_t tiles = tile_count(M, 2 * inter, shape);
   p.tiles = (int)tiles;
-  p.stream_b = streams_b(p.M, p.N, p.K, 1);
   dim3 grid((unsigned)persistent_grid(tiles)), block(512);
   static_assert(tile_threads(4, 2) == 512 && tile_threads(2, 2) == 512 && tile_threads(1, 4) == 512, "");
   hipStream_t st = (hipStream_t)stream;
@@ -1781,7 +1775,6 @@ int hpfp8_linear_backward(const hpfp8_operand* go, const hpfp8_operand* wt, cons
     const int longer = tile_time(shape[1], kblocks[1]) + (accumulate ? accumulate_time(shape[1]) : 0) > tile_time(shape[0], kblocks[0]) ? 1 : 0;
     for (int i = 0; i < 2; ++i) {
       q.gemm[i].tiles = (int)tiles[i];
-      q.gemm[i].stream_b = streams_b(q.gemm[i].M, q.gemm[i].N, q.gemm[i].K, 1);
       q.shape[i] = shape[i];
       q.wgs[i] = (int)(tiles[i] < kXcds ? tiles[i] : (tiles[i] + kXcds - 1) / kXcds * kXcds);
     }

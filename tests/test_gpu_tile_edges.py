@@ -839,22 +839,16 @@ def test_a_weight_that_stays_in_the_caches_is_read_from_them(gpu, grouped):
     assert fastest(weights[:1]) < 0.85 * fastest(weights)
 
 
-def test_products_whose_weight_is_streamed_past_the_caches_have_the_bits_of_those_that_keep_it(gpu):
-    """Weights larger than the Infinity Cache with rows that one low tile reads alone: dense, with the SwiGLU epilogue and grouped by rows
-    (experts with none, one tile's and several tiles' rows); 256 x 256 tiles stream nothing."""
+def test_grouped_products_whose_weight_is_streamed_past_the_caches_have_the_bits_of_those_that_keep_it(gpu):
+    """Experts with rows on both sides of the size from which on rows of b that one low tile reads alone are streamed, among 12 and among
+    70 (two chunks of 64 lanes), with none, one tile's and several tiles' rows; 256 x 256 tiles stream nothing."""
     from hpfp8 import ops
-    k, n, experts = 7168, 10 * 4096, 10
-    b, sb = ops.quantize_128x128(_normal((n, k), 2, gpu, 0.02))
-    for m in (65, 128, 129):
-        a, sa = ops.quantize_1x128(_normal((m, k), 1, gpu), kmajor=True)
-        got, want = _both_tiles(lambda: ops.gemm_blockwise(a, sa, b, sb))
-        assert torch.equal(got, want)
-        (gq, gs), (wq, ws) = _both_tiles(lambda: ops.gemm_blockwise_swiglu_quantize(a, sa, b, sb, fast=True)[:2])
-        assert torch.equal(gq.view(torch.uint8), wq.view(torch.uint8)) and torch.equal(gs, ws)
-    for sizes in ([1, 0, 64, 65, 128, 129, 7, 300, 16, 2], [10] * 10):
-        a, sa = ops.quantize_1x128(_normal((sum(sizes), k), 1, gpu), kmajor=True)
-        offs = torch.tensor(sizes, device=gpu).cumsum(0).int()
-        got, want = _both_tiles(lambda: ops.gemm_grouped_blockwise(a, sa, b.view(experts, 4096, k), sb.view(experts, 32, k // 128), offs))
+    for experts, n, k, counts in ((12, 4096, 7168, [1, 0, 64, 65, 128, 129, 7, 300, 16, 2, 1, 1]), (12, 4096, 7168, [10] * 12), (12, 4096, 7168, [10] * 10 + [0] * 2),
+                                  (70, 2048, 2560, [3] * 30 + [0] * 10 + [70] + [1] * 29)):
+        b, sb = ops.quantize_128x128(_normal((experts * n, k), 2, gpu, 0.02))
+        a, sa = ops.quantize_1x128(_normal((sum(counts), k), 1, gpu), kmajor=True)
+        offs = torch.tensor(counts, device=gpu).cumsum(0).int()
+        got, want = _both_tiles(lambda: ops.gemm_grouped_blockwise(a, sa, b.view(experts, n, k), sb.view(experts, n // 128, k // 128), offs))
         assert torch.equal(got, want)
 
 
