@@ -1360,8 +1360,8 @@ static GroupedTiles pick_grouped(int64_t M, int64_t N, int experts) {
   return M > (int64_t)256 * experts && M / 256 * ((N + 255) / 256) >= 2 * cus ? kHighTiles : kChosenTiles;
 }
 
-static int64_t few_rows(int64_t K) {        // the most rows that count as few
-  return K >= kSkinnyMinK && g_small_gemm_mode.load(std::memory_order_relaxed) == 0 ? kSkinnyMaxRows : 0;
+static int64_t few_rows(int64_t N, int64_t K) {        // the most rows that count as few
+  return K >= kSkinnyMinK && g_small_gemm_mode.load(std::memory_order_relaxed) == 0 ? skinny_rows(N, K) : 0;
 }
 
 // Both products of a linear's backward in one launch (gemm_backward_kernel) where that is shorter by more than a thirty-second: the time
@@ -1410,7 +1410,7 @@ static bool pick_backward(int64_t M, int64_t N, int64_t K, int64_t padded, int l
     shape[0] = shape[1] = mode == 1 ? k256x256 : (mode == 3 ? k128x256 : (mode == 4 ? k128x128 : k64x128));
     return true;
   }
-  if (M <= few_rows(N)) return false;
+  if (M <= few_rows(K, N)) return false;
   const int64_t cus = persistent_grid((int64_t)1 << 40);
   const int64_t kb[2] = {N / BK, padded / BK}, rows[2] = {M, N};
   int64_t apart = (launches - 1) * kLaunchTime;
@@ -1445,9 +1445,10 @@ static bool pick_backward(int64_t M, int64_t N, int64_t K, int64_t padded, int l
 // behind it: what those save on the GPU (weight [8192, 1024], 8 rows 11.6 -> 9.0 us; [36864, 512], 64 rows 9.9 -> 13.5) the second
 // call costs on the host (15 -> 25 us).
 constexpr int64_t kEpilogueMaxK = 2048;
+static_assert(kEpilogueMaxK >= kSkinnyAnyWidthK, "hpfp8_gemm_few_rows knows no width");
 
 static bool try_skinny(const GemmParams& p, SkinnyMode mode, int out_type, hipStream_t stream, int& rc) {
-  if (p.accumulate || p.M > few_rows(p.K)) return false;
+  if (p.accumulate || p.M > few_rows(p.N, p.K)) return false;
   SkinnyParams q{};
   q.a = p.a; q.b = p.b; q.sa = p.sa; q.sb = p.sb; q.lda = p.lda; q.ldb = p.ldb;
   q.sa_sm = p.sa_sm; q.sa_sk = p.sa_sk; q.sb_sn = p.sb_sn; q.sb_sk = p.sb_sk; q.sb_bytes = p.sb_bytes;
@@ -1705,14 +1706,14 @@ int hpfp8_gemm_blockwise_swiglu_quantize(const void* a, int64_t lda, const float
 
 void hpfp8_debug_set_small_gemm(int mode) { g_small_gemm_mode.store(mode >= 1 && mode <= 5 ? mode : 0, std::memory_order_relaxed); }
 
-int64_t hpfp8_gemm_few_rows(int64_t K) { return K >= kEpilogueMaxK ? few_rows(K) : 0; }
+int64_t hpfp8_gemm_few_rows(int64_t K) { return K >= kEpilogueMaxK ? few_rows(kBlock, K) : 0; }
 
 // Up to 8 rows are quantized inside the product (gemm_skinny.hip has the figures).  With few runs of columns and a long contraction
 // every compute unit's chain of k-blocks is longer than in two launches and what those cost more is less: us, 8 rows, two / one
 // [1024, 10240] 11.0 / 10.1, [1024, 12288] 11.6 / 11.4 (1 row 10.4 / 10.9), [2048, 16384] 13.6 / 14.2, [4096, 16384] 16.2 / 14.4.
 int64_t hpfp8_linear_few_rows(int64_t N, int64_t K) {
   if (K > 10240 && 4 * (N / 16) <= 3 * (int64_t)persistent_grid((int64_t)1 << 40)) return 0;
-  return few_rows(K) > kSkinnyMaxRowsBf16 ? kSkinnyMaxRowsBf16 : few_rows(K);
+  return few_rows(kBlock, K) > kSkinnyMaxRowsBf16 ? kSkinnyMaxRowsBf16 : few_rows(kBlock, K);
 }
 
 int hpfp8_linear_few_rows_bf16(const void* x, const void* b, int64_t ldb, const float* sb, int64_t sb_stride_n, int64_t sb_stride_k,

@@ -321,7 +321,12 @@ __global__ __launch_bounds__(skinny_threads(F, QUANT)) void gemm_skinny_kernel(c
 // vector-memory path (1.4 : 1 per KB), and 1.4 times that where a stage is fewer than four k-blocks; taken is the form whose
 // runs cost least, the narrowest of equals.  Over 10 widths from 4096 to 36864, 4 contractions from 4096 to 16384 and 5 row
 // counts this is 0.7 % slower on average than the best of the six forms of each, 14 % at most (24 rows of [18432, 7168]).
-static int skinny_fragments(int64_t N, int me, int cus, bool quant = false) {
+// With a short contraction, and with rows quantized here, a run also costs about what three k-blocks of the narrowest form do, and a
+// contraction that does not fill its last stage the whole of it.  Contractions from 512 to 1920, 1 to 64 rows and 1024 to 131072
+// columns, 12610 sizes: 1.7 % slower than the best form of each on average, without these two terms 3.5 % and up to 78 % ([27008, 896],
+// 8 rows: seven runs of one fragment 10.0 us, two of four 6.1); from 2048 on they gain 0.5 % on average and cost some sizes 5 %.
+static int skinny_fragments(int64_t N, int64_t K, int me, int cus, bool quant = false) {
+  const bool per_run = quant || K < kSkinnyAnyWidthK;
   const int forms[] = {1, 2, 3, 4, 6, 9};
   int best = 0;
   int64_t best_cost = 0;
@@ -329,7 +334,8 @@ static int skinny_fragments(int64_t N, int me, int cus, bool quant = false) {
     if (quant && f > 3) break;
     const int64_t units = (N / 16 + f - 1) / f, runs = (units + cus - 1) / cus;
     const int64_t run = 14 * 2 * f > 10 * (2 * f + me) ? 14 * 2 * f : 10 * (2 * f + me);
-    const int64_t cost = runs * run * (skinny_kstep(me, f, quant) >= 4 ? 10 : 14);
+    const int64_t step = skinny_kstep(me, f, quant), kblocks = per_run ? (K / BK + step - 1) / step * step : K / BK;
+    const int64_t cost = runs * (kblocks * run * (step >= 4 ? 10 : 14) + (per_run ? 1000 : 0));
     if (!best || cost < best_cost) {
       best = f;
       best_cost = cost;
@@ -346,7 +352,7 @@ static void launch_skinny_form(const SkinnyParams& p, int cus, hipStream_t strea
 
 template <int MODE, int ME>
 static void launch_skinny_cols(const SkinnyParams& p, int cus, hipStream_t stream) {
-  switch (skinny_fragments(p.N, ME, cus)) {
+  switch (skinny_fragments(p.N, p.K, ME, cus)) {
     case 1: launch_skinny_form<MODE, ME, 1>(p, cus, stream); break;
     case 2: launch_skinny_form<MODE, ME, 2>(p, cus, stream); break;
     case 3: launch_skinny_form<MODE, ME, 3>(p, cus, stream); break;
@@ -380,7 +386,7 @@ int launch_skinny(const SkinnyParams& p, SkinnyMode mode, int cus, hipStream_t s
 
 template <int MODE>
 static void launch_skinny_bf16(const SkinnyParams& p, int cus, hipStream_t stream) {
-  switch (skinny_fragments(p.N, 2, cus, true)) {
+  switch (skinny_fragments(p.N, p.K, 2, cus, true)) {
     case 1: launch_skinny_form<MODE, 2, 1, true>(p, cus, stream); break;
     case 2: launch_skinny_form<MODE, 2, 2, true>(p, cus, stream); break;
     default: launch_skinny_form<MODE, 2, 3, true>(p, cus, stream); break;

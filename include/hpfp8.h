@@ -388,7 +388,7 @@ int hpfp8_gemm_per_tensor(const void* a, int64_t lda, const float* sa_inv, const
 /* Forms of the GEMMs.  They take the smallest output tile with which a problem is still one tile per compute unit (64 x 64, 64 x 128,
  * 128 x 128, 128 x 256), and otherwise 256 x 256 or, where those would leave most of a second round idle, 128 x 256; the forms grouped by rows take 64 x 64, 64 x 128, 128 x 256 or 256 x 256 ones, which
  * the kernel chooses where the host cannot know.  With at most 64 rows and K >= 512
- * hpfp8_gemm_per_tensor and hpfp8_gemm_blockwise[_pow2] with sb_gran = 128 (no accumulate) take a form that reads b once at
+ * (K < 2048: at most 32 from 24577 columns on, 16 from 98305 on) hpfp8_gemm_per_tensor and hpfp8_gemm_blockwise[_pow2] with sb_gran = 128 (no accumulate) take a form that reads b once at
  * the memory's rate.  Same arithmetic in the same order in all of them: an element of c has the same bits in each, so it
  * depends neither on the number of rows nor on where b's rows stand (a column shard).  Test hook, not part of the path: mode
  * 0 = that rule (default), 1 = always 256 x 256 tiles, 2 = the smallest tile a form has, 3 = 128 x 256, 4 = 128 x 128 and 5 = 64 x
