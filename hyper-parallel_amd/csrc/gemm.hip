@@ -4,7 +4,7 @@
 //   * Both operands are K-contiguous E4M3 codes, so a 16-row x 128-byte slab of either is exactly
 //     one operand of v_mfma_f32_16x16x128_f8f6f4: one matrix instruction consumes one whole
 //     128-wide scaling block, and its fp32 result is promoted into the running accumulator with
-//     one FMA per element (acc += partial * sa * sb).
+//     one FMA per element (acc += partial * (sa * sb)).
 //   * The weight-like operand b feeds the MFMA "A" port and the activation-like operand a the
 //     "B" port: a lane then holds 4 consecutive n for one m, which makes the per-row scale
 //     sa(m,kb) a per-lane constant.
@@ -210,8 +210,9 @@ __device__ __forceinline__ bool next_experts(ExpertChunk& c, const GemmParams& p
 
 // Grouped by rows: the rows of the best tile for the rows that the experts have, 64 (x 128 columns), 128 or 256 (x 256).  What
 // counts is the rounds of one tile per compute unit; rounds cost 26 : 50 : 83 (measured, us with 64 / 128 / 256 rows: 8192
-// rows of one expert [4096, 7168], 16 / 4 / 2 rounds 338 / 213 / 183, bound by arithmetic; 2048 rows over 32 of them evenly, 4 / 2 / 2
-// rounds 165 / 168 / 224, bound by reading b; 64 rows of one, one round each 21 / 41 / 66).  c: the first 64 experts.
+// rows of one expert [4096, 7168], 16 / 4 / 2 rounds 313 / 201 / 178, bound by arithmetic; 2048 rows over 32 of them evenly, 4 / 2 / 2
+// rounds 151 / 144 / 197, bound by reading b; 512 rows of one, one round each 23 / 42 / 64).  What this chooses was the fastest of the
+// three or within 3 % of it in every line of the table at pick_grouped.  c: the first 64 experts.
 __device__ __forceinline__ int grouped_tile_rows(const ExpertChunk& c, const GemmParams& p, int lane) {
   int low = 0, mid = 0, high = 0;
   for (ExpertChunk e = c;;) {
@@ -438,8 +439,9 @@ __device__ __forceinline__ void gemm_tiles(const GemmParams& p, uint8_t* const l
   // (The resource runs on to the end of the tensor rather than to the end of the tile: dense, transfers
   // through a resource that only just covers the rows they touch were measured markedly slower.  Grouped by rows, where most of a
   // tile may be rows of other experts that are not stored, it ends with the tile's own: us with resources that end with the tensor /
-  // with the tile 64 rows of 8 experts [4096, 7168] 39.1 / 36.3, 1024 of 32 [2048, 7168] 107 / 98, 8192 of 32 [4096, 7168] 313 / 299, 131072
-  // 3239 / 3212.)
+  // with the tile, 32 experts [4096, 7168] 512 rows evenly 148 / 141, by Zipf's law 193 / 176, 2048 rows 151 / 145 and 195 / 186, 8192
+  // 258 / 258 and 309 / 301; tiles that are full take the same in both, with the tensor's end for those alone too: 16384 rows of 64 experts
+  // [2048, 2048] evenly 82 / 82, 131072 of 8 3032 / 3033.)
   auto span_bytes = [&](int64_t rows, int64_t ld) {     // up to the end of the last row's K codes
     const int64_t bytes = rows > 0 ? (rows - 1) * ld + K : 0;
     return (int)(bytes < (int64_t)0x7FFFF000 ? bytes : (int64_t)0x7FFFF000);   // 256 rows always fit (host check)
@@ -1342,13 +1344,16 @@ static TileShape pick_shape_swiglu(int64_t M, int64_t N) {
 // tiles are better, with many (or the rows of many with one expert) high ones; the rows of an expert are known on the device
 // only.  Where even the most 64 x 64 or 64 x 128 tiles there can be are one round: those.  Of more than 256 rows per expert on average and
 // two rounds of 256 x 256 tiles or more: those.  In between the kernel chooses (grouped_tile_rows).  us with 64 / 128 / 256 rows per
-// tile, for rows spread evenly / by Zipf's law / half with one expert / all with one:
-//   32 experts [4096, 7168],   512 rows   140 / 139 / 196   155 / 140 / 193   159 / 179 / 197    24 /  44 /  65
-//                             2048 rows   159 / 151 / 211   199 / 179 / 249   190 / 179 / 261    85 /  58 /  77
-//                             8192 rows   445 / 257 / 234   455 / 298 / 356   509 / 343 / 305   337 / 214 / 183
-//   8 experts  [4096, 7168],   512 rows    41 /  57 /  81    54 /  56 /  81    59 /  54 /  84    24 /  43 /  65
-//   16 experts [1024, 4096],  2048 rows    23 /  33 /  48    31 /  32 /  47    32 /  31 /  48    16 /  27 /  40
-//   64 experts [2048, 2048], 16384 rows   156 /  87 /  79   155 /  96 / 122   167 / 115 / 106   115 /  70 /  63
+// tile, for rows spread evenly / by Zipf's law / half with one expert / all with one; one weight for every call, so that those of 8 and 16
+// experts stay in the Infinity Cache (second lines: several in turn, so that none does):
+//   32 experts [4096, 7168],   512 rows   141 / 140 / 189   158 / 177 / 180   156 / 174 / 245    23 /  42 /  64
+//                             2048 rows   151 / 144 / 197   226 / 185 / 251   199 / 182 / 252    77 /  53 /  71
+//                             8192 rows   441 / 249 / 226   484 / 296 / 301   496 / 346 / 295   314 / 201 / 179
+//   8 experts  [4096, 7168],   512 rows    37 /  43 /  66    54 /  43 /  66    54 /  44 /  66    23 /  42 /  64
+//                                          45 /  59 /  80    66 /  60 /  81    64 /  57 /  80    23 /  42 /  64
+//   16 experts [1024, 4096],  2048 rows    16 /  26 /  40    29 /  27 /  40    27 /  27 /  40    15 /  26 /  40
+//                                          22 /  33 /  47    35 /  33 /  47    32 /  32 /  47    16 /  27 /  40
+//   64 experts [2048, 2048], 16384 rows   148 /  75 /  69   150 /  93 / 112   157 / 103 /  98   105 /  65 /  58
 enum GroupedTiles { kSmallestTiles, kLowestTiles, kHighTiles, kChosenTiles, kLowTiles /* test hook: as chosen */ };
 
 static GroupedTiles pick_grouped(int64_t M, int64_t N, int experts) {
@@ -1376,6 +1381,9 @@ static int64_t few_rows(int64_t N, int64_t K) {        // the most rows that cou
 // old values, all tiles of a round at once where they are a launch of their own (two launches / one): block 4096 x 7168 x 7168 448 / 400,
 // 2048 x 7168 x 4096 149 / 131, 1006 x 9472 x 3456 135 / 100, pow2 2048 x 7168 x 4096 137 / 124; without that time in the model pow2 2048 x
 // 7168 x 4096 stayed with two launches, and block 300 x 1024 x 16384 took 49.9 in one where two take 42.6.
+// Drawn over 1 to 8192 tokens and 128 to 16384 features, all recipes: where this chooses one launch (21272 sizes) it takes 0.69 of the two
+// or three launches' time on average and in 1.1 % of them over 3 % more, most often for some hundred tokens, many outputs and few inputs
+// (tensor 73 x 10752 x 1024 30.6 / 35.8), whose first product alone would take 64 x 64 tiles.
 static int64_t tile_time(TileShape shape, int64_t kblocks) {
   switch (shape) {
     case k256x256: return 5000 + 1300 * kblocks;
@@ -1437,16 +1445,15 @@ static bool pick_backward(int64_t M, int64_t N, int64_t K, int64_t padded, int l
   return best_end < apart - apart / 32;
 }
 
-// Few rows of a (decode): bound by reading b once, which the tile kernels do not reach (gemm_skinny.hip; 8 rows of
-// [7168, 16384]: 60 us with 64 x 128 tiles, 20.6 us; 64 rows: 64 and 26.8 us; 37 rows of [36864, 7168]: 81 us with 256 x 256
-// tiles, 41.6 us), with the same bits.  try_skinny hands the problem over if it is one; otherwise false.
-
 // Below this contraction a fused epilogue on tiles is still the better choice with few rows than the few-rows form and a launch
 // behind it: what those save on the GPU (weight [8192, 1024], 8 rows 11.6 -> 9.0 us; [36864, 512], 64 rows 9.9 -> 13.5) the second
 // call costs on the host (15 -> 25 us).
 constexpr int64_t kEpilogueMaxK = 2048;
 static_assert(kEpilogueMaxK >= kSkinnyAnyWidthK, "hpfp8_gemm_few_rows knows no width");
 
+// Few rows of a (decode): bound by reading b once, which the tile kernels do not reach (gemm_skinny.hip; 8 rows of
+// [7168, 16384]: 60 us with 64 x 128 tiles, 20.6 us; 64 rows: 64 and 26.8 us; 37 rows of [36864, 7168]: 81 us with 256 x 256
+// tiles, 41.6 us), with the same bits.  try_skinny hands the problem over if it is one; otherwise false.
 static bool try_skinny(const GemmParams& p, SkinnyMode mode, int out_type, hipStream_t stream, int& rc) {
   if (p.accumulate || p.M > few_rows(p.N, p.K)) return false;
   SkinnyParams q{};
@@ -1584,7 +1591,8 @@ static int blockwise_params(const void* a, int64_t lda, const float* sa, int64_t
   p.c = c; p.ldc = ldc; p.bias = (const uint16_t*)bias;
   p.M = (int)M; p.N = (int)N; p.K = (int)K; p.accumulate = accumulate;
   if (sb_gran == 128) return 1;
-  // per-row b scales travel to LDS as one contiguous 1 KB piece per k-block
+  // per-row b scales are read with unit stride: 1 KB per k-block to LDS (powers of two, 256 x 256 tiles), 256 bytes per fetching wave, or
+  // into registers
   if (K == BK) sb_stride_k = N;     // a single k-block: the stride between k-blocks is never used
   p.sb_sk = sb_stride_k;
   HPFP8_REQUIRE(sb_stride_n == 1 && sb_stride_k >= N && sb_stride_k % 4 == 0 && aligned16(sb), HPFP8_ERR_SHAPE,

@@ -396,9 +396,9 @@ int hpfp8_gemm_per_tensor(const void* a, int64_t lda, const float* sa_inv, const
  * launch). */
 void hpfp8_debug_set_small_gemm(int mode);
 
-/* The largest number of rows of a with which the few-rows form that hpfp8_gemm_blockwise[_pow2] (sb_gran = 128, no accumulate) and
- * hpfp8_gemm_per_tensor have for decode steps is worth more than a fused call at contraction K (0: none): a caller that can choose
- * between a fused call and one of these followed by another launch asks here. */
+/* Whether splitting a fused call pays at contraction K: the largest number of rows of a with which hpfp8_gemm_blockwise[_pow2] (sb_gran =
+ * 128, no accumulate) in its few-rows form, followed by another launch, is the better choice (0: none; below K = 2048 it is none
+ * although that form is taken there). */
 int64_t hpfp8_gemm_few_rows(int64_t K);
 
 /* quantize_1x128 (power-of-two scales with pow2) of x and hpfp8_gemm_blockwise[_pow2] (sb_gran = 128, no accumulate) in one launch, with
