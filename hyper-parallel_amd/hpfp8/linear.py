@@ -14,8 +14,8 @@ Recipes
   "per_tensor" : one scale per tensor (amax -> 448/amax); backward also per tensor.
   "blockwise_pow2" : the blockwise groups with every scale_inv rounded up to a power of two (E8M0
                  scales, as DeepSeek-V3.1 trains with).  gfx950's matrix instruction applies such
-                 scales itself, so the three GEMMs do no scaling arithmetic and run 10 % (forward,
-                 dgrad) to 23 % (wgrad) faster; the price is up to one binade of headroom per group.
+                 scales itself, so the three GEMMs do no scaling arithmetic and run 11 % (forward,
+                 dgrad) to 19 % (wgrad) faster; the price is up to one binade of headroom per group.
                  An extension: the benchmarked recipe is "blockwise" with plain fp32 scales.
 """
 from __future__ import annotations
